@@ -1,0 +1,43 @@
+// pm_affine.h -- element products of parallelepiped elements (pm_affine.hip).
+#pragma once
+#include "pm_elemargs.h"
+
+// Device data of a mesh whose elements are all parallelepipeds (constant
+// Jacobian).  Elements are kept in `ord`, sorted by their lowest equation so
+// that the gathers of neighbouring elements lie close in the vectors.
+struct PmAffine {
+  int numel = 0, nen = 0, nrn = 0;
+  int *ord = nullptr;            // (numel) element of each slot
+  unsigned int *en = nullptr;    // (numel, nen) first free equation << 4 | free dofs of the node
+  unsigned int *gptr = nullptr;  // (nrn + 1) incidences of each row block
+  unsigned int *gsrc = nullptr;  // their offsets in ye
+  unsigned char *gmask = nullptr;  // (nrn) free dofs of the block's node
+  double *ec_op = nullptr;       // (numel, 16) coefficients of the assembled matrix
+  double *ec = nullptr;          // (numel, 16) coefficients of one element loop
+  double *ye = nullptr;          // element vectors
+  int *slot = nullptr;           // (numel) slot of each element
+  double *tab = nullptr;         // reference integrals of the matrix
+  int max_cols = 0;              // widest row block
+  bool op_valid = false;         // ec_op holds the matrix's coefficients
+};
+
+void pm_affine_free(PmAffine *a);
+// builds the data if every element is a parallelepiped (c->affine stays null
+// otherwise, and where memory for it is short)
+int pm_affine_setup(pm_ctx *c, const double *x, const PmHostPattern &pat);
+// element loop isw 2 or 4 of pform_pm: E.b -= p of every element, face loads
+// included; with lhs the matrix, whose coefficients are kept for products
+bool pm_affine_loops(const pm_ctx *c, int isw, int lhs);
+int pm_affine_pform(pm_ctx *c, const ElemArgs &E, int isw, int lhs, int rhs);
+
+// Krylov products through the elements: true when the matrix in c->A is the
+// one whose coefficients are kept
+bool pm_affine_product(const pm_ctx *c);
+
+// the element part of y = A x: element vectors into ye
+void pm_affine_elements(pm_ctx *c, const double *x, const PmScalars *S);
+
+// y = sum of the element vectors (rows times m with scale_m), with the dots
+// y.w and y.y of nv = 0, 1, 2 as workgroup partials; returns the grid
+int pm_affine_gather(pm_ctx *c, double *y, const double *w, const double *m, int nv, bool scale_m,
+                     const PmScalars *S);

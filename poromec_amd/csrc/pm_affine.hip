@@ -1,0 +1,923 @@
+// pm_affine.hip -- element loops and matrix products over parallelepiped
+// elements, without forming element matrices.
+//
+// On an element with a constant Jacobian the integrals of elmt17_pm
+// (Elmlib03.f:2022-2526) and of the Q1/Q1 element separate in the products
+// of Legendre polynomials P_a(r) P_b(s) P_c(t): the 20 serendipity functions
+// span the products with at most one degree 2 and the others <= 1, the 8
+// trilinear ones those with degrees <= 1.  In that basis
+//   * nodal values become coefficients by sums and differences of the
+//     vertices and of the mid-edges (pm_modal_fwd; the transpose
+//     pm_modal_back takes coefficient forces to nodal forces),
+//   * a derivative moves a coefficient one degree down (P1' = P0, P2' = 3 P1),
+//   * the 4^3 (2^3) Gauss rule is exact for every product that occurs, so the
+//     17 derivative modes are orthogonal and D acts on each mode alone.
+// An element's K_e u_e is then ~600 FP64 operations per dof component instead
+// of the 64-point loops' ~2 million per element, and needs its 15
+// coefficients (128 B) instead of the matrix's 37 KB of stored values.
+//
+// Four lanes take an element: lanes 0-2 one displacement component each, lane
+// 3 the pressure; the stress of a mode exchanges gradients inside the quad by
+// DPP.  Element vectors go to ye (one write) and a second kernel sums every
+// node's entries in a fixed order (one read): no atomics, no colours.
+#include <algorithm>
+#include <cmath>
+#include <cstring>
+
+#include "pm_affine.h"
+#include "pm_elemlib.h"
+
+#define PM_EC 16  // doubles of element coefficients
+// 0-8 g[i][x] = d r_i / d x, then det J times: 9 a (1 - b), 10 a b, 11 a c,
+// 12 alpha, 13 1/M, 14 dt perm (+ the Q1/Q1 stabilization), 15 one
+
+template <int CTRL>
+__device__ __forceinline__ double pm_quad(double v) {
+  const long long b = __builtin_bit_cast(long long, v);
+  const int lo = __builtin_amdgcn_mov_dpp((int)(b & 0xffffffffll), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xf, 0xf, true);
+  return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned int)lo);
+}
+#define PM_QP(a, b, c, d) ((a) | ((b) << 2) | ((c) << 4) | ((d) << 6))
+
+__host__ __device__ constexpr int pm_md(int a, int b, int c) { return a * 9 + b * 3 + c; }
+// modes of the element's displacement basis
+template <int NEN>
+__host__ __device__ constexpr bool pm_is_mode(int a, int b, int c) {
+  const int twos = (a == 2) + (b == 2) + (c == 2);
+  return a <= 2 && b <= 2 && c <= 2 && twos <= (NEN == 20 ? 1 : 0);
+}
+
+// sums and differences of the 8 vertex values (not scaled): h[a*4+b*2+c]
+__host__ __device__ __forceinline__ void pm_hadamard8(const double *v, double *h) {
+#pragma unroll
+  for (int c = 0; c < 2; c++) {
+    double q[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) q[k] = c == 0 ? v[k] + v[k + 4] : v[k] - v[k + 4];
+    // vertices of a face: 0 (+,+), 1 (-,+), 2 (-,-), 3 (+,-)
+    const double p1 = q[0] + q[1], m1 = q[0] - q[1], p2 = q[3] + q[2], m2 = q[3] - q[2];
+    h[0 + c] = p1 + p2;
+    h[2 + c] = p1 - p2;
+    h[4 + c] = m1 + m2;
+    h[6 + c] = m1 - m2;
+  }
+}
+// the transpose: h[a*4+b*2+c] to the 8 vertices
+__device__ __forceinline__ void pm_hadamard8t(const double *h, double *v) {
+  double q[2][4];
+#pragma unroll
+  for (int c = 0; c < 2; c++) {
+    const double p1 = h[0 + c] + h[2 + c], p2 = h[0 + c] - h[2 + c];
+    const double m1 = h[4 + c] + h[6 + c], m2 = h[4 + c] - h[6 + c];
+    q[c][0] = p1 + m1;
+    q[c][1] = p1 - m1;
+    q[c][3] = p2 + m2;
+    q[c][2] = p2 - m2;
+  }
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    v[k] = q[0][k] + q[1][k];
+    v[k + 4] = q[0][k] - q[1][k];
+  }
+}
+// the 4 mid-edges of one direction, given in the order (+,+), (-,+), (-,-),
+// (+,-) of the two other directions' signs: e[b*2+c]
+__host__ __device__ __forceinline__ void pm_hadamard4(double a, double b, double c, double d, double *e) {
+  const double p1 = a + b, m1 = a - b, p2 = d + c, m2 = d - c;
+  e[0] = p1 + p2;  // 1
+  e[1] = p1 - p2;  // second sign
+  e[2] = m1 + m2;  // first sign
+  e[3] = m1 - m2;
+}
+
+// nodal values -> Legendre coefficients.  kap = 2/3 for a displacement
+// component; 0 for the pressure, whose degree-2 coefficients vanish (its
+// mid-edge values are passed as zero).
+template <int NEN>
+__host__ __device__ __forceinline__ void pm_modal_fwd(const double *v, double kap, double *co) {
+  double h[8];
+  pm_hadamard8(v, h);
+#pragma unroll
+  for (int i = 0; i < 8; i++) h[i] *= 0.125;
+  if constexpr (NEN == 8) {
+#pragma unroll
+    for (int i = 0; i < 8; i++) co[pm_md(i >> 2, (i >> 1) & 1, i & 1)] = h[i];
+    return;
+  } else {
+    double er[4], es[4], et[4];
+    // first/second sign: (t, s) for r-edges, (t, r) for s-edges, (s, r) for t-edges
+    pm_hadamard4(v[8], v[12], v[14], v[10], er);
+    pm_hadamard4(v[11], v[15], v[13], v[9], es);
+    pm_hadamard4(v[16], v[19], v[18], v[17], et);
+    double b[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) b[i] = h[i];
+#pragma unroll
+    for (int p = 0; p < 2; p++)
+#pragma unroll
+      for (int q = 0; q < 2; q++) {
+        // (2, b = p, c = q): e index = first sign t (c), second sign s (b)
+        const double c2 = kap * (h[0 * 4 + p * 2 + q] - 0.25 * er[q * 2 + p]);
+        co[pm_md(2, p, q)] = c2;
+        b[0 * 4 + p * 2 + q] -= c2;
+        // (a = p, 2, c = q)
+        const double d2 = kap * (h[p * 4 + 0 * 2 + q] - 0.25 * es[q * 2 + p]);
+        co[pm_md(p, 2, q)] = d2;
+        b[p * 4 + 0 * 2 + q] -= d2;
+        // (a = p, b = q, 2)
+        const double f2 = kap * (h[p * 4 + q * 2 + 0] - 0.25 * et[q * 2 + p]);
+        co[pm_md(p, q, 2)] = f2;
+        b[p * 4 + q * 2 + 0] -= f2;
+      }
+#pragma unroll
+    for (int i = 0; i < 8; i++) co[pm_md(i >> 2, (i >> 1) & 1, i & 1)] = b[i];
+  }
+}
+
+// coefficient forces -> nodal forces (the transpose of pm_modal_fwd)
+template <int NEN>
+__device__ __forceinline__ void pm_modal_back(const double *f, double kap, double *v) {
+  double h[8];
+#pragma unroll
+  for (int i = 0; i < 8; i++) h[i] = f[pm_md(i >> 2, (i >> 1) & 1, i & 1)];
+  if constexpr (NEN == 20) {
+    double base[8], er[4], es[4], et[4];
+#pragma unroll
+    for (int i = 0; i < 8; i++) base[i] = h[i];
+#pragma unroll
+    for (int p = 0; p < 2; p++)
+#pragma unroll
+      for (int q = 0; q < 2; q++) {
+        const double w1 = kap * (f[pm_md(2, p, q)] - base[0 * 4 + p * 2 + q]);
+        h[0 * 4 + p * 2 + q] += w1;
+        er[q * 2 + p] = -0.25 * w1;
+        const double w2 = kap * (f[pm_md(p, 2, q)] - base[p * 4 + 0 * 2 + q]);
+        h[p * 4 + 0 * 2 + q] += w2;
+        es[q * 2 + p] = -0.25 * w2;
+        const double w3 = kap * (f[pm_md(p, q, 2)] - base[p * 4 + q * 2 + 0]);
+        h[p * 4 + q * 2 + 0] += w3;
+        et[q * 2 + p] = -0.25 * w3;
+      }
+    auto edge = [](const double *e, double &pp, double &mp, double &mm, double &pm) {
+      const double a = e[0] + e[1], b = e[0] - e[1], c = e[2] + e[3], d = e[2] - e[3];
+      pp = a + c;  // first +, second +
+      mp = a - c;  // first -, second +
+      pm = b + d;  // first +, second -
+      mm = b - d;
+    };
+    edge(er, v[8], v[12], v[14], v[10]);
+    edge(es, v[11], v[15], v[13], v[9]);
+    edge(et, v[16], v[19], v[18], v[17]);
+  }
+#pragma unroll
+  for (int i = 0; i < 8; i++) h[i] *= 0.125;
+  pm_hadamard8t(h, v);
+}
+
+struct AffineArgs {
+  int numel;
+  const int *ord;
+  const unsigned int *en;
+  const double *ec;
+  double *ye;
+  const double *x;  // equation vector (OP)
+  const int *ix;    // (numel, nen) nodes (RHS2, RHS4)
+  const double *u;  // (nnode, 4)
+  const double *dp; // (nnode)
+  const int *mat;
+  const double *e;  // (numat, 15)
+  double grav[3];
+  const PmScalars *S;
+};
+
+enum { AF_OP = 0, AF_RHS2 = 1, AF_RHS4 = 2 };
+
+// offset of a node's values in an element's vector: vertices 4 values,
+// mid-edges 3
+__host__ __device__ constexpr int pm_ye_off(int k) { return k < 8 ? 4 * k : 32 + 3 * (k - 8); }
+__host__ __device__ constexpr int pm_ye_len(int nen) { return nen == 20 ? 68 : 32; }
+
+// Element vectors K_e x_e (AF_OP: x an equation vector, restrained dofs zero;
+// AF_RHS2: x the nodal state) or the isw 4 vectors (AF_RHS4).  Bound by the
+// gathers and the one write of the element vectors.
+template <int NEN, int MODE>
+__global__ __launch_bounds__(PM_WG) void k_affine_elements(AffineArgs A) {
+  if (MODE == AF_OP && A.S != nullptr && A.S->done) return;
+  const int lb = pm_xcd_block(blockIdx.x, gridDim.x);
+  const int slot = lb * (PM_WG / 4) + (threadIdx.x >> 2);
+  if (slot >= A.numel) return;  // whole quads leave together
+  const int c = threadIdx.x & 3;
+  double v[NEN], dpv[8];
+  if constexpr (MODE == AF_OP) {
+    unsigned int w[NEN];
+    const uint4 *wp = reinterpret_cast<const uint4 *>(A.en + (size_t)slot * NEN);
+#pragma unroll
+    for (int k = 0; k < NEN / 4; k++) {
+      const uint4 q = wp[k];
+      w[4 * k] = q.x;
+      w[4 * k + 1] = q.y;
+      w[4 * k + 2] = q.z;
+      w[4 * k + 3] = q.w;
+    }
+    const unsigned int below = (1u << c) - 1u;
+#pragma unroll
+    for (int k = 0; k < NEN; k++) {
+      const unsigned int row = (w[k] >> 4) + __popc(w[k] & below);
+      v[k] = ((w[k] >> c) & 1u) ? A.x[row] : 0.0;
+    }
+  } else {
+    const int4 *np = reinterpret_cast<const int4 *>(A.ix + (size_t)A.ord[slot] * NEN);
+    int no[NEN];
+#pragma unroll
+    for (int k = 0; k < NEN / 4; k++) {
+      const int4 q = np[k];
+      no[4 * k] = q.x;
+      no[4 * k + 1] = q.y;
+      no[4 * k + 2] = q.z;
+      no[4 * k + 3] = q.w;
+    }
+#pragma unroll
+    for (int k = 0; k < NEN; k++) v[k] = (k < 8 || c < 3) ? A.u[(size_t)no[k] * 4 + c] : 0.0;
+    if constexpr (MODE == AF_RHS4)
+#pragma unroll
+      for (int k = 0; k < 8; k++) dpv[k] = A.dp[no[k]];
+  }
+  const double *ec = A.ec + (size_t)slot * PM_EC;
+  // the lane's physical axes in cyclic order: its own first (lane 3: x, y, z)
+  double g[3][3];
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    int ax = (c == 3 ? 0 : c) + k;
+    ax = ax >= 3 ? ax - 3 : ax;
+#pragma unroll
+    for (int i = 0; i < 3; i++) g[k][i] = ec[3 * i + ax];
+  }
+  const bool pr = c == 3;
+  const double dtk = ec[14];
+  const double cA = pr ? -dtk : ec[9], cB = pr ? 0.0 : ec[10], cC = pr ? -dtk : ec[11];
+  const double cR = pr ? 0.0 : 1.0, cP = pr ? 0.0 : -ec[12];
+  const double cM = pr ? -ec[13] : 0.0, cT = pr ? -ec[12] : 0.0;
+  const double kap = pr ? 0.0 : 2.0 / 3.0;
+  double co[27], f[27], dpm[8];
+  pm_modal_fwd<NEN>(v, kap, co);
+  if constexpr (MODE == AF_RHS4) pm_hadamard8(dpv, dpm);  // every lane holds dp
+#pragma unroll
+  for (int i = 0; i < 27; i++) f[i] = 0.0;
+  constexpr double nrm[3] = {2.0, 2.0 / 3.0, 2.0 / 5.0};
+#pragma unroll
+  for (int a = 0; a < 3; a++)
+#pragma unroll
+    for (int b = 0; b < 3; b++)
+#pragma unroll
+      for (int d = 0; d < 3; d++) {
+        if (!pm_is_mode<NEN>(a, b, d)) continue;
+        const bool hr = a < 2 && pm_is_mode<NEN>(a + 1, b, d);
+        const bool hs = b < 2 && pm_is_mode<NEN>(a, b + 1, d);
+        const bool ht = d < 2 && pm_is_mode<NEN>(a, b, d + 1);
+        const bool base = a < 2 && b < 2 && d < 2;  // a pressure mode
+        if (!hr && !hs && !ht && !base) continue;
+        const double nd = nrm[a] * nrm[b] * nrm[d];
+        const double sr = a == 1 ? 3.0 : 1.0, ss = b == 1 ? 3.0 : 1.0, st = d == 1 ? 3.0 : 1.0;
+        double F[3] = {0.0, 0.0, 0.0};
+        if (hr || hs || ht) {
+          const double dr = hr ? sr * co[pm_md(a + 1, b, d)] : 0.0;
+          const double ds = hs ? ss * co[pm_md(a, b + 1, d)] : 0.0;
+          const double dt = ht ? st * co[pm_md(a, b, d + 1)] : 0.0;
+#pragma unroll
+          for (int k = 0; k < 3; k++) {
+            double s = 0.0;
+            if (hr) s = g[k][0] * dr;
+            if (hs) s = hr ? fma(g[k][1], ds, s) : g[k][1] * ds;
+            if (ht) s = (hr || hs) ? fma(g[k][2], dt, s) : g[k][2] * dt;
+            F[k] = s;
+          }
+          const double tr = pm_quad<PM_QP(0, 0, 0, 0)>(F[0]) + pm_quad<PM_QP(1, 1, 1, 1)>(F[0]) +
+                            pm_quad<PM_QP(2, 2, 2, 2)>(F[0]);
+          // shear partners: lane c + 1's gradient along c is its third in
+          // cyclic order, lane c + 2's its second
+          const double r1 = pm_quad<PM_QP(1, 2, 0, 3)>(F[2]);
+          const double r2 = pm_quad<PM_QP(2, 0, 1, 3)>(F[1]);
+          double s0 = fma(cB, tr, cA * F[0]);
+          if (base) {
+            const double p = MODE == AF_RHS4 ? 0.125 * dpm[a * 4 + b * 2 + d]
+                                             : pm_quad<PM_QP(3, 3, 3, 3)>(co[pm_md(a, b, d)]);
+            s0 = fma(cP, p, s0);
+          }
+          double s1 = cC * fma(cR, r1, F[1]);
+          double s2 = cC * fma(cR, r2, F[2]);
+          if (MODE == AF_RHS4 && a + b + d == 0) {  // gravity's flux dt perm rho_f g
+            const double *em = A.e + (size_t)A.mat[A.ord[slot]] * PM_PROP;
+            const double fd = pr ? em[6] * 1.0e-06 * dtk : 0.0;
+            s0 = fma(fd, A.grav[0], s0);
+            s1 = fma(fd, A.grav[1], s1);
+            s2 = fma(fd, A.grav[2], s2);
+          }
+          s0 *= nd;
+          s1 *= nd;
+          s2 *= nd;
+          if (hr) {
+            const double q = fma(g[2][0], s2, fma(g[1][0], s1, g[0][0] * s0));
+            f[pm_md(a + 1, b, d)] = fma(sr, q, f[pm_md(a + 1, b, d)]);
+          }
+          if (hs) {
+            const double q = fma(g[2][1], s2, fma(g[1][1], s1, g[0][1] * s0));
+            f[pm_md(a, b + 1, d)] = fma(ss, q, f[pm_md(a, b + 1, d)]);
+          }
+          if (ht) {
+            const double q = fma(g[2][2], s2, fma(g[1][2], s1, g[0][2] * s0));
+            f[pm_md(a, b, d + 1)] = fma(st, q, f[pm_md(a, b, d + 1)]);
+          }
+          if (base && MODE != AF_RHS4) f[pm_md(a, b, d)] = fma(nd * cT, tr, f[pm_md(a, b, d)]);
+        }
+        if (base && MODE != AF_RHS4)
+          f[pm_md(a, b, d)] = fma(nd * cM, co[pm_md(a, b, d)], f[pm_md(a, b, d)]);
+        if (MODE == AF_RHS4 && a + b + d == 0) {  // - rho g on the displacement rows
+          const double *em = A.e + (size_t)A.mat[A.ord[slot]] * PM_PROP;
+          const double gc = c == 0 ? A.grav[0] : c == 1 ? A.grav[1] : c == 2 ? A.grav[2] : 0.0;
+          f[0] -= nd * ec[15] * (em[5] * 1.0e-06) * gc;
+        }
+      }
+  pm_modal_back<NEN>(f, kap, v);
+  double *y = A.ye + (size_t)slot * pm_ye_len(NEN) + c;
+#pragma unroll
+  for (int k = 0; k < NEN; k++)
+    if (k < 8 || c < 3) y[pm_ye_off(k)] = v[k];
+}
+
+// element coefficients: geometry and material, dt folded in
+__global__ __launch_bounds__(PM_WG) void k_affine_coefs(int numel, int nen, const int *ord,
+                                                        const int *ix, const double *xv,
+                                                        const int *mat, const double *e,
+                                                        double dt, double gmod, int stab,
+                                                        double *ec, int *err) {
+  const int slot = blockIdx.x * PM_WG + threadIdx.x;
+  if (slot >= numel) return;
+  const int el = ord[slot];
+  const int *nodes = ix + (size_t)el * nen;
+  double J[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
+  for (int k = 0; k < 8; k++)
+    for (int j = 0; j < 3; j++) {
+      const double x = 0.125 * xv[(size_t)nodes[k] * 3 + j];
+      J[0][j] += c_rn[k] * x;
+      J[1][j] += c_sn[k] * x;
+      J[2][j] += c_tn[k] * x;
+    }
+  const double det = J[0][0] * (J[1][1] * J[2][2] - J[1][2] * J[2][1]) -
+                     J[0][1] * (J[1][0] * J[2][2] - J[1][2] * J[2][0]) +
+                     J[0][2] * (J[1][0] * J[2][1] - J[1][1] * J[2][0]);
+  if (det <= 1.0e-14) atomicExch(err, PM_ERR_JACOBIAN);
+  double *o = ec + (size_t)slot * PM_EC;
+  // o[3 i + x] = d r_i / d x
+  o[0] = (J[1][1] * J[2][2] - J[1][2] * J[2][1]) / det;
+  o[1] = -(J[1][0] * J[2][2] - J[1][2] * J[2][0]) / det;
+  o[2] = (J[1][0] * J[2][1] - J[1][1] * J[2][0]) / det;
+  o[3] = -(J[0][1] * J[2][2] - J[0][2] * J[2][1]) / det;
+  o[4] = (J[0][0] * J[2][2] - J[0][2] * J[2][0]) / det;
+  o[5] = -(J[0][0] * J[2][1] - J[0][1] * J[2][0]) / det;
+  o[6] = (J[0][1] * J[1][2] - J[0][2] * J[1][1]) / det;
+  o[7] = -(J[0][0] * J[1][2] - J[0][2] * J[1][0]) / det;
+  o[8] = (J[0][0] * J[1][1] - J[0][1] * J[1][0]) / det;
+  const double *em = e + (size_t)mat[el] * PM_PROP;
+  const ElemMat M = elem_material(em, dt, gmod);
+  double dtk = M.dt_perm;
+  if (stab && em[8] != 0.0) {  // the Q1/Q1 element's pressure stabilization (k_q1_isw2)
+    const double h = cbrt(8.0 * det);
+    dtk += em[8] * h * h / M.a;
+  }
+  o[9] = det * M.a * (1.0 - M.b);
+  o[10] = det * M.a * M.b;
+  o[11] = det * M.a * M.c;
+  o[12] = det * M.coef_biot;
+  o[13] = det * M.imod_biot;
+  o[14] = det * dtk;
+  o[15] = det;
+}
+
+// ---------------------------------------------------------------------------
+// sums of the element vectors per node
+// ---------------------------------------------------------------------------
+// Four lanes take a row block (a node) and sum its incidences in ascending
+// slot order; lane c holds dof c.  The entries' offsets and values are loaded
+// four at a time so that a node's loads are in flight together.
+struct GatherArgs {
+  int nrn;
+  const int *fr;
+  const unsigned int *gptr, *gsrc;
+  const unsigned char *gmask;
+  const double *ye;
+};
+
+__device__ __forceinline__ double pm_gather_sum(const GatherArgs &G, int64_t k, int c) {
+  const unsigned int p0 = G.gptr[k], p1 = G.gptr[k + 1];
+  double s = 0.0;
+  for (unsigned int p = p0; p < p1; p += 4) {
+    unsigned int o[4];
+    double t[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) o[j] = G.gsrc[p + j < p1 ? p + j : p0];
+#pragma unroll
+    for (int j = 0; j < 4; j++) t[j] = G.ye[o[j] + (unsigned int)c];
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      if (p + j < p1) s += t[j];
+  }
+  return s;
+}
+
+template <int NV, bool SCALE_M>
+__global__ __launch_bounds__(PM_WG) void k_affine_gather(GatherArgs G, double *__restrict__ y,
+                                                         const double *__restrict__ w,
+                                                         const double *__restrict__ m,
+                                                         double *partials, const PmScalars *S) {
+  if (S != nullptr && S->done) return;
+  const int lb = pm_xcd_block(blockIdx.x, gridDim.x);
+  int64_t k0, k1;
+  pm_chunk(G.nrn, lb, gridDim.x, k0, k1);
+  const int c = threadIdx.x & 3;
+  double v[2] = {0.0, 0.0};
+  for (int64_t k = k0 + (threadIdx.x >> 2); k < k1; k += PM_WG / 4) {
+    const unsigned int mk = G.gmask[k];
+    if (!((mk >> c) & 1u)) continue;
+    const int row = G.fr[k] + __popc(mk & ((1u << c) - 1u));
+    double s = pm_gather_sum(G, k, c);
+    if (SCALE_M) s *= m[row];
+    y[row] = s;
+    if (NV >= 1) v[0] += s * w[row];
+    if (NV >= 2) v[1] += s * s;
+  }
+  pm_block_partials<NV>(v, partials);
+}
+
+__global__ __launch_bounds__(PM_WG) void k_affine_subtract(GatherArgs G, double *b) {
+  const int64_t k = (int64_t)pm_xcd_block(blockIdx.x, gridDim.x) * (PM_WG / 4) + (threadIdx.x >> 2);
+  const int c = threadIdx.x & 3;
+  if (k >= G.nrn) return;
+  const unsigned int mk = G.gmask[k];
+  if (!((mk >> c) & 1u)) return;
+  const int row = G.fr[k] + __popc(mk & ((1u << c) - 1u));
+  b[row] -= pm_gather_sum(G, k, c);
+}
+
+// ---------------------------------------------------------------------------
+// the matrix, one row block per group of lanes
+// ---------------------------------------------------------------------------
+// Integrals over the reference element, m, n nodes and q, s pressure vertices:
+//   R[m][ij][n] = int d_i N_m d_j N_n    M[m][j][q] = int d_j N_m Np_q
+//   T[q][j][n] = M[n][j][q]              Z[q][s] = int Np_q Np_s
+//   L[q][ij][s] = int d_i Np_q d_j Np_s
+template <int NEN>
+struct RefTab {
+  static constexpr int R = 0, M = R + NEN * 9 * NEN, T = M + NEN * 3 * 8, Z = T + 8 * 3 * NEN,
+                       L = Z + 64, SIZE = L + 8 * 9 * 8;
+};
+
+// Each matrix value is written once: the lanes of a group walk the row node's
+// incident elements, lane (b, x) forming the column of node b's component x
+// (then lanes 0..7 the pressure columns), and add into the block's rows in
+// LDS; a node's columns are found in the block's column list by bisection in
+// LDS.  A pair's 3 x 3 block is J^-T R J^-1 contracted with D: ~45
+// multiply-adds a lane instead of 64 Gauss points'.
+template <int NEN>
+__global__ __launch_bounds__(PM_WG) void k_affine_matrix(
+    int nrn, int max_cols, const unsigned int *__restrict__ gptr,
+    const unsigned int *__restrict__ gsrc, const unsigned char *__restrict__ gmask,
+    const unsigned int *__restrict__ en, const double *__restrict__ ec,
+    const double *__restrict__ tab, const int *__restrict__ nr,
+    const int64_t *__restrict__ colptr, const int64_t *__restrict__ valptr,
+    const int *__restrict__ ncol, double *__restrict__ val, int *err) {
+  constexpr int LPB = NEN == 20 ? 64 : 32;  // 60 (24) displacement columns an element
+  constexpr int GR = PM_WG / LPB;
+  using RT = RefTab<NEN>;
+  extern __shared__ double s_dyn[];
+  const int grp = threadIdx.x / LPB, l = threadIdx.x % LPB;
+  double *row = s_dyn + (size_t)grp * max_cols * 4;
+  int *cols = reinterpret_cast<int *>(s_dyn + (size_t)GR * max_cols * 4) + (size_t)grp * max_cols;
+  const int64_t k = (int64_t)pm_xcd_block(blockIdx.x, gridDim.x) * GR + grp;
+  const bool live = k < nrn;
+  const int n = live ? nr[k] : 0;
+  const int64_t cp = live ? colptr[k] : 0;
+  const int cnt = live ? (int)(colptr[k + 1] - cp) : 0;
+  for (int j = l; j < cnt; j += LPB) cols[j] = ncol[cp + j];
+  for (int j = l; j < n * cnt; j += LPB) row[j] = 0.0;
+  __syncthreads();
+  if (!live) return;  // no workgroup barrier follows
+  const unsigned int mk = gmask[k];
+  const unsigned int p0 = gptr[k], p1 = gptr[k + 1];
+  // position of a column in the block (or -1)
+  auto find = [&](int col) {
+    int lo = 0, hi = cnt;
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      if (cols[mid] < col) lo = mid + 1;
+      else hi = mid;
+    }
+    if (lo >= cnt || cols[lo] != col) {  // pattern does not hold the pair
+      atomicExch(err, PM_ERR_STATE);
+      return -1;
+    }
+    return lo;
+  };
+  for (unsigned int p = p0; p < p1; p++) {
+    const unsigned int src = gsrc[p];
+    const unsigned int slot = src / (unsigned int)pm_ye_len(NEN);
+    const int off = (int)(src - slot * (unsigned int)pm_ye_len(NEN));
+    const int a = off < 32 ? off >> 2 : 8 + (off - 32) / 3;  // the row's local node
+    const double *eq = ec + (size_t)slot * PM_EC;
+    double g[9];
+#pragma unroll
+    for (int i = 0; i < 9; i++) g[i] = eq[i];
+    const double cd = eq[9] + eq[10], cb = eq[10], cc = eq[11], al = eq[12];
+    // g g^T
+    double gg[9];
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+      for (int j = 0; j < 3; j++)
+        gg[3 * i + j] = g[3 * i] * g[3 * j] + g[3 * i + 1] * g[3 * j + 1] + g[3 * i + 2] * g[3 * j + 2];
+    if (l < 3 * NEN) {
+      const int b = l / 3, x = l - 3 * b;
+      const unsigned int w = en[(size_t)slot * NEN + b];
+      if ((w >> x) & 1u) {
+        const double gx[3] = {x == 0 ? g[0] : x == 1 ? g[1] : g[2],
+                              x == 0 ? g[3] : x == 1 ? g[4] : g[5],
+                              x == 0 ? g[6] : x == 1 ? g[7] : g[8]};
+        double H[3] = {0, 0, 0}, Ht[3] = {0, 0, 0}, lap = 0.0;
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+#pragma unroll
+          for (int j = 0; j < 3; j++) {
+            const double r = tab[RT::R + (a * 9 + 3 * i + j) * NEN + b];
+            H[i] = fma(r, gx[j], H[i]);    // int d_i N_a dN_b/dx
+            Ht[j] = fma(r, gx[i], Ht[j]);  // int dN_a/dx d_j N_b
+            lap = fma(r, gg[3 * i + j], lap);
+          }
+        const int pos = find((int)((w >> 4) + __popc(w & ((1u << x) - 1u))));
+        int q = 0;
+#pragma unroll
+        for (int y = 0; y < 3; y++) {
+          const double Gyx = g[y] * H[0] + g[3 + y] * H[1] + g[6 + y] * H[2];
+          const double Gxy = g[y] * Ht[0] + g[3 + y] * Ht[1] + g[6 + y] * Ht[2];
+          // row y, column x: D's normal and shear parts
+          const double v = y == x ? cd * Gyx + cc * (lap - Gyx) : cb * Gyx + cc * Gxy;
+          if ((mk >> y) & 1u) {
+            if (pos >= 0) row[q * cnt + pos] += v;
+            q++;
+          }
+        }
+        if (a < 8 && ((mk >> 3) & 1u)) {  // pressure row
+          double v = 0.0;
+#pragma unroll
+          for (int j = 0; j < 3; j++) v = fma(gx[j], tab[RT::T + (a * 3 + j) * NEN + b], v);
+          if (pos >= 0) row[q * cnt + pos] -= al * v;
+        }
+      }
+    }
+    if (l < 8) {  // pressure columns
+      const unsigned int w = en[(size_t)slot * NEN + l];
+      if ((w >> 3) & 1u) {
+        const int pos = find((int)((w >> 4) + __popc(w & 7u)));
+        int q = 0;
+#pragma unroll
+        for (int y = 0; y < 3; y++) {
+          if (!((mk >> y) & 1u)) continue;
+          double v = 0.0;
+#pragma unroll
+          for (int j = 0; j < 3; j++) v = fma(g[3 * j + y], tab[RT::M + (a * 3 + j) * 8 + l], v);
+          if (pos >= 0) row[q * cnt + pos] -= al * v;
+          q++;
+        }
+        if (a < 8 && ((mk >> 3) & 1u)) {
+          double lap = 0.0;
+#pragma unroll
+          for (int i = 0; i < 9; i++) lap = fma(tab[RT::L + (a * 9 + i) * 8 + l], gg[i], lap);
+          const double v = eq[13] * tab[RT::Z + a * 8 + l] + eq[14] * lap;
+          if (pos >= 0) row[q * cnt + pos] -= v;
+        }
+      }
+    }
+    // the next element's lanes add into what these lanes wrote
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+  double *out = val + valptr[k];
+  for (int j = l; j < n * cnt; j += LPB) out[j] = row[j];
+}
+
+// the reference integrals from the shape functions' Legendre coefficients
+template <int NEN>
+static std::vector<double> reference_integrals() {
+  using RT = RefTab<NEN>;
+  std::vector<double> t((size_t)RT::SIZE, 0.0);
+  const double nrm[3] = {2.0, 2.0 / 3.0, 2.0 / 5.0};
+  auto coefs = [](int nodes, int k, double *co) {
+    double v[20] = {0};
+    for (int i = 0; i < 27; i++) co[i] = 0.0;
+    v[k] = 1.0;
+    if (nodes == 20) pm_modal_fwd<20>(v, 2.0 / 3.0, co);
+    else pm_modal_fwd<8>(v, 2.0 / 3.0, co);
+  };
+  auto derive = [](const double *co, int dir, double *d) {
+    for (int i = 0; i < 27; i++) d[i] = 0.0;
+    for (int m = 0; m < 27; m++) {
+      int e[3] = {m / 9, (m / 3) % 3, m % 3};
+      const double s = e[dir] == 2 ? 3.0 : 1.0;
+      if (e[dir] == 0) continue;
+      e[dir]--;
+      d[e[0] * 9 + e[1] * 3 + e[2]] += s * co[m];
+    }
+  };
+  auto dot = [&](const double *p, const double *q) {
+    double s = 0.0;
+    for (int m = 0; m < 27; m++) s += p[m] * q[m] * (nrm[m / 9] * nrm[(m / 3) % 3] * nrm[m % 3]);
+    return s;
+  };
+  double N[20][27], dN[20][3][27], P[8][27], dP[8][3][27];
+  for (int k = 0; k < NEN; k++) {
+    coefs(NEN, k, N[k]);
+    for (int i = 0; i < 3; i++) derive(N[k], i, dN[k][i]);
+  }
+  for (int k = 0; k < 8; k++) {
+    coefs(8, k, P[k]);
+    for (int i = 0; i < 3; i++) derive(P[k], i, dP[k][i]);
+  }
+  for (int m = 0; m < NEN; m++)
+    for (int i = 0; i < 3; i++)
+      for (int j = 0; j < 3; j++)
+        for (int n = 0; n < NEN; n++) t[RT::R + (m * 9 + 3 * i + j) * NEN + n] = dot(dN[m][i], dN[n][j]);
+  for (int q = 0; q < 8; q++) {
+    for (int m = 0; m < NEN; m++)
+      for (int j = 0; j < 3; j++) {
+        const double v = dot(dN[m][j], P[q]);
+        t[RT::M + (m * 3 + j) * 8 + q] = v;
+        t[RT::T + (q * 3 + j) * NEN + m] = v;
+      }
+    for (int s = 0; s < 8; s++) {
+      t[RT::Z + q * 8 + s] = dot(P[q], P[s]);
+      for (int i = 0; i < 3; i++)
+        for (int j = 0; j < 3; j++) t[RT::L + (q * 9 + 3 * i + j) * 8 + s] = dot(dP[q][i], dP[s][j]);
+    }
+  }
+  return t;
+}
+
+// ---------------------------------------------------------------------------
+// host
+// ---------------------------------------------------------------------------
+void pm_affine_free(PmAffine *a) {
+  if (!a) return;
+  for (void *p : {(void *)a->ord, (void *)a->en, (void *)a->gptr, (void *)a->gsrc,
+                  (void *)a->gmask, (void *)a->ec_op, (void *)a->ec, (void *)a->ye,
+                  (void *)a->slot, (void *)a->tab})
+    if (p) (void)hipFree(p);
+  delete a;
+}
+
+// true if the 8 vertices span a parallelepiped: the bilinear and trilinear
+// parts of the map vanish to the rounding of the coordinates.  1e-12 of the
+// edge is what coordinates i * h of a mesh of a few hundred cells leave; the
+// matrix entries then differ by as much, far below the solvers' tolerances.
+static bool is_parallelepiped(const int *v, const double *x) {
+  static const int sr[8] = {1, -1, -1, 1, 1, -1, -1, 1}, ss[8] = {1, 1, -1, -1, 1, 1, -1, -1},
+                   st[8] = {1, 1, 1, 1, -1, -1, -1, -1};
+  double lin = 0.0, rest = 0.0;
+  for (int d = 0; d < 3; d++) {
+    double c[7] = {0, 0, 0, 0, 0, 0, 0};
+    for (int k = 0; k < 8; k++) {
+      const double xk = x[(size_t)(v[k] - 1) * 3 + d];
+      c[0] += sr[k] * xk;
+      c[1] += ss[k] * xk;
+      c[2] += st[k] * xk;
+      c[3] += sr[k] * ss[k] * xk;
+      c[4] += ss[k] * st[k] * xk;
+      c[5] += sr[k] * st[k] * xk;
+      c[6] += sr[k] * ss[k] * st[k] * xk;
+    }
+    for (int i = 0; i < 7; i++)
+      if (!std::isfinite(c[i])) return false;
+    for (int i = 0; i < 3; i++) lin = std::max(lin, std::fabs(c[i]));
+    for (int i = 3; i < 7; i++) rest = std::max(rest, std::fabs(c[i]));
+  }
+  return rest <= 1.0e-12 * lin;
+}
+
+int pm_affine_setup(pm_ctx *c, const double *x, const PmHostPattern &pat) {
+  const std::vector<int> &eq_block = pat.eq_block;
+  const PmHostMesh &m = c->mesh;
+  const int nen = m.nen, numel = m.numel, nrn = c->A.nrn;
+  if (m.neq >= (1 << 28) || (int64_t)numel * pm_ye_len(nen) >= ((int64_t)1 << 32)) return PM_OK;
+  for (int e = 0; e < numel; e++)
+    if (!is_parallelepiped(m.ix20.data() + (size_t)e * 21, x)) return PM_OK;
+  // each node's free dofs: first equation << 4 | mask, and its row block
+  std::vector<unsigned int> word((size_t)m.nnode, 0);
+  std::vector<int> block((size_t)m.nnode, -1);
+  std::vector<unsigned char> mask((size_t)nrn, 0);
+  for (int n = 0; n < m.nnode; n++) {
+    const int nd = m.fnno[n] == 1 ? 4 : 3;
+    unsigned int mk = 0;
+    int first = -1;
+    for (int d = 0; d < nd; d++) {
+      const int q = m.id[(size_t)n * 4 + d];
+      if (q <= 0) continue;
+      if (first < 0) first = q - 1;
+      mk |= 1u << d;
+    }
+    if (first < 0) continue;
+    word[n] = ((unsigned int)first << 4) | mk;
+    block[n] = eq_block[first];
+    mask[block[n]] = (unsigned char)mk;
+  }
+  int max_cols = 0;
+  for (int k = 0; k < nrn; k++)
+    max_cols = std::max(max_cols, (int)(pat.colptr[k + 1] - pat.colptr[k]));
+  // slots: elements by their lowest equation
+  std::vector<int> key((size_t)numel), ord((size_t)numel);
+  {
+    std::vector<int> cnt((size_t)nrn + 2, 0);
+    for (int e = 0; e < numel; e++) {
+      int lo = nrn;
+      for (int k = 0; k < nen; k++) {
+        const int b = block[m.ix20[(size_t)e * 21 + k] - 1];
+        if (b >= 0 && b < lo) lo = b;
+      }
+      key[e] = lo;
+      cnt[lo + 1]++;
+    }
+    for (int k = 0; k <= nrn; k++) cnt[k + 1] += cnt[k];
+    for (int e = 0; e < numel; e++) ord[cnt[key[e]]++] = e;
+  }
+  std::vector<unsigned int> en((size_t)numel * nen), gptr((size_t)nrn + 1, 0);
+  for (int s = 0; s < numel; s++)
+    for (int k = 0; k < nen; k++) {
+      const int n = m.ix20[(size_t)ord[s] * 21 + k] - 1;
+      en[(size_t)s * nen + k] = word[n];
+      if (block[n] >= 0) gptr[block[n] + 1]++;
+    }
+  for (int k = 0; k < nrn; k++) gptr[k + 1] += gptr[k];
+  std::vector<unsigned int> gsrc(std::max<size_t>(gptr[nrn], 1)), fill(gptr.begin(), gptr.end() - 1);
+  for (int s = 0; s < numel; s++)
+    for (int k = 0; k < nen; k++) {
+      const int b = block[m.ix20[(size_t)ord[s] * 21 + k] - 1];
+      if (b >= 0) gsrc[fill[b]++] = (unsigned int)((size_t)s * pm_ye_len(nen) + pm_ye_off(k));
+    }
+  std::vector<int> slot((size_t)numel);
+  for (int s = 0; s < numel; s++) slot[ord[s]] = s;
+  const std::vector<double> tab = nen == 20 ? reference_integrals<20>() : reference_integrals<8>();
+  PmAffine *a = new PmAffine();
+  a->max_cols = max_cols;
+  a->numel = numel;
+  a->nen = nen;
+  a->nrn = nrn;
+  bool ok = true;
+  auto up = [&](void **d, const void *h, size_t bytes) {
+    ok = ok && hipMalloc(d, bytes) == hipSuccess &&
+         (!h || hipMemcpy(*d, h, bytes, hipMemcpyHostToDevice) == hipSuccess);
+  };
+  up((void **)&a->ord, ord.data(), sizeof(int) * ord.size());
+  up((void **)&a->en, en.data(), sizeof(unsigned int) * en.size());
+  up((void **)&a->gptr, gptr.data(), sizeof(unsigned int) * gptr.size());
+  up((void **)&a->gsrc, gsrc.data(), sizeof(unsigned int) * gsrc.size());
+  up((void **)&a->gmask, mask.data(), std::max<size_t>(mask.size(), 1));
+  up((void **)&a->ec_op, nullptr, sizeof(double) * PM_EC * (size_t)numel);
+  up((void **)&a->ec, nullptr, sizeof(double) * PM_EC * (size_t)numel);
+  up((void **)&a->slot, slot.data(), sizeof(int) * slot.size());
+  up((void **)&a->tab, tab.data(), sizeof(double) * tab.size());
+  up((void **)&a->ye, nullptr, sizeof(double) * (size_t)numel * pm_ye_len(nen));
+  if (!ok) {  // the stored-matrix path needs none of this
+    (void)hipGetLastError();
+    pm_affine_free(a);
+    return PM_OK;
+  }
+  c->affine = a;
+  return PM_OK;
+}
+
+// c->affine's element loops stand for elmt17_pm and the Q1/Q1 element with
+// constant properties, summed in any order
+static bool affine_elements(const pm_ctx *c) {
+  return c->affine && !c->ordered && !c->vprop[0];
+}
+
+// From 2 million stored values (16 MB) on.  Below, the stored product is one
+// short kernel and the elements are two: an SQMR iteration on boxes takes
+// 24.4 against 23.4 us at 1.2 M values (hexa20/8 8^3), 24.7 against 31.6 at
+// 4.2 M (12^3); Q1/Q1 25.0 against 24.7 at 1.7 M (16^3), 26.0 against 38.8 at
+// 5.8 M (24^3).
+bool pm_affine_product(const pm_ctx *c) {
+  return affine_elements(c) && c->affine->op_valid && c->A.values_valid && c->A.nnz >= 2000000;
+}
+
+static GatherArgs gather_args(const pm_ctx *c) {
+  const PmAffine *a = c->affine;
+  return GatherArgs{a->nrn, c->A.fr, a->gptr, a->gsrc, a->gmask, a->ye};
+}
+
+template <int MODE>
+static void launch_elements(pm_ctx *c, AffineArgs A) {
+  const int g = ((A.numel + PM_WG / 4 - 1) / (PM_WG / 4) + 7) & ~7;
+  if (c->affine->nen == 20)
+    hipLaunchKernelGGL((k_affine_elements<20, MODE>), dim3(g), dim3(PM_WG), 0, c->stream, A);
+  else
+    hipLaunchKernelGGL((k_affine_elements<8, MODE>), dim3(g), dim3(PM_WG), 0, c->stream, A);
+}
+
+static AffineArgs affine_args(const pm_ctx *c) {
+  AffineArgs A{};
+  const PmAffine *a = c->affine;
+  A.numel = a->numel;
+  A.ord = a->ord;
+  A.en = a->en;
+  A.ye = a->ye;
+  return A;
+}
+
+void pm_affine_elements(pm_ctx *c, const double *x, const PmScalars *S) {
+  AffineArgs A = affine_args(c);
+  A.ec = c->affine->ec_op;
+  A.x = x;
+  A.S = S;
+  launch_elements<AF_OP>(c, A);
+}
+
+int pm_affine_gather(pm_ctx *c, double *y, const double *w, const double *m, int nv, bool scale_m,
+                     const PmScalars *S) {
+  const GatherArgs G = gather_args(c);
+  int g = (G.nrn + PM_WG / 4 - 1) / (PM_WG / 4);
+  g = (std::min(g, PM_MAX_GRID) + 7) & ~7;
+  const dim3 gr(g), bl(PM_WG);
+  if (scale_m) {
+    if (nv == 1)
+      hipLaunchKernelGGL((k_affine_gather<1, true>), gr, bl, 0, c->stream, G, y, w, m,
+                         c->d_partials, S);
+    else
+      hipLaunchKernelGGL((k_affine_gather<0, true>), gr, bl, 0, c->stream, G, y, w, m,
+                         c->d_partials, S);
+  } else if (nv == 2) {
+    hipLaunchKernelGGL((k_affine_gather<2, false>), gr, bl, 0, c->stream, G, y, w, m,
+                       c->d_partials, S);
+  } else if (nv == 1) {
+    hipLaunchKernelGGL((k_affine_gather<1, false>), gr, bl, 0, c->stream, G, y, w, m,
+                       c->d_partials, S);
+  } else {
+    hipLaunchKernelGGL((k_affine_gather<0, false>), gr, bl, 0, c->stream, G, y, w, m,
+                       c->d_partials, S);
+  }
+  return g;
+}
+
+// LDS of a workgroup of k_affine_matrix: every group's rows and column list
+static size_t matrix_lds(const PmAffine *a) {
+  return (size_t)(PM_WG / (a->nen == 20 ? 64 : 32)) * a->max_cols * (4 * sizeof(double) + sizeof(int));
+}
+
+bool pm_affine_loops(const pm_ctx *c, int isw, int lhs) {
+  // row blocks too wide for the 64 KB of LDS a workgroup may ask for keep the
+  // scattered assembly (455 columns; a box's vertex has 270, 108 with Q1/Q1)
+  return affine_elements(c) && (isw != 2 || !lhs || matrix_lds(c->affine) <= 65536);
+}
+
+int pm_affine_pform(pm_ctx *c, const ElemArgs &E, int isw, int lhs, int rhs) {
+  PmAffine *a = c->affine;
+  const PmDevMatrix &M = c->A;
+  double *ec = isw == 2 && lhs ? a->ec_op : a->ec;
+  if (isw == 2 && lhs) a->op_valid = false;
+  hipLaunchKernelGGL(k_affine_coefs, dim3((a->numel + PM_WG - 1) / PM_WG), dim3(PM_WG), 0,
+                     c->stream, a->numel, a->nen, a->ord, E.ix, E.xv, E.mat, E.e, E.dt, E.gmod,
+                     a->nen == 8 && isw == 2, ec, E.err);
+  if (rhs) {
+    AffineArgs A = affine_args(c);
+    A.ec = ec;
+    A.ix = E.ix;
+    A.u = E.u;
+    A.dp = E.dp;
+    A.mat = E.mat;
+    A.e = E.e;
+    for (int d = 0; d < 3; d++) A.grav[d] = E.grav[d];
+    if (isw == 2) launch_elements<AF_RHS2>(c, A);
+    else launch_elements<AF_RHS4>(c, A);
+    if (isw == 4 && c->n_face_elems > 0) {
+      if (a->nen == 20)
+        PM_TRY(pm_hexa20_faces(E, c->n_face_elems, c->d_face_elems, a->slot, a->ye, c->stream));
+      else
+        PM_TRY(pm_q1_faces(E, c->n_face_elems, c->d_face_elems, a->slot, a->ye, c->stream));
+    }
+    const GatherArgs G = gather_args(c);
+    const int g = ((G.nrn + PM_WG / 4 - 1) / (PM_WG / 4) + 7) & ~7;
+    hipLaunchKernelGGL(k_affine_subtract, dim3(g), dim3(PM_WG), 0, c->stream, G, E.b);
+  }
+  if (isw == 2 && lhs) {
+    const int gr = PM_WG / (a->nen == 20 ? 64 : 32);
+    const dim3 g((unsigned)(((a->nrn + gr - 1) / gr + 7) & ~7));
+    const size_t lds = matrix_lds(a);
+    if (a->nen == 20)
+      hipLaunchKernelGGL(k_affine_matrix<20>, g, dim3(PM_WG), lds, c->stream, a->nrn, a->max_cols,
+                         a->gptr, a->gsrc, a->gmask, a->en, ec, a->tab, M.nr, M.colptr, M.valptr,
+                         M.ncol, M.val, E.err);
+    else
+      hipLaunchKernelGGL(k_affine_matrix<8>, g, dim3(PM_WG), lds, c->stream, a->nrn, a->max_cols,
+                         a->gptr, a->gsrc, a->gmask, a->en, ec, a->tab, M.nr, M.colptr, M.valptr,
+                         M.ncol, M.val, E.err);
+  }
+  PM_CHECK_HIP(hipGetLastError());
+  return PM_OK;
+}

@@ -5,6 +5,7 @@
 #include <cstring>
 #include <mutex>
 
+#include "pm_affine.h"
 #include "pm_device.h"
 #include "pm_spmv.h"
 
@@ -70,6 +71,7 @@ pm_ctx::~pm_ctx() {
   FREE(d_tf_out);
   FREE(d_ie);
   FREE(d_vp);
+  pm_affine_free(affine);
   if (batch) pm_batch_free(batch);
   FREE(d_eq_box);
   free_matrix(A);
@@ -80,6 +82,7 @@ pm_ctx::~pm_ctx() {
   FREE(d_mat);
   FREE(d_e);
   FREE(d_eload);
+  FREE(d_face_elems);
   FREE(d_load);
   FREE(d_fload);
   FREE(d_colour_elems);
@@ -176,6 +179,8 @@ int pm_upload_pattern(pm_ctx *c, const PmHostPattern &p) {
     c->batch = nullptr;
   }
   FREE(c->d_eq_box);
+  pm_affine_free(c->affine);  // its row blocks are the old matrix's
+  c->affine = nullptr;
   free_matrix(c->A);
   PmDevMatrix &A = c->A;
   A.nrn = p.nrn;
@@ -421,6 +426,7 @@ static int mesh_setup(pm_ctx *c, int nen, int numel, int nnodev, const int *ix, 
   c->colour_ptr = m.colour_ptr;
   c->mesh.neq = m.neq;
   PM_TRY(ensure_state(c));
+  PM_TRY(pm_affine_setup(c, x, p));
   PM_CHECK_HIP(hipStreamSynchronize(c->stream));
   c->have_mesh = true;
   c->have_materials = false;
@@ -539,6 +545,14 @@ extern "C" int pm_set_materials(pm_ctx *c, int numat, const double *e, const int
   PM_TRY(dupload(c, &c->d_load, ld.data(), ld.size()));
   PM_TRY(dupload(c, &c->d_fload, fl.data(), fl.size()));
   c->has_face_loads = any != 0;
+  std::vector<int> face_elems;
+  for (int el = 0; el < m.numel; el++) {
+    int on = 0;
+    for (int j = 0; j < 6; j++) on |= el14[(size_t)el * 14 + j] | el14[(size_t)el * 14 + 7 + j];
+    if (on) face_elems.push_back(el);
+  }
+  PM_TRY(dupload(c, &c->d_face_elems, face_elems.data(), face_elems.size()));
+  c->n_face_elems = (int)face_elems.size();
   for (int d = 0; d < 3; d++) c->gravity[d] = gravity ? gravity[d] : 0.0;
   c->gravity_mod = gravity_mod;
   // initial_porosity (Pform.f:1331-1376, run by the mesh macro, Main.f:820-828):
@@ -680,6 +694,7 @@ extern "C" int pm_values_upload(pm_ctx *c, const double *ad, const double *al) {
   (void)hipFree(d_al);
   A.values_valid = true;
   A.have32 = false;
+  if (c->affine) c->affine->op_valid = false;  // no longer the elements' matrix
   return PM_OK;
 }
 

@@ -51,3 +51,10 @@ __device__ inline double dev_interpol(const double *xs, const double *ys, double
 // through isw 2 or 4, and the vertex porosity change of isw 7
 int pm_q1_elements(const ElemArgs &A, int isw, hipStream_t stream);
 int pm_q1_porosity(const ElemArgs &A, double *dporo, hipStream_t stream);
+
+// face loads of the n elements in list, added to their element vectors
+// (vertices 4 values, mid-edges 3) at slot[element]
+int pm_hexa20_faces(const ElemArgs &A, int n, const int *list, const int *slot, double *ye,
+                    hipStream_t stream);
+int pm_q1_faces(const ElemArgs &A, int n, const int *list, const int *slot, double *ye,
+                hipStream_t stream);

@@ -20,7 +20,7 @@
 
 #include <algorithm>
 
-#include "pm_elemargs.h"
+#include "pm_affine.h"
 #include "pm_elemlib.h"
 
 __device__ __forceinline__ bool is_elmt18(const ElemArgs &A, int el) {
@@ -382,6 +382,36 @@ __device__ void face_loads(const ElemArgs &A, const int *iqm, const int *iqh,
   }
 }
 
+// face loads alone, one thread per loaded element (the elements of a face of
+// the mesh: few against the volume terms)
+__global__ __launch_bounds__(64) void k_faces20(ElemArgs A, int n, const int *list,
+                                                const int *slot, double *ye) {
+  __shared__ double s_p[64][PM_NST + 1];
+  const int i = blockIdx.x * 64 + threadIdx.x;
+  if (i >= n) return;
+  const int el = list[i];
+  const int *nodes = A.ix + (size_t)el * 20;
+  double xv[8][3];
+  for (int k = 0; k < 8; k++)
+    for (int d = 0; d < 3; d++) xv[k][d] = A.xv[(size_t)nodes[k] * 3 + d];
+  double *p = s_p[threadIdx.x];
+  for (int j = 0; j < PM_NST; j++) p[j] = 0.0;
+  const int *eq14 = A.eload + (size_t)el * 14;
+  face_loads(A, eq14, eq14 + 7, xv, p);
+  double *y = ye + (size_t)slot[el] * PM_NST;
+  for (int k = 0; k < 20; k++) {
+    double *yk = y + (k < 8 ? 4 * k : 32 + 3 * (k - 8));
+    for (int d = 0; d < 3; d++) yk[d] += p[3 * k + d];
+    if (k < 8) yk[3] += p[60 + k];
+  }
+}
+
+int pm_hexa20_faces(const ElemArgs &A, int n, const int *list, const int *slot, double *ye,
+                    hipStream_t stream) {
+  hipLaunchKernelGGL(k_faces20, dim3((n + 63) / 64), dim3(64), 0, stream, A, n, list, slot, ye);
+  return hipGetLastError() == hipSuccess ? PM_OK : PM_ERR_HIP;
+}
+
 __global__ __launch_bounds__(PM_WG) void k_elmt_isw4(ElemArgs A) {
   __shared__ double s_xv[8][3];
   __shared__ double s_u[PM_NST];
@@ -714,8 +744,11 @@ static int read_elem_err(pm_ctx *c) {
 int pm_pform_dev(pm_ctx *c, int isw, int lhs, int rhs, double dt, double t, double *bvec) {
   if (!c->have_mesh || !c->have_materials || !c->have_matrix) return PM_ERR_STATE;
   PM_CHECK_HIP(hipMemsetAsync(c->d_elem_err, 0, sizeof(int), c->stream));
+  const bool affine = (isw == 2 || isw == 4) && pm_affine_loops(c, isw, lhs);
   if (isw == 2 && lhs) {
-    PM_CHECK_HIP(hipMemsetAsync(c->A.val, 0, sizeof(double) * (size_t)c->A.nnz, c->stream));
+    if (!affine)  // the scatter adds; pm_affine_pform writes every value
+      PM_CHECK_HIP(hipMemsetAsync(c->A.val, 0, sizeof(double) * (size_t)c->A.nnz, c->stream));
+    if (c->affine) c->affine->op_valid = false;
     c->A.values_valid = false;
     c->A.have32 = false;
   }
@@ -728,7 +761,8 @@ int pm_pform_dev(pm_ctx *c, int isw, int lhs, int rhs, double dt, double t, doub
     if (isw == 2 && lhs) A.ke = c->d_ke;
     if (rhs) A.pe = c->d_pe;
   }
-  const int ncolour = (int)c->colour_ptr.size() - 1;
+  const int ncolour = affine ? 0 : (int)c->colour_ptr.size() - 1;
+  if (affine) PM_TRY(pm_affine_pform(c, A, isw, lhs, rhs));
   for (int k = 0; k < ncolour; k++) {
     A.elems = c->d_colour_elems + c->colour_ptr[k];
     A.nelem = c->colour_ptr[k + 1] - c->colour_ptr[k];
@@ -760,6 +794,7 @@ int pm_pform_dev(pm_ctx *c, int isw, int lhs, int rhs, double dt, double t, doub
   if (isw == 2 && lhs) {
     PM_TRY(pm_extract_diag(c));
     c->A.values_valid = true;
+    if (affine) c->affine->op_valid = true;
   }
   return PM_OK;
 }

@@ -96,6 +96,7 @@ int64_t pm_host_count_lower(const PmHostPattern &p);
 // ---------------------------------------------------------------------------
 struct PmScalars;  // device-side Krylov scalars (pm_device.h)
 struct PmBatch;    // batching form (pm_batch.hip)
+struct PmAffine;   // parallelepiped elements (pm_affine.hip)
 void pm_batch_free(PmBatch *b);
 
 struct PmDevMatrix {
@@ -141,6 +142,8 @@ struct pm_ctx {
   int numat = 0;
   int *d_eload = nullptr;   // (numel, 14): mechanical 7, hydraulic 7
   int has_face_loads = 0;
+  int *d_face_elems = nullptr;  // elements with face loads
+  int n_face_elems = 0;
   int *d_load = nullptr;    // (200, 3)
   double *d_fload = nullptr;// (200, 5, 1000)
   std::vector<int> h_load;
@@ -213,6 +216,9 @@ struct pm_ctx {
   // so SQMR reaching maxit returns PM_ERR_MAXIT instead of falling back to
   // GMRES (whose basis would need (ngram + 1) more vectors)
   bool no_alloc = false;
+
+  // element products of parallelepiped meshes (null: stored matrix only)
+  PmAffine *affine = nullptr;
 
   // batching form
   PmBatch *batch = nullptr;

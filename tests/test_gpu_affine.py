@@ -1,0 +1,122 @@
+"""Parallelepiped meshes, whose element loops and Krylov products run in the
+element's Legendre modes (pm_affine.hip), against the oracle's Gauss loops.
+
+Bars: the element loops' own (matrix within 1e-13 of the row's largest entry,
+right-hand sides within 1e-13 of max|b|); solutions within 1e-9 of those from
+the stored matrix, the bar of the marches."""
+import dataclasses
+
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from poromec_amd import problem as P
+from test_gpu_elmt07 import _rowwise
+
+pytestmark = pytest.mark.gpu
+
+SHEAR = np.array([[1.0, 0.2, -0.1], [0.15, 0.8, 0.25], [-0.2, 0.1, 1.2]])
+
+
+def _deck(shape, nen, shear=True, seed=3):
+    """Box under gravity, traction and flux, its vertices mapped by SHEAR."""
+    d = P.heterogeneous_box_deck(max(shape), seed=seed, shape=shape, sigma_lnk=0.8, corr_len=2.0,
+                                 dt=0.05, nen=nen, patch_fraction=0.7)
+    if shear:
+        d = dataclasses.replace(d, x=d.x @ SHEAR.T)
+    d.gravity = np.array([0.5, -0.3, -10.0])
+    d.e[:, 5] = 2000.0
+    d.load[1] = (43, 2, 2)
+    d.fload[1, 0, :2] = (0.0, 1e30)
+    d.fload[1, 1, :2] = (1e-3, 1e-3)
+    d.eloadp[np.arange(d.numel) % shape[0] == 0, 5] = 2
+    if nen == 8:
+        d.e[:, 8] = 0.25
+    return d
+
+
+# one element; 63, 64 and 65 of them (a workgroup takes 64); several workgroups
+@pytest.mark.parametrize("nen", [20, 8])
+@pytest.mark.parametrize("shape", [(1, 1, 1), (3, 7, 3), (4, 4, 4), (5, 13, 1), (9, 5, 6)])
+def test_element_loops(shape, nen):
+    from poromec_amd.solver import MefSolver
+    d = _deck(shape, nen)
+    st = O.build_structure(d)
+    m = O.OracleModel(d, st)
+    s = MefSolver(d)
+    rng = np.random.default_rng(11)
+    u = rng.standard_normal((st["nnode"], 4)) * 1e-3
+    dp = rng.standard_normal(st["nnode"]) * 1e-4
+    u[d.nnodev:, 3] = 0.0
+    dp[d.nnodev:] = 0.0
+    m.u[:], m.dp[:] = u, dp
+    s.set_state(u=u, u0=np.zeros_like(u), dp=dp, t=0.0)
+    f = rng.standard_normal(st["neq"]) * 1e-3
+    for isw, lhs in ((2, True), (2, False), (4, False)):
+        m.b[:] = f
+        m.env.t = 0.5
+        m.assemble(isw=isw, lhs=lhs, rhs=True)
+        s.set_vectors(b=f)
+        s.pform(isw, lhs, True, d.dt, 0.5, target="b")
+        b = s.vectors()[1]
+        assert np.abs(b - m.b).max() <= 1e-13 * np.abs(m.b).max(), (isw, lhs)
+    _, _, ad, al = s.export_csrc()
+    assert _rowwise(st["ia"], ad, al, m.ad, m.al[: st["nad"]]) < 1e-13
+    s.close()
+
+
+def _stored(s):
+    """The same matrix in a context that has no elements."""
+    from poromec_amd.solver import CsrcSolver
+    ia, ja, ad, al = s.export_csrc()
+    cs = CsrcSolver(ia, ja)
+    cs.set_values(ad, al)
+    return cs
+
+
+def _rel(a, b):
+    return np.abs(a - b).max() / np.abs(b).max()
+
+
+# meshes just past the size from which products run through the elements, and
+# the same with one vertex moved (no longer parallelepipeds: stored matrix)
+@pytest.mark.parametrize("nen,shape", [(20, (11, 10, 10)), (8, (17, 19, 18))])
+@pytest.mark.parametrize("moved", [False, True])
+def test_products_sqmr(nen, shape, moved):
+    from poromec_amd.solver import MefSolver, SolverConfig
+    d = _deck(shape, nen, shear=False)
+    d.e[:, 8] = 0.0
+    if moved:
+        d.x[np.argmin(np.abs(d.x - 0.5 * np.array(shape)).sum(1)), 2] += 0.05
+    s = MefSolver(d)
+    s.pform(2, True, False, d.dt, d.dt)
+    assert s.matrix_info()["nnz"] > 2_000_000
+    b = np.random.default_rng(5).standard_normal(s.neq)
+    cs = _stored(s)
+    x0, _ = cs.solve(b, SolverConfig(tol=1e-11))
+    for prec in ("fp64", "fp32ir"):
+        x, info = s.solve(b, SolverConfig(tol=1e-11, precision=prec))
+        # the residual is recomputed from the stored matrix
+        assert info["true_rel"] < 1e-9 and _rel(x, x0) < 1e-9, (prec, info)
+    s.close()
+    cs.close()
+
+
+def test_products_other_solvers():
+    from poromec_amd.solver import MefSolver, SolverConfig
+    d = _deck((11, 10, 11), 20)
+    d.idv[:, 3] = 1  # K = K_uu, positive definite
+    s = MefSolver(d)
+    s.pform(2, True, False, d.dt, d.dt)
+    assert s.matrix_info()["nnz"] > 2_000_000
+    b = np.random.default_rng(6).standard_normal(s.neq)
+    cs = _stored(s)
+    x0, _ = cs.solve(b, SolverConfig(solver="pcg", tol=1e-12))
+    for solver, precond in (("pcg", 2), ("bicgstab", 2), ("minres", 5)):
+        x, _ = s.solve(b, SolverConfig(solver=solver, precond=precond, tol=1e-12))
+        assert _rel(x, x0) < 1e-9, solver
+    # GMRES stops on the scaled residual; its rows' scales differ by < 100
+    x, info = s.solve(b, SolverConfig(solver="gmres", tol=1e-7, maxit=20))
+    assert info["true_rel"] < 1e-5
+    s.close()
+    cs.close()
