@@ -18,6 +18,7 @@
 #include <cstring>
 #include <type_traits>
 
+#include "pm_affine.h"
 #include "pm_device.h"
 #include "pm_functors.h"
 #include "pm_spmv.h"
@@ -805,6 +806,23 @@ static void launch_spmv(pm_ctx *c, int use32, const double *x, double *y, const 
   spmv_time_end(c, use32);
 }
 
+// The product of the Krylov loops: through the elements where the mesh allows
+// it (pm_affine.hip; FP64 throughout, also in place of the FP32 values), from
+// the stored matrix otherwise.
+template <int NV, bool SCALE_M, class Epi>
+static void launch_product(pm_ctx *c, int use32, const double *x, double *y, const double *w,
+                           const double *m, PmScalars *S, Epi epi) {
+  if (!pm_affine_product(c)) {
+    launch_spmv<NV, SCALE_M>(c, use32, x, y, w, m, S, epi);
+    return;
+  }
+  spmv_time_begin(c);
+  pm_affine_elements(c, x, S);
+  const int g = pm_affine_gather(c, y, w, m, NV, SCALE_M, S);
+  if (NV > 0) launch_finish<NV>(c, g, S, epi, 0);
+  spmv_time_end(c, use32);
+}
+
 int pm_spmv_dev(pm_ctx *c, const double *x, double *y, int use32) {
   launch_spmv<0, false>(c, use32, x, y, nullptr, nullptr, nullptr, NoEpi{});
   PM_CHECK_HIP(hipGetLastError());
@@ -1269,7 +1287,7 @@ static int run_pcg(pm_ctx *c, int n, const double *b, double *x, const double *m
     int chunk = std::min(next_chunk(launched), maxit - launched);
     for (int it = 0; it < chunk; it++) {
       c->cur_iter = launched + it + 1;
-      launch_spmv<1, false>(c, use32, p, z, p, nullptr, S, PcgAlpha{});
+      launch_product<1, false>(c, use32, p, z, p, nullptr, S, PcgAlpha{});
       (use32 ? info->spmv32 : info->spmv64)++;
       launch_vec<1>(c, n, S, PcgUpd{x, r, z, p, m}, PcgUpdEpi{});
       launch_vec<0>(c, n, S, PcgP{p, z}, FinishEpi{});
@@ -1298,7 +1316,7 @@ static int run_sqmr(pm_ctx *c, int n, const double *b, double *x, const double *
     int chunk = std::min(next_chunk(launched), maxit - launched);
     for (int it = 0; it < chunk; it++) {
       c->cur_iter = launched + it + 1;
-      launch_spmv<1, false>(c, use32, q, t, q, nullptr, S, SqmrSigma{});
+      launch_product<1, false>(c, use32, q, t, q, nullptr, S, SqmrSigma{});
       (use32 ? info->spmv32 : info->spmv64)++;
       launch_vec<2>(c, n, S, SqmrRT{r, t, m}, SqmrRTEpi{});
       launch_vec<0>(c, n, S, SqmrDXQ{d, x, q, t}, SqmrFinishEpi{});
@@ -1331,9 +1349,9 @@ static int run_bicgstab(pm_ctx *c, int n, const double *b, double *x, const doub
     int chunk = std::min(next_chunk(launched), maxit - launched);
     for (int it = 0; it < chunk; it++) {
       c->cur_iter = launched + it + 1;
-      launch_spmv<1, false>(c, use32, z, v, r0, nullptr, S, BcgAlpha{});
+      launch_product<1, false>(c, use32, z, v, r0, nullptr, S, BcgAlpha{});
       launch_vec<1>(c, n, S, BcgS{x, r, z, v, m}, BcgSEpi{});
-      launch_spmv<2, false>(c, use32, z, t, r, nullptr, S, BcgW{});
+      launch_product<2, false>(c, use32, z, t, r, nullptr, S, BcgW{});
       launch_vec<2>(c, n, S, BcgR{x, r, z, t, r0}, BcgREpi{});
       launch_vec<0>(c, n, S, BcgP{p, z, r, v, m}, NoEpi{});
       (use32 ? info->spmv32 : info->spmv64) += 2;
@@ -1363,14 +1381,14 @@ static int run_minres(pm_ctx *c, int n, const double *b, double *x, const double
   for (int cycle = 0; cycle <= nrestart && !done; cycle++) {
     double *v0 = buf[0], *v = buf[1], *p = buf[2], *z0 = buf[3], *z = buf[4], *w00 = buf[5],
            *w0 = buf[6];
-    launch_spmv<0, false>(c, 0, x, z, nullptr, nullptr, S, NoEpi{});
+    launch_product<0, false>(c, 0, x, z, nullptr, nullptr, S, NoEpi{});
     launch_vec<1>(c, n, S, MrStart{b, m, z, v, v0, w0, w00, z0}, MrStartEpi{});
     int launched = 0;
     while (launched < maxit) {
       int chunk = std::min(next_chunk(launched), maxit - launched);
       for (int it = 0; it < chunk; it++) {
         c->cur_iter = total + launched + it + 1;
-        launch_spmv<1, false>(c, use32, z0, p, z0, nullptr, S, MrAlpha{});
+        launch_product<1, false>(c, use32, z0, p, z0, nullptr, S, MrAlpha{});
         (use32 ? info->spmv32 : info->spmv64)++;
         launch_vec<1>(c, n, S, MrP{p, z, v, v0, m}, MrQr{});
         launch_vec<0>(c, n, S, MrW{x, w00, z0, w0}, FinishEpi{});
@@ -1420,7 +1438,7 @@ static int run_gmres(pm_ctx *c, int n, const double *b, double *x, const double 
   launch_vec<1>(c, n, S, GmInitNorm{b, m, x, g(0)}, GmInitNormEpi{tol});
   int done = 0, iter = 0;
   for (int l = 0; l < maxit && !done; l++) {
-    launch_spmv<0, false>(c, 0, x, g(0), nullptr, nullptr, S, NoEpi{});
+    launch_product<0, false>(c, 0, x, g(0), nullptr, nullptr, S, NoEpi{});
     launch_vec<1>(c, n, S, GmRes0{b, m, g(0)}, GmE0{e});
     launch_vec<0>(c, n, S, GmScale{g(0)}, NoEpi{});
     for (int i = 0; i < k; i++) {
@@ -1431,7 +1449,7 @@ static int run_gmres(pm_ctx *c, int n, const double *b, double *x, const double 
         if (c->h_scal->flag == 2 || done) break;
       }
       double *gi = g(i), *gn = g(i + 1);
-      launch_spmv<1, true>(c, use32, gi, gn, gn, m, S, GmTau{});
+      launch_product<1, true>(c, use32, gi, gn, gn, m, S, GmTau{});
       (use32 ? info->spmv32 : info->spmv64)++;
       for (int sweep = 0; sweep < 2; sweep++) {
         // first dot with g0
