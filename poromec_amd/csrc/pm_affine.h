@@ -31,8 +31,8 @@ bool pm_affine_loops(const pm_ctx *c, int isw, int lhs);
 int pm_affine_pform(pm_ctx *c, const ElemArgs &E, int isw, int lhs, int rhs);
 
 // Krylov products through the elements: true when the matrix in c->A is the
-// one whose coefficients are kept
-bool pm_affine_product(const pm_ctx *c);
+// one whose coefficients are kept and large enough for it to pay
+bool pm_affine_product(const pm_ctx *c, int use32);
 
 // the element part of y = A x: element vectors into ye
 void pm_affine_elements(pm_ctx *c, const double *x, const PmScalars *S);

@@ -26,6 +26,7 @@
 
 #include "pm_affine.h"
 #include "pm_elemlib.h"
+#include "pm_fused.h"
 
 #define PM_EC 16  // doubles of element coefficients
 // 0-8 g[i][x] = d r_i / d x, then det J times: 9 a (1 - b), 10 a b, 11 a c,
@@ -198,51 +199,11 @@ enum { AF_OP = 0, AF_RHS2 = 1, AF_RHS4 = 2 };
 __host__ __device__ constexpr int pm_ye_off(int k) { return k < 8 ? 4 * k : 32 + 3 * (k - 8); }
 __host__ __device__ constexpr int pm_ye_len(int nen) { return nen == 20 ? 68 : 32; }
 
-// Element vectors K_e x_e (AF_OP: x an equation vector, restrained dofs zero;
-// AF_RHS2: x the nodal state) or the isw 4 vectors (AF_RHS4).  Bound by the
-// gathers and the one write of the element vectors.
+// One lane's share of an element vector: the nodal values v of component c (3:
+// pressure) become the nodal forces of K_e, or (AF_RHS4) of isw 4.
 template <int NEN, int MODE>
-__global__ __launch_bounds__(PM_WG) void k_affine_elements(AffineArgs A) {
-  if (MODE == AF_OP && A.S != nullptr && A.S->done) return;
-  const int lb = pm_xcd_block(blockIdx.x, gridDim.x);
-  const int slot = lb * (PM_WG / 4) + (threadIdx.x >> 2);
-  if (slot >= A.numel) return;  // whole quads leave together
-  const int c = threadIdx.x & 3;
-  double v[NEN], dpv[8];
-  if constexpr (MODE == AF_OP) {
-    unsigned int w[NEN];
-    const uint4 *wp = reinterpret_cast<const uint4 *>(A.en + (size_t)slot * NEN);
-#pragma unroll
-    for (int k = 0; k < NEN / 4; k++) {
-      const uint4 q = wp[k];
-      w[4 * k] = q.x;
-      w[4 * k + 1] = q.y;
-      w[4 * k + 2] = q.z;
-      w[4 * k + 3] = q.w;
-    }
-    const unsigned int below = (1u << c) - 1u;
-#pragma unroll
-    for (int k = 0; k < NEN; k++) {
-      const unsigned int row = (w[k] >> 4) + __popc(w[k] & below);
-      v[k] = ((w[k] >> c) & 1u) ? A.x[row] : 0.0;
-    }
-  } else {
-    const int4 *np = reinterpret_cast<const int4 *>(A.ix + (size_t)A.ord[slot] * NEN);
-    int no[NEN];
-#pragma unroll
-    for (int k = 0; k < NEN / 4; k++) {
-      const int4 q = np[k];
-      no[4 * k] = q.x;
-      no[4 * k + 1] = q.y;
-      no[4 * k + 2] = q.z;
-      no[4 * k + 3] = q.w;
-    }
-#pragma unroll
-    for (int k = 0; k < NEN; k++) v[k] = (k < 8 || c < 3) ? A.u[(size_t)no[k] * 4 + c] : 0.0;
-    if constexpr (MODE == AF_RHS4)
-#pragma unroll
-      for (int k = 0; k < 8; k++) dpv[k] = A.dp[no[k]];
-  }
+__device__ __forceinline__ void pm_element_vector(const AffineArgs &A, int slot, int c, double *v,
+                                                  const double *dpv) {
   const double *ec = A.ec + (size_t)slot * PM_EC;
   // the lane's physical axes in cyclic order: its own first (lane 3: x, y, z)
   double g[3][3];
@@ -339,10 +300,102 @@ __global__ __launch_bounds__(PM_WG) void k_affine_elements(AffineArgs A) {
         }
       }
   pm_modal_back<NEN>(f, kap, v);
-  double *y = A.ye + (size_t)slot * pm_ye_len(NEN) + c;
+}
+
+template <int NEN>
+__device__ __forceinline__ void pm_store_element(double *ye, int slot, int c, const double *v) {
+  double *y = ye + (size_t)slot * pm_ye_len(NEN) + c;
 #pragma unroll
   for (int k = 0; k < NEN; k++)
     if (k < 8 || c < 3) y[pm_ye_off(k)] = v[k];
+}
+
+// the free-dof words of an element's nodes
+template <int NEN>
+__device__ __forceinline__ void pm_load_words(const unsigned int *en, int slot, unsigned int *w) {
+  const uint4 *wp = reinterpret_cast<const uint4 *>(en + (size_t)slot * NEN);
+#pragma unroll
+  for (int k = 0; k < NEN / 4; k++) {
+    const uint4 q = wp[k];
+    w[4 * k] = q.x;
+    w[4 * k + 1] = q.y;
+    w[4 * k + 2] = q.z;
+    w[4 * k + 3] = q.w;
+  }
+}
+
+// Element vectors K_e x_e (AF_OP: x an equation vector, restrained dofs zero;
+// AF_RHS2: x the nodal state) or the isw 4 vectors (AF_RHS4).  Bound by the
+// gathers and the one write of the element vectors.
+template <int NEN, int MODE>
+__global__ __launch_bounds__(PM_WG) void k_affine_elements(AffineArgs A) {
+  if (MODE == AF_OP && A.S != nullptr && A.S->done) return;
+  const int lb = pm_xcd_block(blockIdx.x, gridDim.x);
+  const int slot = lb * (PM_WG / 4) + (threadIdx.x >> 2);
+  if (slot >= A.numel) return;  // whole quads leave together
+  const int c = threadIdx.x & 3;
+  double v[NEN], dpv[8];
+  if constexpr (MODE == AF_OP) {
+    unsigned int w[NEN];
+    pm_load_words<NEN>(A.en, slot, w);
+    const unsigned int below = (1u << c) - 1u;
+#pragma unroll
+    for (int k = 0; k < NEN; k++) {
+      const unsigned int row = (w[k] >> 4) + __popc(w[k] & below);
+      v[k] = ((w[k] >> c) & 1u) ? A.x[row] : 0.0;
+    }
+  } else {
+    const int4 *np = reinterpret_cast<const int4 *>(A.ix + (size_t)A.ord[slot] * NEN);
+    int no[NEN];
+#pragma unroll
+    for (int k = 0; k < NEN / 4; k++) {
+      const int4 q = np[k];
+      no[4 * k] = q.x;
+      no[4 * k + 1] = q.y;
+      no[4 * k + 2] = q.z;
+      no[4 * k + 3] = q.w;
+    }
+#pragma unroll
+    for (int k = 0; k < NEN; k++) v[k] = (k < 8 || c < 3) ? A.u[(size_t)no[k] * 4 + c] : 0.0;
+    if constexpr (MODE == AF_RHS4)
+#pragma unroll
+      for (int k = 0; k < 8; k++) dpv[k] = A.dp[no[k]];
+  }
+  pm_element_vector<NEN, MODE>(A, slot, c, v, dpv);
+  pm_store_element<NEN>(A.ye, slot, c, v);
+}
+
+// Pass A of the fused iteration (pm_fused.h), element part: the element
+// vectors of q_new = t + beta q, formed at the gathered nodes.
+template <int NEN, PmMethod MT>
+__global__ __launch_bounds__(PM_WG) void k_affine_pass_elements(AffineArgs A, PmVecs V,
+                                                                PmIterState *st, int cur,
+                                                                int first, double tol, int nblk,
+                                                                const double *pb) {
+  const PmIter s = pm_iter_begin<MT>(st, cur, first, tol, nblk, pb);
+  if (blockIdx.x == 0 && threadIdx.x == 0) st->it[cur ^ 1] = s;
+  if (s.done || s.pending) return;
+  const int lb = pm_xcd_block(blockIdx.x, gridDim.x);
+  const int c = threadIdx.x & 3;
+  const unsigned int below = (1u << c) - 1u;
+  // contiguous tiles of 64 elements per workgroup
+  const int tiles = (A.numel + PM_WG / 4 - 1) / (PM_WG / 4);
+  int64_t t0, t1;
+  pm_chunk(tiles, lb, gridDim.x, t0, t1);
+  for (int64_t t = t0; t < t1; t++) {
+    const int slot = (int)t * (PM_WG / 4) + (threadIdx.x >> 2);
+    if (slot >= A.numel) return;  // whole quads, in the last tile
+    unsigned int w[NEN];
+    pm_load_words<NEN>(A.en, slot, w);
+    double v[NEN];
+#pragma unroll
+    for (int k = 0; k < NEN; k++) {
+      const unsigned int row = (w[k] >> 4) + __popc(w[k] & below);
+      v[k] = ((w[k] >> c) & 1u) ? V.t[row] + s.beta * V.q[row] : 0.0;
+    }
+    pm_element_vector<NEN, AF_OP>(A, slot, c, v, nullptr);
+    pm_store_element<NEN>(A.ye, slot, c, v);
+  }
 }
 
 // element coefficients: geometry and material, dt folded in
@@ -447,6 +500,31 @@ __global__ __launch_bounds__(PM_WG) void k_affine_gather(GatherArgs G, double *_
     if (NV >= 2) v[1] += s * s;
   }
   pm_block_partials<NV>(v, partials);
+}
+
+// Pass A, node part: y = A q_new with the row's update and the dot q_new . y
+template <PmMethod MT>
+__global__ __launch_bounds__(PM_WG) void k_affine_pass_gather(GatherArgs G, PmVecs V,
+                                                              const PmIterState *st, int nxt,
+                                                              double *pa) {
+  const PmIter s = st->it[nxt];  // written by the element part
+  if (s.done) return;
+  const int lb = pm_xcd_block(blockIdx.x, gridDim.x);
+  int64_t k0, k1;
+  pm_chunk(G.nrn, lb, gridDim.x, k0, k1);
+  const int c = threadIdx.x & 3;
+  double v[1] = {0.0};
+  for (int64_t k = k0 + (threadIdx.x >> 2); k < k1; k += PM_WG / 4) {
+    const unsigned int mk = G.gmask[k];
+    if (!((mk >> c) & 1u)) continue;
+    const int row = G.fr[k] + __popc(mk & ((1u << c) - 1u));
+    const double qn = pm_row_update<MT>(V, s, row);
+    if (s.pending) continue;
+    const double y = pm_gather_sum(G, k, c);
+    V.y[row] = y;
+    v[0] += y * qn;
+  }
+  pm_block_partials<1>(v, pa);
 }
 
 __global__ __launch_bounds__(PM_WG) void k_affine_subtract(GatherArgs G, double *b) {
@@ -798,13 +876,16 @@ static bool affine_elements(const pm_ctx *c) {
   return c->affine && !c->ordered && !c->vprop[0];
 }
 
-// From 2 million stored values (16 MB) on.  Below, the stored product is one
-// short kernel and the elements are two: an SQMR iteration on boxes takes
-// 24.4 against 23.4 us at 1.2 M values (hexa20/8 8^3), 24.7 against 31.6 at
-// 4.2 M (12^3); Q1/Q1 25.0 against 24.7 at 1.7 M (16^3), 26.0 against 38.8 at
-// 5.8 M (24^3).
-bool pm_affine_product(const pm_ctx *c) {
-  return affine_elements(c) && c->affine->op_valid && c->A.values_valid && c->A.nnz >= 2000000;
+// From 3.6 million stored values on with FP64 values, 4.5 with FP32: below,
+// the stored product is the shorter chain (one pass against two).  An SQMR
+// iteration on boxes, stored / elements, FP64 and FP32: hexa20/8 11^3 (3.2 M
+// values) 17.1 / 19.2 us and 14.6 / 19.3, 12^3 (4.2 M) 20.1 / 19.1 and 16.7 /
+// 19.3, 14^3 (6.7 M) 24.4 / 19.6 and 20.7 / 19.5; Q1/Q1 18^3 (2.4 M) 15.2 /
+// 17.1 and 14.4 / 17.0, 20^3 (3.3 M) 18.2 / 16.8 and 16.0 / 17.0, 24^3 (5.8 M)
+// 23.6 / 17.4 and 20.0 / 17.5.
+bool pm_affine_product(const pm_ctx *c, int use32) {
+  return affine_elements(c) && c->affine->op_valid && c->A.values_valid &&
+         c->A.nnz >= (use32 ? 4500000 : 3600000);
 }
 
 static GatherArgs gather_args(const pm_ctx *c) {
@@ -863,6 +944,33 @@ int pm_affine_gather(pm_ctx *c, double *y, const double *w, const double *m, int
                        c->d_partials, S);
   }
   return g;
+}
+
+template <PmMethod MT>
+static int affine_pass(pm_ctx *c, const PmVecs &V, PmIterState *st, int cur, int first, double tol,
+                       int nblk, const double *pb, double *pa) {
+  AffineArgs A = affine_args(c);
+  A.ec = c->affine->ec_op;
+  // at most 2048 workgroups: each sums the partials of pass B again
+  const int tiles = (A.numel + PM_WG / 4 - 1) / (PM_WG / 4);
+  const int ge = (std::min(tiles, PM_MAX_GRID) + 7) & ~7;
+  if (c->affine->nen == 20)
+    hipLaunchKernelGGL((k_affine_pass_elements<20, MT>), dim3(ge), dim3(PM_WG), 0, c->stream, A, V,
+                       st, cur, first, tol, nblk, pb);
+  else
+    hipLaunchKernelGGL((k_affine_pass_elements<8, MT>), dim3(ge), dim3(PM_WG), 0, c->stream, A, V,
+                       st, cur, first, tol, nblk, pb);
+  const GatherArgs G = gather_args(c);
+  const int g = (std::min((G.nrn + PM_WG / 4 - 1) / (PM_WG / 4), PM_MAX_GRID) + 7) & ~7;
+  hipLaunchKernelGGL(k_affine_pass_gather<MT>, dim3(g), dim3(PM_WG), 0, c->stream, G, V, st,
+                     cur ^ 1, pa);
+  return g;
+}
+
+int pm_affine_pass(pm_ctx *c, PmMethod mt, const PmVecs &V, PmIterState *st, int cur, int first,
+                   double tol, int nblk, const double *pb, double *pa) {
+  return mt == PM_IT_SQMR ? affine_pass<PM_IT_SQMR>(c, V, st, cur, first, tol, nblk, pb, pa)
+                          : affine_pass<PM_IT_PCG>(c, V, st, cur, first, tol, nblk, pb, pa);
 }
 
 // LDS of a workgroup of k_affine_matrix: every group's rows and column list

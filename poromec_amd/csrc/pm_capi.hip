@@ -7,6 +7,7 @@
 
 #include "pm_affine.h"
 #include "pm_device.h"
+#include "pm_fused.h"
 #include "pm_spmv.h"
 
 static thread_local char g_last_error[512] = "";
@@ -104,6 +105,8 @@ pm_ctx::~pm_ctx() {
   FREE(d_partials);
   FREE(d_counter);
   FREE(d_scal);
+  FREE(d_iter);
+  if (h_iter) hipHostFree(h_iter);
   if (h_scal) hipHostFree(h_scal);
   if (ev0) hipEventDestroy(ev0);
   if (ev1) hipEventDestroy(ev1);
@@ -150,6 +153,9 @@ extern "C" int pm_ctx_create(pm_ctx **out, int device) {
   chk(hipMemset(c->d_counter, 0, sizeof(unsigned int)));
   chk(hipMalloc(&c->d_scal, sizeof(PmScalars)));
   chk(hipMemset(c->d_scal, 0, sizeof(PmScalars)));
+  chk(hipMalloc(&c->d_iter, sizeof(PmIterState)));
+  chk(hipMemset(c->d_iter, 0, sizeof(PmIterState)));
+  chk(hipHostMalloc((void **)&c->h_iter, sizeof(PmIter), hipHostMallocDefault));
   chk(hipHostMalloc((void **)&c->h_scal, sizeof(PmScalars), hipHostMallocDefault));
   chk(hipMalloc(&c->d_elem_err, sizeof(int)));
   if (rc != PM_OK) {

@@ -1,0 +1,126 @@
+// pm_fused.h -- scalars of the fused SQMR and PCG iterations (pm_fused.hip).
+//
+// An iteration is a product pass A and a vector pass B.  Each pass leaves
+// workgroup partials of its dots; the workgroups of the next pass sum them
+// again, all in the same fixed order, and so all hold the same scalars
+// without a finisher kernel between the passes.  Workgroup 0 writes the
+// scalars for the passes after that one.  A pass never reads what its own
+// launch writes: A takes slot it & 1 to slot (it + 1) & 1, B writes PmStep.
+#pragma once
+#include "pm_device.h"
+
+enum PmMethod { PM_IT_SQMR, PM_IT_PCG };
+
+struct PmIter {
+  double conv;         // stop threshold of the recurrence residual
+  double ro, tau, v0;  // SQMR: rho, tau, theta; PCG: ro = r . M^-1 r
+  double t1, t2, beta; // coefficients of the pending update of d and q
+  double resid;        // recurrence residual of the last finished iteration
+  int done;            // 0 running, 1 converged, < 0 PM_ERR_* code
+  int pending;         // converged (1) or broken down (< 0): this pass A still
+                       // makes the finished iteration's update, then done
+  int it;              // iterations started
+  int pad;
+};
+struct PmStep {
+  double alpha;
+  int broken;  // the product's dot vanished (SQMR)
+  int pad;
+};
+struct PmIterState {  // device
+  PmIter it[2];
+  PmStep step;
+};
+
+// Scalars of the iteration that pass A starts: from the partials of pass B
+// of the last one (first: of the initial vectors), RPSQMR (Iters.f:6100-6436)
+// and PCG (Iters.f:299-595).  Called by whole workgroups; every thread
+// receives the same values.
+template <PmMethod MT>
+__device__ __forceinline__ PmIter pm_iter_begin(const PmIterState *st, int cur, int first, double tol,
+                                                int nblk, const double *partials) {
+  PmIter s = st->it[cur];
+  if (first) {
+    double r[2];
+    pm_sum_partials<2>(nblk, partials, r);
+    s.v0 = s.t1 = s.t2 = s.beta = 0.0;
+    s.resid = 0.0;
+    s.done = s.pending = 0;
+    s.it = 1;
+    if (MT == PM_IT_SQMR) {
+      s.conv = tol * sqrt(fabs(r[0]));
+      s.tau = sqrt(r[0]);
+      s.ro = r[1];
+    } else {
+      s.conv = tol * sqrt(fabs(r[1]));
+      s.tau = 0.0;
+      s.ro = r[1];
+    }
+    return s;
+  }
+  if (s.done) return s;
+  if (s.pending) {  // the update was made by the last pass A
+    s.done = s.pending;
+    return s;
+  }
+  if (MT == PM_IT_SQMR && st->step.broken) {
+    s.done = PM_ERR_BREAKDOWN;
+    return s;
+  }
+  double r[2];
+  pm_sum_partials<2>(nblk, partials, r);
+  if (MT == PM_IT_SQMR) {
+    const double normr = sqrt(r[0]);
+    const double vn = normr / s.tau;
+    const double cn = 1.0 / sqrt(1.0 + vn * vn);
+    s.tau = s.tau * vn * cn;
+    s.t1 = cn * cn * s.v0 * s.v0;
+    s.t2 = cn * cn * st->step.alpha;
+    s.v0 = vn;
+    if (s.ro == 0.0) {
+      s.pending = PM_ERR_BREAKDOWN;
+      return s;
+    }
+    s.beta = r[1] / s.ro;
+    s.ro = r[1];
+    s.resid = normr;
+    if (normr < s.conv) s.pending = 1;
+  } else {
+    s.beta = r[1] / s.ro;
+    s.ro = r[1];
+    s.resid = sqrt(fabs(r[1]));
+    if (s.resid < s.conv) s.pending = 1;
+  }
+  if (!s.pending) s.it += 1;
+  return s;
+}
+
+// vectors of an iteration: q_new = t + beta q; SQMR also d = t1 d + t2 q,
+// x += d (PCG moves x in pass B)
+struct PmVecs {
+  const double *t, *q;
+  double *qn, *d, *x, *y;
+};
+
+// one row of pass A's update; returns q_new
+template <PmMethod MT>
+__device__ __forceinline__ double pm_row_update(const PmVecs &V, const PmIter &s, int64_t i) {
+  const double qi = V.q[i];
+  if (MT == PM_IT_SQMR) {
+    const double di = s.t1 * V.d[i] + s.t2 * qi;
+    V.d[i] = di;
+    V.x[i] = V.x[i] + di;
+  }
+  const double qn = V.t[i] + s.beta * qi;
+  V.qn[i] = qn;
+  return qn;
+}
+
+// pass A through the elements (pm_affine.hip); returns the grid of its partials
+int pm_affine_pass(pm_ctx *c, PmMethod mt, const PmVecs &V, PmIterState *st, int cur, int first,
+                   double tol, int nblk, const double *pb, double *pa);
+
+// true if the solve can run fused
+bool pm_fused_usable(const pm_ctx *c, int use32);
+int pm_fused_solve(pm_ctx *c, PmMethod mt, int n, const double *b, double *x, const double *m,
+                   double tol, int maxit, int use32, pm_solve_info *info, int *converged);

@@ -97,6 +97,8 @@ int64_t pm_host_count_lower(const PmHostPattern &p);
 struct PmScalars;  // device-side Krylov scalars (pm_device.h)
 struct PmBatch;    // batching form (pm_batch.hip)
 struct PmAffine;   // parallelepiped elements (pm_affine.hip)
+struct PmIterState;  // fused iterations (pm_fused.h)
+struct PmIter;
 void pm_batch_free(PmBatch *b);
 
 struct PmDevMatrix {
@@ -192,6 +194,8 @@ struct pm_ctx {
   unsigned int *d_counter = nullptr;
   PmScalars *d_scal = nullptr;
   PmScalars *h_scal = nullptr; // pinned mirror
+  PmIterState *d_iter = nullptr;  // scalars of the fused iterations
+  PmIter *h_iter = nullptr;       // pinned mirror
   int red_blocks = 1024;
   // live SpMV timing (measurement hook): an event pair around every SpMV a
   // single-system solver launches, harvested after each host sync; pairs
@@ -261,5 +265,8 @@ int pm_batch_true_res(pm_ctx *c, const double *b, const double *x, double *res,
 int pm_adjoint_dev(pm_ctx *c, int nsteps, double dt, const pm_solver_cfg *cfg, int nsens,
                    const int *sensor_dof, const double *target, int ckpt_every, double *J,
                    double *grad_logE, double *grad_logk);
+void pm_spmv_time_begin(pm_ctx *c);
+void pm_spmv_time_end(pm_ctx *c, int use32);
 void pm_spmv_harvest(pm_ctx *c, int done, int iter);
+void pm_progress(int launched, double resid);
 int pm_batch_spmv_dev(pm_ctx *c, const double *x, double *y, int use32);

@@ -21,6 +21,7 @@
 #include "pm_affine.h"
 #include "pm_device.h"
 #include "pm_functors.h"
+#include "pm_fused.h"
 #include "pm_spmv.h"
 #include <vector>
 
@@ -735,7 +736,7 @@ struct SpmvDots {  // the dots fused into the fast SpMV: y.w and y.y
   }
 };
 
-static void spmv_time_begin(pm_ctx *c) {
+void pm_spmv_time_begin(pm_ctx *c) {
   c->tev_open = false;
   if (!c->time_spmv || (c->spmv_seq++ % c->time_spmv) != 0) return;  // every time_spmv-th
   if ((size_t)(2 * c->tev_used + 2) > c->tev.size()) {
@@ -753,7 +754,7 @@ static void spmv_time_begin(pm_ctx *c) {
   c->tev_open = true;
 }
 
-static void spmv_time_end(pm_ctx *c, int use32) {
+void pm_spmv_time_end(pm_ctx *c, int use32) {
   if (!c->tev_open) return;
   c->tev_open = false;
   (void)hipEventRecord(c->tev[2 * c->tev_used + 1], c->stream);
@@ -801,9 +802,9 @@ static void launch_spmv_raw(pm_ctx *c, int use32, const double *x, double *y, co
 template <int NV, bool SCALE_M, class Epi>
 static void launch_spmv(pm_ctx *c, int use32, const double *x, double *y, const double *w,
                         const double *m, PmScalars *S, Epi epi) {
-  spmv_time_begin(c);
+  pm_spmv_time_begin(c);
   launch_spmv_raw<NV, SCALE_M>(c, use32, x, y, w, m, S, epi);
-  spmv_time_end(c, use32);
+  pm_spmv_time_end(c, use32);
 }
 
 // The product of the Krylov loops: through the elements where the mesh allows
@@ -812,15 +813,15 @@ static void launch_spmv(pm_ctx *c, int use32, const double *x, double *y, const 
 template <int NV, bool SCALE_M, class Epi>
 static void launch_product(pm_ctx *c, int use32, const double *x, double *y, const double *w,
                            const double *m, PmScalars *S, Epi epi) {
-  if (!pm_affine_product(c)) {
+  if (!pm_affine_product(c, use32)) {
     launch_spmv<NV, SCALE_M>(c, use32, x, y, w, m, S, epi);
     return;
   }
-  spmv_time_begin(c);
+  pm_spmv_time_begin(c);
   pm_affine_elements(c, x, S);
   const int g = pm_affine_gather(c, y, w, m, NV, SCALE_M, S);
   if (NV > 0) launch_finish<NV>(c, g, S, epi, 0);
-  spmv_time_end(c, use32);
+  pm_spmv_time_end(c, use32);
 }
 
 int pm_spmv_dev(pm_ctx *c, const double *x, double *y, int use32) {
@@ -837,28 +838,30 @@ int pm_spmv_fused_dev(pm_ctx *c, const double *x, double *y, int use32) {
   return PM_OK;
 }
 
+// PM_PROGRESS_SECONDS=s (opt-in): the solve's iteration and recurrence
+// residual on stderr every s seconds (long solves under a watchdog)
+void pm_progress(int launched, double resid) {
+  static const double progress_s = [] {
+    const char *e = std::getenv("PM_PROGRESS_SECONDS");
+    return e ? std::atof(e) : 0.0;
+  }();
+  if (progress_s <= 0.0) return;
+  static thread_local auto last = std::chrono::steady_clock::now();
+  const auto now = std::chrono::steady_clock::now();
+  if (std::chrono::duration<double>(now - last).count() >= progress_s) {
+    std::fprintf(stderr, "[pm_solve] %d iterations launched, residual %.3e\n", launched, resid);
+    std::fflush(stderr);
+    last = now;
+  }
+}
+
 static int poll_done(pm_ctx *c, int *done, int *iter) {
   PM_CHECK_HIP(hipMemcpyAsync(c->h_scal, c->d_scal, sizeof(PmScalars), hipMemcpyDeviceToHost,
                               c->stream));
   PM_CHECK_HIP(hipStreamSynchronize(c->stream));
   *done = c->h_scal->done;
   *iter = c->h_scal->iter;
-  // PM_PROGRESS_SECONDS=s (opt-in): the solve's iteration and recurrence
-  // residual on stderr every s seconds (long solves under a watchdog)
-  static const double progress_s = [] {
-    const char *e = std::getenv("PM_PROGRESS_SECONDS");
-    return e ? std::atof(e) : 0.0;
-  }();
-  if (progress_s > 0.0) {
-    static thread_local auto last = std::chrono::steady_clock::now();
-    const auto now = std::chrono::steady_clock::now();
-    if (std::chrono::duration<double>(now - last).count() >= progress_s) {
-      std::fprintf(stderr, "[pm_solve] %d iterations launched, residual %.3e\n", c->cur_iter,
-                   c->h_scal->resid);
-      std::fflush(stderr);
-      last = now;
-    }
-  }
+  pm_progress(c->cur_iter, c->h_scal->resid);
   if (c->tev_used) pm_spmv_harvest(c, *done, *iter);
   return PM_OK;
 }
@@ -1278,6 +1281,11 @@ static int zero_diag_check(pm_ctx *c);
 
 static int run_pcg(pm_ctx *c, int n, const double *b, double *x, const double *m, double tol,
                    int maxit, int use32, pm_solve_info *info) {
+  if (pm_fused_usable(c, use32)) {
+    int ok = 0;
+    PM_TRY(pm_fused_solve(c, PM_IT_PCG, n, b, x, m, tol, maxit, use32, info, &ok));
+    return ok ? PM_OK : PM_ERR_MAXIT;
+  }
   double *r = c->d_wk[0], *z = c->d_wk[1], *p = c->d_wk[2];
   PmScalars *S = c->d_scal;
   PM_TRY(reset_scalars(c));
@@ -1309,6 +1317,15 @@ static int run_sqmr(pm_ctx *c, int n, const double *b, double *x, const double *
   double *t = c->d_wk[0], *r = c->d_wk[1], *q = c->d_wk[2], *d = c->d_wk[3];
   PmScalars *S = c->d_scal;
   *failed = 0;
+  if (pm_fused_usable(c, use32)) {
+    int ok = 0;
+    PM_TRY(pm_fused_solve(c, PM_IT_SQMR, n, b, x, m, tol, maxit, use32, info, &ok));
+    if (!ok) {
+      *failed = 1;
+      info->iters += maxit;
+    }
+    return PM_OK;
+  }
   PM_TRY(reset_scalars(c));
   launch_vec<2>(c, n, S, SqmrInit{b, m, x, r, q, d}, SqmrInitEpi{tol});
   int launched = 0, done = 0, iter = 0;
