@@ -9,9 +9,10 @@ struct PmAffine {
   int numel = 0, nen = 0, nrn = 0;
   int *ord = nullptr;            // (numel) element of each slot
   unsigned int *en = nullptr;    // (numel, nen) first free equation << 4 | free dofs of the node
-  unsigned int *gptr = nullptr;  // (nrn + 1) incidences of each row block
-  unsigned int *gsrc = nullptr;  // their offsets in ye
-  unsigned char *gmask = nullptr;  // (nrn) free dofs of the block's node
+  int stride = 0;                // incidences kept per row block (the most any has, to 4)
+  unsigned int *gnode = nullptr; // (nrn) the block's first row << 4 | free dofs
+  unsigned int *gsrc = nullptr;  // (nrn, stride) offsets of its entries in ye, then `zero`
+  unsigned int zero = 0;         // offset of four zeros in ye
   double *ec_op = nullptr;       // (numel, 16) coefficients of the assembled matrix
   double *ec = nullptr;          // (numel, 16) coefficients of one element loop
   double *ye = nullptr;          // element vectors

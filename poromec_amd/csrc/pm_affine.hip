@@ -372,9 +372,6 @@ __global__ __launch_bounds__(PM_WG) void k_affine_pass_elements(AffineArgs A, Pm
                                                                 PmIterState *st, int cur,
                                                                 int first, double tol, int nblk,
                                                                 const double *pb) {
-  const PmIter s = pm_iter_begin<MT>(st, cur, first, tol, nblk, pb);
-  if (blockIdx.x == 0 && threadIdx.x == 0) st->it[cur ^ 1] = s;
-  if (s.done || s.pending) return;
   const int lb = pm_xcd_block(blockIdx.x, gridDim.x);
   const int c = threadIdx.x & 3;
   const unsigned int below = (1u << c) - 1u;
@@ -382,17 +379,31 @@ __global__ __launch_bounds__(PM_WG) void k_affine_pass_elements(AffineArgs A, Pm
   const int tiles = (A.numel + PM_WG / 4 - 1) / (PM_WG / 4);
   int64_t t0, t1;
   pm_chunk(tiles, lb, gridDim.x, t0, t1);
+  double tv[NEN], qv[NEN];
+  auto gather = [&](int64_t t) {
+    const int slot = (int)t * (PM_WG / 4) + (threadIdx.x >> 2);
+    if (t >= t1 || slot >= A.numel) return;
+    unsigned int w[NEN];
+    pm_load_words<NEN>(A.en, slot, w);
+#pragma unroll
+    for (int k = 0; k < NEN; k++) {
+      const bool on = (w[k] >> c) & 1u;
+      const unsigned int row = on ? (w[k] >> 4) + __popc(w[k] & below) : 0u;
+      tv[k] = on ? V.t[row] : 0.0;
+      qv[k] = on ? V.q[row] : 0.0;
+    }
+  };
+  gather(t0);  // in flight while the scalars are formed
+  const PmIter s = pm_iter_begin<MT>(st, cur, first, tol, nblk, pb);
+  if (blockIdx.x == 0 && threadIdx.x == 0) st->it[cur ^ 1] = s;
+  if (s.done || s.pending) return;
   for (int64_t t = t0; t < t1; t++) {
     const int slot = (int)t * (PM_WG / 4) + (threadIdx.x >> 2);
     if (slot >= A.numel) return;  // whole quads, in the last tile
-    unsigned int w[NEN];
-    pm_load_words<NEN>(A.en, slot, w);
+    if (t > t0) gather(t);
     double v[NEN];
 #pragma unroll
-    for (int k = 0; k < NEN; k++) {
-      const unsigned int row = (w[k] >> 4) + __popc(w[k] & below);
-      v[k] = ((w[k] >> c) & 1u) ? V.t[row] + s.beta * V.q[row] : 0.0;
-    }
+    for (int k = 0; k < NEN; k++) v[k] = tv[k] + s.beta * qv[k];
     pm_element_vector<NEN, AF_OP>(A, slot, c, v, nullptr);
     pm_store_element<NEN>(A.ye, slot, c, v);
   }
@@ -450,30 +461,38 @@ __global__ __launch_bounds__(PM_WG) void k_affine_coefs(int numel, int nen, cons
 // ---------------------------------------------------------------------------
 // sums of the element vectors per node
 // ---------------------------------------------------------------------------
-// Four lanes take a row block (a node) and sum its incidences in ascending
-// slot order; lane c holds dof c.  The entries' offsets and values are loaded
-// four at a time so that a node's loads are in flight together.
+// Four lanes take a row block (a node) and sum its incidences, eight at a
+// time in a fixed tree; lane c holds dof c.  Every node has `stride` offsets
+// (8 in a box; the mid-edges' last four and a boundary node's missing ones
+// point to a zero), so their loads need no pointer first.
 struct GatherArgs {
-  int nrn;
-  const int *fr;
-  const unsigned int *gptr, *gsrc;
-  const unsigned char *gmask;
+  int nrn, stride;
+  const unsigned int *gnode;  // (nrn) first row << 4 | free dofs
+  const unsigned int *gsrc;   // (nrn, stride) offsets in ye; past the last, of a zero
   const double *ye;
+  unsigned int zero;
 };
 
 __device__ __forceinline__ double pm_gather_sum(const GatherArgs &G, int64_t k, int c) {
-  const unsigned int p0 = G.gptr[k], p1 = G.gptr[k + 1];
+  const uint4 *src = reinterpret_cast<const uint4 *>(G.gsrc + (size_t)k * G.stride);
   double s = 0.0;
-  for (unsigned int p = p0; p < p1; p += 4) {
-    unsigned int o[4];
-    double t[4];
-#pragma unroll
-    for (int j = 0; j < 4; j++) o[j] = G.gsrc[p + j < p1 ? p + j : p0];
-#pragma unroll
-    for (int j = 0; j < 4; j++) t[j] = G.ye[o[j] + (unsigned int)c];
-#pragma unroll
-    for (int j = 0; j < 4; j++)
-      if (p + j < p1) s += t[j];
+  for (int p = 0; p < G.stride; p += 8) {
+    const uint4 a = src[p / 4];
+    const uint4 b = p + 4 < G.stride ? src[p / 4 + 1] : uint4{G.zero, G.zero, G.zero, G.zero};
+    double t[8];
+    t[0] = G.ye[a.x + (unsigned int)c];
+    t[1] = G.ye[a.y + (unsigned int)c];
+    t[2] = G.ye[a.z + (unsigned int)c];
+    t[3] = G.ye[a.w + (unsigned int)c];
+    if (b.x != G.zero) {  // mid-edges have four at most
+      t[4] = G.ye[b.x + (unsigned int)c];
+      t[5] = G.ye[b.y + (unsigned int)c];
+      t[6] = G.ye[b.z + (unsigned int)c];
+      t[7] = G.ye[b.w + (unsigned int)c];
+    } else {
+      t[4] = t[5] = t[6] = t[7] = 0.0;
+    }
+    s += ((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]));
   }
   return s;
 }
@@ -490,9 +509,9 @@ __global__ __launch_bounds__(PM_WG) void k_affine_gather(GatherArgs G, double *_
   const int c = threadIdx.x & 3;
   double v[2] = {0.0, 0.0};
   for (int64_t k = k0 + (threadIdx.x >> 2); k < k1; k += PM_WG / 4) {
-    const unsigned int mk = G.gmask[k];
-    if (!((mk >> c) & 1u)) continue;
-    const int row = G.fr[k] + __popc(mk & ((1u << c) - 1u));
+    const unsigned int w4 = G.gnode[k];
+    if (!((w4 >> c) & 1u)) continue;
+    const unsigned int row = (w4 >> 4) + __popc(w4 & ((1u << c) - 1u));
     double s = pm_gather_sum(G, k, c);
     if (SCALE_M) s *= m[row];
     y[row] = s;
@@ -515,25 +534,25 @@ __global__ __launch_bounds__(PM_WG) void k_affine_pass_gather(GatherArgs G, PmVe
   const int c = threadIdx.x & 3;
   double v[1] = {0.0};
   for (int64_t k = k0 + (threadIdx.x >> 2); k < k1; k += PM_WG / 4) {
-    const unsigned int mk = G.gmask[k];
-    if (!((mk >> c) & 1u)) continue;
-    const int row = G.fr[k] + __popc(mk & ((1u << c) - 1u));
+    const unsigned int w4 = G.gnode[k];
+    if (!((w4 >> c) & 1u)) continue;
+    const unsigned int row = (w4 >> 4) + __popc(w4 & ((1u << c) - 1u));
+    const double y = s.pending ? 0.0 : pm_gather_sum(G, k, c);
     const double qn = pm_row_update<MT>(V, s, row);
     if (s.pending) continue;
-    const double y = pm_gather_sum(G, k, c);
     V.y[row] = y;
     v[0] += y * qn;
   }
-  pm_block_partials<1>(v, pa);
+  pm_dots_partials<1>(v, pa);
 }
 
 __global__ __launch_bounds__(PM_WG) void k_affine_subtract(GatherArgs G, double *b) {
   const int64_t k = (int64_t)pm_xcd_block(blockIdx.x, gridDim.x) * (PM_WG / 4) + (threadIdx.x >> 2);
   const int c = threadIdx.x & 3;
   if (k >= G.nrn) return;
-  const unsigned int mk = G.gmask[k];
-  if (!((mk >> c) & 1u)) return;
-  const int row = G.fr[k] + __popc(mk & ((1u << c) - 1u));
+  const unsigned int w4 = G.gnode[k];
+  if (!((w4 >> c) & 1u)) return;
+  const unsigned int row = (w4 >> 4) + __popc(w4 & ((1u << c) - 1u));
   b[row] -= pm_gather_sum(G, k, c);
 }
 
@@ -558,8 +577,8 @@ struct RefTab {
 // multiply-adds a lane instead of 64 Gauss points'.
 template <int NEN>
 __global__ __launch_bounds__(PM_WG) void k_affine_matrix(
-    int nrn, int max_cols, const unsigned int *__restrict__ gptr,
-    const unsigned int *__restrict__ gsrc, const unsigned char *__restrict__ gmask,
+    int nrn, int max_cols, int stride, unsigned int zero, const unsigned int *__restrict__ gsrc,
+    const unsigned int *__restrict__ gnode,
     const unsigned int *__restrict__ en, const double *__restrict__ ec,
     const double *__restrict__ tab, const int *__restrict__ nr,
     const int64_t *__restrict__ colptr, const int64_t *__restrict__ valptr,
@@ -580,8 +599,7 @@ __global__ __launch_bounds__(PM_WG) void k_affine_matrix(
   for (int j = l; j < n * cnt; j += LPB) row[j] = 0.0;
   __syncthreads();
   if (!live) return;  // no workgroup barrier follows
-  const unsigned int mk = gmask[k];
-  const unsigned int p0 = gptr[k], p1 = gptr[k + 1];
+  const unsigned int mk = gnode[k] & 15u;
   // position of a column in the block (or -1)
   auto find = [&](int col) {
     int lo = 0, hi = cnt;
@@ -596,8 +614,9 @@ __global__ __launch_bounds__(PM_WG) void k_affine_matrix(
     }
     return lo;
   };
-  for (unsigned int p = p0; p < p1; p++) {
-    const unsigned int src = gsrc[p];
+  for (int p = 0; p < stride; p++) {
+    const unsigned int src = gsrc[(size_t)k * stride + p];
+    if (src == zero) break;
     const unsigned int slot = src / (unsigned int)pm_ye_len(NEN);
     const int off = (int)(src - slot * (unsigned int)pm_ye_len(NEN));
     const int a = off < 32 ? off >> 2 : 8 + (off - 32) / 3;  // the row's local node
@@ -744,8 +763,8 @@ static std::vector<double> reference_integrals() {
 // ---------------------------------------------------------------------------
 void pm_affine_free(PmAffine *a) {
   if (!a) return;
-  for (void *p : {(void *)a->ord, (void *)a->en, (void *)a->gptr, (void *)a->gsrc,
-                  (void *)a->gmask, (void *)a->ec_op, (void *)a->ec, (void *)a->ye,
+  for (void *p : {(void *)a->ord, (void *)a->en, (void *)a->gsrc, (void *)a->gnode,
+                  (void *)a->ec_op, (void *)a->ec, (void *)a->ye,
                   (void *)a->slot, (void *)a->tab})
     if (p) (void)hipFree(p);
   delete a;
@@ -783,13 +802,13 @@ int pm_affine_setup(pm_ctx *c, const double *x, const PmHostPattern &pat) {
   const std::vector<int> &eq_block = pat.eq_block;
   const PmHostMesh &m = c->mesh;
   const int nen = m.nen, numel = m.numel, nrn = c->A.nrn;
-  if (m.neq >= (1 << 28) || (int64_t)numel * pm_ye_len(nen) >= ((int64_t)1 << 32)) return PM_OK;
+  if (m.neq >= (1 << 28) || (int64_t)numel * pm_ye_len(nen) + 4 >= ((int64_t)1 << 32)) return PM_OK;
   for (int e = 0; e < numel; e++)
     if (!is_parallelepiped(m.ix20.data() + (size_t)e * 21, x)) return PM_OK;
   // each node's free dofs: first equation << 4 | mask, and its row block
   std::vector<unsigned int> word((size_t)m.nnode, 0);
   std::vector<int> block((size_t)m.nnode, -1);
-  std::vector<unsigned char> mask((size_t)nrn, 0);
+  std::vector<unsigned int> gnode((size_t)nrn, 0);
   for (int n = 0; n < m.nnode; n++) {
     const int nd = m.fnno[n] == 1 ? 4 : 3;
     unsigned int mk = 0;
@@ -803,7 +822,7 @@ int pm_affine_setup(pm_ctx *c, const double *x, const PmHostPattern &pat) {
     if (first < 0) continue;
     word[n] = ((unsigned int)first << 4) | mk;
     block[n] = eq_block[first];
-    mask[block[n]] = (unsigned char)mk;
+    gnode[block[n]] = word[n];
   }
   int max_cols = 0;
   for (int k = 0; k < nrn; k++)
@@ -824,25 +843,33 @@ int pm_affine_setup(pm_ctx *c, const double *x, const PmHostPattern &pat) {
     for (int k = 0; k <= nrn; k++) cnt[k + 1] += cnt[k];
     for (int e = 0; e < numel; e++) ord[cnt[key[e]]++] = e;
   }
-  std::vector<unsigned int> en((size_t)numel * nen), gptr((size_t)nrn + 1, 0);
+  std::vector<unsigned int> en((size_t)numel * nen);
+  std::vector<int> cnt((size_t)nrn, 0);
   for (int s = 0; s < numel; s++)
     for (int k = 0; k < nen; k++) {
       const int n = m.ix20[(size_t)ord[s] * 21 + k] - 1;
       en[(size_t)s * nen + k] = word[n];
-      if (block[n] >= 0) gptr[block[n] + 1]++;
+      if (block[n] >= 0) cnt[block[n]]++;
     }
-  for (int k = 0; k < nrn; k++) gptr[k + 1] += gptr[k];
-  std::vector<unsigned int> gsrc(std::max<size_t>(gptr[nrn], 1)), fill(gptr.begin(), gptr.end() - 1);
+  const int stride = ((nrn > 0 ? *std::max_element(cnt.begin(), cnt.end()) : 0) + 3) & ~3;
+  if (stride > 32) return PM_OK;  // a fan of elements: keep the stored matrix
+  const unsigned int zero = (unsigned int)((size_t)numel * pm_ye_len(nen));
+  std::vector<unsigned int> gsrc((size_t)nrn * stride, zero);
+  std::fill(cnt.begin(), cnt.end(), 0);
   for (int s = 0; s < numel; s++)
     for (int k = 0; k < nen; k++) {
       const int b = block[m.ix20[(size_t)ord[s] * 21 + k] - 1];
-      if (b >= 0) gsrc[fill[b]++] = (unsigned int)((size_t)s * pm_ye_len(nen) + pm_ye_off(k));
+      if (b >= 0)
+        gsrc[(size_t)b * stride + cnt[b]++] =
+            (unsigned int)((size_t)s * pm_ye_len(nen) + pm_ye_off(k));
     }
   std::vector<int> slot((size_t)numel);
   for (int s = 0; s < numel; s++) slot[ord[s]] = s;
   const std::vector<double> tab = nen == 20 ? reference_integrals<20>() : reference_integrals<8>();
   PmAffine *a = new PmAffine();
   a->max_cols = max_cols;
+  a->stride = stride;
+  a->zero = zero;
   a->numel = numel;
   a->nen = nen;
   a->nrn = nrn;
@@ -853,14 +880,15 @@ int pm_affine_setup(pm_ctx *c, const double *x, const PmHostPattern &pat) {
   };
   up((void **)&a->ord, ord.data(), sizeof(int) * ord.size());
   up((void **)&a->en, en.data(), sizeof(unsigned int) * en.size());
-  up((void **)&a->gptr, gptr.data(), sizeof(unsigned int) * gptr.size());
   up((void **)&a->gsrc, gsrc.data(), sizeof(unsigned int) * gsrc.size());
-  up((void **)&a->gmask, mask.data(), std::max<size_t>(mask.size(), 1));
+  up((void **)&a->gnode, gnode.data(), sizeof(unsigned int) * gnode.size());
   up((void **)&a->ec_op, nullptr, sizeof(double) * PM_EC * (size_t)numel);
   up((void **)&a->ec, nullptr, sizeof(double) * PM_EC * (size_t)numel);
   up((void **)&a->slot, slot.data(), sizeof(int) * slot.size());
   up((void **)&a->tab, tab.data(), sizeof(double) * tab.size());
-  up((void **)&a->ye, nullptr, sizeof(double) * (size_t)numel * pm_ye_len(nen));
+  // the element vectors, then four zeros for the gathers' missing entries
+  up((void **)&a->ye, nullptr, sizeof(double) * ((size_t)zero + 4));
+  ok = ok && hipMemset(a->ye + zero, 0, 4 * sizeof(double)) == hipSuccess;
   if (!ok) {  // the stored-matrix path needs none of this
     (void)hipGetLastError();
     pm_affine_free(a);
@@ -890,7 +918,7 @@ bool pm_affine_product(const pm_ctx *c, int use32) {
 
 static GatherArgs gather_args(const pm_ctx *c) {
   const PmAffine *a = c->affine;
-  return GatherArgs{a->nrn, c->A.fr, a->gptr, a->gsrc, a->gmask, a->ye};
+  return GatherArgs{a->nrn, a->stride, a->gnode, a->gsrc, a->ye, a->zero};
 }
 
 template <int MODE>
@@ -1019,11 +1047,11 @@ int pm_affine_pform(pm_ctx *c, const ElemArgs &E, int isw, int lhs, int rhs) {
     const size_t lds = matrix_lds(a);
     if (a->nen == 20)
       hipLaunchKernelGGL(k_affine_matrix<20>, g, dim3(PM_WG), lds, c->stream, a->nrn, a->max_cols,
-                         a->gptr, a->gsrc, a->gmask, a->en, ec, a->tab, M.nr, M.colptr, M.valptr,
+                         a->stride, a->zero, a->gsrc, a->gnode, a->en, ec, a->tab, M.nr, M.colptr, M.valptr,
                          M.ncol, M.val, E.err);
     else
       hipLaunchKernelGGL(k_affine_matrix<8>, g, dim3(PM_WG), lds, c->stream, a->nrn, a->max_cols,
-                         a->gptr, a->gsrc, a->gmask, a->en, ec, a->tab, M.nr, M.colptr, M.valptr,
+                         a->stride, a->zero, a->gsrc, a->gnode, a->en, ec, a->tab, M.nr, M.colptr, M.valptr,
                          M.ncol, M.val, E.err);
   }
   PM_CHECK_HIP(hipGetLastError());

@@ -8,6 +8,7 @@
 // launch writes: A takes slot it & 1 to slot (it + 1) & 1, B writes PmStep.
 #pragma once
 #include "pm_device.h"
+#include "pm_spmv.h"
 
 enum PmMethod { PM_IT_SQMR, PM_IT_PCG };
 
@@ -32,6 +33,48 @@ struct PmIterState {  // device
   PmStep step;
 };
 
+// Sums of the partials of nblk workgroups, the same in every workgroup: as
+// pm_sum_partials, the wavefront sums by DPP instead of six LDS permutes each
+// (they sit on every pass's critical path).
+template <int NV>
+__device__ __forceinline__ void pm_sum_dots(int nblk, const double *partials, double *out) {
+  __shared__ double sh[NV][PM_WAVES];
+  double acc[NV];
+#pragma unroll
+  for (int i = 0; i < NV; i++) acc[i] = 0.0;
+  for (int b = threadIdx.x; b < nblk; b += PM_WG)
+#pragma unroll
+    for (int i = 0; i < NV; i++) acc[i] += partials[(size_t)b * NV + i];
+#pragma unroll
+  for (int i = 0; i < NV; i++) {
+    const double w = pm_group_sum<64>(acc[i]);
+    if ((threadIdx.x & 63) == 63) sh[i][threadIdx.x >> 6] = w;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < NV; i++) {
+    out[i] = sh[i][0];
+    for (int w = 1; w < PM_WAVES; w++) out[i] += sh[i][w];
+  }
+}
+
+// workgroup partials of NV dots, DPP sums
+template <int NV>
+__device__ __forceinline__ void pm_dots_partials(const double *v, double *partials) {
+  __shared__ double sh[NV][PM_WAVES];
+#pragma unroll
+  for (int i = 0; i < NV; i++) {
+    const double w = pm_group_sum<64>(v[i]);
+    if ((threadIdx.x & 63) == 63) sh[i][threadIdx.x >> 6] = w;
+  }
+  __syncthreads();
+  if (threadIdx.x < NV) {
+    double acc = sh[threadIdx.x][0];
+    for (int w = 1; w < PM_WAVES; w++) acc += sh[threadIdx.x][w];
+    partials[(size_t)blockIdx.x * NV + threadIdx.x] = acc;
+  }
+}
+
 // Scalars of the iteration that pass A starts: from the partials of pass B
 // of the last one (first: of the initial vectors), RPSQMR (Iters.f:6100-6436)
 // and PCG (Iters.f:299-595).  Called by whole workgroups; every thread
@@ -42,7 +85,7 @@ __device__ __forceinline__ PmIter pm_iter_begin(const PmIterState *st, int cur, 
   PmIter s = st->it[cur];
   if (first) {
     double r[2];
-    pm_sum_partials<2>(nblk, partials, r);
+    pm_sum_dots<2>(nblk, partials, r);
     s.v0 = s.t1 = s.t2 = s.beta = 0.0;
     s.resid = 0.0;
     s.done = s.pending = 0;
@@ -68,7 +111,7 @@ __device__ __forceinline__ PmIter pm_iter_begin(const PmIterState *st, int cur, 
     return s;
   }
   double r[2];
-  pm_sum_partials<2>(nblk, partials, r);
+  pm_sum_dots<2>(nblk, partials, r);
   if (MT == PM_IT_SQMR) {
     const double normr = sqrt(r[0]);
     const double vn = normr / s.tau;

@@ -75,7 +75,7 @@ __global__ __launch_bounds__(PM_WG) void k_stored_pass(
       }
     }
   }
-  pm_block_partials<1>(dot, pa);
+  pm_dots_partials<1>(dot, pa);
 }
 
 // ---------------------------------------------------------------------------
@@ -95,7 +95,7 @@ __global__ __launch_bounds__(PM_WG) void k_fused_init(int64_t n, const double *b
     v[0] += bi * bi;
     v[1] += bi * ti;
   }
-  pm_block_partials<2>(v, pb);
+  pm_dots_partials<2>(v, pb);
 }
 
 template <PmMethod MT>
@@ -112,7 +112,7 @@ __global__ __launch_bounds__(PM_WG) void k_fused_b(int64_t n, PmIterState *st, i
   const bool on = i < i1;
   double yi = on ? y[i] : 0.0, ri = on ? r[i] : 0.0, mi = on ? m[i] : 0.0;
   double sum[1];
-  pm_sum_partials<1>(nblk, pa, sum);
+  pm_sum_dots<1>(nblk, pa, sum);
   if (MT == PM_IT_SQMR && sum[0] == 0.0) {
     if (blockIdx.x == 0 && threadIdx.x == 0) st->step.broken = 1;
     return;
@@ -138,7 +138,7 @@ __global__ __launch_bounds__(PM_WG) void k_fused_b(int64_t n, PmIterState *st, i
       mi = m[i];
     }
   }
-  pm_block_partials<2>(v, pb);
+  pm_dots_partials<2>(v, pb);
 }
 
 // the update and the stop test of the last iteration launched
