@@ -18,11 +18,14 @@
 //
 // Four lanes take an element: lanes 0-2 one displacement component each, lane
 // 3 the pressure; the stress of a mode exchanges gradients inside the quad by
-// DPP.  Element vectors go to ye (one write) and a second kernel sums every
-// node's entries in a fixed order (one read): no atomics, no colours.
+// DPP.  A wavefront sums the vectors of 16 neighbouring elements in LDS and
+// writes the patch's nodes to ye; a second kernel sums every node's patches in
+// a fixed order: no colours, the same result every time.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <functional>
+#include <thread>
 
 #include "pm_affine.h"
 #include "pm_elemlib.h"
@@ -177,9 +180,12 @@ __device__ __forceinline__ void pm_modal_back(const double *f, double kap, doubl
 }
 
 struct AffineArgs {
-  int numel;
+  int npatch, max_nodes;
+  const int *ps;             // (npatch + 1) first slot of each patch
+  const unsigned int *pn;    // (npatch + 1) first entry of each patch in pw
+  const unsigned int *pw;    // free-dof words of the patches' nodes
+  const unsigned short *loc; // (numel, nen) patch node of each element node
   const int *ord;
-  const unsigned int *en;
   const double *ec;
   double *ye;
   const double *x;  // equation vector (OP)
@@ -193,11 +199,6 @@ struct AffineArgs {
 };
 
 enum { AF_OP = 0, AF_RHS2 = 1, AF_RHS4 = 2 };
-
-// offset of a node's values in an element's vector: vertices 4 values,
-// mid-edges 3
-__host__ __device__ constexpr int pm_ye_off(int k) { return k < 8 ? 4 * k : 32 + 3 * (k - 8); }
-__host__ __device__ constexpr int pm_ye_len(int nen) { return nen == 20 ? 68 : 32; }
 
 // One lane's share of an element vector: the nodal values v of component c (3:
 // pressure) become the nodal forces of K_e, or (AF_RHS4) of isw 4.
@@ -302,111 +303,158 @@ __device__ __forceinline__ void pm_element_vector(const AffineArgs &A, int slot,
   pm_modal_back<NEN>(f, kap, v);
 }
 
-template <int NEN>
-__device__ __forceinline__ void pm_store_element(double *ye, int slot, int c, const double *v) {
-  double *y = ye + (size_t)slot * pm_ye_len(NEN) + c;
-#pragma unroll
-  for (int k = 0; k < NEN; k++)
-    if (k < 8 || c < 3) y[pm_ye_off(k)] = v[k];
+// ---------------------------------------------------------------------------
+// patches
+// ---------------------------------------------------------------------------
+// A wavefront takes a patch of up to 16 elements (a brick of 4 x 2 x 2 in a
+// box).  It reads every node of the patch once into LDS, forms the element
+// vectors, adds them up in LDS and writes one vector per patch node, 2.3
+// (hexa20/8: 141 nodes for 320 element nodes) to 2.8 times (Q1/Q1: 45 for
+// 128) fewer values than element vectors are.  The additions are LDS atomics
+// in a fixed order: a wavefront's instructions execute in turn, and within
+// one no two elements share the node (checked when the patches are built).
+__device__ __forceinline__ void pm_wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
 }
 
-// the free-dof words of an element's nodes
-template <int NEN>
-__device__ __forceinline__ void pm_load_words(const unsigned int *en, int slot, unsigned int *w) {
-  const uint4 *wp = reinterpret_cast<const uint4 *>(en + (size_t)slot * NEN);
+// doubles of LDS a wavefront needs: the patch's nodes and a dummy for
+// restrained ones, four values each
+__host__ __device__ inline int pm_patch_lds(int max_nodes) { return (max_nodes + 1) * 4; }
+
+// buf holds the patch nodes' values (AF_OP) on entry and their sums on exit,
+// n4 = 4 * nodes values; written to ye
+template <int NEN, int MODE>
+__device__ __forceinline__ void pm_patch(const AffineArgs &A, int p, int lane, int n4, double *buf) {
+  const int c = lane & 3;
+  const int slot = A.ps[p] + (lane >> 2);
+  const bool on = slot < A.ps[p + 1];
+  double v[NEN], dpv[8];
+  int l[NEN];
+  if (on) {
+    const uint2 *lp = reinterpret_cast<const uint2 *>(A.loc + (size_t)slot * NEN);
 #pragma unroll
-  for (int k = 0; k < NEN / 4; k++) {
-    const uint4 q = wp[k];
-    w[4 * k] = q.x;
-    w[4 * k + 1] = q.y;
-    w[4 * k + 2] = q.z;
-    w[4 * k + 3] = q.w;
+    for (int k = 0; k < NEN / 4; k++) {
+      const uint2 q = lp[k];
+      l[4 * k] = (int)(q.x & 0xffffu) * 4 + c;
+      l[4 * k + 1] = (int)(q.x >> 16) * 4 + c;
+      l[4 * k + 2] = (int)(q.y & 0xffffu) * 4 + c;
+      l[4 * k + 3] = (int)(q.y >> 16) * 4 + c;
+    }
+    if constexpr (MODE == AF_OP) {
+#pragma unroll
+      for (int k = 0; k < NEN; k++) v[k] = buf[l[k]];
+    } else {
+      const int4 *np = reinterpret_cast<const int4 *>(A.ix + (size_t)A.ord[slot] * NEN);
+      int no[NEN];
+#pragma unroll
+      for (int k = 0; k < NEN / 4; k++) {
+        const int4 q = np[k];
+        no[4 * k] = q.x;
+        no[4 * k + 1] = q.y;
+        no[4 * k + 2] = q.z;
+        no[4 * k + 3] = q.w;
+      }
+#pragma unroll
+      for (int k = 0; k < NEN; k++) v[k] = (k < 8 || c < 3) ? A.u[(size_t)no[k] * 4 + c] : 0.0;
+      if constexpr (MODE == AF_RHS4)
+#pragma unroll
+        for (int k = 0; k < 8; k++) dpv[k] = A.dp[no[k]];
+    }
+    pm_element_vector<NEN, MODE>(A, slot, c, v, dpv);
   }
+  pm_wave_lds_fence();  // every element has its values: the buffer turns into the sums
+  for (int i = lane; i < n4 + 4; i += 64) buf[i] = 0.0;
+  pm_wave_lds_fence();
+  if (on) {
+#pragma unroll
+    for (int k = 0; k < NEN; k++)
+      if (k < 8 || c < 3)
+        __hip_atomic_fetch_add(&buf[l[k]], v[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+  }
+  pm_wave_lds_fence();
+  double *y = A.ye + (size_t)A.pn[p] * 4;
+  for (int i = lane; i < n4; i += 64) y[i] = buf[i];
+  pm_wave_lds_fence();
 }
 
-// Element vectors K_e x_e (AF_OP: x an equation vector, restrained dofs zero;
-// AF_RHS2: x the nodal state) or the isw 4 vectors (AF_RHS4).  Bound by the
-// gathers and the one write of the element vectors.
+// row of dof c in a free-dof word
+__device__ __forceinline__ unsigned int pm_word_row(unsigned int w, int c) {
+  return (w >> 4) + __popc(w & ((1u << c) - 1u));
+}
+
+// Patch vectors of K_e x_e (AF_OP: x an equation vector, restrained dofs
+// zero; AF_RHS2: the nodal state) or of isw 4 (AF_RHS4).
 template <int NEN, int MODE>
 __global__ __launch_bounds__(PM_WG) void k_affine_elements(AffineArgs A) {
   if (MODE == AF_OP && A.S != nullptr && A.S->done) return;
-  const int lb = pm_xcd_block(blockIdx.x, gridDim.x);
-  const int slot = lb * (PM_WG / 4) + (threadIdx.x >> 2);
-  if (slot >= A.numel) return;  // whole quads leave together
-  const int c = threadIdx.x & 3;
-  double v[NEN], dpv[8];
-  if constexpr (MODE == AF_OP) {
-    unsigned int w[NEN];
-    pm_load_words<NEN>(A.en, slot, w);
-    const unsigned int below = (1u << c) - 1u;
-#pragma unroll
-    for (int k = 0; k < NEN; k++) {
-      const unsigned int row = (w[k] >> 4) + __popc(w[k] & below);
-      v[k] = ((w[k] >> c) & 1u) ? A.x[row] : 0.0;
+  extern __shared__ double s_dyn[];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 3;
+  double *buf = s_dyn + (size_t)wave * pm_patch_lds(A.max_nodes);
+  const int p = pm_xcd_block(blockIdx.x, gridDim.x) * PM_WAVES + wave;
+  if (p >= A.npatch) return;
+  const unsigned int n0 = A.pn[p];
+  const int n4 = (int)(A.pn[p + 1] - n0) * 4;
+  if (MODE == AF_OP) {
+    for (int i = lane; i < n4 + 4; i += 64) {
+      const unsigned int w = i < n4 ? A.pw[n0 + (i >> 2)] : 0u;
+      buf[i] = ((w >> c) & 1u) ? A.x[pm_word_row(w, c)] : 0.0;
     }
-  } else {
-    const int4 *np = reinterpret_cast<const int4 *>(A.ix + (size_t)A.ord[slot] * NEN);
-    int no[NEN];
-#pragma unroll
-    for (int k = 0; k < NEN / 4; k++) {
-      const int4 q = np[k];
-      no[4 * k] = q.x;
-      no[4 * k + 1] = q.y;
-      no[4 * k + 2] = q.z;
-      no[4 * k + 3] = q.w;
-    }
-#pragma unroll
-    for (int k = 0; k < NEN; k++) v[k] = (k < 8 || c < 3) ? A.u[(size_t)no[k] * 4 + c] : 0.0;
-    if constexpr (MODE == AF_RHS4)
-#pragma unroll
-      for (int k = 0; k < 8; k++) dpv[k] = A.dp[no[k]];
+    pm_wave_lds_fence();
   }
-  pm_element_vector<NEN, MODE>(A, slot, c, v, dpv);
-  pm_store_element<NEN>(A.ye, slot, c, v);
+  pm_patch<NEN, MODE>(A, p, lane, n4, buf);
 }
 
-// Pass A of the fused iteration (pm_fused.h), element part: the element
-// vectors of q_new = t + beta q, formed at the gathered nodes.
+// Pass A of the fused iteration (pm_fused.h), element part: the patch vectors
+// of q_new = t + beta q.  The first patch's nodes are loaded while the scalars
+// are formed.
 template <int NEN, PmMethod MT>
 __global__ __launch_bounds__(PM_WG) void k_affine_pass_elements(AffineArgs A, PmVecs V,
                                                                 PmIterState *st, int cur,
                                                                 int first, double tol, int nblk,
                                                                 const double *pb) {
-  const int lb = pm_xcd_block(blockIdx.x, gridDim.x);
-  const int c = threadIdx.x & 3;
-  const unsigned int below = (1u << c) - 1u;
-  // contiguous tiles of 64 elements per workgroup
-  const int tiles = (A.numel + PM_WG / 4 - 1) / (PM_WG / 4);
-  int64_t t0, t1;
-  pm_chunk(tiles, lb, gridDim.x, t0, t1);
-  double tv[NEN], qv[NEN];
-  auto gather = [&](int64_t t) {
-    const int slot = (int)t * (PM_WG / 4) + (threadIdx.x >> 2);
-    if (t >= t1 || slot >= A.numel) return;
-    unsigned int w[NEN];
-    pm_load_words<NEN>(A.en, slot, w);
+  extern __shared__ double s_dyn[];
+  constexpr int NB = NEN == 20 ? 10 : 3;  // 160 or 48 nodes in registers
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 3;
+  double *buf = s_dyn + (size_t)wave * pm_patch_lds(A.max_nodes);
+  const int p = pm_xcd_block(blockIdx.x, gridDim.x) * PM_WAVES + wave;
+  const bool on = p < A.npatch;
+  const unsigned int n0 = on ? A.pn[p] : 0u;
+  const int n4 = on ? (int)(A.pn[p + 1] - n0) * 4 : 0;
+  double tv[NB], qv[NB];
+  unsigned int wv[NB];
 #pragma unroll
-    for (int k = 0; k < NEN; k++) {
-      const bool on = (w[k] >> c) & 1u;
-      const unsigned int row = on ? (w[k] >> 4) + __popc(w[k] & below) : 0u;
-      tv[k] = on ? V.t[row] : 0.0;
-      qv[k] = on ? V.q[row] : 0.0;
-    }
-  };
-  gather(t0);  // in flight while the scalars are formed
-  const PmIter s = pm_iter_begin<MT>(st, cur, first, tol, nblk, pb);
-  if (blockIdx.x == 0 && threadIdx.x == 0) st->it[cur ^ 1] = s;
-  if (s.done || s.pending) return;
-  for (int64_t t = t0; t < t1; t++) {
-    const int slot = (int)t * (PM_WG / 4) + (threadIdx.x >> 2);
-    if (slot >= A.numel) return;  // whole quads, in the last tile
-    if (t > t0) gather(t);
-    double v[NEN];
-#pragma unroll
-    for (int k = 0; k < NEN; k++) v[k] = tv[k] + s.beta * qv[k];
-    pm_element_vector<NEN, AF_OP>(A, slot, c, v, nullptr);
-    pm_store_element<NEN>(A.ye, slot, c, v);
+  for (int b = 0; b < NB; b++) {
+    // no branches around the loads: past the nodes lane 0's word, restrained
+    // dofs row 0, dropped below
+    const int i = b * 64 + lane;
+    wv[b] = A.pw[i < n4 ? n0 + (unsigned int)(i >> 2) : 0u];
   }
+#pragma unroll
+  for (int b = 0; b < NB; b++) {
+    const unsigned int row = (wv[b] >> c) & 1u ? pm_word_row(wv[b], c) : 0u;
+    tv[b] = V.t[row];
+    qv[b] = V.q[row];
+  }
+  double beta;
+  {
+    const PmIter s = pm_iter_begin<MT>(st, cur, first, tol, nblk, pb);
+    if (blockIdx.x == 0 && threadIdx.x == 0) st->it[cur ^ 1] = s;
+    if (s.done || s.pending || !on) return;
+    beta = s.beta;
+  }
+#pragma unroll
+  for (int b = 0; b < NB; b++) {
+    const int i = b * 64 + lane;
+    if (i < n4 + 4) buf[i] = i < n4 && ((wv[b] >> c) & 1u) ? tv[b] + beta * qv[b] : 0.0;
+  }
+  for (int i = NB * 64 + lane; i < n4 + 4; i += 64) {
+    const unsigned int w = i < n4 ? A.pw[n0 + (i >> 2)] : 0u;
+    const unsigned int row = pm_word_row(w, c);
+    buf[i] = ((w >> c) & 1u) ? V.t[row] + beta * V.q[row] : 0.0;
+  }
+  pm_wave_lds_fence();
+  pm_patch<NEN, AF_OP>(A, p, lane, n4, buf);
 }
 
 // element coefficients: geometry and material, dt folded in
@@ -459,12 +507,12 @@ __global__ __launch_bounds__(PM_WG) void k_affine_coefs(int numel, int nen, cons
 }
 
 // ---------------------------------------------------------------------------
-// sums of the element vectors per node
+// sums of the patch vectors per node
 // ---------------------------------------------------------------------------
-// Four lanes take a row block (a node) and sum its incidences, eight at a
-// time in a fixed tree; lane c holds dof c.  Every node has `stride` offsets
-// (8 in a box; the mid-edges' last four and a boundary node's missing ones
-// point to a zero), so their loads need no pointer first.
+// Four lanes take a row block (a node) and sum its patches' entries, eight at
+// a time in a fixed tree; lane c holds dof c.  Every node has `stride` offsets
+// (8 in a box, two or three of them used on average; the others point to a
+// zero), so their loads need no pointer first.
 struct GatherArgs {
   int nrn, stride;
   const unsigned int *gnode;  // (nrn) first row << 4 | free dofs
@@ -484,7 +532,7 @@ __device__ __forceinline__ double pm_gather_sum(const GatherArgs &G, int64_t k, 
     t[1] = G.ye[a.y + (unsigned int)c];
     t[2] = G.ye[a.z + (unsigned int)c];
     t[3] = G.ye[a.w + (unsigned int)c];
-    if (b.x != G.zero) {  // mid-edges have four at most
+    if (b.x != G.zero) {  // only the nodes of five patches and more
       t[4] = G.ye[b.x + (unsigned int)c];
       t[5] = G.ye[b.y + (unsigned int)c];
       t[6] = G.ye[b.z + (unsigned int)c];
@@ -556,6 +604,20 @@ __global__ __launch_bounds__(PM_WG) void k_affine_subtract(GatherArgs G, double 
   b[row] -= pm_gather_sum(G, k, c);
 }
 
+// b -= the face loads of each loaded node's elements, in list order
+__global__ __launch_bounds__(256) void k_face_subtract(int n4, const int *node, const int *ptr,
+                                                       const int *src, const double *fv,
+                                                       const int *eq, double *b) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= n4) return;
+  const int j = i >> 2, c = i & 3;
+  const int row = eq[(size_t)node[j] * 4 + c];
+  if (row < 0) return;
+  double s = 0.0;
+  for (int q = ptr[j]; q < ptr[j + 1]; q++) s += fv[(size_t)src[q] * 4 + c];
+  b[row] -= s;
+}
+
 // ---------------------------------------------------------------------------
 // the matrix, one row block per group of lanes
 // ---------------------------------------------------------------------------
@@ -577,7 +639,7 @@ struct RefTab {
 // multiply-adds a lane instead of 64 Gauss points'.
 template <int NEN>
 __global__ __launch_bounds__(PM_WG) void k_affine_matrix(
-    int nrn, int max_cols, int stride, unsigned int zero, const unsigned int *__restrict__ gsrc,
+    int nrn, int max_cols, int mstride, const unsigned int *__restrict__ minc,
     const unsigned int *__restrict__ gnode,
     const unsigned int *__restrict__ en, const double *__restrict__ ec,
     const double *__restrict__ tab, const int *__restrict__ nr,
@@ -614,12 +676,11 @@ __global__ __launch_bounds__(PM_WG) void k_affine_matrix(
     }
     return lo;
   };
-  for (int p = 0; p < stride; p++) {
-    const unsigned int src = gsrc[(size_t)k * stride + p];
-    if (src == zero) break;
-    const unsigned int slot = src / (unsigned int)pm_ye_len(NEN);
-    const int off = (int)(src - slot * (unsigned int)pm_ye_len(NEN));
-    const int a = off < 32 ? off >> 2 : 8 + (off - 32) / 3;  // the row's local node
+  for (int p = 0; p < mstride; p++) {
+    const unsigned int code = minc[(size_t)k * mstride + p];
+    if (code == 0xffffffffu) break;
+    const unsigned int slot = code >> 5;
+    const int a = (int)(code & 31u);  // the row's local node
     const double *eq = ec + (size_t)slot * PM_EC;
     double g[9];
 #pragma unroll
@@ -763,9 +824,9 @@ static std::vector<double> reference_integrals() {
 // ---------------------------------------------------------------------------
 void pm_affine_free(PmAffine *a) {
   if (!a) return;
-  for (void *p : {(void *)a->ord, (void *)a->en, (void *)a->gsrc, (void *)a->gnode,
-                  (void *)a->ec_op, (void *)a->ec, (void *)a->ye,
-                  (void *)a->slot, (void *)a->tab})
+  for (void *p : {(void *)a->ord, (void *)a->ps, (void *)a->pn, (void *)a->pw, (void *)a->loc,
+                  (void *)a->en, (void *)a->gsrc, (void *)a->gnode, (void *)a->minc,
+                  (void *)a->ec_op, (void *)a->ec, (void *)a->ye, (void *)a->tab})
     if (p) (void)hipFree(p);
   delete a;
 }
@@ -798,11 +859,106 @@ static bool is_parallelepiped(const int *v, const double *x) {
   return rest <= 1.0e-12 * lin;
 }
 
+// Slots and patches: the elements of each connected part of the mesh split in
+// two along its longest side (in mean element sizes), again and again, at
+// multiples of 16 elements, so that only a part's last patch is not full.
+static void element_patches(const PmHostMesh &m, const double *x, std::vector<int> &ord,
+                            std::vector<int> &ps) {
+  const int numel = m.numel, L = 16;
+  std::vector<float> cen((size_t)numel * 3);
+  double size[3] = {0, 0, 0};
+  std::vector<int> part((size_t)m.nnodev);
+  for (int n = 0; n < m.nnodev; n++) part[n] = n;
+  auto root = [&](int n) {
+    while (part[n] != n) n = part[n] = part[part[n]];
+    return n;
+  };
+  for (int e = 0; e < numel; e++) {
+    const int *v = m.ix20.data() + (size_t)e * 21;
+    const int r = root(v[0] - 1);
+    for (int k = 1; k < 8; k++) {
+      const int q = root(v[k] - 1);
+      if (q != r) part[q] = r;
+    }
+    for (int d = 0; d < 3; d++) {
+      double lo = x[(size_t)(v[0] - 1) * 3 + d], hi = lo, sum = 0.0;
+      for (int k = 0; k < 8; k++) {
+        const double xk = x[(size_t)(v[k] - 1) * 3 + d];
+        lo = std::min(lo, xk);
+        hi = std::max(hi, xk);
+        sum += xk;
+      }
+      cen[(size_t)e * 3 + d] = (float)(0.125 * sum);
+      size[d] += hi - lo;
+    }
+  }
+  for (int d = 0; d < 3; d++)
+    if (!(size[d] > 0.0)) size[d] = 1.0;
+  for (int e = 0; e < numel; e++)
+    for (int d = 0; d < 3; d++) cen[(size_t)e * 3 + d] *= (float)(numel / size[d]);
+  // parts in the order of their lowest equation, as the matrix has them
+  std::vector<int> key((size_t)m.nnodev, INT32_MAX);
+  for (int e = 0; e < numel; e++) {
+    int lo = INT32_MAX;
+    for (int k = 0; k < m.nen; k++)
+      for (int d = 0; d < 4; d++) {
+        const int q = m.id[(size_t)(m.ix20[(size_t)e * 21 + k] - 1) * 4 + d];
+        if (q > 0) lo = std::min(lo, q);
+      }
+    int &kr = key[root(m.ix20[(size_t)e * 21] - 1)];
+    kr = std::min(kr, lo);
+  }
+  ord.resize((size_t)numel);
+  std::vector<std::pair<int, int>> pk((size_t)numel);
+  for (int e = 0; e < numel; e++) {
+    const int r = root(m.ix20[(size_t)e * 21] - 1);
+    pk[e] = {key[r] == INT32_MAX ? INT32_MAX : key[r], r};
+    ord[e] = e;
+  }
+  std::stable_sort(ord.begin(), ord.end(), [&](int a, int b) { return pk[a] < pk[b]; });
+  std::function<void(int, int, int)> split = [&](int lo, int hi, int fork) {
+    const int n = hi - lo;
+    if (n <= L) return;
+    float mn[3] = {1e30f, 1e30f, 1e30f}, mx[3] = {-1e30f, -1e30f, -1e30f};
+    for (int i = lo; i < hi; i++)
+      for (int d = 0; d < 3; d++) {
+        const float v = cen[(size_t)ord[i] * 3 + d];
+        mn[d] = std::min(mn[d], v);
+        mx[d] = std::max(mx[d], v);
+      }
+    int ax = 0;
+    for (int d = 1; d < 3; d++)
+      if (mx[d] - mn[d] > (mx[ax] - mn[ax]) * 1.001f + 0.01f) ax = d;
+    const int mid = lo + ((n + L - 1) / L) / 2 * L;
+    std::nth_element(ord.begin() + lo, ord.begin() + mid, ord.begin() + hi, [&](int a, int b) {
+      const float va = cen[(size_t)a * 3 + ax], vb = cen[(size_t)b * 3 + ax];
+      return va != vb ? va < vb : a < b;
+    });
+    if (fork > 0 && n > 20000) {
+      std::thread t([&] { split(lo, mid, fork - 1); });
+      split(mid, hi, fork - 1);
+      t.join();
+    } else {
+      split(lo, mid, 0);
+      split(mid, hi, 0);
+    }
+  };
+  ps.assign(1, 0);
+  for (int a = 0; a < numel;) {
+    int b = a + 1;
+    while (b < numel && pk[ord[b]] == pk[ord[a]]) b++;
+    split(a, b, 3);
+    for (int q = a; q < b; q += L) ps.push_back(std::min(q + L, b));
+    a = b;
+  }
+}
+
 int pm_affine_setup(pm_ctx *c, const double *x, const PmHostPattern &pat) {
   const std::vector<int> &eq_block = pat.eq_block;
   const PmHostMesh &m = c->mesh;
   const int nen = m.nen, numel = m.numel, nrn = c->A.nrn;
-  if (m.neq >= (1 << 28) || (int64_t)numel * pm_ye_len(nen) + 4 >= ((int64_t)1 << 32)) return PM_OK;
+  if (m.neq >= (1 << 28) || (int64_t)numel * nen * 4 + 4 >= ((int64_t)1 << 32) || numel >= (1 << 27))
+    return PM_OK;
   for (int e = 0; e < numel; e++)
     if (!is_parallelepiped(m.ix20.data() + (size_t)e * 21, x)) return PM_OK;
   // each node's free dofs: first equation << 4 | mask, and its row block
@@ -827,50 +983,73 @@ int pm_affine_setup(pm_ctx *c, const double *x, const PmHostPattern &pat) {
   int max_cols = 0;
   for (int k = 0; k < nrn; k++)
     max_cols = std::max(max_cols, (int)(pat.colptr[k + 1] - pat.colptr[k]));
-  // slots: elements by their lowest equation
-  std::vector<int> key((size_t)numel), ord((size_t)numel);
-  {
-    std::vector<int> cnt((size_t)nrn + 2, 0);
-    for (int e = 0; e < numel; e++) {
-      int lo = nrn;
+  std::vector<int> ord, ps;
+  element_patches(m, x, ord, ps);
+  const int npatch = (int)ps.size() - 1;
+  // patch nodes in the order the elements meet them; restrained nodes share
+  // the dummy after the last
+  std::vector<unsigned int> en((size_t)numel * nen), pn((size_t)npatch + 1, 0), pw;
+  std::vector<int> pblock;  // row block of each entry of pw
+  std::vector<unsigned short> loc((size_t)numel * nen);
+  std::vector<int> at((size_t)m.nnode, -1), seen((size_t)m.nnode, -1);
+  std::vector<int> pcnt((size_t)nrn, 0), mcnt((size_t)nrn, 0);
+  int max_nodes = 0, step = 0;
+  pw.reserve((size_t)numel * nen / 2);
+  pblock.reserve((size_t)numel * nen / 2);
+  for (int p = 0; p < npatch; p++) {
+    const int n0 = (int)pw.size();
+    for (int s = ps[p]; s < ps[p + 1]; s++)
       for (int k = 0; k < nen; k++) {
-        const int b = block[m.ix20[(size_t)e * 21 + k] - 1];
-        if (b >= 0 && b < lo) lo = b;
+        const int n = m.ix20[(size_t)ord[s] * 21 + k] - 1;
+        en[(size_t)s * nen + k] = word[n];
+        if (block[n] < 0) continue;
+        mcnt[block[n]]++;
+        if (at[n] < n0) {
+          at[n] = (int)pw.size();
+          pw.push_back(word[n]);
+          pblock.push_back(block[n]);
+          pcnt[block[n]]++;
+        }
       }
-      key[e] = lo;
-      cnt[lo + 1]++;
-    }
-    for (int k = 0; k <= nrn; k++) cnt[k + 1] += cnt[k];
-    for (int e = 0; e < numel; e++) ord[cnt[key[e]]++] = e;
+    const int nn = (int)pw.size() - n0;
+    max_nodes = std::max(max_nodes, nn);
+    for (int k = 0; k < nen; k++, step++)
+      for (int s = ps[p]; s < ps[p + 1]; s++) {
+        const int n = m.ix20[(size_t)ord[s] * 21 + k] - 1;
+        loc[(size_t)s * nen + k] = (unsigned short)(block[n] < 0 ? nn : at[n] - n0);
+        if (seen[n] == step) return PM_OK;  // two elements add to a node at once
+        seen[n] = step;
+      }
+    pn[p + 1] = (unsigned int)pw.size();
   }
-  std::vector<unsigned int> en((size_t)numel * nen);
-  std::vector<int> cnt((size_t)nrn, 0);
-  for (int s = 0; s < numel; s++)
-    for (int k = 0; k < nen; k++) {
-      const int n = m.ix20[(size_t)ord[s] * 21 + k] - 1;
-      en[(size_t)s * nen + k] = word[n];
-      if (block[n] >= 0) cnt[block[n]]++;
-    }
-  const int stride = ((nrn > 0 ? *std::max_element(cnt.begin(), cnt.end()) : 0) + 3) & ~3;
-  if (stride > 32) return PM_OK;  // a fan of elements: keep the stored matrix
-  const unsigned int zero = (unsigned int)((size_t)numel * pm_ye_len(nen));
-  std::vector<unsigned int> gsrc((size_t)nrn * stride, zero);
-  std::fill(cnt.begin(), cnt.end(), 0);
+  auto widest = [](const std::vector<int> &v) {
+    return ((v.empty() ? 0 : *std::max_element(v.begin(), v.end())) + 3) & ~3;
+  };
+  const int stride = widest(pcnt), mstride = widest(mcnt);
+  if (stride > 32 || mstride > 32) return PM_OK;  // a fan of elements: keep the stored matrix
+  // LDS of a workgroup of patches: 64 KB (a brick's 141 nodes take 18 KB)
+  if ((size_t)pm_patch_lds(max_nodes) * PM_WAVES * sizeof(double) > 65536) return PM_OK;
+  const unsigned int zero = pn[npatch] * 4u;
+  std::vector<unsigned int> gsrc((size_t)nrn * stride, zero),
+      minc((size_t)nrn * mstride, 0xffffffffu);
+  std::fill(pcnt.begin(), pcnt.end(), 0);
+  std::fill(mcnt.begin(), mcnt.end(), 0);
+  for (size_t i = 0; i < pw.size(); i++)
+    gsrc[(size_t)pblock[i] * stride + pcnt[pblock[i]]++] = (unsigned int)i * 4u;
   for (int s = 0; s < numel; s++)
     for (int k = 0; k < nen; k++) {
       const int b = block[m.ix20[(size_t)ord[s] * 21 + k] - 1];
-      if (b >= 0)
-        gsrc[(size_t)b * stride + cnt[b]++] =
-            (unsigned int)((size_t)s * pm_ye_len(nen) + pm_ye_off(k));
+      if (b >= 0) minc[(size_t)b * mstride + mcnt[b]++] = ((unsigned int)s << 5) | (unsigned int)k;
     }
-  std::vector<int> slot((size_t)numel);
-  for (int s = 0; s < numel; s++) slot[ord[s]] = s;
   const std::vector<double> tab = nen == 20 ? reference_integrals<20>() : reference_integrals<8>();
   PmAffine *a = new PmAffine();
   a->max_cols = max_cols;
   a->stride = stride;
   a->zero = zero;
   a->numel = numel;
+  a->npatch = npatch;
+  a->max_nodes = max_nodes;
+  a->mstride = mstride;
   a->nen = nen;
   a->nrn = nrn;
   bool ok = true;
@@ -879,14 +1058,18 @@ int pm_affine_setup(pm_ctx *c, const double *x, const PmHostPattern &pat) {
          (!h || hipMemcpy(*d, h, bytes, hipMemcpyHostToDevice) == hipSuccess);
   };
   up((void **)&a->ord, ord.data(), sizeof(int) * ord.size());
+  up((void **)&a->ps, ps.data(), sizeof(int) * ps.size());
+  up((void **)&a->pn, pn.data(), sizeof(unsigned int) * pn.size());
+  up((void **)&a->pw, pw.data(), sizeof(unsigned int) * std::max<size_t>(pw.size(), 1));
+  up((void **)&a->loc, loc.data(), sizeof(unsigned short) * loc.size());
+  up((void **)&a->minc, minc.data(), sizeof(unsigned int) * std::max<size_t>(minc.size(), 1));
   up((void **)&a->en, en.data(), sizeof(unsigned int) * en.size());
   up((void **)&a->gsrc, gsrc.data(), sizeof(unsigned int) * gsrc.size());
   up((void **)&a->gnode, gnode.data(), sizeof(unsigned int) * gnode.size());
   up((void **)&a->ec_op, nullptr, sizeof(double) * PM_EC * (size_t)numel);
   up((void **)&a->ec, nullptr, sizeof(double) * PM_EC * (size_t)numel);
-  up((void **)&a->slot, slot.data(), sizeof(int) * slot.size());
   up((void **)&a->tab, tab.data(), sizeof(double) * tab.size());
-  // the element vectors, then four zeros for the gathers' missing entries
+  // the patch vectors, then four zeros for the gathers' missing entries
   up((void **)&a->ye, nullptr, sizeof(double) * ((size_t)zero + 4));
   ok = ok && hipMemset(a->ye + zero, 0, 4 * sizeof(double)) == hipSuccess;
   if (!ok) {  // the stored-matrix path needs none of this
@@ -921,21 +1104,30 @@ static GatherArgs gather_args(const pm_ctx *c) {
   return GatherArgs{a->nrn, a->stride, a->gnode, a->gsrc, a->ye, a->zero};
 }
 
+static size_t patch_lds(const PmAffine *a) {
+  return (size_t)pm_patch_lds(a->max_nodes) * PM_WAVES * sizeof(double);
+}
+
 template <int MODE>
 static void launch_elements(pm_ctx *c, AffineArgs A) {
-  const int g = ((A.numel + PM_WG / 4 - 1) / (PM_WG / 4) + 7) & ~7;
+  const int g = ((A.npatch + PM_WAVES - 1) / PM_WAVES + 7) & ~7;
+  const size_t lds = patch_lds(c->affine);
   if (c->affine->nen == 20)
-    hipLaunchKernelGGL((k_affine_elements<20, MODE>), dim3(g), dim3(PM_WG), 0, c->stream, A);
+    hipLaunchKernelGGL((k_affine_elements<20, MODE>), dim3(g), dim3(PM_WG), lds, c->stream, A);
   else
-    hipLaunchKernelGGL((k_affine_elements<8, MODE>), dim3(g), dim3(PM_WG), 0, c->stream, A);
+    hipLaunchKernelGGL((k_affine_elements<8, MODE>), dim3(g), dim3(PM_WG), lds, c->stream, A);
 }
 
 static AffineArgs affine_args(const pm_ctx *c) {
   AffineArgs A{};
   const PmAffine *a = c->affine;
-  A.numel = a->numel;
+  A.npatch = a->npatch;
+  A.max_nodes = a->max_nodes;
+  A.ps = a->ps;
+  A.pn = a->pn;
+  A.pw = a->pw;
+  A.loc = a->loc;
   A.ord = a->ord;
-  A.en = a->en;
   A.ye = a->ye;
   return A;
 }
@@ -979,14 +1171,13 @@ static int affine_pass(pm_ctx *c, const PmVecs &V, PmIterState *st, int cur, int
                        int nblk, const double *pb, double *pa) {
   AffineArgs A = affine_args(c);
   A.ec = c->affine->ec_op;
-  // at most 2048 workgroups: each sums the partials of pass B again
-  const int tiles = (A.numel + PM_WG / 4 - 1) / (PM_WG / 4);
-  const int ge = (std::min(tiles, PM_MAX_GRID) + 7) & ~7;
+  const int ge = ((A.npatch + PM_WAVES - 1) / PM_WAVES + 7) & ~7;
+  const size_t lds = patch_lds(c->affine);
   if (c->affine->nen == 20)
-    hipLaunchKernelGGL((k_affine_pass_elements<20, MT>), dim3(ge), dim3(PM_WG), 0, c->stream, A, V,
+    hipLaunchKernelGGL((k_affine_pass_elements<20, MT>), dim3(ge), dim3(PM_WG), lds, c->stream, A, V,
                        st, cur, first, tol, nblk, pb);
   else
-    hipLaunchKernelGGL((k_affine_pass_elements<8, MT>), dim3(ge), dim3(PM_WG), 0, c->stream, A, V,
+    hipLaunchKernelGGL((k_affine_pass_elements<8, MT>), dim3(ge), dim3(PM_WG), lds, c->stream, A, V,
                        st, cur, first, tol, nblk, pb);
   const GatherArgs G = gather_args(c);
   const int g = (std::min((G.nrn + PM_WG / 4 - 1) / (PM_WG / 4), PM_MAX_GRID) + 7) & ~7;
@@ -1031,15 +1222,16 @@ int pm_affine_pform(pm_ctx *c, const ElemArgs &E, int isw, int lhs, int rhs) {
     for (int d = 0; d < 3; d++) A.grav[d] = E.grav[d];
     if (isw == 2) launch_elements<AF_RHS2>(c, A);
     else launch_elements<AF_RHS4>(c, A);
-    if (isw == 4 && c->n_face_elems > 0) {
-      if (a->nen == 20)
-        PM_TRY(pm_hexa20_faces(E, c->n_face_elems, c->d_face_elems, a->slot, a->ye, c->stream));
-      else
-        PM_TRY(pm_q1_faces(E, c->n_face_elems, c->d_face_elems, a->slot, a->ye, c->stream));
-    }
     const GatherArgs G = gather_args(c);
     const int g = ((G.nrn + PM_WG / 4 - 1) / (PM_WG / 4) + 7) & ~7;
     hipLaunchKernelGGL(k_affine_subtract, dim3(g), dim3(PM_WG), 0, c->stream, G, E.b);
+    if (isw == 4 && c->n_face_elems > 0) {
+      if (a->nen == 20) PM_TRY(pm_hexa20_faces(E, c->n_face_elems, c->d_face_elems, c->d_face_vec, c->stream));
+      else PM_TRY(pm_q1_faces(E, c->n_face_elems, c->d_face_elems, c->d_face_vec, c->stream));
+      const int n4 = c->n_face_nodes * 4;
+      hipLaunchKernelGGL(k_face_subtract, dim3((n4 + 255) / 256), dim3(256), 0, c->stream, n4,
+                         c->d_face_node, c->d_face_ptr, c->d_face_src, c->d_face_vec, E.eq, E.b);
+    }
   }
   if (isw == 2 && lhs) {
     const int gr = PM_WG / (a->nen == 20 ? 64 : 32);
@@ -1047,11 +1239,11 @@ int pm_affine_pform(pm_ctx *c, const ElemArgs &E, int isw, int lhs, int rhs) {
     const size_t lds = matrix_lds(a);
     if (a->nen == 20)
       hipLaunchKernelGGL(k_affine_matrix<20>, g, dim3(PM_WG), lds, c->stream, a->nrn, a->max_cols,
-                         a->stride, a->zero, a->gsrc, a->gnode, a->en, ec, a->tab, M.nr, M.colptr, M.valptr,
+                         a->mstride, a->minc, a->gnode, a->en, ec, a->tab, M.nr, M.colptr, M.valptr,
                          M.ncol, M.val, E.err);
     else
       hipLaunchKernelGGL(k_affine_matrix<8>, g, dim3(PM_WG), lds, c->stream, a->nrn, a->max_cols,
-                         a->stride, a->zero, a->gsrc, a->gnode, a->en, ec, a->tab, M.nr, M.colptr, M.valptr,
+                         a->mstride, a->minc, a->gnode, a->en, ec, a->tab, M.nr, M.colptr, M.valptr,
                          M.ncol, M.val, E.err);
   }
   PM_CHECK_HIP(hipGetLastError());

@@ -84,6 +84,10 @@ pm_ctx::~pm_ctx() {
   FREE(d_e);
   FREE(d_eload);
   FREE(d_face_elems);
+  FREE(d_face_node);
+  FREE(d_face_ptr);
+  FREE(d_face_src);
+  FREE(d_face_vec);
   FREE(d_load);
   FREE(d_fload);
   FREE(d_colour_elems);
@@ -559,6 +563,32 @@ extern "C" int pm_set_materials(pm_ctx *c, int numat, const double *e, const int
   }
   PM_TRY(dupload(c, &c->d_face_elems, face_elems.data(), face_elems.size()));
   c->n_face_elems = (int)face_elems.size();
+  {
+    // the loaded elements' nodes and, per node, its entries in their vectors
+    const int nen = m.nen;
+    std::vector<int> at((size_t)m.nnode, -1), node, ptr(1, 0);
+    for (int el : face_elems)
+      for (int k = 0; k < nen; k++) {
+        const int n = m.ix20[(size_t)el * 21 + k] - 1;
+        if (at[n] < 0) {
+          at[n] = (int)node.size();
+          node.push_back(n);
+          ptr.push_back(0);
+        }
+        ptr[at[n] + 1]++;
+      }
+    for (size_t j = 1; j < ptr.size(); j++) ptr[j] += ptr[j - 1];
+    std::vector<int> src((size_t)ptr.back()), fill(ptr.begin(), ptr.end() - 1);
+    for (size_t i = 0; i < face_elems.size(); i++)
+      for (int k = 0; k < nen; k++)
+        src[fill[at[m.ix20[(size_t)face_elems[i] * 21 + k] - 1]]++] = (int)(i * nen + k);
+    c->n_face_nodes = (int)node.size();
+    PM_TRY(dupload(c, &c->d_face_node, node.data(), node.size()));
+    PM_TRY(dupload(c, &c->d_face_ptr, ptr.data(), ptr.size()));
+    PM_TRY(dupload(c, &c->d_face_src, src.data(), src.size()));
+    PM_TRY(dalloc(&c->d_face_vec, src.size() * 4));
+    PM_CHECK_HIP(hipStreamSynchronize(c->stream));
+  }
   for (int d = 0; d < 3; d++) c->gravity[d] = gravity ? gravity[d] : 0.0;
   c->gravity_mod = gravity_mod;
   // initial_porosity (Pform.f:1331-1376, run by the mesh macro, Main.f:820-828):

@@ -52,9 +52,6 @@ __device__ inline double dev_interpol(const double *xs, const double *ys, double
 int pm_q1_elements(const ElemArgs &A, int isw, hipStream_t stream);
 int pm_q1_porosity(const ElemArgs &A, double *dporo, hipStream_t stream);
 
-// face loads of the n elements in list, added to their element vectors
-// (vertices 4 values, mid-edges 3) at slot[element]
-int pm_hexa20_faces(const ElemArgs &A, int n, const int *list, const int *slot, double *ye,
-                    hipStream_t stream);
-int pm_q1_faces(const ElemArgs &A, int n, const int *list, const int *slot, double *ye,
-                hipStream_t stream);
+// face loads of the n elements in list: four values for every node of each
+int pm_hexa20_faces(const ElemArgs &A, int n, const int *list, double *fv, hipStream_t stream);
+int pm_q1_faces(const ElemArgs &A, int n, const int *list, double *fv, hipStream_t stream);

@@ -384,8 +384,7 @@ __device__ void face_loads(const ElemArgs &A, const int *iqm, const int *iqh,
 
 // face loads alone, one thread per loaded element (the elements of a face of
 // the mesh: few against the volume terms)
-__global__ __launch_bounds__(64) void k_faces20(ElemArgs A, int n, const int *list,
-                                                const int *slot, double *ye) {
+__global__ __launch_bounds__(64) void k_faces20(ElemArgs A, int n, const int *list, double *fv) {
   __shared__ double s_p[64][PM_NST + 1];
   const int i = blockIdx.x * 64 + threadIdx.x;
   if (i >= n) return;
@@ -398,17 +397,14 @@ __global__ __launch_bounds__(64) void k_faces20(ElemArgs A, int n, const int *li
   for (int j = 0; j < PM_NST; j++) p[j] = 0.0;
   const int *eq14 = A.eload + (size_t)el * 14;
   face_loads(A, eq14, eq14 + 7, xv, p);
-  double *y = ye + (size_t)slot[el] * PM_NST;
   for (int k = 0; k < 20; k++) {
-    double *yk = y + (k < 8 ? 4 * k : 32 + 3 * (k - 8));
-    for (int d = 0; d < 3; d++) yk[d] += p[3 * k + d];
-    if (k < 8) yk[3] += p[60 + k];
+    for (int d = 0; d < 3; d++) fv[((size_t)i * 20 + k) * 4 + d] = p[3 * k + d];
+    fv[((size_t)i * 20 + k) * 4 + 3] = k < 8 ? p[60 + k] : 0.0;
   }
 }
 
-int pm_hexa20_faces(const ElemArgs &A, int n, const int *list, const int *slot, double *ye,
-                    hipStream_t stream) {
-  hipLaunchKernelGGL(k_faces20, dim3((n + 63) / 64), dim3(64), 0, stream, A, n, list, slot, ye);
+int pm_hexa20_faces(const ElemArgs &A, int n, const int *list, double *fv, hipStream_t stream) {
+  hipLaunchKernelGGL(k_faces20, dim3((n + 63) / 64), dim3(64), 0, stream, A, n, list, fv);
   return hipGetLastError() == hipSuccess ? PM_OK : PM_ERR_HIP;
 }
 

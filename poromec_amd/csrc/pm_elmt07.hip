@@ -273,8 +273,7 @@ __device__ void q1_face_loads(const ElemArgs &A, const int *iqm, const int *iqh,
 }
 
 // face loads alone, one thread per loaded element
-__global__ __launch_bounds__(64) void k_q1_faces(ElemArgs A, int n, const int *list,
-                                                 const int *slot, double *ye) {
+__global__ __launch_bounds__(64) void k_q1_faces(ElemArgs A, int n, const int *list, double *fv) {
   __shared__ double s_p[64][Q1_NST + 1];
   const int i = blockIdx.x * 64 + threadIdx.x;
   if (i >= n) return;
@@ -287,16 +286,14 @@ __global__ __launch_bounds__(64) void k_q1_faces(ElemArgs A, int n, const int *l
   for (int j = 0; j < Q1_NST; j++) p[j] = 0.0;
   const int *eq14 = A.eload + (size_t)el * 14;
   q1_face_loads(A, eq14, eq14 + 7, xv, p);
-  double *y = ye + (size_t)slot[el] * Q1_NST;
   for (int k = 0; k < 8; k++) {
-    for (int d = 0; d < 3; d++) y[4 * k + d] += p[3 * k + d];
-    y[4 * k + 3] += p[24 + k];
+    for (int d = 0; d < 3; d++) fv[((size_t)i * 8 + k) * 4 + d] = p[3 * k + d];
+    fv[((size_t)i * 8 + k) * 4 + 3] = p[24 + k];
   }
 }
 
-int pm_q1_faces(const ElemArgs &A, int n, const int *list, const int *slot, double *ye,
-                hipStream_t stream) {
-  hipLaunchKernelGGL(k_q1_faces, dim3((n + 63) / 64), dim3(64), 0, stream, A, n, list, slot, ye);
+int pm_q1_faces(const ElemArgs &A, int n, const int *list, double *fv, hipStream_t stream) {
+  hipLaunchKernelGGL(k_q1_faces, dim3((n + 63) / 64), dim3(64), 0, stream, A, n, list, fv);
   return hipGetLastError() == hipSuccess ? PM_OK : PM_ERR_HIP;
 }
 

@@ -146,6 +146,10 @@ struct pm_ctx {
   int has_face_loads = 0;
   int *d_face_elems = nullptr;  // elements with face loads
   int n_face_elems = 0;
+  // their nodes, each node's entries in the face vectors (4 values each)
+  int n_face_nodes = 0;
+  int *d_face_node = nullptr, *d_face_ptr = nullptr, *d_face_src = nullptr;
+  double *d_face_vec = nullptr;
   int *d_load = nullptr;    // (200, 3)
   double *d_fload = nullptr;// (200, 5, 1000)
   std::vector<int> h_load;
