@@ -8,6 +8,7 @@
 struct PmAffine {
   int numel = 0, nen = 0, nrn = 0;
   int *ord = nullptr;            // (numel) element of each slot
+  int lpe = 4;                   // lanes an element: 64 / lpe elements a patch
   int npatch = 0, max_nodes = 0; // patches, most nodes in one
   int *ps = nullptr;             // (npatch + 1) first slot of each patch
   unsigned int *pn = nullptr;    // (npatch + 1) first entry of each patch in pw

@@ -12,15 +12,17 @@
 //   * a derivative moves a coefficient one degree down (P1' = P0, P2' = 3 P1),
 //   * the 4^3 (2^3) Gauss rule is exact for every product that occurs, so the
 //     17 derivative modes are orthogonal and D acts on each mode alone.
-// An element's K_e u_e is then ~600 FP64 operations per dof component instead
-// of the 64-point loops' ~2 million per element, and needs its 15
-// coefficients (128 B) instead of the matrix's 37 KB of stored values.
+// An element's K_e u_e is then ~2800 FP64 instructions (Q1/Q1 ~1300) instead
+// of the 64-point loops' ~2 million operations, and needs its 15 coefficients
+// (128 B) instead of the matrix's 37 KB of stored values.
 //
-// Four lanes take an element: lanes 0-2 one displacement component each, lane
-// 3 the pressure; the stress of a mode exchanges gradients inside the quad by
-// DPP.  A wavefront sums the vectors of 16 neighbouring elements in LDS and
-// writes the patch's nodes to ye; a second kernel sums every node's patches in
-// a fixed order: no colours, the same result every time.
+// In small meshes four lanes take an element: lanes 0-2 one displacement
+// component each, lane 3 the pressure; the stress of a mode exchanges
+// gradients inside the quad by DPP (6500 instructions per 64 elements, but
+// four times the wavefronts).  A wavefront sums the vectors of its 64 or 16
+// neighbouring elements in LDS and writes the patch's nodes to ye; a second
+// kernel sums every node's patches in a fixed order: no colours, the same
+// result every time.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -303,14 +305,231 @@ __device__ __forceinline__ void pm_element_vector(const AffineArgs &A, int slot,
   pm_modal_back<NEN>(f, kap, v);
 }
 
+// The same with one lane per element, all four components in its registers:
+// no exchanges, a quarter of the instructions per element; for meshes large
+// enough to fill the chip with 64 elements a wavefront.  x: 4 components of
+// every node on entry, the nodal forces on exit.  The transforms' 1/8 each way
+// and the modes' norms are folded into the material coefficients.
+template <int NEN>
+__device__ __forceinline__ void pm_modal_fwd8(const double *v, double *co) {  // 8 x coefficients
+  double h[8];
+  pm_hadamard8(v, h);
+  if constexpr (NEN == 20) {
+    double er[4], es[4], et[4];
+    pm_hadamard4(v[8], v[12], v[14], v[10], er);
+    pm_hadamard4(v[11], v[15], v[13], v[9], es);
+    pm_hadamard4(v[16], v[19], v[18], v[17], et);
+    double b[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) b[i] = h[i];
+    constexpr double k1 = 2.0 / 3.0, k2 = -4.0 / 3.0;
+#pragma unroll
+    for (int p = 0; p < 2; p++)
+#pragma unroll
+      for (int q = 0; q < 2; q++) {
+        const double c2 = fma(k2, er[q * 2 + p], k1 * h[0 * 4 + p * 2 + q]);
+        const double d2 = fma(k2, es[q * 2 + p], k1 * h[p * 4 + 0 * 2 + q]);
+        const double f2 = fma(k2, et[q * 2 + p], k1 * h[p * 4 + q * 2 + 0]);
+        co[pm_md(2, p, q)] = c2;
+        co[pm_md(p, 2, q)] = d2;
+        co[pm_md(p, q, 2)] = f2;
+        b[0 * 4 + p * 2 + q] -= c2;
+        b[p * 4 + 0 * 2 + q] -= d2;
+        b[p * 4 + q * 2 + 0] -= f2;
+      }
+#pragma unroll
+    for (int i = 0; i < 8; i++) h[i] = b[i];
+  }
+#pragma unroll
+  for (int i = 0; i < 8; i++) co[pm_md(i >> 2, (i >> 1) & 1, i & 1)] = h[i];
+}
+
+// 8 x the transpose
+template <int NEN>
+__device__ __forceinline__ void pm_modal_back8(const double *f, double *v) {
+  double h[8];
+#pragma unroll
+  for (int i = 0; i < 8; i++) h[i] = f[pm_md(i >> 2, (i >> 1) & 1, i & 1)];
+  if constexpr (NEN == 20) {
+    double base[8], er[4], es[4], et[4];
+#pragma unroll
+    for (int i = 0; i < 8; i++) base[i] = h[i];
+    constexpr double k1 = 2.0 / 3.0, k2 = -4.0 / 3.0;
+#pragma unroll
+    for (int p = 0; p < 2; p++)
+#pragma unroll
+      for (int q = 0; q < 2; q++) {
+        const double w1 = f[pm_md(2, p, q)] - base[0 * 4 + p * 2 + q];
+        const double w2 = f[pm_md(p, 2, q)] - base[p * 4 + 0 * 2 + q];
+        const double w3 = f[pm_md(p, q, 2)] - base[p * 4 + q * 2 + 0];
+        h[0 * 4 + p * 2 + q] = fma(k1, w1, h[0 * 4 + p * 2 + q]);
+        h[p * 4 + 0 * 2 + q] = fma(k1, w2, h[p * 4 + 0 * 2 + q]);
+        h[p * 4 + q * 2 + 0] = fma(k1, w3, h[p * 4 + q * 2 + 0]);
+        er[q * 2 + p] = k2 * w1;
+        es[q * 2 + p] = k2 * w2;
+        et[q * 2 + p] = k2 * w3;
+      }
+    auto edge = [](const double *e, double &pp, double &mp, double &mm, double &pm) {
+      const double a = e[0] + e[1], b = e[0] - e[1], c = e[2] + e[3], d = e[2] - e[3];
+      pp = a + c;
+      mp = a - c;
+      pm = b + d;
+      mm = b - d;
+    };
+    edge(er, v[8], v[12], v[14], v[10]);
+    edge(es, v[11], v[15], v[13], v[9]);
+    edge(et, v[16], v[19], v[18], v[17]);
+  }
+  pm_hadamard8t(h, v);
+}
+
+// adds v to f, or starts it
+__device__ __forceinline__ void pm_acc(bool &on, double &f, double k, double v) {
+  f = on ? fma(k, v, f) : k * v;
+  on = true;
+}
+
+template <int NEN, int MODE>
+__device__ __forceinline__ void pm_element_lane(const AffineArgs &A, int slot,
+                                                double (&x)[4][NEN], const double *dpv) {
+  const double *ec = A.ec + (size_t)slot * PM_EC;
+  double g[3][3];  // g[i][y] = d r_i / d y
+#pragma unroll
+  for (int i = 0; i < 3; i++)
+#pragma unroll
+    for (int y = 0; y < 3; y++) g[i][y] = ec[3 * i + y];
+  constexpr double s64 = 1.0 / 64.0;
+  const double cA = s64 * ec[9], cB = s64 * ec[10], cC = s64 * ec[11], cP = -s64 * ec[12];
+  const double cM = -s64 * ec[13], cK = -s64 * ec[14];
+  double co[4][27], f[4][27];
+#pragma unroll
+  for (int c = 0; c < 3; c++) pm_modal_fwd8<NEN>(x[c], co[c]);
+  pm_modal_fwd8<8>(x[3], co[3]);
+  double dpm[8];
+  if constexpr (MODE == AF_RHS4) pm_hadamard8(dpv, dpm);
+  bool fon[4][27];
+#pragma unroll
+  for (int c = 0; c < 4; c++)
+#pragma unroll
+    for (int i = 0; i < 27; i++) {
+      fon[c][i] = false;
+      f[c][i] = 0.0;
+    }
+  constexpr double nrm[3] = {2.0, 2.0 / 3.0, 2.0 / 5.0};
+#pragma unroll
+  for (int a = 0; a < 3; a++)
+#pragma unroll
+    for (int b = 0; b < 3; b++)
+#pragma unroll
+      for (int d = 0; d < 3; d++) {
+        if (!pm_is_mode<NEN>(a, b, d)) continue;
+        const int e[3] = {a, b, d};
+        const double nd = nrm[a] * nrm[b] * nrm[d];
+        const bool base = a < 2 && b < 2 && d < 2;
+        const int m = pm_md(a, b, d);
+        bool has[3], hasp[3];
+        int src[3];
+        double sc[3];
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+          const int q[3] = {a + (i == 0), b + (i == 1), d + (i == 2)};
+          has[i] = e[i] < 2 && pm_is_mode<NEN>(q[0], q[1], q[2]);
+          hasp[i] = e[i] < 1 && pm_is_mode<8>(q[0], q[1], q[2]);
+          src[i] = q[0] * 9 + q[1] * 3 + q[2];
+          sc[i] = e[i] == 1 ? 3.0 : 1.0;
+        }
+        const bool any = has[0] || has[1] || has[2];
+        double tr = 0.0;
+        if (any) {
+          double F[3][3];  // F[u][y] = d u / d y
+#pragma unroll
+          for (int u = 0; u < 3; u++) {
+            bool on[3] = {false, false, false};
+#pragma unroll
+            for (int i = 0; i < 3; i++) {
+              if (!has[i]) continue;
+              const double di = sc[i] == 1.0 ? co[u][src[i]] : sc[i] * co[u][src[i]];
+#pragma unroll
+              for (int y = 0; y < 3; y++) {
+                F[u][y] = on[y] ? fma(g[i][y], di, F[u][y]) : g[i][y] * di;
+                on[y] = true;
+              }
+            }
+          }
+          tr = F[0][0] + F[1][1] + F[2][2];
+          double T = (nd * cB) * tr;
+          if (base) T = fma(nd * cP, MODE == AF_RHS4 ? dpm[a * 4 + b * 2 + d] : co[3][m], T);
+          double S[3][3];
+#pragma unroll
+          for (int u = 0; u < 3; u++) S[u][u] = fma(nd * cA, F[u][u], T);
+          S[0][1] = S[1][0] = (nd * cC) * (F[0][1] + F[1][0]);
+          S[1][2] = S[2][1] = (nd * cC) * (F[1][2] + F[2][1]);
+          S[0][2] = S[2][0] = (nd * cC) * (F[0][2] + F[2][0]);
+#pragma unroll
+          for (int u = 0; u < 3; u++)
+#pragma unroll
+            for (int i = 0; i < 3; i++) {
+              if (!has[i]) continue;
+              const double q = fma(g[i][2], S[u][2], fma(g[i][1], S[u][1], g[i][0] * S[u][0]));
+              if (sc[i] == 1.0) {
+                f[u][src[i]] = fon[u][src[i]] ? f[u][src[i]] + q : q;
+                fon[u][src[i]] = true;
+              } else {
+                pm_acc(fon[u][src[i]], f[u][src[i]], sc[i], q);
+              }
+            }
+        }
+        if (hasp[0] || hasp[1] || hasp[2]) {
+          double P[3];
+          bool on = false;
+#pragma unroll
+          for (int i = 0; i < 3; i++) {
+            if (!hasp[i]) continue;
+#pragma unroll
+            for (int y = 0; y < 3; y++)
+              P[y] = on ? fma(g[i][y], co[3][src[i]], P[y]) : g[i][y] * co[3][src[i]];
+            on = true;
+          }
+#pragma unroll
+          for (int y = 0; y < 3; y++) P[y] *= nd * cK;
+          if (MODE == AF_RHS4 && a + b + d == 0) {  // gravity's flux dt perm rho_f g
+            const double *em = A.e + (size_t)A.mat[A.ord[slot]] * PM_PROP;
+            const double fd = nd * 0.125 * ec[14] * (em[6] * 1.0e-06);
+#pragma unroll
+            for (int y = 0; y < 3; y++) P[y] = fma(fd, A.grav[y], P[y]);
+          }
+#pragma unroll
+          for (int i = 0; i < 3; i++) {
+            if (!hasp[i]) continue;
+            const double q = fma(g[i][2], P[2], fma(g[i][1], P[1], g[i][0] * P[0]));
+            f[3][src[i]] = fon[3][src[i]] ? f[3][src[i]] + q : q;
+            fon[3][src[i]] = true;
+          }
+        }
+        if (base && MODE != AF_RHS4) {
+          pm_acc(fon[3][m], f[3][m], nd * cM, co[3][m]);
+          if (any) pm_acc(fon[3][m], f[3][m], nd * cP, tr);
+        }
+        if (MODE == AF_RHS4 && a + b + d == 0) {  // - rho g on the displacement rows
+          const double *em = A.e + (size_t)A.mat[A.ord[slot]] * PM_PROP;
+          const double w = -nd * 0.125 * ec[15] * (em[5] * 1.0e-06);
+#pragma unroll
+          for (int u = 0; u < 3; u++) pm_acc(fon[u][m], f[u][m], w, A.grav[u]);
+        }
+      }
+#pragma unroll
+  for (int c = 0; c < 3; c++) pm_modal_back8<NEN>(f[c], x[c]);
+  pm_modal_back8<8>(f[3], x[3]);
+}
+
 // ---------------------------------------------------------------------------
 // patches
 // ---------------------------------------------------------------------------
-// A wavefront takes a patch of up to 16 elements (a brick of 4 x 2 x 2 in a
-// box).  It reads every node of the patch once into LDS, forms the element
-// vectors, adds them up in LDS and writes one vector per patch node, 2.3
-// (hexa20/8: 141 nodes for 320 element nodes) to 2.8 times (Q1/Q1: 45 for
-// 128) fewer values than element vectors are.  The additions are LDS atomics
+// A wavefront takes a patch of up to 64 (16) elements, a brick of 4 x 4 x 4
+// (4 x 2 x 2) in a box.  It reads every node of the patch once into LDS, forms
+// the element vectors, adds them up in LDS and writes one vector per patch
+// node: 425 (141) nodes for 1280 (320) element nodes with hexa20/8, 125 (45)
+// for 512 (128) with Q1/Q1.  The additions are LDS atomics
 // in a fixed order: a wavefront's instructions execute in turn, and within
 // one no two elements share the node (checked when the patches are built).
 __device__ __forceinline__ void pm_wave_lds_fence() {
@@ -318,11 +537,16 @@ __device__ __forceinline__ void pm_wave_lds_fence() {
   __builtin_amdgcn_wave_barrier();
 }
 
+// wavefronts of a workgroup: two where a patch's nodes take 14 KB of LDS
+__host__ __device__ constexpr int pm_patch_waves(int nen, int lpe) {
+  return nen == 20 && lpe == 1 ? 2 : PM_WAVES;
+}
+
 // doubles of LDS a wavefront needs: the patch's nodes and a dummy for
 // restrained ones, four values each
 __host__ __device__ inline int pm_patch_lds(int max_nodes) { return (max_nodes + 1) * 4; }
 
-// buf holds the patch nodes' values (AF_OP) on entry and their sums on exit,
+// four lanes an element: buf holds the patch nodes' values (AF_OP) on entry and their sums on exit,
 // n4 = 4 * nodes values; written to ye
 template <int NEN, int MODE>
 __device__ __forceinline__ void pm_patch(const AffineArgs &A, int p, int lane, int n4, double *buf) {
@@ -378,46 +602,112 @@ __device__ __forceinline__ void pm_patch(const AffineArgs &A, int p, int lane, i
   pm_wave_lds_fence();
 }
 
+// One lane an element, 64 elements a patch.  buf is component-major here (ld values a component), so that the lanes' nodes fall
+// on different banks.
+template <int NEN, int MODE>
+__device__ __forceinline__ void pm_patch_lane(const AffineArgs &A, int p, int lane, int n4, int ld,
+                                              double *buf) {
+  const int slot = A.ps[p] + lane;
+  const bool on = slot < A.ps[p + 1];
+  double x[4][NEN], dpv[8];
+  int l[NEN];
+  if (on) {
+    const uint2 *lp = reinterpret_cast<const uint2 *>(A.loc + (size_t)slot * NEN);
+#pragma unroll
+    for (int k = 0; k < NEN / 4; k++) {
+      const uint2 q = lp[k];
+      l[4 * k] = (int)(q.x & 0xffffu);
+      l[4 * k + 1] = (int)(q.x >> 16);
+      l[4 * k + 2] = (int)(q.y & 0xffffu);
+      l[4 * k + 3] = (int)(q.y >> 16);
+    }
+    if constexpr (MODE == AF_OP) {
+#pragma unroll
+      for (int c = 0; c < 4; c++)
+#pragma unroll
+        for (int k = 0; k < (c < 3 ? NEN : 8); k++) x[c][k] = buf[c * ld + l[k]];
+    } else {
+      const int *no = A.ix + (size_t)A.ord[slot] * NEN;
+#pragma unroll
+      for (int k = 0; k < NEN; k++) {
+        const double2 *up = reinterpret_cast<const double2 *>(A.u + (size_t)no[k] * 4);
+        const double2 q0 = up[0], q1 = up[1];
+        x[0][k] = q0.x;
+        x[1][k] = q0.y;
+        x[2][k] = q1.x;
+        x[3][k] = q1.y;
+        if (MODE == AF_RHS4 && k < 8) dpv[k] = A.dp[no[k]];
+      }
+    }
+    pm_element_lane<NEN, MODE>(A, slot, x, dpv);
+  }
+  pm_wave_lds_fence();
+  for (int i = lane; i < 4 * ld; i += 64) buf[i] = 0.0;
+  pm_wave_lds_fence();
+  if (on) {
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+#pragma unroll
+      for (int k = 0; k < (c < 3 ? NEN : 8); k++)
+        __hip_atomic_fetch_add(&buf[c * ld + l[k]], x[c][k], __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_WAVEFRONT);
+  }
+  pm_wave_lds_fence();
+  double *y = A.ye + (size_t)A.pn[p] * 4;
+  for (int i = lane; i < n4; i += 64) y[i] = buf[(i & 3) * ld + (i >> 2)];
+  pm_wave_lds_fence();
+}
+
 // row of dof c in a free-dof word
 __device__ __forceinline__ unsigned int pm_word_row(unsigned int w, int c) {
   return (w >> 4) + __popc(w & ((1u << c) - 1u));
 }
 
+// place of value i = 4 * node + component in a patch's buffer
+template <int LPE>
+__device__ __forceinline__ int pm_at(int i, int ld) {
+  return LPE == 4 ? i : (i & 3) * ld + (i >> 2);
+}
+
 // Patch vectors of K_e x_e (AF_OP: x an equation vector, restrained dofs
-// zero; AF_RHS2: the nodal state) or of isw 4 (AF_RHS4).
-template <int NEN, int MODE>
-__global__ __launch_bounds__(PM_WG) void k_affine_elements(AffineArgs A) {
+// zero; AF_RHS2: the nodal state) or of isw 4 (AF_RHS4); LPE lanes an element.
+template <int NEN, int MODE, int LPE>
+__global__ __launch_bounds__(64 * pm_patch_waves(NEN, LPE)) void k_affine_elements(AffineArgs A) {
   if (MODE == AF_OP && A.S != nullptr && A.S->done) return;
   extern __shared__ double s_dyn[];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 3;
+  const int ld = A.max_nodes + 1;
   double *buf = s_dyn + (size_t)wave * pm_patch_lds(A.max_nodes);
-  const int p = pm_xcd_block(blockIdx.x, gridDim.x) * PM_WAVES + wave;
+  const int p = pm_xcd_block(blockIdx.x, gridDim.x) * pm_patch_waves(NEN, LPE) + wave;
   if (p >= A.npatch) return;
   const unsigned int n0 = A.pn[p];
   const int n4 = (int)(A.pn[p + 1] - n0) * 4;
   if (MODE == AF_OP) {
     for (int i = lane; i < n4 + 4; i += 64) {
       const unsigned int w = i < n4 ? A.pw[n0 + (i >> 2)] : 0u;
-      buf[i] = ((w >> c) & 1u) ? A.x[pm_word_row(w, c)] : 0.0;
+      buf[pm_at<LPE>(i, ld)] = ((w >> c) & 1u) ? A.x[pm_word_row(w, c)] : 0.0;
     }
     pm_wave_lds_fence();
   }
-  pm_patch<NEN, MODE>(A, p, lane, n4, buf);
+  if constexpr (LPE == 4) pm_patch<NEN, MODE>(A, p, lane, n4, buf);
+  else pm_patch_lane<NEN, MODE>(A, p, lane, n4, ld, buf);
 }
 
 // Pass A of the fused iteration (pm_fused.h), element part: the patch vectors
-// of q_new = t + beta q.  The first patch's nodes are loaded while the scalars
-// are formed.
-template <int NEN, PmMethod MT>
-__global__ __launch_bounds__(PM_WG) void k_affine_pass_elements(AffineArgs A, PmVecs V,
+// of q_new = t + beta q, a patch per wavefront.  The patch's nodes are loaded
+// while the scalars are formed.
+template <int NEN, PmMethod MT, int LPE>
+__global__ __launch_bounds__(64 * pm_patch_waves(NEN, LPE)) void k_affine_pass_elements(AffineArgs A, PmVecs V,
                                                                 PmIterState *st, int cur,
                                                                 int first, double tol, int nblk,
                                                                 const double *pb) {
   extern __shared__ double s_dyn[];
-  constexpr int NB = NEN == 20 ? 10 : 3;  // 160 or 48 nodes in registers
+  // nodes in registers, 16 a step: 160 or 48 (four lanes an element), 432 or 128
+  constexpr int NB = LPE == 4 ? (NEN == 20 ? 10 : 3) : (NEN == 20 ? 27 : 8);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 3;
+  const int ld = A.max_nodes + 1;
   double *buf = s_dyn + (size_t)wave * pm_patch_lds(A.max_nodes);
-  const int p = pm_xcd_block(blockIdx.x, gridDim.x) * PM_WAVES + wave;
+  const int p = pm_xcd_block(blockIdx.x, gridDim.x) * pm_patch_waves(NEN, LPE) + wave;
   const bool on = p < A.npatch;
   const unsigned int n0 = on ? A.pn[p] : 0u;
   const int n4 = on ? (int)(A.pn[p + 1] - n0) * 4 : 0;
@@ -438,7 +728,7 @@ __global__ __launch_bounds__(PM_WG) void k_affine_pass_elements(AffineArgs A, Pm
   }
   double beta;
   {
-    const PmIter s = pm_iter_begin<MT>(st, cur, first, tol, nblk, pb);
+    const PmIter s = pm_iter_begin<MT, pm_patch_waves(NEN, LPE)>(st, cur, first, tol, nblk, pb);
     if (blockIdx.x == 0 && threadIdx.x == 0) st->it[cur ^ 1] = s;
     if (s.done || s.pending || !on) return;
     beta = s.beta;
@@ -446,15 +736,17 @@ __global__ __launch_bounds__(PM_WG) void k_affine_pass_elements(AffineArgs A, Pm
 #pragma unroll
   for (int b = 0; b < NB; b++) {
     const int i = b * 64 + lane;
-    if (i < n4 + 4) buf[i] = i < n4 && ((wv[b] >> c) & 1u) ? tv[b] + beta * qv[b] : 0.0;
+    if (i < n4 + 4)
+      buf[pm_at<LPE>(i, ld)] = i < n4 && ((wv[b] >> c) & 1u) ? tv[b] + beta * qv[b] : 0.0;
   }
-  for (int i = NB * 64 + lane; i < n4 + 4; i += 64) {
+  for (int i = NB * 64 + lane; i < n4 + 4; i += 64) {  // a wider patch
     const unsigned int w = i < n4 ? A.pw[n0 + (i >> 2)] : 0u;
     const unsigned int row = pm_word_row(w, c);
-    buf[i] = ((w >> c) & 1u) ? V.t[row] + beta * V.q[row] : 0.0;
+    buf[pm_at<LPE>(i, ld)] = ((w >> c) & 1u) ? V.t[row] + beta * V.q[row] : 0.0;
   }
   pm_wave_lds_fence();
-  pm_patch<NEN, AF_OP>(A, p, lane, n4, buf);
+  if constexpr (LPE == 4) pm_patch<NEN, AF_OP>(A, p, lane, n4, buf);
+  else pm_patch_lane<NEN, AF_OP>(A, p, lane, n4, ld, buf);
 }
 
 // element coefficients: geometry and material, dt folded in
@@ -861,10 +1153,10 @@ static bool is_parallelepiped(const int *v, const double *x) {
 
 // Slots and patches: the elements of each connected part of the mesh split in
 // two along its longest side (in mean element sizes), again and again, at
-// multiples of 16 elements, so that only a part's last patch is not full.
-static void element_patches(const PmHostMesh &m, const double *x, std::vector<int> &ord,
+// multiples of L elements, so that only a part's last patch is not full.
+static void element_patches(const PmHostMesh &m, const double *x, int L, std::vector<int> &ord,
                             std::vector<int> &ps) {
-  const int numel = m.numel, L = 16;
+  const int numel = m.numel;
   std::vector<float> cen((size_t)numel * 3);
   double size[3] = {0, 0, 0};
   std::vector<int> part((size_t)m.nnodev);
@@ -984,7 +1276,12 @@ int pm_affine_setup(pm_ctx *c, const double *x, const PmHostPattern &pat) {
   for (int k = 0; k < nrn; k++)
     max_cols = std::max(max_cols, (int)(pat.colptr[k + 1] - pat.colptr[k]));
   std::vector<int> ord, ps;
-  element_patches(m, x, ord, ps);
+  // one lane an element from 50,000 elements (800 wavefronts): below, four
+  // times the wavefronts hide more latency.  SQMR iteration, four lanes / one:
+  // Q1/Q1 32^3 18.1 / 18.3 us, 40^3 24.1 / 22.9, 64^3 65.7 / 51.9; hexa20/8
+  // 24^3 21.1 / 26.1, 32^3 30.6 / 33.2, 40^3 50.8 / 46.4, 48^3 79.8 / 76.3.
+  const int lpe = numel >= 50000 ? 1 : 4;
+  element_patches(m, x, 64 / lpe, ord, ps);
   const int npatch = (int)ps.size() - 1;
   // patch nodes in the order the elements meet them; restrained nodes share
   // the dummy after the last
@@ -1027,8 +1324,9 @@ int pm_affine_setup(pm_ctx *c, const double *x, const PmHostPattern &pat) {
   };
   const int stride = widest(pcnt), mstride = widest(mcnt);
   if (stride > 32 || mstride > 32) return PM_OK;  // a fan of elements: keep the stored matrix
-  // LDS of a workgroup of patches: 64 KB (a brick's 141 nodes take 18 KB)
-  if ((size_t)pm_patch_lds(max_nodes) * PM_WAVES * sizeof(double) > 65536) return PM_OK;
+  // a workgroup of patches may ask for 64 KB of LDS (bricks take 27 KB at most)
+  if ((size_t)pm_patch_lds(max_nodes) * pm_patch_waves(nen, lpe) * sizeof(double) > 65536)
+    return PM_OK;
   const unsigned int zero = pn[npatch] * 4u;
   std::vector<unsigned int> gsrc((size_t)nrn * stride, zero),
       minc((size_t)nrn * mstride, 0xffffffffu);
@@ -1048,6 +1346,7 @@ int pm_affine_setup(pm_ctx *c, const double *x, const PmHostPattern &pat) {
   a->zero = zero;
   a->numel = numel;
   a->npatch = npatch;
+  a->lpe = lpe;
   a->max_nodes = max_nodes;
   a->mstride = mstride;
   a->nen = nen;
@@ -1105,17 +1404,22 @@ static GatherArgs gather_args(const pm_ctx *c) {
 }
 
 static size_t patch_lds(const PmAffine *a) {
-  return (size_t)pm_patch_lds(a->max_nodes) * PM_WAVES * sizeof(double);
+  return (size_t)pm_patch_lds(a->max_nodes) * pm_patch_waves(a->nen, a->lpe) * sizeof(double);
 }
 
 template <int MODE>
 static void launch_elements(pm_ctx *c, AffineArgs A) {
-  const int g = ((A.npatch + PM_WAVES - 1) / PM_WAVES + 7) & ~7;
+  const int pw = pm_patch_waves(c->affine->nen, c->affine->lpe);
+  const dim3 g(((A.npatch + pw - 1) / pw + 7) & ~7), bl(64 * pw);
   const size_t lds = patch_lds(c->affine);
-  if (c->affine->nen == 20)
-    hipLaunchKernelGGL((k_affine_elements<20, MODE>), dim3(g), dim3(PM_WG), lds, c->stream, A);
-  else
-    hipLaunchKernelGGL((k_affine_elements<8, MODE>), dim3(g), dim3(PM_WG), lds, c->stream, A);
+  auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, g, bl, lds, c->stream, A); };
+  if (c->affine->nen == 20) {
+    if (c->affine->lpe == 4) go(k_affine_elements<20, MODE, 4>);
+    else go(k_affine_elements<20, MODE, 1>);
+  } else {
+    if (c->affine->lpe == 4) go(k_affine_elements<8, MODE, 4>);
+    else go(k_affine_elements<8, MODE, 1>);
+  }
 }
 
 static AffineArgs affine_args(const pm_ctx *c) {
@@ -1171,14 +1475,19 @@ static int affine_pass(pm_ctx *c, const PmVecs &V, PmIterState *st, int cur, int
                        int nblk, const double *pb, double *pa) {
   AffineArgs A = affine_args(c);
   A.ec = c->affine->ec_op;
-  const int ge = ((A.npatch + PM_WAVES - 1) / PM_WAVES + 7) & ~7;
+  const int pw = pm_patch_waves(c->affine->nen, c->affine->lpe);
+  const dim3 ge(((A.npatch + pw - 1) / pw + 7) & ~7), bl(64 * pw);
   const size_t lds = patch_lds(c->affine);
-  if (c->affine->nen == 20)
-    hipLaunchKernelGGL((k_affine_pass_elements<20, MT>), dim3(ge), dim3(PM_WG), lds, c->stream, A, V,
-                       st, cur, first, tol, nblk, pb);
-  else
-    hipLaunchKernelGGL((k_affine_pass_elements<8, MT>), dim3(ge), dim3(PM_WG), lds, c->stream, A, V,
-                       st, cur, first, tol, nblk, pb);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, ge, bl, lds, c->stream, A, V, st, cur, first, tol, nblk, pb);
+  };
+  if (c->affine->nen == 20) {
+    if (c->affine->lpe == 4) go(k_affine_pass_elements<20, MT, 4>);
+    else go(k_affine_pass_elements<20, MT, 1>);
+  } else {
+    if (c->affine->lpe == 4) go(k_affine_pass_elements<8, MT, 4>);
+    else go(k_affine_pass_elements<8, MT, 1>);
+  }
   const GatherArgs G = gather_args(c);
   const int g = (std::min((G.nrn + PM_WG / 4 - 1) / (PM_WG / 4), PM_MAX_GRID) + 7) & ~7;
   hipLaunchKernelGGL(k_affine_pass_gather<MT>, dim3(g), dim3(PM_WG), 0, c->stream, G, V, st,

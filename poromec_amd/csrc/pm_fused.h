@@ -36,13 +36,13 @@ struct PmIterState {  // device
 // Sums of the partials of nblk workgroups, the same in every workgroup: as
 // pm_sum_partials, the wavefront sums by DPP instead of six LDS permutes each
 // (they sit on every pass's critical path).
-template <int NV>
+template <int NV, int WAVES = PM_WAVES>
 __device__ __forceinline__ void pm_sum_dots(int nblk, const double *partials, double *out) {
-  __shared__ double sh[NV][PM_WAVES];
+  __shared__ double sh[NV][WAVES];
   double acc[NV];
 #pragma unroll
   for (int i = 0; i < NV; i++) acc[i] = 0.0;
-  for (int b = threadIdx.x; b < nblk; b += PM_WG)
+  for (int b = threadIdx.x; b < nblk; b += WAVES * 64)
 #pragma unroll
     for (int i = 0; i < NV; i++) acc[i] += partials[(size_t)b * NV + i];
 #pragma unroll
@@ -54,7 +54,7 @@ __device__ __forceinline__ void pm_sum_dots(int nblk, const double *partials, do
 #pragma unroll
   for (int i = 0; i < NV; i++) {
     out[i] = sh[i][0];
-    for (int w = 1; w < PM_WAVES; w++) out[i] += sh[i][w];
+    for (int w = 1; w < WAVES; w++) out[i] += sh[i][w];
   }
 }
 
@@ -79,13 +79,13 @@ __device__ __forceinline__ void pm_dots_partials(const double *v, double *partia
 // of the last one (first: of the initial vectors), RPSQMR (Iters.f:6100-6436)
 // and PCG (Iters.f:299-595).  Called by whole workgroups; every thread
 // receives the same values.
-template <PmMethod MT>
+template <PmMethod MT, int WAVES = PM_WAVES>
 __device__ __forceinline__ PmIter pm_iter_begin(const PmIterState *st, int cur, int first, double tol,
                                                 int nblk, const double *partials) {
   PmIter s = st->it[cur];
   if (first) {
     double r[2];
-    pm_sum_dots<2>(nblk, partials, r);
+    pm_sum_dots<2, WAVES>(nblk, partials, r);
     s.v0 = s.t1 = s.t2 = s.beta = 0.0;
     s.resid = 0.0;
     s.done = s.pending = 0;
@@ -111,7 +111,7 @@ __device__ __forceinline__ PmIter pm_iter_begin(const PmIterState *st, int cur, 
     return s;
   }
   double r[2];
-  pm_sum_dots<2>(nblk, partials, r);
+  pm_sum_dots<2, WAVES>(nblk, partials, r);
   if (MT == PM_IT_SQMR) {
     const double normr = sqrt(r[0]);
     const double vn = normr / s.tau;

@@ -173,14 +173,15 @@ static int stored_pass(pm_ctx *c, const VT *val, const PmVecs &V, PmIterState *s
                        int first, double tol, int nblk, const double *pb, double *pa) {
   const PmDevMatrix &A = c->A;
   int g = (A.nrn + PM_WG / 64 - 1) / (PM_WG / 64);
-  g = (std::min(g, 1024) + 7) & ~7;
+  g = (std::min(g, PM_MAX_GRID) + 7) & ~7;
   hipLaunchKernelGGL((k_stored_pass<VT, 3, MT>), dim3(g), dim3(PM_WG), 0, c->stream, A.nrn, A.fr,
                      A.nr, A.colptr, A.valptr, A.ncol, val, V, st, cur, first, tol, nblk, pb, pa);
   return g;
 }
 
 // grid of the vector passes: a row per thread up to 512 workgroups (their
-// partials are summed by every workgroup of the next pass A), 1024 beyond
+// partials are summed by every workgroup of the next pass A; two rows a thread
+// measured the same, four 0.5-1 us an iteration more), 1024 beyond
 static int vec_grid(int64_t n) {
   const int64_t g = (n + PM_WG - 1) / PM_WG;
   return (int)((std::min<int64_t>(g, n > 2000000 ? 1024 : 512) + 7) & ~7);

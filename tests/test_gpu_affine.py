@@ -65,6 +65,38 @@ def test_element_loops(shape, nen):
     s.close()
 
 
+# one lane an element (from 50,000 on), the last patch one element short of
+# full: against the Gauss loops of the same mesh with a vertex moved by 1e-9
+# (no parallelepipeds any more; the entries move by ~1e-9 of the largest)
+@pytest.mark.parametrize("nen,shape", [(20, (37, 39, 35)), (8, (39, 37, 35))])
+def test_element_loops_one_lane(nen, shape):
+    from poromec_amd.solver import MefSolver
+    d = _deck(shape, nen)
+    assert d.numel > 50000
+    moved = dataclasses.replace(d, x=d.x.copy())
+    moved.x[d.nnodev // 2, 2] += 1e-9
+    out = []
+    rng = np.random.default_rng(12)
+    for deck in (d, moved):
+        s = MefSolver(deck)
+        if not out:
+            u = rng.standard_normal((s.nnode, 4)) * 1e-3
+            u[d.nnodev:, 3] = 0.0
+            dp = rng.standard_normal(s.nnode) * 1e-4
+            f = rng.standard_normal(s.neq)
+        s.set_state(u=u, u0=np.zeros_like(u), dp=dp, t=0.0)
+        s.set_vectors(b0=np.zeros(s.neq), b=np.zeros(s.neq))
+        s.pform(4, False, True, d.dt, 0.5, target="b0")
+        s.pform(2, True, True, d.dt, 0.5, target="b")
+        b0, b, _ = s.vectors()
+        out.append((b0, b, s.spmv(f)))
+        s.close()
+    for a, b in zip(*out):
+        scale = np.abs(b).max()
+        assert np.abs(a - b).max() <= 1e-7 * scale
+        assert np.median(np.abs(a - b)) <= 1e-14 * scale  # rows away from the vertex
+
+
 def _stored(s):
     """The same matrix in a context that has no elements."""
     from poromec_amd.solver import CsrcSolver
