@@ -26,6 +26,7 @@ struct PmAffine {
   double *ye = nullptr;          // patch vectors, 4 values a node
   double *tab = nullptr;         // reference integrals of the matrix
   int max_cols = 0;              // widest row block
+  std::vector<int> patch_block;  // (host) a row block of each patch, -1: no free node
   bool op_valid = false;         // ec_op holds the matrix's coefficients
 };
 

@@ -696,19 +696,19 @@ __global__ __launch_bounds__(64 * pm_patch_waves(NEN, LPE)) void k_affine_elemen
 // Pass A of the fused iteration (pm_fused.h), element part: the patch vectors
 // of q_new = t + beta q, a patch per wavefront.  The patch's nodes are loaded
 // while the scalars are formed.
-template <int NEN, PmMethod MT, int LPE>
-__global__ __launch_bounds__(64 * pm_patch_waves(NEN, LPE)) void k_affine_pass_elements(AffineArgs A, PmVecs V,
-                                                                PmIterState *st, int cur,
-                                                                int first, double tol, int nblk,
-                                                                const double *pb) {
+template <int NEN, PmMethod MT, int LPE, bool BATCH>
+__global__ __launch_bounds__(64 * pm_patch_waves(NEN, LPE)) void k_affine_pass_elements(
+    AffineArgs A, PmVecs V, PmIterState *st, int cur, int first, double tol, int nblk,
+    const double *pb, PmMap M) {
   extern __shared__ double s_dyn[];
   // nodes in registers, 16 a step: 160 or 48 (four lanes an element), 432 or 128
   constexpr int NB = LPE == 4 ? (NEN == 20 ? 10 : 3) : (NEN == 20 ? 27 : 8);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 3;
   const int ld = A.max_nodes + 1;
   double *buf = s_dyn + (size_t)wave * pm_patch_lds(A.max_nodes);
-  const int p = pm_xcd_block(blockIdx.x, gridDim.x) * pm_patch_waves(NEN, LPE) + wave;
-  const bool on = p < A.npatch;
+  const PmPart P = pm_part<BATCH, PM_PASS_ELEMS>(M, A.npatch, st, pb, nblk, nullptr);
+  const int p = (int)P.lo + P.wg * pm_patch_waves(NEN, LPE) + wave;
+  const bool on = p < P.hi;
   const unsigned int n0 = on ? A.pn[p] : 0u;
   const int n4 = on ? (int)(A.pn[p + 1] - n0) * 4 : 0;
   double tv[NB], qv[NB];
@@ -728,8 +728,9 @@ __global__ __launch_bounds__(64 * pm_patch_waves(NEN, LPE)) void k_affine_pass_e
   }
   double beta;
   {
-    const PmIter s = pm_iter_begin<MT, pm_patch_waves(NEN, LPE)>(st, cur, first, tol, nblk, pb);
-    if (blockIdx.x == 0 && threadIdx.x == 0) st->it[cur ^ 1] = s;
+    const PmIter s =
+        pm_iter_begin<MT, pm_patch_waves(NEN, LPE), BATCH>(P.st, cur, first, tol, P.nin, P.in);
+    if (P.wg == 0 && threadIdx.x == 0) P.st->it[cur ^ 1] = s;
     if (s.done || s.pending || !on) return;
     beta = s.beta;
   }
@@ -862,15 +863,15 @@ __global__ __launch_bounds__(PM_WG) void k_affine_gather(GatherArgs G, double *_
 }
 
 // Pass A, node part: y = A q_new with the row's update and the dot q_new . y
-template <PmMethod MT>
+template <PmMethod MT, bool BATCH>
 __global__ __launch_bounds__(PM_WG) void k_affine_pass_gather(GatherArgs G, PmVecs V,
-                                                              const PmIterState *st, int nxt,
-                                                              double *pa) {
-  const PmIter s = st->it[nxt];  // written by the element part
+                                                              PmIterState *st, int nxt, double *pa,
+                                                              PmMap M) {
+  const PmPart P = pm_part<BATCH, PM_PASS_NODES>(M, G.nrn, st, nullptr, 0, pa);
+  const PmIter s = P.st->it[nxt];  // written by the element part
   if (s.done) return;
-  const int lb = pm_xcd_block(blockIdx.x, gridDim.x);
   int64_t k0, k1;
-  pm_chunk(G.nrn, lb, gridDim.x, k0, k1);
+  pm_share(P, k0, k1);
   const int c = threadIdx.x & 3;
   double v[1] = {0.0};
   for (int64_t k = k0 + (threadIdx.x >> 2); k < k1; k += PM_WG / 4) {
@@ -883,7 +884,7 @@ __global__ __launch_bounds__(PM_WG) void k_affine_pass_gather(GatherArgs G, PmVe
     V.y[row] = y;
     v[0] += y * qn;
   }
-  pm_dots_partials<1>(v, pa);
+  pm_dots_partials<1>(v, P.out, P.slot);
 }
 
 __global__ __launch_bounds__(PM_WG) void k_affine_subtract(GatherArgs G, double *b) {
@@ -1290,6 +1291,7 @@ int pm_affine_setup(pm_ctx *c, const double *x, const PmHostPattern &pat) {
   std::vector<unsigned short> loc((size_t)numel * nen);
   std::vector<int> at((size_t)m.nnode, -1), seen((size_t)m.nnode, -1);
   std::vector<int> pcnt((size_t)nrn, 0), mcnt((size_t)nrn, 0);
+  std::vector<int> patch_block((size_t)npatch, -1);
   int max_nodes = 0, step = 0;
   pw.reserve((size_t)numel * nen / 2);
   pblock.reserve((size_t)numel * nen / 2);
@@ -1318,6 +1320,7 @@ int pm_affine_setup(pm_ctx *c, const double *x, const PmHostPattern &pat) {
         seen[n] = step;
       }
     pn[p + 1] = (unsigned int)pw.size();
+    patch_block[p] = nn > 0 ? pblock[n0] : -1;
   }
   auto widest = [](const std::vector<int> &v) {
     return ((v.empty() ? 0 : *std::max_element(v.begin(), v.end())) + 3) & ~3;
@@ -1347,6 +1350,7 @@ int pm_affine_setup(pm_ctx *c, const double *x, const PmHostPattern &pat) {
   a->numel = numel;
   a->npatch = npatch;
   a->lpe = lpe;
+  a->patch_block = std::move(patch_block);
   a->max_nodes = max_nodes;
   a->mstride = mstride;
   a->nen = nen;
@@ -1470,28 +1474,33 @@ int pm_affine_gather(pm_ctx *c, double *y, const double *w, const double *m, int
   return g;
 }
 
+// the element part's kernel for the mesh, called with it
+template <PmMethod MT, bool BATCH, class Go>
+static void pass_elements(const PmAffine *a, Go go) {
+  if (a->nen == 20) {
+    if (a->lpe == 4) go(k_affine_pass_elements<20, MT, 4, BATCH>);
+    else go(k_affine_pass_elements<20, MT, 1, BATCH>);
+  } else {
+    if (a->lpe == 4) go(k_affine_pass_elements<8, MT, 4, BATCH>);
+    else go(k_affine_pass_elements<8, MT, 1, BATCH>);
+  }
+}
+
 template <PmMethod MT>
 static int affine_pass(pm_ctx *c, const PmVecs &V, PmIterState *st, int cur, int first, double tol,
                        int nblk, const double *pb, double *pa) {
   AffineArgs A = affine_args(c);
   A.ec = c->affine->ec_op;
-  const int pw = pm_patch_waves(c->affine->nen, c->affine->lpe);
+  const int pw = pm_affine_patch_waves(c);
   const dim3 ge(((A.npatch + pw - 1) / pw + 7) & ~7), bl(64 * pw);
   const size_t lds = patch_lds(c->affine);
-  auto go = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, ge, bl, lds, c->stream, A, V, st, cur, first, tol, nblk, pb);
-  };
-  if (c->affine->nen == 20) {
-    if (c->affine->lpe == 4) go(k_affine_pass_elements<20, MT, 4>);
-    else go(k_affine_pass_elements<20, MT, 1>);
-  } else {
-    if (c->affine->lpe == 4) go(k_affine_pass_elements<8, MT, 4>);
-    else go(k_affine_pass_elements<8, MT, 1>);
-  }
+  pass_elements<MT, false>(c->affine, [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, ge, bl, lds, c->stream, A, V, st, cur, first, tol, nblk, pb, PmMap{});
+  });
   const GatherArgs G = gather_args(c);
   const int g = (std::min((G.nrn + PM_WG / 4 - 1) / (PM_WG / 4), PM_MAX_GRID) + 7) & ~7;
-  hipLaunchKernelGGL(k_affine_pass_gather<MT>, dim3(g), dim3(PM_WG), 0, c->stream, G, V, st,
-                     cur ^ 1, pa);
+  hipLaunchKernelGGL((k_affine_pass_gather<MT, false>), dim3(g), dim3(PM_WG), 0, c->stream, G, V,
+                     st, cur ^ 1, pa, PmMap{});
   return g;
 }
 
@@ -1499,6 +1508,46 @@ int pm_affine_pass(pm_ctx *c, PmMethod mt, const PmVecs &V, PmIterState *st, int
                    double tol, int nblk, const double *pb, double *pa) {
   return mt == PM_IT_SQMR ? affine_pass<PM_IT_SQMR>(c, V, st, cur, first, tol, nblk, pb, pa)
                           : affine_pass<PM_IT_PCG>(c, V, st, cur, first, tol, nblk, pb, pa);
+}
+
+template <PmMethod MT>
+static void affine_pass_boxes(pm_ctx *c, const PmVecs &V, PmIterState *st, int cur, int first,
+                              double tol, const double *pb, double *pa, const PmMap &elems,
+                              int n_elems, const PmMap &nodes, int n_nodes) {
+  AffineArgs A = affine_args(c);
+  A.ec = c->affine->ec_op;
+  const size_t lds = patch_lds(c->affine);
+  pass_elements<MT, true>(c->affine, [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(n_elems), dim3(64 * pm_affine_patch_waves(c)), lds, c->stream,
+                       A, V, st, cur, first, tol, 0, pb, elems);
+  });
+  hipLaunchKernelGGL((k_affine_pass_gather<MT, true>), dim3(n_nodes), dim3(PM_WG), 0, c->stream,
+                     gather_args(c), V, st, cur ^ 1, pa, nodes);
+}
+
+void pm_affine_pass_boxes(pm_ctx *c, PmMethod mt, const PmVecs &V, PmIterState *st, int cur,
+                          int first, double tol, const double *pb, double *pa, const PmMap &elems,
+                          int n_elems, const PmMap &nodes, int n_nodes) {
+  if (mt == PM_IT_SQMR)
+    affine_pass_boxes<PM_IT_SQMR>(c, V, st, cur, first, tol, pb, pa, elems, n_elems, nodes, n_nodes);
+  else
+    affine_pass_boxes<PM_IT_PCG>(c, V, st, cur, first, tol, pb, pa, elems, n_elems, nodes, n_nodes);
+}
+
+int pm_affine_patch_waves(const pm_ctx *c) { return pm_patch_waves(c->affine->nen, c->affine->lpe); }
+
+bool pm_affine_box_patches(const pm_ctx *c, const std::vector<int> &blk0, std::vector<int> &p0) {
+  const std::vector<int> &pb = c->affine->patch_block;
+  const int nbox = (int)blk0.size() - 1;
+  p0.assign(nbox + 1, 0);
+  int box = 0;
+  for (size_t p = 0; p < pb.size(); p++) {
+    if (pb[p] < 0) continue;  // no free node: with the patch before
+    if (pb[p] < blk0[box]) return false;  // patches out of the boxes' order
+    while (pb[p] >= blk0[box + 1]) p0[++box] = (int)p;
+  }
+  while (box < nbox) p0[++box] = (int)pb.size();
+  return true;
 }
 
 // LDS of a workgroup of k_affine_matrix: every group's rows and column list

@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "pm_functors.h"
+#include "pm_fused.h"
 #include "pm_spmv.h"
 
 struct PmBatch {
@@ -35,8 +36,10 @@ struct PmBatch {
   static constexpr int kGraphKey = 20;
   uintptr_t graph_key[kGraphKey] = {};
   int use_graph = 1;
+  PmFusedBoxes *fused = nullptr;  // solves through the elements
   int rebalance = 1;  // hand converged boxes' workgroups to the open ones
   ~PmBatch() {
+    pm_fused_boxes_free(fused);
     if (graph) (void)hipGraphExecDestroy(graph);
     (void)hipFree(d_wg_box);
     (void)hipFree(d_wg0);
@@ -409,6 +412,30 @@ int pm_batch_krylov(pm_ctx *c, int solver, int maxit, double tol, const double *
   if (solver != PM_SOLVER_SQMR && solver != PM_SOLVER_PCG) return PM_ERR_UNSUPPORTED;
   // the box ranges must describe the matrix the kernels are about to read
   if (B->eq0[B->nbox] != c->A.neq || B->blk0[B->nbox] != c->A.nrn) return PM_ERR_STATE;
+  {
+    std::vector<int> done;
+    std::vector<double> resid;
+    int launched = 0, usable = 0;
+    PM_TRY(pm_fused_batch_solve(c, &B->fused, B->eq0, B->blk0,
+                                solver == PM_SOLVER_SQMR ? PM_IT_SQMR : PM_IT_PCG, b, x, m, tol,
+                                maxit, use32, cap_stragglers, B->last_iters, done, resid, &launched,
+                                &usable));
+    if (usable) {
+      int worst = 0, maxiter = 0;
+      for (int k = 0; k < B->nbox; k++) {
+        if (done[k] < 0) worst = done[k];
+        else if (done[k] == 0 && worst == 0) worst = PM_ERR_MAXIT;
+        if (done[k] == 0) B->last_iters[k] = 0;  // as the open boxes of the loop below
+        maxiter = std::max(maxiter, B->last_iters[k]);
+        info->resid = k == 0 ? resid[k] : std::max(info->resid, resid[k]);
+        B->h_S[k].done = done[k];
+      }
+      (use32 ? info->spmv32 : info->spmv64) += launched;
+      info->iters += maxiter;
+      info->used_solver = solver;
+      return worst;
+    }
+  }
   PM_TRY(breset(c));
   if (solver == PM_SOLVER_PCG) {
     double *r = c->d_wk[0], *z = c->d_wk[1], *p = c->d_wk[2];

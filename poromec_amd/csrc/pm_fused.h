@@ -60,7 +60,7 @@ __device__ __forceinline__ void pm_sum_dots(int nblk, const double *partials, do
 
 // workgroup partials of NV dots, DPP sums
 template <int NV>
-__device__ __forceinline__ void pm_dots_partials(const double *v, double *partials) {
+__device__ __forceinline__ void pm_dots_partials(const double *v, double *partials, int wg) {
   __shared__ double sh[NV][PM_WAVES];
 #pragma unroll
   for (int i = 0; i < NV; i++) {
@@ -71,7 +71,7 @@ __device__ __forceinline__ void pm_dots_partials(const double *v, double *partia
   if (threadIdx.x < NV) {
     double acc = sh[threadIdx.x][0];
     for (int w = 1; w < PM_WAVES; w++) acc += sh[threadIdx.x][w];
-    partials[(size_t)blockIdx.x * NV + threadIdx.x] = acc;
+    partials[(size_t)wg * NV + threadIdx.x] = acc;
   }
 }
 
@@ -79,7 +79,7 @@ __device__ __forceinline__ void pm_dots_partials(const double *v, double *partia
 // of the last one (first: of the initial vectors), RPSQMR (Iters.f:6100-6436)
 // and PCG (Iters.f:299-595).  Called by whole workgroups; every thread
 // receives the same values.
-template <PmMethod MT, int WAVES = PM_WAVES>
+template <PmMethod MT, int WAVES = PM_WAVES, bool BATCH = false>
 __device__ __forceinline__ PmIter pm_iter_begin(const PmIterState *st, int cur, int first, double tol,
                                                 int nblk, const double *partials) {
   PmIter s = st->it[cur];
@@ -98,6 +98,10 @@ __device__ __forceinline__ PmIter pm_iter_begin(const PmIterState *st, int cur, 
       s.conv = tol * sqrt(fabs(r[1]));
       s.tau = 0.0;
       s.ro = r[1];
+    }
+    if (BATCH && r[0] == 0.0) {  // a box without load: x = 0
+      s.done = 1;
+      s.it = 0;
     }
     return s;
   }
@@ -158,6 +162,84 @@ __device__ __forceinline__ double pm_row_update(const PmVecs &V, const PmIter &s
   V.qn[i] = qn;
   return qn;
 }
+
+// The batching form: every box its own scalars, partials and workgroups.  A
+// pass's workgroups are listed in a map (x box, y the workgroup's number among
+// the box's, z their number) that holds the open boxes only; a box's own
+// numbers never change, so neither do its sums.
+struct PmBoxInfo {
+  int p0, p1, k0, k1, e0, e1;  // patches, row blocks, equations
+  int na, abase, nb, bbase;    // workgroups of passes A (node part) and B, first partials
+};
+struct PmMap {
+  const int4 *wg;
+  const PmBoxInfo *box;
+};
+
+// a workgroup's part of a pass: number `wg` of `nwg`, on items [lo, hi)
+struct PmPart {
+  int wg, nwg, slot;  // slot: of its partials
+  int64_t lo, hi;
+  PmIterState *st;
+  const double *in;
+  int nin;
+  double *out;
+};
+enum PmPass { PM_PASS_ELEMS, PM_PASS_NODES, PM_PASS_B };
+
+template <bool BATCH, PmPass PASS>
+__device__ __forceinline__ PmPart pm_part(const PmMap &M, int64_t n, PmIterState *st,
+                                          const double *in, int nin, double *out) {
+  if constexpr (BATCH) {
+    const int4 w = M.wg[blockIdx.x];
+    const PmBoxInfo B = M.box[w.x];
+    PmPart P{w.y, w.z, w.y, 0, 0, st + w.x, nullptr, 0, nullptr};
+    if (PASS == PM_PASS_ELEMS) {
+      P.lo = B.p0;
+      P.hi = B.p1;
+    } else if (PASS == PM_PASS_NODES) {
+      P.lo = B.k0;
+      P.hi = B.k1;
+    } else {
+      P.lo = B.e0;
+      P.hi = B.e1;
+    }
+    P.in = PASS == PM_PASS_B ? in + B.abase : in + 2 * B.bbase;
+    P.nin = PASS == PM_PASS_B ? B.na : B.nb;
+    P.out = PASS == PM_PASS_B ? out + 2 * B.bbase : out + B.abase;
+    return P;
+  } else {
+    return PmPart{pm_xcd_block(blockIdx.x, gridDim.x), (int)gridDim.x, (int)blockIdx.x, 0, n, st,
+                  in, nin, out};
+  }
+}
+// the part's contiguous share of its items
+__device__ __forceinline__ void pm_share(const PmPart &P, int64_t &a, int64_t &b) {
+  pm_chunk(P.hi - P.lo, P.wg, P.nwg, a, b);
+  a += P.lo;
+  b += P.lo;
+}
+
+// pass A of every open box through the elements: maps of the element and the
+// node part
+void pm_affine_pass_boxes(pm_ctx *c, PmMethod mt, const PmVecs &V, PmIterState *st, int cur,
+                          int first, double tol, const double *pb, double *pa, const PmMap &elems,
+                          int n_elems, const PmMap &nodes, int n_nodes);
+// patches of the row blocks [blk0[b], blk0[b + 1]); false if they do not split so
+bool pm_affine_box_patches(const pm_ctx *c, const std::vector<int> &blk0, std::vector<int> &p0);
+int pm_affine_patch_waves(const pm_ctx *c);
+
+struct PmFusedBoxes;  // buffers of the batched solve
+void pm_fused_boxes_free(PmFusedBoxes *f);
+// SQMR or PCG on every box (eq0, blk0: nbox + 1 first equations and blocks);
+// iters and done per box (1 converged, < 0 error, 0 open).  cap != 0: once
+// half the boxes have converged at iteration L, stop at 4 L.  *usable = 0 and
+// nothing done where the elements do not serve.
+int pm_fused_batch_solve(pm_ctx *c, PmFusedBoxes **fb, const std::vector<int> &eq0,
+                         const std::vector<int> &blk0, PmMethod mt, const double *b, double *x,
+                         const double *m, double tol, int maxit, int use32, int cap,
+                         std::vector<int> &iters, std::vector<int> &done,
+                         std::vector<double> &resid, int *launched, int *usable);
 
 // pass A through the elements (pm_affine.hip); returns the grid of its partials
 int pm_affine_pass(pm_ctx *c, PmMethod mt, const PmVecs &V, PmIterState *st, int cur, int first,

@@ -75,17 +75,20 @@ __global__ __launch_bounds__(PM_WG) void k_stored_pass(
       }
     }
   }
-  pm_dots_partials<1>(dot, pa);
+  pm_dots_partials<1>(dot, pa, blockIdx.x);
 }
 
 // ---------------------------------------------------------------------------
 // initial vectors and pass B
 // ---------------------------------------------------------------------------
+template <bool BATCH>
 __global__ __launch_bounds__(PM_WG) void k_fused_init(int64_t n, const double *b, const double *m,
                                                       double *x, double *r, double *t, double *q,
-                                                      double *d, double *pb) {
+                                                      double *d, double *pb, PmMap M) {
+  const PmPart P = pm_part<BATCH, PM_PASS_B>(M, n, nullptr, nullptr, 0, pb);
   double v[2] = {0.0, 0.0};
-  for (int64_t i = (int64_t)blockIdx.x * PM_WG + threadIdx.x; i < n; i += (int64_t)gridDim.x * PM_WG) {
+  const int64_t i0 = P.lo + (int64_t)P.slot * PM_WG + threadIdx.x;
+  for (int64_t i = i0; i < P.hi; i += (int64_t)P.nwg * PM_WG) {
     const double bi = b[i], ti = bi * m[i];
     x[i] = 0.0;
     r[i] = bi;
@@ -95,32 +98,34 @@ __global__ __launch_bounds__(PM_WG) void k_fused_init(int64_t n, const double *b
     v[0] += bi * bi;
     v[1] += bi * ti;
   }
-  pm_dots_partials<2>(v, pb);
+  pm_dots_partials<2>(v, P.out, P.slot);
 }
 
-template <PmMethod MT>
+template <PmMethod MT, bool BATCH>
 __global__ __launch_bounds__(PM_WG) void k_fused_b(int64_t n, PmIterState *st, int nxt, int nblk,
                                                    const double *pa, const double *y,
                                                    const double *m, const double *q, double *x,
-                                                   double *r, double *t, double *pb) {
-  const PmIter s = st->it[nxt];
+                                                   double *r, double *t, double *pb, PmMap M) {
+  const PmPart P = pm_part<BATCH, PM_PASS_B>(M, n, st, pa, nblk, pb);
+  const PmIter s = P.st->it[nxt];
   if (s.done || s.pending) return;
-  // XCD-contiguous chunks; the first row's loads do not wait for the sums
+  // contiguous shares; the first row's loads do not wait for the sums
   int64_t i0, i1;
-  pm_chunk(n, pm_xcd_block(blockIdx.x, gridDim.x), gridDim.x, i0, i1);
+  pm_share(P, i0, i1);
   int64_t i = i0 + threadIdx.x;
   const bool on = i < i1;
   double yi = on ? y[i] : 0.0, ri = on ? r[i] : 0.0, mi = on ? m[i] : 0.0;
   double sum[1];
-  pm_sum_dots<1>(nblk, pa, sum);
+  pm_sum_dots<1>(P.nin, P.in, sum);
+  const bool lead = P.wg == 0 && threadIdx.x == 0;
   if (MT == PM_IT_SQMR && sum[0] == 0.0) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) st->step.broken = 1;
+    if (lead) P.st->step.broken = 1;
     return;
   }
   const double alpha = s.ro / sum[0];
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    st->step.alpha = alpha;
-    st->step.broken = 0;
+  if (lead) {
+    P.st->step.alpha = alpha;
+    P.st->step.broken = 0;
   }
   double v[2] = {0.0, 0.0};
   while (i < i1) {
@@ -138,20 +143,27 @@ __global__ __launch_bounds__(PM_WG) void k_fused_b(int64_t n, PmIterState *st, i
       mi = m[i];
     }
   }
-  pm_dots_partials<2>(v, pb);
+  pm_dots_partials<2>(v, P.out, P.slot);
 }
 
 // the update and the stop test of the last iteration launched
-template <PmMethod MT>
+template <PmMethod MT, bool BATCH>
 __global__ __launch_bounds__(PM_WG) void k_fused_tail(int64_t n, PmVecs V, PmIterState *st, int cur,
-                                                      int nblk, const double *pb) {
-  PmIter s = pm_iter_begin<MT>(st, cur, 0, 0.0, nblk, pb);
+                                                      int nblk, const double *pb, PmMap M) {
+  PmPart P = pm_part<BATCH, PM_PASS_B>(M, n, st, pb, nblk, nullptr);
+  if (BATCH) {  // pass B's partials come in here
+    const PmBoxInfo B = M.box[M.wg[blockIdx.x].x];
+    P.in = pb + 2 * B.bbase;
+    P.nin = B.nb;
+  }
+  PmIter s = pm_iter_begin<MT>(P.st, cur, 0, 0.0, P.nin, P.in);
   const bool update = !s.done;
   if (s.pending) s.done = s.pending;
-  if (blockIdx.x == 0 && threadIdx.x == 0) st->it[cur ^ 1] = s;
+  if (P.wg == 0 && threadIdx.x == 0) P.st->it[cur ^ 1] = s;
   if (!update) return;
-  for (int64_t i = (int64_t)blockIdx.x * PM_WG + threadIdx.x; i < n; i += (int64_t)gridDim.x * PM_WG)
-    (void)pm_row_update<MT>(V, s, i);
+  int64_t i0, i1;
+  pm_share(P, i0, i1);
+  for (int64_t i = i0 + threadIdx.x; i < i1; i += PM_WG) (void)pm_row_update<MT>(V, s, i);
 }
 
 // ---------------------------------------------------------------------------
@@ -197,8 +209,8 @@ static int solve(pm_ctx *c, int n, const double *b, double *x, const double *m, 
   *converged = 0;
   const bool elems = pm_affine_product(c, use32);
   const int gv = vec_grid(n);
-  hipLaunchKernelGGL(k_fused_init, dim3(gv), dim3(PM_WG), 0, c->stream, (int64_t)n, b, m, x, r, t,
-                     q[0], d, pb);
+  hipLaunchKernelGGL(k_fused_init<false>, dim3(gv), dim3(PM_WG), 0, c->stream, (int64_t)n, b, m, x,
+                     r, t, q[0], d, pb, PmMap{});
   int launched = 0;
   PmIter h{};
   while (launched < maxit) {
@@ -213,16 +225,16 @@ static int solve(pm_ctx *c, int n, const double *b, double *x, const double *m, 
           : use32 ? stored_pass<float, MT>(c, c->A.val32, V, st, cur, it == 0, tol, gv, pb, pa)
                   : stored_pass<double, MT>(c, c->A.val, V, st, cur, it == 0, tol, gv, pb, pa);
       pm_spmv_time_end(c, use32);
-      hipLaunchKernelGGL(k_fused_b<MT>, dim3(gv), dim3(PM_WG), 0, c->stream, (int64_t)n, st,
-                         cur ^ 1, ga, pa, y, m, V.qn, x, r, t, pb);
+      hipLaunchKernelGGL((k_fused_b<MT, false>), dim3(gv), dim3(PM_WG), 0, c->stream, (int64_t)n,
+                         st, cur ^ 1, ga, pa, y, m, V.qn, x, r, t, pb, PmMap{});
       (use32 ? info->spmv32 : info->spmv64)++;
     }
     launched += chunk;
     int last = launched & 1;  // slot written by the last pass A
     if (launched >= maxit) {
       const PmVecs V{t, q[last], q[last ^ 1], d, x, y};
-      hipLaunchKernelGGL(k_fused_tail<MT>, dim3(gv), dim3(PM_WG), 0, c->stream, (int64_t)n, V, st,
-                         last, gv, pb);
+      hipLaunchKernelGGL((k_fused_tail<MT, false>), dim3(gv), dim3(PM_WG), 0, c->stream, (int64_t)n,
+                         V, st, last, gv, pb, PmMap{});
       last ^= 1;
     }
     PM_CHECK_HIP(hipGetLastError());
@@ -248,4 +260,172 @@ int pm_fused_solve(pm_ctx *c, PmMethod mt, int n, const double *b, double *x, co
                    double tol, int maxit, int use32, pm_solve_info *info, int *converged) {
   return mt == PM_IT_SQMR ? solve<PM_IT_SQMR>(c, n, b, x, m, tol, maxit, use32, info, converged)
                           : solve<PM_IT_PCG>(c, n, b, x, m, tol, maxit, use32, info, converged);
+}
+
+// ---------------------------------------------------------------------------
+// every box of a batch its own solve
+// ---------------------------------------------------------------------------
+struct PmFusedBoxes {
+  int nbox = 0;
+  std::vector<PmBoxInfo> box;
+  PmBoxInfo *d_box = nullptr;
+  int4 *d_wg = nullptr;  // the three maps, one after the other
+  size_t wg_cap = 0;
+  PmIterState *d_st = nullptr, *h_st = nullptr;
+  double *d_part = nullptr;
+  size_t pa_len = 0;
+  ~PmFusedBoxes() {
+    (void)hipFree(d_box);
+    (void)hipFree(d_wg);
+    (void)hipFree(d_st);
+    (void)hipFree(d_part);
+    if (h_st) (void)hipHostFree(h_st);
+  }
+};
+
+void pm_fused_boxes_free(PmFusedBoxes *f) { delete f; }
+
+static int boxes_setup(pm_ctx *c, PmFusedBoxes **fb, const std::vector<int> &eq0,
+                       const std::vector<int> &blk0) {
+  std::vector<int> p0;
+  if (!pm_affine_box_patches(c, blk0, p0)) return PM_OK;
+  const int nbox = (int)eq0.size() - 1, pw = pm_affine_patch_waves(c);
+  PmFusedBoxes *f = new PmFusedBoxes();
+  f->nbox = nbox;
+  f->box.resize(nbox);
+  size_t na = 0, nb = 0, ne = 0;
+  for (int b = 0; b < nbox; b++) {
+    PmBoxInfo &B = f->box[b];
+    B.p0 = p0[b];
+    B.p1 = p0[b + 1];
+    B.k0 = blk0[b];
+    B.k1 = blk0[b + 1];
+    B.e0 = eq0[b];
+    B.e1 = eq0[b + 1];
+    // as in the single solve: 64 nodes and a row per thread a workgroup, up
+    // to 256 and 128 workgroups a box
+    B.na = std::min(256, std::max(1, (B.k1 - B.k0 + PM_WG / 4 - 1) / (PM_WG / 4)));
+    B.nb = std::min(128, std::max(1, (B.e1 - B.e0 + PM_WG - 1) / PM_WG));
+    B.abase = (int)na;
+    B.bbase = (int)nb;
+    na += B.na;
+    nb += B.nb;
+    ne += std::max(1, (B.p1 - B.p0 + pw - 1) / pw);
+  }
+  f->pa_len = na;
+  f->wg_cap = ne + na + nb;
+  bool ok = hipMalloc((void **)&f->d_box, sizeof(PmBoxInfo) * nbox) == hipSuccess &&
+            hipMalloc((void **)&f->d_wg, sizeof(int4) * f->wg_cap) == hipSuccess &&
+            hipMalloc((void **)&f->d_st, sizeof(PmIterState) * nbox) == hipSuccess &&
+            hipMalloc((void **)&f->d_part, sizeof(double) * (na + 2 * nb)) == hipSuccess &&
+            hipHostMalloc((void **)&f->h_st, sizeof(PmIterState) * nbox, hipHostMallocDefault) ==
+                hipSuccess &&
+            hipMemcpy(f->d_box, f->box.data(), sizeof(PmBoxInfo) * nbox, hipMemcpyHostToDevice) ==
+                hipSuccess;
+  if (!ok) {  // the stored-matrix batch needs none of this
+    (void)hipGetLastError();
+    delete f;
+    return PM_OK;
+  }
+  *fb = f;
+  return PM_OK;
+}
+
+template <PmMethod MT>
+static int batch_solve(pm_ctx *c, PmFusedBoxes *f, const double *b, double *x, const double *m,
+                       double tol, int maxit, int use32, int cap, std::vector<int> &iters,
+                       std::vector<int> &done, std::vector<double> &resid, int *out_launched) {
+  double *y = c->d_wk[0], *r = c->d_wk[1], *t = c->d_wk[2], *d = c->d_wk[3];
+  double *q[2] = {c->d_wk[4], c->d_wk[5]};
+  double *pa = f->d_part, *pb = f->d_part + f->pa_len;
+  const int nbox = f->nbox, pw = pm_affine_patch_waves(c);
+  PmIterState *st = f->d_st;
+  done.assign(nbox, 0);
+  iters.assign(nbox, 0);
+  resid.assign(nbox, 0.0);
+  // maps of the open boxes' workgroups; a box keeps its own numbers
+  PmMap me{nullptr, f->d_box}, mn = me, mb = me;
+  int ne = 0, nn = 0, nv = 0;
+  auto build = [&]() -> int {
+    std::vector<int4> w;
+    for (int pass = 0; pass < 3; pass++) {
+      const size_t at = w.size();
+      for (int k = 0; k < nbox; k++) {
+        if (done[k]) continue;
+        const PmBoxInfo &B = f->box[k];
+        const int g = pass == 0 ? std::max(1, (B.p1 - B.p0 + pw - 1) / pw) : pass == 1 ? B.na : B.nb;
+        for (int i = 0; i < g; i++) w.push_back(int4{k, i, g, 0});
+      }
+      (pass == 0 ? me : pass == 1 ? mn : mb).wg = f->d_wg + at;
+      (pass == 0 ? ne : pass == 1 ? nn : nv) = (int)(w.size() - at);
+    }
+    if (!w.empty())
+      PM_CHECK_HIP(hipMemcpy(f->d_wg, w.data(), sizeof(int4) * w.size(), hipMemcpyHostToDevice));
+    return PM_OK;
+  };
+  PM_TRY(build());
+  hipLaunchKernelGGL(k_fused_init<true>, dim3(nv), dim3(PM_WG), 0, c->stream, (int64_t)0, b, m, x, r,
+                     t, q[0], d, pb, mb);
+  int launched = 0, open = nbox, open_last = nbox, half_at = -1;
+  while (open > 0 && launched < maxit) {
+    if (cap && half_at >= 0 && launched >= 4 * std::max(half_at, 64)) break;
+    const int chunk = std::min(launched < 32 ? 8 : 32, maxit - launched);
+    for (int k = 0; k < chunk; k++) {
+      const int it = launched + k, cur = it & 1;
+      const PmVecs V{t, q[cur], q[cur ^ 1], d, x, y};
+      pm_affine_pass_boxes(c, MT, V, st, cur, it == 0, tol, pb, pa, me, ne, mn, nn);
+      hipLaunchKernelGGL((k_fused_b<MT, true>), dim3(nv), dim3(PM_WG), 0, c->stream, (int64_t)0, st,
+                         cur ^ 1, 0, pa, y, m, V.qn, x, r, t, pb, mb);
+    }
+    launched += chunk;
+    int last = launched & 1;
+    const bool end = launched >= maxit ||
+                     (cap && half_at >= 0 && launched >= 4 * std::max(half_at, 64));
+    if (end) {
+      const PmVecs V{t, q[last], q[last ^ 1], d, x, y};
+      hipLaunchKernelGGL((k_fused_tail<MT, true>), dim3(nv), dim3(PM_WG), 0, c->stream, (int64_t)0,
+                         V, st, last, 0, pb, mb);
+      last ^= 1;
+    }
+    PM_CHECK_HIP(hipGetLastError());
+    PM_CHECK_HIP(hipMemcpyAsync(f->h_st, st, sizeof(PmIterState) * nbox, hipMemcpyDeviceToHost,
+                                c->stream));
+    PM_CHECK_HIP(hipStreamSynchronize(c->stream));
+    double worst = 0.0;
+    for (int k = 0; k < nbox; k++) {
+      if (done[k]) continue;
+      const PmIter &s = f->h_st[k].it[last];
+      iters[k] = s.it;
+      resid[k] = s.resid;
+      worst = std::max(worst, s.resid);
+      done[k] = s.done ? s.done : s.pending;  // pending: the last pass A made the update
+      open -= done[k] != 0;
+    }
+    pm_progress(launched, worst);
+    if (half_at < 0 && 2 * (nbox - open) >= nbox) half_at = launched;
+    if (end) break;
+    // the finished boxes' workgroups leave when a quarter of them is idle
+    if (open > 0 && 4 * open <= 3 * open_last) {
+      PM_TRY(build());
+      open_last = open;
+    }
+  }
+  *out_launched = launched;
+  return PM_OK;
+}
+
+int pm_fused_batch_solve(pm_ctx *c, PmFusedBoxes **fb, const std::vector<int> &eq0,
+                         const std::vector<int> &blk0, PmMethod mt, const double *b, double *x,
+                         const double *m, double tol, int maxit, int use32, int cap,
+                         std::vector<int> &iters, std::vector<int> &done,
+                         std::vector<double> &resid, int *launched, int *usable) {
+  *usable = 0;
+  if (!pm_affine_product(c, use32)) return PM_OK;
+  if (!*fb) PM_TRY(boxes_setup(c, fb, eq0, blk0));
+  if (!*fb) return PM_OK;
+  *usable = 1;
+  return mt == PM_IT_SQMR ? batch_solve<PM_IT_SQMR>(c, *fb, b, x, m, tol, maxit, use32, cap, iters,
+                                                    done, resid, launched)
+                          : batch_solve<PM_IT_PCG>(c, *fb, b, x, m, tol, maxit, use32, cap, iters,
+                                                   done, resid, launched);
 }

@@ -189,3 +189,42 @@ def test_fused_iterations(nen, shape, solver):
         with pytest.raises(PmError):
             s.solve(np.zeros(s.neq), SolverConfig(tol=1e-11))
     s.close()
+
+
+# the batched solve through the elements: boxes of different sizes, the middle
+# one with a zero right-hand side, against each box alone (RCM numbers every
+# box as it does alone, one range after the other)
+@pytest.mark.parametrize("nen,ns", [(20, (9, 3, 12)), (8, (18, 5, 20))])
+@pytest.mark.parametrize("solver,prec", [("sqmr", "fp64"), ("sqmr", "fp32ir"), ("pcg", "fp64")])
+def test_batch_through_elements(nen, ns, solver, prec):
+    from poromec_amd.solver import MefSolver, SolverConfig
+    decks = [P.heterogeneous_box_deck(n, seed=n, corr_len=n / 2, dt=0.1, nen=nen) for n in ns]
+    big, off = P.concat_decks(decks)
+    s = MefSolver(big)
+    assert s.matrix_info()["nnz"] > 4_500_000
+    s.batch_define(off)
+    s.pform(2, True, False, big.dt, big.dt)
+    rng = np.random.default_rng(9)
+    singles = [MefSolver(d) for d in decks]
+    bs = [rng.standard_normal(o.neq) if k != 1 else np.zeros(o.neq) for k, o in enumerate(singles)]
+    # fp32ir cannot meet much less than 1e-10 of a random load
+    tol = 1e-12 if prec == "fp64" else 1e-10
+    cfg = SolverConfig(solver=solver, tol=tol, precision=prec)
+    for _ in range(2):  # the second solve reuses the first one's buffers
+        x, info = s.solve(np.concatenate(bs), cfg)
+    at = 0
+    for k, o in enumerate(singles):
+        part = x[at: at + o.neq]
+        at += o.neq
+        if k == 1:
+            assert not part.any()
+        else:
+            o.pform(2, True, False, big.dt, big.dt)
+            ref, _ = o.solve(bs[k], SolverConfig(tol=1e-12))
+            assert _rel(part, ref) < (1e-9 if prec == "fp64" else 1e-7), k
+        o.close()
+    if prec == "fp64":
+        assert s.batch_iters()[1] == 0
+    else:
+        assert info["true_rel"] < 1e-10
+    s.close()
