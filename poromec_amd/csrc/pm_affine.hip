@@ -924,17 +924,33 @@ struct RefTab {
                        L = Z + 64, SIZE = L + 8 * 9 * 8;
 };
 
+// g g^T of every element, the symmetric products of its coefficients
+__global__ __launch_bounds__(PM_WG) void k_affine_metric(int numel, const double *ec, double *gg) {
+  const int slot = blockIdx.x * PM_WG + threadIdx.x;
+  if (slot >= numel) return;
+  const double *g = ec + (size_t)slot * PM_EC;
+  double *o = gg + (size_t)slot * PM_EC;
+#pragma unroll
+  for (int i = 0; i < 3; i++)
+#pragma unroll
+    for (int j = 0; j < 3; j++)
+      o[3 * i + j] = g[3 * i] * g[3 * j] + g[3 * i + 1] * g[3 * j + 1] + g[3 * i + 2] * g[3 * j + 2];
+}
+
 // Each matrix value is written once: the lanes of a group walk the row node's
 // incident elements, lane (b, x) forming the column of node b's component x
 // (then lanes 0..7 the pressure columns), and add into the block's rows in
-// LDS; a node's columns are found in the block's column list by bisection in
 // LDS.  A pair's 3 x 3 block is J^-T R J^-1 contracted with D: ~45
-// multiply-adds a lane instead of 64 Gauss points'.
+// multiply-adds a lane instead of 64 Gauss points'.  Bound by instruction
+// issue, so the places of all the elements' nodes in the block's column list
+// are found first, a node a lane (bisection in LDS): three searches a row
+// block instead of sixteen (hexa20/8 vertices); with 64 lanes a block its
+// elements' data are scalar loads.
 template <int NEN>
 __global__ __launch_bounds__(PM_WG) void k_affine_matrix(
     int nrn, int max_cols, int mstride, const unsigned int *__restrict__ minc,
-    const unsigned int *__restrict__ gnode,
-    const unsigned int *__restrict__ en, const double *__restrict__ ec,
+    const unsigned int *__restrict__ gnode, const unsigned int *__restrict__ en,
+    const double *__restrict__ ec, const double *__restrict__ gg_all,
     const double *__restrict__ tab, const int *__restrict__ nr,
     const int64_t *__restrict__ colptr, const int64_t *__restrict__ valptr,
     const int *__restrict__ ncol, double *__restrict__ val, int *err) {
@@ -942,9 +958,14 @@ __global__ __launch_bounds__(PM_WG) void k_affine_matrix(
   constexpr int GR = PM_WG / LPB;
   using RT = RefTab<NEN>;
   extern __shared__ double s_dyn[];
-  const int grp = threadIdx.x / LPB, l = threadIdx.x % LPB;
+  int grp = threadIdx.x / LPB;
+  const int l = threadIdx.x % LPB;
+  if (LPB == 64) grp = __builtin_amdgcn_readfirstlane(grp);
   double *row = s_dyn + (size_t)grp * max_cols * 4;
   int *cols = reinterpret_cast<int *>(s_dyn + (size_t)GR * max_cols * 4) + (size_t)grp * max_cols;
+  // place << 4 | free dofs of every node of the incident elements
+  int *place = reinterpret_cast<int *>(s_dyn + (size_t)GR * max_cols * 4) + (size_t)GR * max_cols +
+               (size_t)grp * mstride * NEN;
   const int64_t k = (int64_t)pm_xcd_block(blockIdx.x, gridDim.x) * GR + grp;
   const bool live = k < nrn;
   const int n = live ? nr[k] : 0;
@@ -954,96 +975,93 @@ __global__ __launch_bounds__(PM_WG) void k_affine_matrix(
   for (int j = l; j < n * cnt; j += LPB) row[j] = 0.0;
   __syncthreads();
   if (!live) return;  // no workgroup barrier follows
-  const unsigned int mk = gnode[k] & 15u;
-  // position of a column in the block (or -1)
-  auto find = [&](int col) {
+  const unsigned int *inc = minc + (size_t)k * mstride;
+  for (int i = l; i < mstride * NEN; i += LPB) {
+    const int p = i / NEN, b = i - p * NEN;
+    const unsigned int code = inc[p];
+    if (code == 0xffffffffu) break;
+    const unsigned int w = en[(size_t)(code >> 5) * NEN + b];
     int lo = 0, hi = cnt;
+    const int col = (int)(w >> 4);
     while (lo < hi) {
       const int mid = (lo + hi) >> 1;
       if (cols[mid] < col) lo = mid + 1;
       else hi = mid;
     }
-    if (lo >= cnt || cols[lo] != col) {  // pattern does not hold the pair
+    unsigned int m = w & 15u;
+    if (m && (lo >= cnt || cols[lo] != col)) {  // pattern does not hold the pair
       atomicExch(err, PM_ERR_STATE);
-      return -1;
+      m = 0;
     }
-    return lo;
-  };
+    place[i] = (lo << 4) | (int)m;
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  const unsigned int mk = gnode[k] & 15u;
+  const int q1 = (int)(mk & 1u), q2 = (int)__popc(mk & 3u), q3 = (int)__popc(mk & 7u);
+  double *r0 = row, *r1 = row + q1 * cnt, *r2 = row + q2 * cnt, *r3 = row + q3 * cnt;
+  const int b = l / 3, x = l - 3 * b;
   for (int p = 0; p < mstride; p++) {
-    const unsigned int code = minc[(size_t)k * mstride + p];
+    unsigned int code = inc[p];
+    if (LPB == 64) code = __builtin_amdgcn_readfirstlane(code);
     if (code == 0xffffffffu) break;
     const unsigned int slot = code >> 5;
     const int a = (int)(code & 31u);  // the row's local node
-    const double *eq = ec + (size_t)slot * PM_EC;
+    const double *eq = ec + (size_t)slot * PM_EC, *gg = gg_all + (size_t)slot * PM_EC;
     double g[9];
 #pragma unroll
     for (int i = 0; i < 9; i++) g[i] = eq[i];
-    const double cd = eq[9] + eq[10], cb = eq[10], cc = eq[11], al = eq[12];
-    // g g^T
-    double gg[9];
-#pragma unroll
-    for (int i = 0; i < 3; i++)
-#pragma unroll
-      for (int j = 0; j < 3; j++)
-        gg[3 * i + j] = g[3 * i] * g[3 * j] + g[3 * i + 1] * g[3 * j + 1] + g[3 * i + 2] * g[3 * j + 2];
+    const double cb = eq[10], cd = eq[9] + cb, cc = eq[11], al = eq[12];
     if (l < 3 * NEN) {
-      const int b = l / 3, x = l - 3 * b;
-      const unsigned int w = en[(size_t)slot * NEN + b];
-      if ((w >> x) & 1u) {
+      const int w = place[p * NEN + b];
+      if ((w >> x) & 1) {
+        const int pos = (w >> 4) + __popc(w & ((1 << x) - 1));
         const double gx[3] = {x == 0 ? g[0] : x == 1 ? g[1] : g[2],
                               x == 0 ? g[3] : x == 1 ? g[4] : g[5],
                               x == 0 ? g[6] : x == 1 ? g[7] : g[8]};
+        const double *tr = tab + RT::R + a * 9 * NEN + b;
         double H[3] = {0, 0, 0}, Ht[3] = {0, 0, 0}, lap = 0.0;
 #pragma unroll
         for (int i = 0; i < 3; i++)
 #pragma unroll
           for (int j = 0; j < 3; j++) {
-            const double r = tab[RT::R + (a * 9 + 3 * i + j) * NEN + b];
+            const double r = tr[(3 * i + j) * NEN];
             H[i] = fma(r, gx[j], H[i]);    // int d_i N_a dN_b/dx
             Ht[j] = fma(r, gx[i], Ht[j]);  // int dN_a/dx d_j N_b
             lap = fma(r, gg[3 * i + j], lap);
           }
-        const int pos = find((int)((w >> 4) + __popc(w & ((1u << x) - 1u))));
-        int q = 0;
+        // row y, column x: D's normal and shear parts
+        double v[3];
 #pragma unroll
         for (int y = 0; y < 3; y++) {
-          const double Gyx = g[y] * H[0] + g[3 + y] * H[1] + g[6 + y] * H[2];
-          const double Gxy = g[y] * Ht[0] + g[3 + y] * Ht[1] + g[6 + y] * Ht[2];
-          // row y, column x: D's normal and shear parts
-          const double v = y == x ? cd * Gyx + cc * (lap - Gyx) : cb * Gyx + cc * Gxy;
-          if ((mk >> y) & 1u) {
-            if (pos >= 0) row[q * cnt + pos] += v;
-            q++;
-          }
+          const double Gyx = fma(g[6 + y], H[2], fma(g[3 + y], H[1], g[y] * H[0]));
+          const double Gxy = fma(g[6 + y], Ht[2], fma(g[3 + y], Ht[1], g[y] * Ht[0]));
+          v[y] = y == x ? fma(cd, Gyx, cc * (lap - Gyx)) : fma(cb, Gyx, cc * Gxy);
         }
-        if (a < 8 && ((mk >> 3) & 1u)) {  // pressure row
-          double v = 0.0;
-#pragma unroll
-          for (int j = 0; j < 3; j++) v = fma(gx[j], tab[RT::T + (a * 3 + j) * NEN + b], v);
-          if (pos >= 0) row[q * cnt + pos] -= al * v;
+        if (mk & 1u) r0[pos] += v[0];
+        if (mk & 2u) r1[pos] += v[1];
+        if (mk & 4u) r2[pos] += v[2];
+        if (a < 8 && (mk & 8u)) {  // pressure row
+          const double *tt = tab + RT::T + a * 3 * NEN + b;
+          r3[pos] -= al * fma(gx[2], tt[2 * NEN], fma(gx[1], tt[NEN], gx[0] * tt[0]));
         }
       }
     }
     if (l < 8) {  // pressure columns
-      const unsigned int w = en[(size_t)slot * NEN + l];
-      if ((w >> 3) & 1u) {
-        const int pos = find((int)((w >> 4) + __popc(w & 7u)));
-        int q = 0;
-#pragma unroll
-        for (int y = 0; y < 3; y++) {
-          if (!((mk >> y) & 1u)) continue;
-          double v = 0.0;
-#pragma unroll
-          for (int j = 0; j < 3; j++) v = fma(g[3 * j + y], tab[RT::M + (a * 3 + j) * 8 + l], v);
-          if (pos >= 0) row[q * cnt + pos] -= al * v;
-          q++;
-        }
-        if (a < 8 && ((mk >> 3) & 1u)) {
+      const int w = place[p * NEN + l];
+      if (w & 8) {
+        const int pos = (w >> 4) + __popc(w & 7);
+        const double *tm = tab + RT::M + a * 3 * 8 + l;
+        const double m0 = al * tm[0], m1 = al * tm[8], m2 = al * tm[16];
+        if (mk & 1u) r0[pos] -= fma(g[6], m2, fma(g[3], m1, g[0] * m0));
+        if (mk & 2u) r1[pos] -= fma(g[7], m2, fma(g[4], m1, g[1] * m0));
+        if (mk & 4u) r2[pos] -= fma(g[8], m2, fma(g[5], m1, g[2] * m0));
+        if (a < 8 && (mk & 8u)) {
+          const double *tl = tab + RT::L + a * 9 * 8 + l;
           double lap = 0.0;
 #pragma unroll
-          for (int i = 0; i < 9; i++) lap = fma(tab[RT::L + (a * 9 + i) * 8 + l], gg[i], lap);
-          const double v = eq[13] * tab[RT::Z + a * 8 + l] + eq[14] * lap;
-          if (pos >= 0) row[q * cnt + pos] -= v;
+          for (int i = 0; i < 9; i++) lap = fma(tl[i * 8], gg[i], lap);
+          r3[pos] -= fma(eq[14], lap, eq[13] * tab[RT::Z + a * 8 + l]);
         }
       }
     }
@@ -1550,14 +1568,15 @@ bool pm_affine_box_patches(const pm_ctx *c, const std::vector<int> &blk0, std::v
   return true;
 }
 
-// LDS of a workgroup of k_affine_matrix: every group's rows and column list
+// LDS of a workgroup of k_affine_matrix: every group's rows, columns and places
 static size_t matrix_lds(const PmAffine *a) {
-  return (size_t)(PM_WG / (a->nen == 20 ? 64 : 32)) * a->max_cols * (4 * sizeof(double) + sizeof(int));
+  return (size_t)(PM_WG / (a->nen == 20 ? 64 : 32)) *
+         (a->max_cols * (4 * sizeof(double) + sizeof(int)) + a->mstride * a->nen * sizeof(int));
 }
 
 bool pm_affine_loops(const pm_ctx *c, int isw, int lhs) {
   // row blocks too wide for the 64 KB of LDS a workgroup may ask for keep the
-  // scattered assembly (455 columns; a box's vertex has 270, 108 with Q1/Q1)
+  // scattered assembly (437 columns; a box's vertex has 270, 108 with Q1/Q1)
   return affine_elements(c) && (isw != 2 || !lhs || matrix_lds(c->affine) <= 65536);
 }
 
@@ -1595,13 +1614,15 @@ int pm_affine_pform(pm_ctx *c, const ElemArgs &E, int isw, int lhs, int rhs) {
     const int gr = PM_WG / (a->nen == 20 ? 64 : 32);
     const dim3 g((unsigned)(((a->nrn + gr - 1) / gr + 7) & ~7));
     const size_t lds = matrix_lds(a);
+    hipLaunchKernelGGL(k_affine_metric, dim3((a->numel + PM_WG - 1) / PM_WG), dim3(PM_WG), 0,
+                       c->stream, a->numel, ec, a->ec);
     if (a->nen == 20)
       hipLaunchKernelGGL(k_affine_matrix<20>, g, dim3(PM_WG), lds, c->stream, a->nrn, a->max_cols,
-                         a->mstride, a->minc, a->gnode, a->en, ec, a->tab, M.nr, M.colptr, M.valptr,
+                         a->mstride, a->minc, a->gnode, a->en, ec, a->ec, a->tab, M.nr, M.colptr, M.valptr,
                          M.ncol, M.val, E.err);
     else
       hipLaunchKernelGGL(k_affine_matrix<8>, g, dim3(PM_WG), lds, c->stream, a->nrn, a->max_cols,
-                         a->mstride, a->minc, a->gnode, a->en, ec, a->tab, M.nr, M.colptr, M.valptr,
+                         a->mstride, a->minc, a->gnode, a->en, ec, a->ec, a->tab, M.nr, M.colptr, M.valptr,
                          M.ncol, M.val, E.err);
   }
   PM_CHECK_HIP(hipGetLastError());
