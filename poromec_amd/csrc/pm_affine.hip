@@ -868,21 +868,34 @@ __global__ __launch_bounds__(PM_WG) void k_affine_pass_gather(GatherArgs G, PmVe
                                                               PmIterState *st, int nxt, double *pa,
                                                               PmMap M) {
   const PmPart P = pm_part<BATCH, PM_PASS_NODES>(M, G.nrn, st, nullptr, 0, pa);
-  const PmIter s = P.st->it[nxt];  // written by the element part
-  if (s.done) return;
   int64_t k0, k1;
   pm_share(P, k0, k1);
   const int c = threadIdx.x & 3;
   double v[1] = {0.0};
-  for (int64_t k = k0 + (threadIdx.x >> 2); k < k1; k += PM_WG / 4) {
-    const unsigned int w4 = G.gnode[k];
-    if (!((w4 >> c) & 1u)) continue;
-    const unsigned int row = (w4 >> 4) + __popc(w4 & ((1u << c) - 1u));
-    const double y = s.pending ? 0.0 : pm_gather_sum(G, k, c);
-    const double qn = pm_row_update<MT>(V, s, row);
-    if (s.pending) continue;
-    V.y[row] = y;
-    v[0] += y * qn;
+  int64_t k = k0 + (threadIdx.x >> 2);
+  // the first node's sum does not wait for the scalars
+  unsigned int w4 = 0;
+  double y = 0.0;
+  if (k < k1) {
+    w4 = G.gnode[k];
+    y = pm_gather_sum(G, k, c);
+  }
+  const PmIter s = P.st->it[nxt];  // written by the element part
+  if (s.done) return;
+  while (k < k1) {
+    if ((w4 >> c) & 1u) {
+      const unsigned int row = (w4 >> 4) + __popc(w4 & ((1u << c) - 1u));
+      const double qn = pm_row_update<MT>(V, s, row);
+      if (!s.pending) {
+        V.y[row] = y;
+        v[0] += y * qn;
+      }
+    }
+    k += PM_WG / 4;
+    if (k < k1) {
+      w4 = G.gnode[k];
+      y = pm_gather_sum(G, k, c);
+    }
   }
   pm_dots_partials<1>(v, P.out, P.slot);
 }
@@ -1034,9 +1047,9 @@ __global__ __launch_bounds__(PM_WG) void k_affine_matrix(
         double v[3];
 #pragma unroll
         for (int y = 0; y < 3; y++) {
-          const double Gyx = fma(g[6 + y], H[2], fma(g[3 + y], H[1], g[y] * H[0]));
-          const double Gxy = fma(g[6 + y], Ht[2], fma(g[3 + y], Ht[1], g[y] * Ht[0]));
-          v[y] = y == x ? fma(cd, Gyx, cc * (lap - Gyx)) : fma(cb, Gyx, cc * Gxy);
+          const double Gyx = g[y] * H[0] + g[3 + y] * H[1] + g[6 + y] * H[2];
+          const double Gxy = g[y] * Ht[0] + g[3 + y] * Ht[1] + g[6 + y] * Ht[2];
+          v[y] = y == x ? cd * Gyx + cc * (lap - Gyx) : cb * Gyx + cc * Gxy;
         }
         if (mk & 1u) r0[pos] += v[0];
         if (mk & 2u) r1[pos] += v[1];
@@ -1052,16 +1065,16 @@ __global__ __launch_bounds__(PM_WG) void k_affine_matrix(
       if (w & 8) {
         const int pos = (w >> 4) + __popc(w & 7);
         const double *tm = tab + RT::M + a * 3 * 8 + l;
-        const double m0 = al * tm[0], m1 = al * tm[8], m2 = al * tm[16];
-        if (mk & 1u) r0[pos] -= fma(g[6], m2, fma(g[3], m1, g[0] * m0));
-        if (mk & 2u) r1[pos] -= fma(g[7], m2, fma(g[4], m1, g[1] * m0));
-        if (mk & 4u) r2[pos] -= fma(g[8], m2, fma(g[5], m1, g[2] * m0));
+        const double m0 = tm[0], m1 = tm[8], m2 = tm[16];
+        if (mk & 1u) r0[pos] -= al * fma(g[6], m2, fma(g[3], m1, g[0] * m0));
+        if (mk & 2u) r1[pos] -= al * fma(g[7], m2, fma(g[4], m1, g[1] * m0));
+        if (mk & 4u) r2[pos] -= al * fma(g[8], m2, fma(g[5], m1, g[2] * m0));
         if (a < 8 && (mk & 8u)) {
           const double *tl = tab + RT::L + a * 9 * 8 + l;
           double lap = 0.0;
 #pragma unroll
           for (int i = 0; i < 9; i++) lap = fma(tl[i * 8], gg[i], lap);
-          r3[pos] -= fma(eq[14], lap, eq[13] * tab[RT::Z + a * 8 + l]);
+          r3[pos] -= eq[13] * tab[RT::Z + a * 8 + l] + eq[14] * lap;
         }
       }
     }

@@ -20,49 +20,73 @@
 // ---------------------------------------------------------------------------
 // pass A on the stored matrix: a wavefront per node block, UNR columns a lane
 // ---------------------------------------------------------------------------
+template <typename VT, int UNR>
+struct PmStoredPart {  // UNR columns a lane of a node block: values, t and q
+  VT w[UNR][4];
+  double t[UNR], q[UNR];
+  __device__ __forceinline__ void load(const PmBlockMeta &m, int j0, int lane, const int *ncol,
+                                       const VT *val, const PmVecs &V) {
+    // past the block's columns a lane takes the last one and drops it after
+    // the load; past its rows, row 0 (summed, never stored)
+    int col[UNR];
+#pragma unroll
+    for (int u = 0; u < UNR; u++) {
+      const int j = j0 + u * 64 + lane, jc = j < m.c ? j : m.c - 1;
+      col[u] = ncol[m.cp + jc];
+#pragma unroll
+      for (int k = 0; k < 4; k++) w[u][k] = val[m.vp + (int64_t)(k < m.n ? k : 0) * m.c + jc];
+    }
+#pragma unroll
+    for (int u = 0; u < UNR; u++) {
+      t[u] = V.t[col[u]];
+      q[u] = V.q[col[u]];
+    }
+  }
+  __device__ __forceinline__ void add(const PmBlockMeta &m, int j0, int lane, double beta,
+                                      double *a) const {
+#pragma unroll
+    for (int u = 0; u < UNR; u++) {
+      const double xq = t[u] + beta * q[u];
+      const double x = j0 + u * 64 + lane < m.c ? xq : 0.0;
+#pragma unroll
+      for (int k = 0; k < 4; k++) a[k] += (double)w[u][k] * x;
+    }
+  }
+};
+
+// The first block's loads are in flight while the scalars form.
 template <typename VT, int UNR, PmMethod MT>
 __global__ __launch_bounds__(PM_WG) void k_stored_pass(
     int nrn, const int *__restrict__ fr, const int *__restrict__ nr,
     const int64_t *__restrict__ colptr, const int64_t *__restrict__ valptr,
     const int *__restrict__ ncol, const VT *__restrict__ val, PmVecs V, PmIterState *st, int cur,
     int first, double tol, int nblk, const double *pb, double *pa) {
-  const PmIter s = pm_iter_begin<MT>(st, cur, first, tol, nblk, pb);
-  if (blockIdx.x == 0 && threadIdx.x == 0) st->it[cur ^ 1] = s;
-  if (s.done) return;
   constexpr int GROUPS = PM_WG / 64;
   const int lane = threadIdx.x & 63;
   const int grp = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / 64));
   const int lb = pm_xcd_block(blockIdx.x, gridDim.x);
   int64_t k0, k1;
   pm_chunk(nrn, lb, gridDim.x, k0, k1);
+  int64_t k = k0 + grp;
+  PmBlockMeta m = pm_uniform<64>(pm_block_meta(k, k1, colptr, valptr, nr));
+  PmStoredPart<VT, UNR> D;
+  int f = 0;
+  if (k < k1) {
+    D.load(m, 0, lane, ncol, val, V);
+    f = fr[k];
+  }
+  const PmIter s = pm_iter_begin<MT>(st, cur, first, tol, nblk, pb);
+  if (blockIdx.x == 0 && threadIdx.x == 0) st->it[cur ^ 1] = s;
+  if (s.done) return;
   const int qr = pm_row_of(lane);
   double dot[1] = {0.0};
-  for (int64_t k = k0 + grp; k < k1; k += GROUPS) {
-    const PmBlockMeta m = pm_uniform<64>(pm_block_meta(k, k1, colptr, valptr, nr));
-    const int f = fr[k];
+  while (k < k1) {
     double a[4] = {0.0, 0.0, 0.0, 0.0};
     if (!s.pending) {
-      for (int j0 = 0; j0 < m.c; j0 += UNR * 64) {
-        // past the block's columns a lane takes the last one and drops it
-        // after the load; past its rows, row 0 (summed, never stored)
-        int col[UNR];
-        VT w[UNR][4];
-#pragma unroll
-        for (int u = 0; u < UNR; u++) {
-          const int j = j0 + u * 64 + lane, jc = j < m.c ? j : m.c - 1;
-          col[u] = ncol[m.cp + jc];
-#pragma unroll
-          for (int q = 0; q < 4; q++) w[u][q] = val[m.vp + (int64_t)(q < m.n ? q : 0) * m.c + jc];
-        }
-        double xq[UNR];
-#pragma unroll
-        for (int u = 0; u < UNR; u++) xq[u] = V.t[col[u]] + s.beta * V.q[col[u]];
-#pragma unroll
-        for (int u = 0; u < UNR; u++) {
-          const double x = j0 + u * 64 + lane < m.c ? xq[u] : 0.0;
-#pragma unroll
-          for (int q = 0; q < 4; q++) a[q] += (double)w[u][q] * x;
-        }
+      D.add(m, 0, lane, s.beta, a);
+      for (int j0 = UNR * 64; j0 < m.c; j0 += UNR * 64) {
+        D.load(m, j0, lane, ncol, val, V);
+        D.add(m, j0, lane, s.beta, a);
       }
     }
     const double y = pm_rows4_sum<64>(lane, a);
@@ -73,6 +97,12 @@ __global__ __launch_bounds__(PM_WG) void k_stored_pass(
         V.y[row] = y;
         dot[0] += y * qn;
       }
+    }
+    k += GROUPS;
+    if (k < k1) {
+      m = pm_uniform<64>(pm_block_meta(k, k1, colptr, valptr, nr));
+      D.load(m, 0, lane, ncol, val, V);
+      f = fr[k];
     }
   }
   pm_dots_partials<1>(dot, pa, blockIdx.x);
@@ -107,14 +137,14 @@ __global__ __launch_bounds__(PM_WG) void k_fused_b(int64_t n, PmIterState *st, i
                                                    const double *m, const double *q, double *x,
                                                    double *r, double *t, double *pb, PmMap M) {
   const PmPart P = pm_part<BATCH, PM_PASS_B>(M, n, st, pa, nblk, pb);
-  const PmIter s = P.st->it[nxt];
-  if (s.done || s.pending) return;
-  // contiguous shares; the first row's loads do not wait for the sums
+  // contiguous shares; the first row's loads wait for neither scalars nor sums
   int64_t i0, i1;
   pm_share(P, i0, i1);
   int64_t i = i0 + threadIdx.x;
-  const bool on = i < i1;
-  double yi = on ? y[i] : 0.0, ri = on ? r[i] : 0.0, mi = on ? m[i] : 0.0;
+  const int64_t il = i < i1 ? i : P.lo;
+  double yi = y[il], ri = r[il], mi = m[il];
+  const PmIter s = P.st->it[nxt];
+  if (s.done || s.pending) return;
   double sum[1];
   pm_sum_dots<1>(P.nin, P.in, sum);
   const bool lead = P.wg == 0 && threadIdx.x == 0;
