@@ -73,6 +73,12 @@ pm_ctx::~pm_ctx() {
   FREE(d_ie);
   FREE(d_vp);
   pm_affine_free(affine);
+  pm_stage_free(stage);
+  FREE(d_spmv);
+  FREE(d_csrc_ia);
+  FREE(d_csrc_ja);
+  FREE(d_csrc_ad);
+  FREE(d_csrc_al);
   if (batch) pm_batch_free(batch);
   FREE(d_eq_box);
   free_matrix(A);
@@ -191,6 +197,11 @@ int pm_upload_pattern(pm_ctx *c, const PmHostPattern &p) {
   FREE(c->d_eq_box);
   pm_affine_free(c->affine);  // its row blocks are the old matrix's
   c->affine = nullptr;
+  FREE(c->d_spmv);
+  FREE(c->d_csrc_ia);
+  FREE(c->d_csrc_ja);
+  FREE(c->d_csrc_ad);
+  FREE(c->d_csrc_al);
   free_matrix(c->A);
   PmDevMatrix &A = c->A;
   A.nrn = p.nrn;
@@ -669,12 +680,12 @@ extern "C" int pm_solve(pm_ctx *c, const pm_solver_cfg *cfg, const double *b, do
     PM_TRY(dalloc(&c->d_m, (size_t)n));
   }
   if (b)
-    PM_CHECK_HIP(hipMemcpyAsync(c->d_b, b, sizeof(double) * n, hipMemcpyHostToDevice, c->stream));
+    PM_TRY(pm_h2d(c, c->d_b, b, sizeof(double) * n));
   pm_solve_info local;
   pm_solve_info *inf = info ? info : &local;
   int rc = pm_solve_dev(c, cfg, c->d_b, c->d_x0, inf);
   if (rc == PM_OK && x) {
-    PM_CHECK_HIP(hipMemcpyAsync(x, c->d_x0, sizeof(double) * n, hipMemcpyDeviceToHost, c->stream));
+    PM_TRY(pm_d2h(c, x, c->d_x0, sizeof(double) * n));
     PM_CHECK_HIP(hipStreamSynchronize(c->stream));
   }
   return rc;
@@ -709,25 +720,22 @@ extern "C" int pm_values_upload(pm_ctx *c, const double *ad, const double *al) {
   PM_CHECK_HIP(hipSetDevice(c->device));
   const int neq = c->A.neq;
   const int64_t nad = c->csrc_ia[neq] - 1;
-  int64_t *d_ia = nullptr;
-  int *d_ja = nullptr;
-  double *d_ad = nullptr, *d_al = nullptr;
-  PM_TRY(dupload(c, &d_ia, c->csrc_ia.data(), (size_t)neq + 1));
-  PM_TRY(dupload(c, &d_ja, c->csrc_ja.data(), (size_t)nad));
-  PM_TRY(dupload(c, &d_ad, ad, (size_t)neq));
-  if (nad > 0) PM_TRY(dupload(c, &d_al, al, (size_t)nad));
-  else PM_TRY(dalloc(&d_al, 1));
+  if (!c->d_csrc_al) {  // kept until the next pattern
+    PM_TRY(dupload(c, &c->d_csrc_ia, c->csrc_ia.data(), (size_t)neq + 1));
+    PM_TRY(dupload(c, &c->d_csrc_ja, c->csrc_ja.data(), (size_t)nad));
+    PM_TRY(dalloc(&c->d_csrc_ad, (size_t)neq));
+    PM_TRY(dalloc(&c->d_csrc_al, (size_t)nad));
+  }
+  PM_TRY(pm_h2d(c, c->d_csrc_ad, ad, sizeof(double) * (size_t)neq));
+  if (nad > 0) PM_TRY(pm_h2d(c, c->d_csrc_al, al, sizeof(double) * (size_t)nad));
   PmDevMatrix &A = c->A;
   PM_CHECK_HIP(hipMemsetAsync(A.val, 0, sizeof(double) * (size_t)A.nnz, c->stream));
-  hipLaunchKernelGGL(k_csrc_values, dim3((neq + 255) / 256), dim3(256), 0, c->stream, neq, d_ia,
-                     d_ja, d_ad, d_al, A.eq_block, A.fr, A.colptr, A.valptr, A.ncol, A.val);
+  hipLaunchKernelGGL(k_csrc_values, dim3((neq + 255) / 256), dim3(256), 0, c->stream, neq,
+                     c->d_csrc_ia, c->d_csrc_ja, c->d_csrc_ad, c->d_csrc_al, A.eq_block, A.fr,
+                     A.colptr, A.valptr, A.ncol, A.val);
   PM_CHECK_HIP(hipGetLastError());
   PM_TRY(pm_extract_diag(c));
   PM_CHECK_HIP(hipStreamSynchronize(c->stream));
-  (void)hipFree(d_ia);
-  (void)hipFree(d_ja);
-  (void)hipFree(d_ad);
-  (void)hipFree(d_al);
   A.values_valid = true;
   A.have32 = false;
   if (c->affine) c->affine->op_valid = false;  // no longer the elements' matrix
@@ -739,17 +747,14 @@ extern "C" int pm_spmv(pm_ctx *c, const double *x, double *y) {
   if (!c->have_matrix || !c->A.values_valid) return PM_ERR_STATE;
   PM_CHECK_HIP(hipSetDevice(c->device));
   const int n = c->A.neq;
-  double *dx = nullptr, *dy = nullptr;
-  PM_CHECK_HIP(hipMalloc(&dx, sizeof(double) * n));
-  PM_CHECK_HIP(hipMalloc(&dy, sizeof(double) * n));
-  PM_CHECK_HIP(hipMemcpyAsync(dx, x, sizeof(double) * n, hipMemcpyHostToDevice, c->stream));
+  if (!c->d_spmv) PM_TRY(dalloc(&c->d_spmv, (size_t)n * 2));  // kept until the next pattern
+  double *dx = c->d_spmv, *dy = dx + n;
+  PM_TRY(pm_h2d(c, dx, x, sizeof(double) * n));
   int rc = pm_spmv_dev(c, dx, dy, 0);
   if (rc == PM_OK) {
-    PM_CHECK_HIP(hipMemcpyAsync(y, dy, sizeof(double) * n, hipMemcpyDeviceToHost, c->stream));
+    PM_TRY(pm_d2h(c, y, dy, sizeof(double) * n));
     PM_CHECK_HIP(hipStreamSynchronize(c->stream));
   }
-  hipFree(dx);
-  hipFree(dy);
   return rc;
 }
 
@@ -784,14 +789,14 @@ extern "C" int pm_export_csrc(pm_ctx *c, int64_t *ia, int *ja, double *ad, doubl
     if (ja)
       PM_CHECK_HIP(hipMemcpyAsync(ja, d_ja, sizeof(int) * nad, hipMemcpyDeviceToHost, c->stream));
     if (al)
-      PM_CHECK_HIP(hipMemcpyAsync(al, d_al, sizeof(double) * nad, hipMemcpyDeviceToHost, c->stream));
+      PM_TRY(pm_d2h(c, al, d_al, sizeof(double) * nad));
     PM_CHECK_HIP(hipStreamSynchronize(c->stream));
     FREE(d_ia);
     FREE(d_ja);
     FREE(d_al);
   }
   if (ad)
-    PM_CHECK_HIP(hipMemcpyAsync(ad, A.diag, sizeof(double) * neq, hipMemcpyDeviceToHost, c->stream));
+    PM_TRY(pm_d2h(c, ad, A.diag, sizeof(double) * neq));
   PM_CHECK_HIP(hipStreamSynchronize(c->stream));
   FREE(d_cnt);
   return PM_OK;
@@ -802,11 +807,11 @@ extern "C" int pm_set_state(pm_ctx *c, const double *u, const double *u0, const 
   if (!c || !c->have_mesh) return PM_ERR_STATE;
   PM_CHECK_HIP(hipSetDevice(c->device));
   const size_t nn = (size_t)c->mesh.nnode;
-  if (u) PM_CHECK_HIP(hipMemcpyAsync(c->d_u, u, sizeof(double) * nn * 4, hipMemcpyHostToDevice, c->stream));
-  if (u0) PM_CHECK_HIP(hipMemcpyAsync(c->d_u0, u0, sizeof(double) * nn * 4, hipMemcpyHostToDevice, c->stream));
-  if (dp) PM_CHECK_HIP(hipMemcpyAsync(c->d_dp, dp, sizeof(double) * nn, hipMemcpyHostToDevice, c->stream));
+  if (u) PM_TRY(pm_h2d(c, c->d_u, u, sizeof(double) * nn * 4));
+  if (u0) PM_TRY(pm_h2d(c, c->d_u0, u0, sizeof(double) * nn * 4));
+  if (dp) PM_TRY(pm_h2d(c, c->d_dp, dp, sizeof(double) * nn));
   if (porosity)
-    PM_CHECK_HIP(hipMemcpyAsync(c->d_poro, porosity, sizeof(double) * nn, hipMemcpyHostToDevice, c->stream));
+    PM_TRY(pm_h2d(c, c->d_poro, porosity, sizeof(double) * nn));
   PM_CHECK_HIP(hipStreamSynchronize(c->stream));
   c->t = t;
   return PM_OK;
@@ -817,11 +822,11 @@ extern "C" int pm_get_state(pm_ctx *c, double *u, double *u0, double *dp, double
   if (!c || !c->have_mesh) return PM_ERR_STATE;
   PM_CHECK_HIP(hipSetDevice(c->device));
   const size_t nn = (size_t)c->mesh.nnode;
-  if (u) PM_CHECK_HIP(hipMemcpyAsync(u, c->d_u, sizeof(double) * nn * 4, hipMemcpyDeviceToHost, c->stream));
-  if (u0) PM_CHECK_HIP(hipMemcpyAsync(u0, c->d_u0, sizeof(double) * nn * 4, hipMemcpyDeviceToHost, c->stream));
-  if (dp) PM_CHECK_HIP(hipMemcpyAsync(dp, c->d_dp, sizeof(double) * nn, hipMemcpyDeviceToHost, c->stream));
+  if (u) PM_TRY(pm_d2h(c, u, c->d_u, sizeof(double) * nn * 4));
+  if (u0) PM_TRY(pm_d2h(c, u0, c->d_u0, sizeof(double) * nn * 4));
+  if (dp) PM_TRY(pm_d2h(c, dp, c->d_dp, sizeof(double) * nn));
   if (porosity)
-    PM_CHECK_HIP(hipMemcpyAsync(porosity, c->d_poro, sizeof(double) * nn, hipMemcpyDeviceToHost, c->stream));
+    PM_TRY(pm_d2h(c, porosity, c->d_poro, sizeof(double) * nn));
   PM_CHECK_HIP(hipStreamSynchronize(c->stream));
   if (t) *t = c->t;
   return PM_OK;
@@ -831,9 +836,9 @@ extern "C" int pm_get_vectors(pm_ctx *c, double *b0, double *b, double *x0) {
   if (!c || !c->have_matrix) return PM_ERR_STATE;
   PM_CHECK_HIP(hipSetDevice(c->device));
   const size_t n = (size_t)c->A.neq;
-  if (b0 && c->d_b0) PM_CHECK_HIP(hipMemcpyAsync(b0, c->d_b0, sizeof(double) * n, hipMemcpyDeviceToHost, c->stream));
-  if (b && c->d_b) PM_CHECK_HIP(hipMemcpyAsync(b, c->d_b, sizeof(double) * n, hipMemcpyDeviceToHost, c->stream));
-  if (x0 && c->d_x0) PM_CHECK_HIP(hipMemcpyAsync(x0, c->d_x0, sizeof(double) * n, hipMemcpyDeviceToHost, c->stream));
+  if (b0 && c->d_b0) PM_TRY(pm_d2h(c, b0, c->d_b0, sizeof(double) * n));
+  if (b && c->d_b) PM_TRY(pm_d2h(c, b, c->d_b, sizeof(double) * n));
+  if (x0 && c->d_x0) PM_TRY(pm_d2h(c, x0, c->d_x0, sizeof(double) * n));
   PM_CHECK_HIP(hipStreamSynchronize(c->stream));
   return PM_OK;
 }
@@ -842,9 +847,9 @@ extern "C" int pm_set_vectors(pm_ctx *c, const double *b0, const double *b, cons
   if (!c || !c->have_matrix) return PM_ERR_STATE;
   PM_CHECK_HIP(hipSetDevice(c->device));
   const size_t n = (size_t)c->A.neq;
-  if (b0 && c->d_b0) PM_CHECK_HIP(hipMemcpyAsync(c->d_b0, b0, sizeof(double) * n, hipMemcpyHostToDevice, c->stream));
-  if (b && c->d_b) PM_CHECK_HIP(hipMemcpyAsync(c->d_b, b, sizeof(double) * n, hipMemcpyHostToDevice, c->stream));
-  if (x0 && c->d_x0) PM_CHECK_HIP(hipMemcpyAsync(c->d_x0, x0, sizeof(double) * n, hipMemcpyHostToDevice, c->stream));
+  if (b0 && c->d_b0) PM_TRY(pm_h2d(c, c->d_b0, b0, sizeof(double) * n));
+  if (b && c->d_b) PM_TRY(pm_h2d(c, c->d_b, b, sizeof(double) * n));
+  if (x0 && c->d_x0) PM_TRY(pm_h2d(c, c->d_x0, x0, sizeof(double) * n));
   PM_CHECK_HIP(hipStreamSynchronize(c->stream));
   return PM_OK;
 }

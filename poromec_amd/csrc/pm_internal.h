@@ -98,6 +98,8 @@ struct PmScalars;  // device-side Krylov scalars (pm_device.h)
 struct PmBatch;    // batching form (pm_batch.hip)
 struct PmAffine;   // parallelepiped elements (pm_affine.hip)
 struct PmIterState;  // fused iterations (pm_fused.h)
+struct PmStage;      // pinned pieces of large copies (pm_copy.cpp)
+void pm_stage_free(PmStage *s);
 struct PmIter;
 void pm_batch_free(PmBatch *b);
 
@@ -225,6 +227,13 @@ struct pm_ctx {
   // GMRES (whose basis would need (ngram + 1) more vectors)
   bool no_alloc = false;
 
+  PmStage *stage = nullptr;
+  double *d_spmv = nullptr;  // pm_spmv's two vectors
+  // the caller's CSRC pattern on the device (pm_struct_upload)
+  int64_t *d_csrc_ia = nullptr;
+  int *d_csrc_ja = nullptr;
+  double *d_csrc_ad = nullptr, *d_csrc_al = nullptr;
+
   // element products of parallelepiped meshes (null: stored matrix only)
   PmAffine *affine = nullptr;
 
@@ -235,6 +244,9 @@ struct pm_ctx {
   ~pm_ctx();
 };
 
+// copies of the caller's arrays on the context's stream (pm_copy.cpp)
+int pm_h2d(pm_ctx *c, void *dst, const void *src, size_t bytes);
+int pm_d2h(pm_ctx *c, void *dst, const void *src, size_t bytes);
 int pm_upload_pattern(pm_ctx *c, const PmHostPattern &p);
 int pm_dev_alloc(pm_ctx *c, void **ptr, size_t bytes);
 int pm_ensure_workspace(pm_ctx *c, int n);

@@ -346,8 +346,7 @@ int pm_tform_dev(pm_ctx *c, double *tx, double *txe, double *txb, double *flux) 
   const size_t len[4] = {(size_t)nn * 6, (size_t)nn * 6, (size_t)nn * 6, (size_t)nn * 3};
   for (int i = 0; i < 4; i++)
     if (dst[i])
-      PM_CHECK_HIP(hipMemcpyAsync(dst[i], outs[i], sizeof(double) * len[i],
-                                  hipMemcpyDeviceToHost, c->stream));
+      PM_TRY(pm_d2h(c, dst[i], outs[i], sizeof(double) * len[i]));
   PM_CHECK_HIP(hipStreamSynchronize(c->stream));
   return err ? err : PM_OK;
 }
