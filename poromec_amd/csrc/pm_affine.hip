@@ -27,6 +27,8 @@
 #include <cmath>
 #include <cstring>
 #include <functional>
+#include <new>
+#include <system_error>
 #include <thread>
 
 #include "pm_affine.h"
@@ -1258,14 +1260,16 @@ static void element_patches(const PmHostMesh &m, const double *x, int L, std::ve
       const float va = cen[(size_t)a * 3 + ax], vb = cen[(size_t)b * 3 + ax];
       return va != vb ? va < vb : a < b;
     });
+    std::thread t;
     if (fork > 0 && n > 20000) {
-      std::thread t([&] { split(lo, mid, fork - 1); });
-      split(mid, hi, fork - 1);
-      t.join();
-    } else {
-      split(lo, mid, 0);
-      split(mid, hi, 0);
+      try {
+        t = std::thread([&] { split(lo, mid, fork - 1); });
+      } catch (const std::system_error &) {  // no more threads: this one does both halves
+      }
     }
+    if (!t.joinable()) split(lo, mid, fork - 1);
+    split(mid, hi, fork - 1);
+    if (t.joinable()) t.join();
   };
   ps.assign(1, 0);
   for (int a = 0; a < numel;) {
@@ -1277,7 +1281,7 @@ static void element_patches(const PmHostMesh &m, const double *x, int L, std::ve
   }
 }
 
-int pm_affine_setup(pm_ctx *c, const double *x, const PmHostPattern &pat) {
+static int affine_setup(pm_ctx *c, const double *x, const PmHostPattern &pat) {
   const std::vector<int> &eq_block = pat.eq_block;
   const PmHostMesh &m = c->mesh;
   const int nen = m.nen, numel = m.numel, nrn = c->A.nrn;
@@ -1413,6 +1417,14 @@ int pm_affine_setup(pm_ctx *c, const double *x, const PmHostPattern &pat) {
   }
   c->affine = a;
   return PM_OK;
+}
+
+int pm_affine_setup(pm_ctx *c, const double *x, const PmHostPattern &pat) {
+  try {
+    return affine_setup(c, x, pat);
+  } catch (const std::bad_alloc &) {  // the stored-matrix path needs none of this
+    return PM_OK;
+  }
 }
 
 // c->affine's element loops stand for elmt17_pm and the Q1/Q1 element with
