@@ -303,7 +303,7 @@ static void bspmv_shape(pm_ctx *c, int cfg, const VT *val, const double *x, doub
 
 template <int NV, class Epi>
 static void bspmv(pm_ctx *c, int use32, const double *x, double *y, const double *w, Epi epi) {
-  const int cfg = c->spmv_cfg[use32 ? 1 : 0];
+  const int set = c->spmv_cfg[use32 ? 1 : 0], cfg = set < 0 ? 2 : set;
   if (use32) bspmv_shape<float, NV>(c, cfg, c->A.val32, x, y, w);
   else bspmv_shape<double, NV>(c, cfg, c->A.val, x, y, w);
   if (NV > 0) bfinish<NV>(c, epi, 0);

@@ -216,8 +216,9 @@ struct pm_ctx {
   int tev_used = 0;
   double spmv_ms[2] = {0.0, 0.0};   // FP64, FP32 values
   long long spmv_n[2] = {0, 0};
-  // SpMV shape (index into the tuner's table) per value precision
-  int spmv_cfg[2] = {2, 2};
+  // SpMV shape (index into the tuner's table) per value precision; -1: not
+  // tuned nor set (pm_spmv_shape chooses)
+  int spmv_cfg[2] = {-1, -1};
   int spmv_tuned[2] = {0, 0};
   // reference summation order: every reduction a sequential left-to-right
   // sum, the SpMV in the order of matvec_csrc_sym_pm (slow; for parity)

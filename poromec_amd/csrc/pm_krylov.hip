@@ -161,7 +161,10 @@ __global__ __launch_bounds__(PM_WG) void k_spmv_pf(
 // the length bits (mbcnt), with no LDS.  The descriptors of a block's first
 // pass are loaded one block ahead, as k_spmv_pf does with column indices.
 // Loads past a run read the next columns' values (or the 4 values of padding
-// after the array) and are multiplied by zero; rows past the block's count
+// after the array), which count as zero, so that an infinite value stays in
+// its row; a lane without a run loads past the resources' ends and moves
+// nothing (us before and after: hexa20/8 40^3 289 -> 282, Q1/Q1 64^3 258 ->
+// 233 with shape 14, 195 -> 192 with shape 15); rows past the block's count
 // accumulate into sums that are not stored.
 // FP32 values: at least 6 waves per SIMD (two runs per lane then fit in 80
 // VGPRs without spills, against 101 and 4 waves unbounded)
@@ -508,7 +511,7 @@ __global__ __launch_bounds__(PM_WG, sizeof(VT) == 4 ? 6 : 1) void k_spmv_chg(
       u4 wv[U][4][VPR];
 #pragma unroll
       for (int u = 0; u < U; u++) {
-        const unsigned int o = (voff + off[u]) * (unsigned int)sizeof(VT);
+        const unsigned int o = len[u] > 0 ? (voff + off[u]) * (unsigned int)sizeof(VT) : PM_PAST_END;
 #pragma unroll
         for (int q = 0; q < 4; q++)
 #pragma unroll
@@ -520,11 +523,11 @@ __global__ __launch_bounds__(PM_WG, sizeof(VT) == 4 ? 6 : 1) void k_spmv_chg(
       double xv[U][4];
 #pragma unroll
       for (int u = 0; u < U; u++) {
-        const unsigned int col = d[u] >> 2;
+        const unsigned int xo = len[u] > 0 ? (d[u] >> 2) * 8u : 0xffffff00u;
 #pragma unroll
         for (int kk = 0; kk < 4; kk++) {
-          const double xc = pm_bload<double, 0>(xr, (col + (unsigned int)kk) * 8u);
-          xv[u][kk] = kk < len[u] ? xc : 0.0;
+          const double xc = pm_bload<double, 0>(xr, xo + (unsigned int)kk * 8u);
+          xv[u][kk] = kk == 0 || kk < len[u] ? xc : 0.0;
         }
       }
       if (h0 == 0)  // the next blocks' first descriptors, behind this pass's loads
@@ -539,7 +542,8 @@ __global__ __launch_bounds__(PM_WG, sizeof(VT) == 4 ? 6 : 1) void k_spmv_chg(
           VT v[4];
           __builtin_memcpy(v, &wv[u][q][0], sizeof(v));
 #pragma unroll
-          for (int kk = 0; kk < 4; kk++) a[q] += (double)v[kk] * xv[u][kk];
+          for (int kk = 0; kk < 4; kk++)
+            a[q] += (double)(kk == 0 || kk < len[u] ? v[kk] : VT(0)) * xv[u][kk];
         }
     }
 #pragma unroll
@@ -604,6 +608,27 @@ static int spmv_grid(int nrn, int lanes) {
   if (g < 8) g = 8;
   if (g > PM_SPMV_MAX_GRID) g = PM_SPMV_MAX_GRID;
   return (g + 7) & ~7;
+}
+
+// The shape of a product that was neither tuned nor set: one run of columns
+// per lane for the meshes' matrices, 32 lanes a block (two blocks a
+// wavefront) where its runs fill them once, one or two runs for 64 lanes
+// where they do not.  us, (64, 3) / shape 14 / shape 15:
+//   Q1/Q1 (27 runs)  20^3 FP64 17.4 / 13.7 / 9.2, 32^3 66 / 40 / 26,
+//                    64^3 321 / 233 / 192, FP32 220 / 144 / 118
+//   hexa20/8 (~45)   8^3 FP64 8.5 / 7.5 / 8.2, 16^3 33.5 / 27.0 / 23.1,
+//                    24^3 96 / 72 / 65, 32^3 203 / 158 / 161, 40^3 381 / 282 / 306,
+//                    FP32 16^3 26.5 / 20.6 / 21.9, 40^3 274 / 170 / 212
+// Under a million values the launch is most of it (hexa20/8 6^3: 7.6 / 6.7 /
+// 7.1), and a matrix of short runs would leave three of a lane's four values
+// unused.
+static int pm_spmv_shape(const pm_ctx *c, int use32) {
+  const int set = c->spmv_cfg[use32 ? 1 : 0];
+  if (set >= 0) return set;
+  const PmDevMatrix &A = c->A;
+  if (A.nnz < 1000000 || A.ncols < 2 * A.nchunks) return 2;
+  if (A.nchunks <= (int64_t)32 * A.nrn) return 15;
+  return !use32 && A.nnz < 64000000 ? 15 : 14;
 }
 
 template <typename VT, int NV, bool SCALE_M>
@@ -793,7 +818,7 @@ static void launch_spmv_raw(pm_ctx *c, int use32, const double *x, double *y, co
     if (NV > 0) launch_vec<NV>(c, A.neq, S, SpmvDots<NV>{y, w}, epi, 0);
     return;
   }
-  const int cfg = c->spmv_cfg[use32 ? 1 : 0];
+  const int cfg = pm_spmv_shape(c, use32);
   const int g = use32 ? launch_spmv_shape<float, NV, SCALE_M>(c, cfg, A.val32, x, y, w, m, S)
                       : launch_spmv_shape<double, NV, SCALE_M>(c, cfg, A.val, x, y, w, m, S);
   if (NV > 0) launch_finish<NV>(c, g, S, epi, 0);

@@ -320,6 +320,7 @@ __device__ __forceinline__ void pm_spmv_block(int lane, const PmBlockMeta &m,
 
 // Runs of <= 4 consecutive columns, one per lane (k_spmv_ch, k_spmv_b_ch):
 // a block's metadata, and one pass of UNR runs per lane.
+#define PM_PAST_END 0x80000000u  // byte offset past any block's values
 struct PmRunMeta {
   int64_t vp, hp;
   int c, n, nh;
@@ -378,7 +379,8 @@ __device__ __forceinline__ unsigned int pm_run_pass(int lane, int h0, const PmRu
   u4 w[UNR][4][VPR];
 #pragma unroll
   for (int u = 0; u < UNR; u++) {
-    const unsigned int o = off[u] * (unsigned int)sizeof(VT);
+    // a lane without a run reads past the resources' ends: zeros
+    const unsigned int o = len[u] > 0 ? off[u] * (unsigned int)sizeof(VT) : PM_PAST_END;
 #pragma unroll
     for (int q = 0; q < 4; q++)
 #pragma unroll
@@ -389,11 +391,11 @@ __device__ __forceinline__ unsigned int pm_run_pass(int lane, int h0, const PmRu
   double xv[UNR][4];
 #pragma unroll
   for (int u = 0; u < UNR; u++) {
-    const unsigned int col = d[u] >> 2;
+    const unsigned int xo = len[u] > 0 ? (d[u] >> 2) * 8u : 0xffffff00u;
 #pragma unroll
     for (int k = 0; k < 4; k++) {
-      const double xc = pm_bload<double, 0>(xr, (col + (unsigned int)k) * 8u);
-      xv[u][k] = k < len[u] ? xc : 0.0;
+      const double xc = pm_bload<double, 0>(xr, xo + (unsigned int)k * 8u);
+      xv[u][k] = k == 0 || k < len[u] ? xc : 0.0;
     }
   }
   if (PREFETCH) {
@@ -408,7 +410,8 @@ __device__ __forceinline__ unsigned int pm_run_pass(int lane, int h0, const PmRu
       VT v[4];
       __builtin_memcpy(v, &w[u][q][0], sizeof(v));
 #pragma unroll
-      for (int k = 0; k < 4; k++) a[q] += (double)v[k] * xv[u][k];
+      for (int k = 0; k < 4; k++)
+        a[q] += (double)(k == 0 || k < len[u] ? v[k] : VT(0)) * xv[u][k];
     }
   return base;
 }
