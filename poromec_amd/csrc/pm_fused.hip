@@ -108,6 +108,136 @@ __global__ __launch_bounds__(PM_WG) void k_stored_pass(
   pm_dots_partials<1>(dot, pa, blockIdx.x);
 }
 
+// The same with one run of <= 4 columns per lane and 32 lanes per block
+// (k_spmv_chg's layout; two blocks a wavefront): a third of the index words
+// and of the loads a column, two runs' descriptors and the first runs' values
+// and gathers in flight while the scalars form.
+template <typename VT>
+struct PmRunPart {  // a lane's run: values of the block's rows, t and q
+  int len;
+  VT v[4][4];
+  double t[4], q[4];
+  // base: the block's columns before this pass, returned after it
+  __device__ __forceinline__ unsigned int load(unsigned int d, bool valid, unsigned long long gmask,
+                                               unsigned int base, unsigned int voff,
+                                               unsigned int rowb, __amdgpu_buffer_rsrc_t vr,
+                                               __amdgpu_buffer_rsrc_t tr,
+                                               __amdgpu_buffer_rsrc_t qr) {
+    const unsigned int l1 = d & 3u;
+    const unsigned long long bv = __ballot(valid) & gmask;
+    const unsigned long long b0 = __ballot(valid && (l1 & 1u)) & gmask;
+    const unsigned long long b1 = __ballot(valid && (l1 & 2u)) & gmask;
+    const unsigned int off =
+        base + pm_lanes_below(bv) + pm_lanes_below(b0) + 2u * pm_lanes_below(b1);
+    len = valid ? (int)l1 + 1 : 0;
+    // a lane without a run reads past the resources' ends: zeros
+    const unsigned int o = valid ? (voff + off) * (unsigned int)sizeof(VT) : PM_PAST_END;
+    const unsigned int xo = valid ? (d >> 2) * 8u : 0xffffff00u;
+    typedef unsigned int u4 __attribute__((ext_vector_type(4)));
+    constexpr int VPR = sizeof(VT) == 4 ? 1 : 2;  // 16-byte loads a row
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      u4 w[VPR];
+#pragma unroll
+      for (int h = 0; h < VPR; h++)
+        w[h] = __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(
+                                          vr, o + (unsigned int)k * rowb + 16u * h, 0, 0));
+      __builtin_memcpy(v[k], w, sizeof(v[k]));
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      t[j] = pm_bload<double, 0>(tr, xo + (unsigned int)j * 8u);
+      q[j] = pm_bload<double, 0>(qr, xo + (unsigned int)j * 8u);
+    }
+    return base + (unsigned int)(__popcll(bv) + __popcll(b0) + 2 * __popcll(b1));
+  }
+  __device__ __forceinline__ void add(double beta, double *a) const {
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const bool in = j == 0 || j < len;  // past the run: other columns, other rows
+      const double xq = t[j] + beta * q[j];
+      const double x = in ? xq : 0.0;
+#pragma unroll
+      for (int k = 0; k < 4; k++) a[k] += (double)(in ? v[k][j] : VT(0)) * x;
+    }
+  }
+};
+
+template <typename VT, PmMethod MT>
+__global__ __launch_bounds__(PM_WG) void k_stored_runs(
+    int nrn, int neq, const int *__restrict__ fr, const int *__restrict__ nr,
+    const int64_t *__restrict__ colptr, const int64_t *__restrict__ valptr,
+    const int64_t *__restrict__ chptr, const unsigned int *__restrict__ chunk,
+    const VT *__restrict__ val, PmVecs V, PmIterState *st, int cur, int first, double tol,
+    int nblk, const double *pb, double *pa) {
+  constexpr int GROUPS = PM_WG / 64;
+  const int lane = threadIdx.x & 63, gi = lane >> 5, gl = lane & 31;
+  const unsigned long long gmask = 0xffffffffull << (gi * 32);
+  const int grp = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / 64));
+  const int lb = pm_xcd_block(blockIdx.x, gridDim.x);
+  int64_t p0, p1;
+  pm_chunk(((int64_t)nrn + 1) / 2, lb, gridDim.x, p0, p1);
+  int64_t p = p0 + grp;
+  const __amdgpu_buffer_rsrc_t tr = pm_rsrc(V.t, (unsigned int)neq * 8u);
+  const __amdgpu_buffer_rsrc_t qr = pm_rsrc(V.q, (unsigned int)neq * 8u);
+  PmBlocksMeta<2> m;
+  PmRunMeta me;
+  PmRunPart<VT> D;
+  unsigned int d1 = 0, base = 0;
+  int f = 0;
+  auto descriptor = [&](int h0) {  // of run h0 + gl of the group's block
+    const __amdgpu_buffer_rsrc_t hr =
+        pm_rsrc(chunk + m.b[0].hp, (unsigned int)(m.b[0].nh + m.b[1].nh) * 4u);
+    const unsigned int at = (unsigned int)(me.hp - m.b[0].hp) + (unsigned int)(h0 + gl);
+    return (unsigned int)__builtin_amdgcn_raw_buffer_load_b32(hr, at * 4u, 0, 0);
+  };
+  auto load = [&](int h0, unsigned int d) {
+    const __amdgpu_buffer_rsrc_t vr =
+        pm_rsrc(val + m.b[0].vp,
+                (unsigned int)(m.b[0].n * m.b[0].c + m.b[1].n * m.b[1].c + 3) *
+                    (unsigned int)sizeof(VT));
+    base = D.load(d, h0 + gl < me.nh, gmask, base, (unsigned int)(me.vp - m.b[0].vp),
+                  (unsigned int)me.c * (unsigned int)sizeof(VT), vr, tr, qr);
+  };
+  auto start = [&] {
+    m = pm_blocks_meta<2>(p, p1, nrn, colptr, valptr, nr, chptr);
+    me = pm_pick<2>(m, gi);
+    const unsigned int d0 = descriptor(0);
+    d1 = descriptor(32);
+    f = me.n > 0 ? fr[2 * p + gi] : 0;
+    base = 0;
+    load(0, d0);
+  };
+  if (p < p1) start();
+  const PmIter s = pm_iter_begin<MT>(st, cur, first, tol, nblk, pb);
+  if (blockIdx.x == 0 && threadIdx.x == 0) st->it[cur ^ 1] = s;
+  if (s.done) return;
+  const int row = pm_row_of(gl);
+  double dot[1] = {0.0};
+  while (p < p1) {
+    double a[4] = {0.0, 0.0, 0.0, 0.0};
+    if (!s.pending) {
+      D.add(s.beta, a);
+      const int passes = max(m.b[0].nh, m.b[1].nh);  // the wavefront's
+      for (int h0 = 32; h0 < passes; h0 += 32) {
+        load(h0, h0 == 32 ? d1 : descriptor(h0));
+        D.add(s.beta, a);
+      }
+    }
+    const double y = pm_rows4_sum<32>(gl, a);
+    if (gl < 4 && row < me.n) {
+      const double qn = pm_row_update<MT>(V, s, f + row);
+      if (!s.pending) {
+        V.y[f + row] = y;
+        dot[0] += y * qn;
+      }
+    }
+    p += GROUPS;
+    if (p < p1) start();
+  }
+  pm_dots_partials<1>(dot, pa, blockIdx.x);
+}
+
 // ---------------------------------------------------------------------------
 // initial vectors and pass B
 // ---------------------------------------------------------------------------
@@ -199,21 +329,42 @@ __global__ __launch_bounds__(PM_WG) void k_fused_tail(int64_t n, PmVecs V, PmIte
 // ---------------------------------------------------------------------------
 // driver
 // ---------------------------------------------------------------------------
-// Always through the elements; on the stored matrix up to 12 million values
-// (FP32: 24).  Beyond, the product's two gathers a column cost more than the
-// finishers: an SQMR iteration, three passes with the tuned SpMV shape / fused,
-// takes 44.5 / 33.6 us at 12.2 M values (hexa20/8 17^3), 57.9 / 47.3 at 20 M,
-// 88.8 / 102 at 35 M; Q1/Q1 41.5 / 41.7 at 13.8 M (32^3), 61.0 / 76.1 at 27 M;
-// FP32 59.2 / 57.1 at 35 M, Q1/Q1 53.5 / 53.8 at 27 M.
+// The stored product by runs of columns from 2 million values on where the
+// runs are long enough to fill a lane's four values.  us an SQMR iteration,
+// by columns / by runs: hexa20/8 1.2 M 11.8 / 12.2, 2.4 M 13.3 / 13.3, 3.2 M
+// 17.2 / 14.2, 6.7 M 25.6 / 22.3, 12.2 M 33.8 / 34.5, 20 M 48.4 / 44.8; Q1/Q1
+// 2.4 M 15.2 / 12.6, 5.8 M 23.1 / 20.4, 13.8 M 40.0 / 34.2; FP32 values 14.7 /
+// 13.6 at 3.2 M, Q1/Q1 34.1 / 30.7 at 13.8 M.
+static bool stored_runs(const PmDevMatrix &A) {
+  return A.nnz >= 2000000 && A.ncols >= 2 * A.nchunks;
+}
+
+// Always through the elements; on the stored matrix by runs up to 30 million
+// values (FP32: 40), by columns up to 12 (24).  Beyond, the product's two
+// gathers a column cost more than the finishers: an SQMR iteration in three
+// passes / by runs takes 52.4 / 44.8 us at 20 M values (hexa20/8 20^3), 84.8 /
+// 85.3 at 35 M, 136 / 145 at 56 M; Q1/Q1 61.3 / 52.8 at 27 M (40^3), 110 / 115
+// at 47 M; FP32 60.3 / 52.7 at 35 M, 81.3 / 87.5 at 56 M, Q1/Q1 73.7 / 64.2 at
+// 47 M.  By columns 41.5 / 41.7 at 13.8 M.
 bool pm_fused_usable(const pm_ctx *c, int use32) {
   if (c->ordered) return false;
-  return pm_affine_product(c, use32) || c->A.nnz <= (use32 ? 24000000 : 12000000);
+  const int64_t most = stored_runs(c->A) ? (use32 ? 40000000 : 30000000)
+                                         : (use32 ? 24000000 : 12000000);
+  return pm_affine_product(c, use32) || c->A.nnz <= most;
 }
 
 template <typename VT, PmMethod MT>
 static int stored_pass(pm_ctx *c, const VT *val, const PmVecs &V, PmIterState *st, int cur,
                        int first, double tol, int nblk, const double *pb, double *pa) {
   const PmDevMatrix &A = c->A;
+  if (stored_runs(A)) {
+    int g = (A.nrn + PM_WG / 32 - 1) / (PM_WG / 32);
+    g = (std::min(g, PM_MAX_GRID) + 7) & ~7;
+    hipLaunchKernelGGL((k_stored_runs<VT, MT>), dim3(g), dim3(PM_WG), 0, c->stream, A.nrn, A.neq,
+                       A.fr, A.nr, A.colptr, A.valptr, A.chptr, A.chunk, val, V, st, cur, first,
+                       tol, nblk, pb, pa);
+    return g;
+  }
   int g = (A.nrn + PM_WG / 64 - 1) / (PM_WG / 64);
   g = (std::min(g, PM_MAX_GRID) + 7) & ~7;
   hipLaunchKernelGGL((k_stored_pass<VT, 3, MT>), dim3(g), dim3(PM_WG), 0, c->stream, A.nrn, A.fr,

@@ -368,34 +368,6 @@ __global__ __launch_bounds__(PM_WG, sizeof(VT) == 4 ? 6 : 1) void k_spmv_cha(
 // (or zero past the last) and are never written.  The next group of
 // blocks' descriptors are loaded during the first pass.  XCD sweep mapping
 // over the groups of blocks.
-template <int G>
-struct PmBlocksMeta {
-  PmRunMeta b[G];
-};
-
-template <int G>
-__device__ __forceinline__ PmBlocksMeta<G> pm_blocks_meta(int64_t p, int64_t p1, int nrn,
-                                                          const int64_t *__restrict__ colptr,
-                                                          const int64_t *__restrict__ valptr,
-                                                          const int *__restrict__ nr,
-                                                          const int64_t *__restrict__ chptr) {
-  PmBlocksMeta<G> m;
-  const int64_t k = p < p1 ? (int64_t)G * p : (int64_t)nrn;  // past the range: empty blocks
-#pragma unroll
-  for (int j = 0; j < G; j++) m.b[j] = pm_run_meta(k + j, nrn, colptr, valptr, nr, chptr);
-  return m;
-}
-
-// the block of lane group gi among the G scalar metadata sets
-template <int G>
-__device__ __forceinline__ PmRunMeta pm_pick(const PmBlocksMeta<G> &m, int gi) {
-  PmRunMeta r = m.b[0];
-#pragma unroll
-  for (int j = 1; j < G; j++)
-    if (gi == j) r = m.b[j];
-  return r;
-}
-
 template <typename VT, int LPB, int U, int NV, bool SCALE_M>
 __global__ __launch_bounds__(PM_WG, sizeof(VT) == 4 ? 6 : 1) void k_spmv_chg(
     int nrn, int neq, const int *__restrict__ fr, const int *__restrict__ nr,

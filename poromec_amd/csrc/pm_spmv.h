@@ -342,6 +342,35 @@ __device__ __forceinline__ PmRunMeta pm_run_meta(int64_t k, int64_t k1,
   return m;
 }
 
+// the metadata of G consecutive blocks, one per group of 64 / G lanes
+template <int G>
+struct PmBlocksMeta {
+  PmRunMeta b[G];
+};
+
+template <int G>
+__device__ __forceinline__ PmBlocksMeta<G> pm_blocks_meta(int64_t p, int64_t p1, int nrn,
+                                                          const int64_t *__restrict__ colptr,
+                                                          const int64_t *__restrict__ valptr,
+                                                          const int *__restrict__ nr,
+                                                          const int64_t *__restrict__ chptr) {
+  PmBlocksMeta<G> m;
+  const int64_t k = p < p1 ? (int64_t)G * p : (int64_t)nrn;  // past the range: empty blocks
+#pragma unroll
+  for (int j = 0; j < G; j++) m.b[j] = pm_run_meta(k + j, nrn, colptr, valptr, nr, chptr);
+  return m;
+}
+
+// the block of lane group gi among the G scalar metadata sets
+template <int G>
+__device__ __forceinline__ PmRunMeta pm_pick(const PmBlocksMeta<G> &m, int gi) {
+  PmRunMeta r = m.b[0];
+#pragma unroll
+  for (int j = 1; j < G; j++)
+    if (gi == j) r = m.b[j];
+  return r;
+}
+
 __device__ __forceinline__ unsigned int pm_lanes_below(unsigned long long mask) {
   return __builtin_amdgcn_mbcnt_hi((unsigned int)(mask >> 32),
                                    __builtin_amdgcn_mbcnt_lo((unsigned int)mask, 0u));

@@ -54,3 +54,34 @@ def test_infinite_value_stays_in_its_rows(nen, n):
         assert np.abs(y[~hit] - y0[~hit]).max() <= 1e-13 * np.abs(y0).max()
         cs.close()
     s.close()
+
+
+# the fused iterations' stored product by runs of columns, on blocks of <= 32
+# runs (Q1/Q1) and of up to 77, given as a matrix alone.  The system: the
+# mesh's, scaled symmetrically to entries of one size, with a constant diagonal
+# of twice the largest row sum, so its condition number is at most 3 and a
+# residual of sqrt(k + 1) tol (SQMR's bound, k < 100) an error of 30 tol.
+@pytest.mark.parametrize("solver", ["sqmr", "pcg"])
+@pytest.mark.parametrize("prec", ["fp64", "fp32ir"])
+@pytest.mark.parametrize("nen,n", [(8, 18), (20, 10)])
+def test_fused_iterations_by_runs(nen, n, prec, solver):
+    from poromec_amd.solver import CsrcSolver, SolverConfig
+    s, (ia, ja, ad, al, rows), L = _system(nen, n)
+    assert s.matrix_info()["nnz"] >= 2_000_000
+    one = np.ones(s.neq)
+    sc = 1.0 / np.sqrt(abs(L) @ one + abs(L).T @ one + np.abs(ad))
+    al = al * sc[rows] * sc[ja - 1]
+    L.data[:] = al
+    big = 2.0 * (abs(L) @ one + abs(L).T @ one).max()
+    b = np.random.default_rng(2).standard_normal(s.neq)
+    ref = np.zeros(s.neq)
+    for _ in range(60):  # Jacobi: halves the error at least
+        ref = (b - L @ ref - L.T @ ref) / big
+    cs = CsrcSolver(ia, ja)
+    cs.set_values(np.full(s.neq, big), al)
+    tol = 1e-12 if prec == "fp64" else 1e-10
+    x, info = cs.solve(b, SolverConfig(solver=solver, tol=tol, precision=prec))
+    assert info["iters"] < 100
+    assert np.linalg.norm(x - ref) <= 30 * tol * np.linalg.norm(ref)
+    cs.close()
+    s.close()
