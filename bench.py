@@ -13,7 +13,8 @@ element (element type 7, the mesh kept as read), default n = 128: the
 configuration's 128^3-cell mesh at its nominal 8.6M dofs.
 
 The FP32+IR form (FP32 matrix values and Jacobi inside an FP64
-iterative-refinement loop) runs first, then the FP64 form, each from the zero
+iterative-refinement loop; this box's elements being parallelepipeds, its
+products go through the elements in FP64 all the same) runs first, then the FP64 form, each from the zero
 state: W untimed warmup steps, then K timed steps -- both clamped to what
 fits the wall-clock budget (--budget, default 450 s for the whole run), with
 at least one timed FP32+IR step; the JSON line reports the steps actually
@@ -99,6 +100,27 @@ def csr_bytes(info):
     """Bytes of the same product as a plain full CSR (int32 columns, FP64
     values, int64 row pointers, x once, y once)."""
     return 12 * info["nnz"] + 8 * (info["neq"] + 1) + 16 * info["neq"]
+
+
+def through_elements(solver, use32):
+    """Whether the solves' products go through the elements (parallelepiped
+    meshes), which are FP64 also in the FP32+IR form."""
+    q = getattr(solver, "products_through_elements", None)
+    return bool(q and q(use32))
+
+
+def element_pass_bytes(nen, numel, neq):
+    """Bytes the pass "q = t + beta q, d and x updated, y = A q, q.y" of an SQMR
+    iteration cannot do without when the product goes through the elements:
+    16 coefficients and 2 bytes per node an element, t and q read, d and x
+    read and written, q and y written."""
+    return numel * (128 + 2 * nen) + 64 * neq
+
+
+def element_pass_flops(nen, numel):
+    """FP64 operations of the element vectors (one lane an element; a
+    multiply-add counts two), as the compiled kernel has them."""
+    return numel * (2435 if nen == 20 else 1005)
 
 
 def measured_traffic(prec, shape, info):
@@ -640,12 +662,20 @@ def main():
     # stream around every live_every-th solver SpMV), per value precision
     b32 = spmv_bytes(info, 4, fused_dot=True, shape=shapes["fp32"]["best"])
     b64 = spmv_bytes(info, 8, fused_dot=True, shape=shapes["fp64"]["best"])
+    alg32 = spmv_alg_bytes(info, 8 if args.only == "fp64" else 4)
+    alg64 = spmv_alg_bytes(info, 8)
+    nen = 8 if q1 else 20
+    elems32, elems64 = through_elements(solver, True), through_elements(solver, False)
+    if args.only == "fp64":
+        elems32 = elems64
+    if elems32:
+        b32 = alg32 = element_pass_bytes(nen, deck.numel, solver.neq)
+    if elems64:
+        b64 = alg64 = element_pass_bytes(nen, deck.numel, solver.neq)
     if args.only == "fp64":  # the timed form's SpMV is the FP64 one
         b32, live32 = b64, {"fp32_ms": live32["fp64_ms"], "fp32_n": live32["fp64_n"]}
     ms32 = live32["fp32_ms"] / max(live32["fp32_n"], 1)
     ms64 = live64["fp64_ms"] / max(live64["fp64_n"], 1) if live64 else None
-    alg32 = spmv_alg_bytes(info, 8 if args.only == "fp64" else 4)
-    alg64 = spmv_alg_bytes(info, 8)
     first = "fp64" if args.only == "fp64" else "fp32"
     log(f"SpMV in the timed steps (every {args.live_every}th launch timed): {first} {ms32:.3f} ms x "
         f"{live32['fp32_n']}" + (f", fp64 {ms64:.3f} ms x {live64['fp64_n']}" if ms64 else ""))
@@ -674,8 +704,19 @@ def main():
         except Exception as exc:  # the oracle is test infrastructure: optional here
             log(f"cpu baseline skipped: {exc}")
 
-    traffic32 = (measured_traffic("fp64", shapes["fp64"]["best"], info) if args.only == "fp64"
+    traffic32 = (None if elems32 else measured_traffic("fp64", shapes["fp64"]["best"], info)
+                 if args.only == "fp64"
                  else measured_traffic("fp32", shapes["fp32"]["best"], info))
+    if elems32:
+        kernel = (f"k_affine_pass_elements<{nen}, SQMR, 1, false> + k_affine_pass_gather<SQMR, "
+                  "false> (product through the elements in FP64, with the q, d, x update and "
+                  "the q.y dot)")
+    elif args.only == "fp64":
+        kernel = (spmv_kernel_name("fp64", shapes["fp64"]["best"])
+                  + " (FP64 node-block SpMV with the fused q.t dot)")
+    else:
+        kernel = (spmv_kernel_name("fp32", shapes["fp32"]["best"])
+                  + " (FP32 node-block SpMV with the fused q.t dot)")
     out = {
         "metric": METRIC,
         "value": 1e3 / ms_step32,
@@ -687,7 +728,7 @@ def main():
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": "f64" if args.only == "fp64" else "f32-spmv/f64-ir",
+        "dtype": "f64" if args.only == "fp64" or elems32 else "f32-spmv/f64-ir",
         "data": "synthetic",
         "config": {
             "workload": (f"Biot u-p {'Q1/Q1 hexa8' if q1 else 'hexa20/8'} box {n}^3 cells "
@@ -715,17 +756,16 @@ def main():
             "spmv_ms": ms32, "spmv_launches_timed": live32["fp32_n"],
             "spmv_GBps_algorithmic": alg32 / ms32 / 1e6, "spmv_GBps_compulsory": b32 / ms32 / 1e6},
         "speedup_fp32ir_vs_fp64": (fp64["ms_per_step"] / ms_step32) if fp64 else None,
-        "spmv": {"tuned_shapes": shapes, "fp32_alg_bytes": alg32, "fp64_alg_bytes": alg64,
+        "spmv": {"products": {"fp32ir": "elements" if elems32 else "stored",
+                              "fp64": "elements" if elems64 else "stored"},
+                 "tuned_shapes": shapes, "fp32_alg_bytes": alg32, "fp64_alg_bytes": alg64,
                  "fp32_compulsory_bytes": b32, "fp64_compulsory_bytes": b64},
         "roofline": {"bound": "hbm",
-                     "kernel": (spmv_kernel_name("fp64", shapes["fp64"]["best"])
-                                + " (FP64 node-block SpMV with the fused q.t dot)")
-                     if args.only == "fp64" else
-                     (spmv_kernel_name("fp32", shapes["fp32"]["best"])
-                      + " (FP32 node-block SpMV with the fused q.t dot)"),
+                     "kernel": kernel,
                      "achieved": alg32 / ms32 / 1e6, "peak": HBM_PEAK_GBPS, "unit": "GB/s",
                      "frac": alg32 / ms32 / 1e6 / HBM_PEAK_GBPS,
                      "traffic": traffic32,
+                     "TFLOPs": (element_pass_flops(nen, deck.numel) / ms32 / 1e9) if elems32 else None,
                      "algorithmic_bytes": alg32,
                      "compulsory_bytes": b32,
                      "achieved_compulsory": b32 / ms32 / 1e6,
@@ -775,8 +815,9 @@ def q1_nominal_leg(args, cfg32, cfg64, left, margin):
         live = s.spmv_timing(0)
         key = "fp32" if name == "fp32ir" else "fp64"
         ms = live[key + "_ms"] / max(live[key + "_n"], 1)
-        comp = spmv_bytes(info, 4 if name == "fp32ir" else 8, fused_dot=True,
-                          shape=shapes[key])
+        comp = (element_pass_bytes(8, d.numel, s.neq) if through_elements(s, name == "fp32ir")
+                else spmv_bytes(info, 4 if name == "fp32ir" else 8, fused_dot=True,
+                                shape=shapes[key]))
         res[name] = {"s_per_step": wall, "time_steps_per_s": 1.0 / wall,
                      "krylov_iters": sum(inf["iters"]), "max_true_rel": max(inf["true_rel"]),
                      "spmv_ms": ms, "spmv_GBps_compulsory": comp / ms / 1e6}

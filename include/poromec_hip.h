@@ -51,7 +51,8 @@ typedef struct pm_ctx pm_ctx;
 
 /* arithmetic of the Krylov solve */
 #define PM_PREC_FP64 0   /* everything in FP64 (the oracle form) */
-#define PM_PREC_FP32IR 1 /* FP32 matrix values and Jacobi inside FP64 iterative refinement */
+#define PM_PREC_FP32IR 1 /* FP32 matrix values and Jacobi inside FP64 iterative refinement (FP64
+                            products where they go through the elements) */
 
 typedef struct {
   int solver;      /* PM_SOLVER_* (reference default 11) */
@@ -324,10 +325,19 @@ int pm_bench_spmv(pm_ctx *ctx, int use32, int reps, double *ms_per_launch);
  * level when the shape changes, and stay fixed until the next change. */
 #define PM_SPMV_SHAPES 16
 int pm_tune_spmv(pm_ctx *ctx, int use32, int reps, int *best, double *ms_per_shape);
-/* Selects SpMV shape `shape` (0 .. PM_SPMV_SHAPES-1) without timing. */
+/* Selects SpMV shape `shape` (0 .. PM_SPMV_SHAPES-1) without timing.  Neither
+ * tuned nor set, the shape is chosen by the matrix's size and run lengths.
+ * The shapes are those of the stored product by itself: products through the
+ * elements and the fused iterations on smaller matrices have their own. */
 int pm_set_spmv_shape(pm_ctx *ctx, int use32, int shape);
-/* Live SpMV timing: with on = k > 0 every k-th SpMV the single-system
- * solvers launch is bracketed by HIP events on the library's stream (launches
+/* 1 where the Krylov loops form the product of the current matrix from the
+ * elements (FP64; meshes of parallelepipeds with enough stored values), 0
+ * where they read the stored values. */
+int pm_products_through_elements(pm_ctx *ctx, int use32);
+/* Live SpMV timing: with on = k > 0 every k-th product the single-system
+ * solvers launch (of SQMR and PCG in two passes: the first, which also updates
+ * q, d and x; FP32 for the FP32+IR form's products, also where they go through
+ * the elements) is bracketed by HIP events on the library's stream (launches
  * skipped after convergence are not counted; on = 0 switches it off).  stats
  * (may be NULL) receives what was accumulated since the previous call --
  * {ms FP64, launches timed FP64, ms FP32, launches timed FP32} -- and the

@@ -534,6 +534,14 @@ __device__ __forceinline__ void pm_element_lane(const AffineArgs &A, int slot,
 // for 512 (128) with Q1/Q1.  The additions are LDS atomics
 // in a fixed order: a wavefront's instructions execute in turn, and within
 // one no two elements share the node (checked when the patches are built).
+//
+// Large meshes wait for memory (hexa20/8 87^3: 1.6 GFLOP, 46 us of issue and
+// 0.4 GB in 206 us; 425 nodes of LDS allow eleven wavefronts a CU), small ones
+// for the chain load, transform, stress, transform, store (24^3: 10.8 us).
+// With the node part the product of an SQMR iteration takes 0.41 ms at 87^3
+// against 2.9 ms from the stored matrix in FP64 and 1.9 in FP32, Q1/Q1 64^3
+// 40 us against 192 and 118; without patches it was 71 us there, with patches
+// of four lanes an element 54.
 __device__ __forceinline__ void pm_wave_lds_fence() {
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
@@ -548,8 +556,8 @@ __host__ __device__ constexpr int pm_patch_waves(int nen, int lpe) {
 // restrained ones, four values each
 __host__ __device__ inline int pm_patch_lds(int max_nodes) { return (max_nodes + 1) * 4; }
 
-// four lanes an element: buf holds the patch nodes' values (AF_OP) on entry and their sums on exit,
-// n4 = 4 * nodes values; written to ye
+// four lanes an element: buf holds the patch nodes' values (AF_OP) on entry and
+// their sums on exit, n4 = 4 * nodes values; written to ye
 template <int NEN, int MODE>
 __device__ __forceinline__ void pm_patch(const AffineArgs &A, int p, int lane, int n4, double *buf) {
   const int c = lane & 3;
@@ -604,8 +612,8 @@ __device__ __forceinline__ void pm_patch(const AffineArgs &A, int p, int lane, i
   pm_wave_lds_fence();
 }
 
-// One lane an element, 64 elements a patch.  buf is component-major here (ld values a component), so that the lanes' nodes fall
-// on different banks.
+// One lane an element, 64 elements a patch.  buf is component-major here (ld
+// values a component), so that the lanes' nodes fall on different banks.
 template <int NEN, int MODE>
 __device__ __forceinline__ void pm_patch_lane(const AffineArgs &A, int p, int lane, int n4, int ld,
                                               double *buf) {
@@ -673,6 +681,8 @@ __device__ __forceinline__ int pm_at(int i, int ld) {
 
 // Patch vectors of K_e x_e (AF_OP: x an equation vector, restrained dofs
 // zero; AF_RHS2: the nodal state) or of isw 4 (AF_RHS4); LPE lanes an element.
+// The right-hand sides of hexa20/8 40^3 take 20 us and 12 us to subtract; eight
+// colours of one workgroup an element took 4.3 ms (isw 4).
 template <int NEN, int MODE, int LPE>
 __global__ __launch_bounds__(64 * pm_patch_waves(NEN, LPE)) void k_affine_elements(AffineArgs A) {
   if (MODE == AF_OP && A.S != nullptr && A.S->done) return;
@@ -752,7 +762,9 @@ __global__ __launch_bounds__(64 * pm_patch_waves(NEN, LPE)) void k_affine_pass_e
   else pm_patch_lane<NEN, AF_OP>(A, p, lane, n4, ld, buf);
 }
 
-// element coefficients: geometry and material, dt folded in
+// element coefficients: geometry and material, dt folded in.  One lane an
+// element, bound by its scattered vertex loads: 10 us at 64,000 elements, 300
+// at 2.1 M, once a pass over the elements.
 __global__ __launch_bounds__(PM_WG) void k_affine_coefs(int numel, int nen, const int *ord,
                                                         const int *ix, const double *xv,
                                                         const int *mat, const double *e,
@@ -807,7 +819,9 @@ __global__ __launch_bounds__(PM_WG) void k_affine_coefs(int numel, int nen, cons
 // Four lanes take a row block (a node) and sum its patches' entries, eight at
 // a time in a fixed tree; lane c holds dof c.  Every node has `stride` offsets
 // (8 in a box, two or three of them used on average; the others point to a
-// zero), so their loads need no pointer first.
+// zero), so their loads need no pointer first.  Bound by memory: with SQMR's
+// updates 0.79 GB in 194 us at hexa20/8 87^3 (4.1 TB/s), 174 us at Q1/Q1 128^3;
+// 5-6 us, a chain of three loads, where the vectors stay in cache.
 struct GatherArgs {
   int nrn, stride;
   const unsigned int *gnode;  // (nrn) first row << 4 | free dofs
@@ -960,7 +974,10 @@ __global__ __launch_bounds__(PM_WG) void k_affine_metric(int numel, const double
 // issue, so the places of all the elements' nodes in the block's column list
 // are found first, a node a lane (bisection in LDS): three searches a row
 // block instead of sixteen (hexa20/8 vertices); with 64 lanes a block its
-// elements' data are scalar loads.
+// elements' data are scalar loads.  hexa20/8 40^3: 1.87 ms (2.53 with the
+// places searched one by one) against 8.3 in eight colours of one workgroup an
+// element; 87^3 19.0 against 67; Q1/Q1 64^3 1.60 against 3.6, 128^3 12.4
+// against 20.  The sums keep a multiply and an add apart, in the row's order.
 template <int NEN>
 __global__ __launch_bounds__(PM_WG) void k_affine_matrix(
     int nrn, int max_cols, int mstride, const unsigned int *__restrict__ minc,
@@ -1436,10 +1453,10 @@ static bool affine_elements(const pm_ctx *c) {
 // From 3.6 million stored values on with FP64 values, 4.5 with FP32: below,
 // the stored product is the shorter chain (one pass against two).  An SQMR
 // iteration on boxes, stored / elements, FP64 and FP32: hexa20/8 11^3 (3.2 M
-// values) 17.1 / 19.2 us and 14.6 / 19.3, 12^3 (4.2 M) 20.1 / 19.1 and 16.7 /
-// 19.3, 14^3 (6.7 M) 24.4 / 19.6 and 20.7 / 19.5; Q1/Q1 18^3 (2.4 M) 15.2 /
-// 17.1 and 14.4 / 17.0, 20^3 (3.3 M) 18.2 / 16.8 and 16.0 / 17.0, 24^3 (5.8 M)
-// 23.6 / 17.4 and 20.0 / 17.5.
+// values) 14.2 / 17.2 us and 13.6 / 16.6, 12^3 (4.2 M) 17.5 / 16.9 and 15.3 /
+// 16.3, 14^3 (6.7 M) 22.3 / 16.5 and 20.1 / 16.6; Q1/Q1 18^3 (2.4 M) 12.6 /
+// 15.6 and 12.7 / 15.7, 20^3 (3.3 M) 14.9 / 16.0 and 14.0 / 16.3, 24^3 (5.8 M)
+// 20.4 / 16.0 and 18.3 / 15.8.
 bool pm_affine_product(const pm_ctx *c, int use32) {
   return affine_elements(c) && c->affine->op_valid && c->A.values_valid &&
          c->A.nnz >= (use32 ? 4500000 : 3600000);

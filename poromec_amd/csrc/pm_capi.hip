@@ -1098,6 +1098,10 @@ extern "C" int pm_tune_spmv(pm_ctx *c, int use32, int reps, int *best, double *m
   return PM_OK;
 }
 
+extern "C" int pm_products_through_elements(pm_ctx *c, int use32) {
+  return c && c->have_matrix && !c->ordered && pm_affine_product(c, use32) ? 1 : 0;
+}
+
 extern "C" int pm_set_spmv_shape(pm_ctx *c, int use32, int shape) {
   if (!c || shape < 0 || shape >= PM_SPMV_NCFG) return PM_ERR_ARG;
   c->spmv_cfg[use32 ? 1 : 0] = shape;

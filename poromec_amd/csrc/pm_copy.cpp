@@ -5,7 +5,8 @@
 // through pinned pieces instead, several threads at once: each waits for its
 // piece's DMA, then moves it to or from the caller's memory, so the DMA of one
 // piece, the memory copies of others and the first touch of the caller's pages
-// overlap.
+// overlap: the stress fields of a hexa20/8 40^3 box (45 MB out) 3.45 -> 2.70
+// ms a call.
 #include <algorithm>
 #include <atomic>
 #include <cstring>

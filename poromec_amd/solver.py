@@ -285,6 +285,11 @@ class MefSolver:
                 "pm_tune_spmv")
         return best.value, ms
 
+    def products_through_elements(self, use32: bool) -> bool:
+        """Whether a solve of the current matrix forms its products from the
+        elements (FP64 throughout) instead of the stored values."""
+        return bool(self.lib.pm_products_through_elements(self.ctx, int(use32)))
+
     def set_spmv_shape(self, use32: bool, shape: int):
         L.check(self.lib.pm_set_spmv_shape(self.ctx, int(use32), int(shape)), "pm_set_spmv_shape")
 
