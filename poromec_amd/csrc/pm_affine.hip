@@ -1336,14 +1336,14 @@ static int affine_setup(pm_ctx *c, const double *x, const PmHostPattern &pat) {
   const int lpe = numel >= 50000 ? 1 : 4;
   element_patches(m, x, 64 / lpe, ord, ps);
   const int npatch = (int)ps.size() - 1;
-  // patch nodes in the order the elements meet them; restrained nodes share
-  // the dummy after the last
+  // patch nodes; restrained nodes share the dummy after the last
   std::vector<unsigned int> en((size_t)numel * nen), pn((size_t)npatch + 1, 0), pw;
   std::vector<int> pblock;  // row block of each entry of pw
   std::vector<unsigned short> loc((size_t)numel * nen);
   std::vector<int> at((size_t)m.nnode, -1), seen((size_t)m.nnode, -1);
   std::vector<int> pcnt((size_t)nrn, 0), mcnt((size_t)nrn, 0);
   std::vector<int> patch_block((size_t)npatch, -1);
+  std::vector<int> nodes;  // of a patch
   int max_nodes = 0, step = 0;
   pw.reserve((size_t)numel * nen / 2);
   pblock.reserve((size_t)numel * nen / 2);
@@ -1356,12 +1356,20 @@ static int affine_setup(pm_ctx *c, const double *x, const PmHostPattern &pat) {
         if (block[n] < 0) continue;
         mcnt[block[n]]++;
         if (at[n] < n0) {
-          at[n] = (int)pw.size();
-          pw.push_back(word[n]);
-          pblock.push_back(block[n]);
-          pcnt[block[n]]++;
+          at[n] = n0;
+          nodes.push_back(n);
         }
       }
+    // in the order of their equations: neighbouring lanes read and write
+    // neighbouring entries of the vectors
+    std::sort(nodes.begin(), nodes.end(), [&](int i, int j) { return word[i] < word[j]; });
+    for (int n : nodes) {
+      at[n] = (int)pw.size();
+      pw.push_back(word[n]);
+      pblock.push_back(block[n]);
+      pcnt[block[n]]++;
+    }
+    nodes.clear();
     const int nn = (int)pw.size() - n0;
     max_nodes = std::max(max_nodes, nn);
     for (int k = 0; k < nen; k++, step++)
