@@ -536,11 +536,11 @@ __device__ __forceinline__ void pm_element_lane(const AffineArgs &A, int slot,
 // one no two elements share the node (checked when the patches are built).
 //
 // Large meshes wait for memory (hexa20/8 87^3: 1.6 GFLOP, 46 us of issue and
-// 0.4 GB in 206 us; 425 nodes of LDS allow eleven wavefronts a CU), small ones
+// 0.4 GB in 199 us; 425 nodes of LDS allow eleven wavefronts a CU), small ones
 // for the chain load, transform, stress, transform, store (24^3: 10.8 us).
-// With the node part the product of an SQMR iteration takes 0.41 ms at 87^3
+// With the node part the product of an SQMR iteration takes 0.37 ms at 87^3
 // against 2.9 ms from the stored matrix in FP64 and 1.9 in FP32, Q1/Q1 64^3
-// 40 us against 192 and 118; without patches it was 71 us there, with patches
+// 38 us against 192 and 118; without patches it was 71 us there, with patches
 // of four lanes an element 54.
 __device__ __forceinline__ void pm_wave_lds_fence() {
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -820,7 +820,8 @@ __global__ __launch_bounds__(PM_WG) void k_affine_coefs(int numel, int nen, cons
 // a time in a fixed tree; lane c holds dof c.  Every node has `stride` offsets
 // (8 in a box, two or three of them used on average; the others point to a
 // zero), so their loads need no pointer first.  Bound by memory: with SQMR's
-// updates 0.79 GB in 194 us at hexa20/8 87^3 (4.1 TB/s), 174 us at Q1/Q1 128^3;
+// updates 0.79 GB in 172 us at hexa20/8 87^3 (4.6 TB/s), 157 us at Q1/Q1 128^3
+// (194 and 174 with the patches' nodes in the elements' order);
 // 5-6 us, a chain of three loads, where the vectors stay in cache.
 struct GatherArgs {
   int nrn, stride;
