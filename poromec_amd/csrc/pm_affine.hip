@@ -1334,6 +1334,7 @@ static int affine_setup(pm_ctx *c, const double *x, const PmHostPattern &pat) {
   // times the wavefronts hide more latency.  SQMR iteration, four lanes / one:
   // Q1/Q1 32^3 18.1 / 18.3 us, 40^3 24.1 / 22.9, 64^3 65.7 / 51.9; hexa20/8
   // 24^3 21.1 / 26.1, 32^3 30.6 / 33.2, 40^3 50.8 / 46.4, 48^3 79.8 / 76.3.
+  // (With the patches' nodes in the order of their equations 64^3 takes 48.7, 48^3 69.9.)
   const int lpe = numel >= 50000 ? 1 : 4;
   element_patches(m, x, 64 / lpe, ord, ps);
   const int npatch = (int)ps.size() - 1;
