@@ -26,7 +26,8 @@ struct PmAffine {
   double *ye = nullptr;          // patch vectors, 4 values a node
   double *tab = nullptr;         // reference integrals of the matrix
   int max_cols = 0;              // widest row block
-  std::vector<int> patch_block;  // (host) a row block of each patch, -1: no free node
+  // (host) the first and last row block of each patch's nodes, -1: no free node
+  std::vector<int> patch_first, patch_last;
   bool op_valid = false;         // ec_op holds the matrix's coefficients
 };
 

@@ -1344,7 +1344,7 @@ static int affine_setup(pm_ctx *c, const double *x, const PmHostPattern &pat) {
   std::vector<unsigned short> loc((size_t)numel * nen);
   std::vector<int> at((size_t)m.nnode, -1), seen((size_t)m.nnode, -1);
   std::vector<int> pcnt((size_t)nrn, 0), mcnt((size_t)nrn, 0);
-  std::vector<int> patch_block((size_t)npatch, -1);
+  std::vector<int> patch_first((size_t)npatch, -1), patch_last((size_t)npatch, -1);
   std::vector<int> nodes;  // of a patch
   int max_nodes = 0, step = 0;
   pw.reserve((size_t)numel * nen / 2);
@@ -1382,7 +1382,10 @@ static int affine_setup(pm_ctx *c, const double *x, const PmHostPattern &pat) {
         seen[n] = step;
       }
     pn[p + 1] = (unsigned int)pw.size();
-    patch_block[p] = nn > 0 ? pblock[n0] : -1;
+    if (nn > 0) {
+      patch_first[p] = pblock[n0];
+      patch_last[p] = pblock.back();
+    }
   }
   auto widest = [](const std::vector<int> &v) {
     return ((v.empty() ? 0 : *std::max_element(v.begin(), v.end())) + 3) & ~3;
@@ -1412,7 +1415,8 @@ static int affine_setup(pm_ctx *c, const double *x, const PmHostPattern &pat) {
   a->numel = numel;
   a->npatch = npatch;
   a->lpe = lpe;
-  a->patch_block = std::move(patch_block);
+  a->patch_first = std::move(patch_first);
+  a->patch_last = std::move(patch_last);
   a->max_nodes = max_nodes;
   a->mstride = mstride;
   a->nen = nen;
@@ -1607,16 +1611,19 @@ void pm_affine_pass_boxes(pm_ctx *c, PmMethod mt, const PmVecs &V, PmIterState *
 int pm_affine_patch_waves(const pm_ctx *c) { return pm_patch_waves(c->affine->nen, c->affine->lpe); }
 
 bool pm_affine_box_patches(const pm_ctx *c, const std::vector<int> &blk0, std::vector<int> &p0) {
-  const std::vector<int> &pb = c->affine->patch_block;
+  const std::vector<int> &first = c->affine->patch_first, &last = c->affine->patch_last;
   const int nbox = (int)blk0.size() - 1;
   p0.assign(nbox + 1, 0);
   int box = 0;
-  for (size_t p = 0; p < pb.size(); p++) {
-    if (pb[p] < 0) continue;  // no free node: with the patch before
-    if (pb[p] < blk0[box]) return false;  // patches out of the boxes' order
-    while (pb[p] >= blk0[box + 1]) p0[++box] = (int)p;
+  for (size_t p = 0; p < first.size(); p++) {
+    if (first[p] < 0) continue;  // no free node: with the patch before
+    if (first[p] < blk0[box]) return false;  // patches out of the boxes' order
+    while (first[p] >= blk0[box + 1]) p0[++box] = (int)p;
+    // elements of two boxes that share restrained nodes: every box has scalars
+    // of its own, a patch can have one box's only
+    if (last[p] >= blk0[box + 1]) return false;
   }
-  while (box < nbox) p0[++box] = (int)pb.size();
+  while (box < nbox) p0[++box] = (int)first.size();
   return true;
 }
 

@@ -228,3 +228,26 @@ def test_batch_through_elements(nen, ns, solver, prec):
     else:
         assert info["true_rel"] < 1e-10
     s.close()
+
+
+# two boxes that meet in a plane of restrained nodes: no equation couples them,
+# but their elements are neighbours, and a patch must not take from both (nine
+# elements a layer, sixteen a patch: the one at the plane would).  Supports
+# every twelve layers keep the system's condition that of a short column.
+def test_batch_boxes_sharing_restrained_nodes():
+    from poromec_amd.solver import MefSolver, SolverConfig
+    shape, cut = (3, 3, 1400), 501
+    d = P.heterogeneous_box_deck(3, seed=6, shape=shape, corr_len=4.0, dt=0.1, nen=8)
+    d.idv[d.x[:, 2] % 12 == 0, :3] = 1
+    d.idv[d.x[:, 2] == cut] = 1
+    s = MefSolver(d, reorder=False)  # as read: one box's equations after the other's
+    s.pform(2, True, False, d.dt, d.dt)
+    assert s.matrix_info()["nnz"] > 3_600_000 and s.products_through_elements(False)
+    b = np.random.default_rng(10).standard_normal(s.neq)
+    cs = _stored(s)
+    x0, _ = cs.solve(b, SolverConfig(tol=1e-12))
+    s.batch_define([0, 9 * cut, d.numel])
+    x, info = s.solve(b, SolverConfig(tol=1e-12))
+    assert _rel(x, x0) < 1e-9, info
+    s.close()
+    cs.close()
