@@ -1440,7 +1440,8 @@ static int affine_setup(pm_ctx *c, const double *x, const PmHostPattern &pat) {
   up((void **)&a->tab, tab.data(), sizeof(double) * tab.size());
   // the patch vectors, then four zeros for the gathers' missing entries
   up((void **)&a->ye, nullptr, sizeof(double) * ((size_t)zero + 4));
-  ok = ok && hipMemset(a->ye + zero, 0, 4 * sizeof(double)) == hipSuccess;
+  // on the stream of its readers, which the null stream does not wait for
+  ok = ok && hipMemsetAsync(a->ye + zero, 0, 4 * sizeof(double), c->stream) == hipSuccess;
   if (!ok) {  // the stored-matrix path needs none of this
     (void)hipGetLastError();
     pm_affine_free(a);

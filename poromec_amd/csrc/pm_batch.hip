@@ -661,7 +661,7 @@ int pm_batch_define_dev(pm_ctx *c, int nbox, const int *elem_off) {
     if (e != hipSuccess && rc == PM_OK) rc = PM_ERR_HIP;
   };
   chk(hipMalloc(&B->d_counters, sizeof(unsigned int) * nbox));
-  chk(hipMemset(B->d_counters, 0, sizeof(unsigned int) * nbox));
+  chk(hipMemsetAsync(B->d_counters, 0, sizeof(unsigned int) * nbox, c->stream));
   chk(hipMalloc(&B->d_partials, sizeof(double) * 2 * B->G));
   chk(hipMalloc(&B->d_S, sizeof(PmScalars) * nbox));
   chk(hipHostMalloc((void **)&B->h_S, sizeof(PmScalars) * nbox, hipHostMallocDefault));

@@ -160,11 +160,11 @@ extern "C" int pm_ctx_create(pm_ctx **out, int device) {
   chk(hipEventCreate(&c->ev1));
   chk(hipMalloc(&c->d_partials, sizeof(double) * 8192 * 4));
   chk(hipMalloc(&c->d_counter, sizeof(unsigned int)));
-  chk(hipMemset(c->d_counter, 0, sizeof(unsigned int)));
+  chk(hipMemsetAsync(c->d_counter, 0, sizeof(unsigned int), c->stream));
   chk(hipMalloc(&c->d_scal, sizeof(PmScalars)));
-  chk(hipMemset(c->d_scal, 0, sizeof(PmScalars)));
+  chk(hipMemsetAsync(c->d_scal, 0, sizeof(PmScalars), c->stream));
   chk(hipMalloc(&c->d_iter, sizeof(PmIterState)));
-  chk(hipMemset(c->d_iter, 0, sizeof(PmIterState)));
+  chk(hipMemsetAsync(c->d_iter, 0, sizeof(PmIterState), c->stream));
   chk(hipHostMalloc((void **)&c->h_iter, sizeof(PmIter), hipHostMallocDefault));
   chk(hipHostMalloc((void **)&c->h_scal, sizeof(PmScalars), hipHostMallocDefault));
   chk(hipMalloc(&c->d_elem_err, sizeof(int)));

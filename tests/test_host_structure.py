@@ -79,3 +79,11 @@ def test_abi_exports_every_declared_symbol():
     lib = C.CDLL(str(ROOT / "poromec_amd" / "libpmhip.so"))
     for name in sorted(declared):
         assert hasattr(lib, name), name
+
+
+def test_device_clears_are_on_the_context_stream():
+    """A context's stream does not wait for the null stream, on which a plain
+    hipMemset runs and may still be running when the call returns: what the
+    kernels read is cleared on their own stream."""
+    for src in sorted((ROOT / "poromec_amd" / "csrc").glob("*.*")):
+        assert not re.search(r"\bhipMemset\(", src.read_text()), src.name
