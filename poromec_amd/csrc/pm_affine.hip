@@ -24,7 +24,6 @@
 // kernel sums every node's patches in a fixed order: no colours, the same
 // result every time.
 #include <algorithm>
-#include <cmath>
 #include <cstring>
 #include <functional>
 #include <new>
@@ -34,6 +33,7 @@
 #include "pm_affine.h"
 #include "pm_elemlib.h"
 #include "pm_fused.h"
+#include "pm_patches.h"
 
 #define PM_EC 16  // doubles of element coefficients
 // 0-8 g[i][x] = d r_i / d x, then det J times: 9 a (1 - b), 10 a b, 11 a c,
@@ -1175,34 +1175,6 @@ void pm_affine_free(PmAffine *a) {
   delete a;
 }
 
-// true if the 8 vertices span a parallelepiped: the bilinear and trilinear
-// parts of the map vanish to the rounding of the coordinates.  1e-12 of the
-// edge is what coordinates i * h of a mesh of a few hundred cells leave; the
-// matrix entries then differ by as much, far below the solvers' tolerances.
-static bool is_parallelepiped(const int *v, const double *x) {
-  static const int sr[8] = {1, -1, -1, 1, 1, -1, -1, 1}, ss[8] = {1, 1, -1, -1, 1, 1, -1, -1},
-                   st[8] = {1, 1, 1, 1, -1, -1, -1, -1};
-  double lin = 0.0, rest = 0.0;
-  for (int d = 0; d < 3; d++) {
-    double c[7] = {0, 0, 0, 0, 0, 0, 0};
-    for (int k = 0; k < 8; k++) {
-      const double xk = x[(size_t)(v[k] - 1) * 3 + d];
-      c[0] += sr[k] * xk;
-      c[1] += ss[k] * xk;
-      c[2] += st[k] * xk;
-      c[3] += sr[k] * ss[k] * xk;
-      c[4] += ss[k] * st[k] * xk;
-      c[5] += sr[k] * st[k] * xk;
-      c[6] += sr[k] * ss[k] * st[k] * xk;
-    }
-    for (int i = 0; i < 7; i++)
-      if (!std::isfinite(c[i])) return false;
-    for (int i = 0; i < 3; i++) lin = std::max(lin, std::fabs(c[i]));
-    for (int i = 3; i < 7; i++) rest = std::max(rest, std::fabs(c[i]));
-  }
-  return rest <= 1.0e-12 * lin;
-}
-
 // Slots and patches: the elements of each connected part of the mesh split in
 // two along its longest side (in mean element sizes), again and again, at
 // multiples of L elements, so that only a part's last patch is not full.
@@ -1306,7 +1278,7 @@ static int affine_setup(pm_ctx *c, const double *x, const PmHostPattern &pat) {
   if (m.neq >= (1 << 28) || (int64_t)numel * nen * 4 + 4 >= ((int64_t)1 << 32) || numel >= (1 << 27))
     return PM_OK;
   for (int e = 0; e < numel; e++)
-    if (!is_parallelepiped(m.ix20.data() + (size_t)e * 21, x)) return PM_OK;
+    if (!pm_is_parallelepiped(m.ix20.data() + (size_t)e * 21, x)) return PM_OK;
   // each node's free dofs: first equation << 4 | mask, and its row block
   std::vector<unsigned int> word((size_t)m.nnode, 0);
   std::vector<int> block((size_t)m.nnode, -1);

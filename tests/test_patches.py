@@ -1,0 +1,85 @@
+"""Host geometry of the element products (pm_patches.cpp), compiled alone for
+the CPU."""
+import ctypes as C
+import subprocess
+from pathlib import Path
+
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from poromec_amd import problem as P
+
+CSRC = Path(__file__).resolve().parents[1] / "poromec_amd" / "csrc"
+WRAP = r"""
+#include "pm_patches.h"
+extern "C" int parallelepiped(const int *v, const double *x) { return pm_is_parallelepiped(v, x); }
+"""
+
+
+@pytest.fixture(scope="module")
+def patches(tmp_path_factory):
+    d = tmp_path_factory.mktemp("patches")
+    (d / "wrap.cpp").write_text(WRAP)
+    so = d / "patches.so"
+    subprocess.run(["g++", "-std=c++17", "-O2", "-shared", "-fPIC", "-pthread", f"-I{CSRC}",
+                    str(d / "wrap.cpp"), str(CSRC / "pm_patches.cpp"), "-o", str(so)], check=True)
+    return C.CDLL(str(so))
+
+
+def _parallelepiped(lib, ix, x):
+    v = np.ascontiguousarray(ix[:8], np.int32)
+    x = np.ascontiguousarray(x, np.float64)
+    return bool(lib.parallelepiped(v.ctypes.data_as(C.c_void_p), x.ctypes.data_as(C.c_void_p)))
+
+
+SHEAR = np.array([[1.0, 0.2, -0.1], [0.15, 0.8, 0.25], [-0.2, 0.1, 1.2]])
+
+
+@pytest.mark.parametrize("aspect", [1.0, 100.0, 1e4])
+def test_parallelepipeds_of_any_aspect(patches, aspect):
+    """A vertex moved by d along an edge h changes each of the four bilinear
+    and trilinear parts by d / 4h of the edge's own linear part (4 h)."""
+    ix, x = P.box_mesh(1, 1, 1, h=(1.0, 1.0, 1.0 / aspect))
+    assert _parallelepiped(patches, ix[0], x)
+    assert _parallelepiped(patches, ix[0], x[:, [2, 0, 1]])
+    assert _parallelepiped(patches, ix[0], x @ SHEAR.T)
+    for axis, h in ((0, 1.0), (1, 1.0), (2, 1.0 / aspect)):
+        for k in (0, 7):  # a vertex at the origin and one that is not
+            for f, ok in ((0.5, True), (2.0, False)):
+                y = x.copy()
+                y[ix[0, 6] - 1 if k == 0 else ix[0, 0] - 1, axis] += f * 4e-12 * h
+                assert _parallelepiped(patches, ix[0], y) == ok, (axis, k, f)
+    flat = x.copy()
+    flat[:, 2] = 0.0
+    assert not _parallelepiped(patches, ix[0], flat)
+    flat[0, 0] = np.nan
+    assert not _parallelepiped(patches, ix[0], flat)
+
+
+@pytest.mark.parametrize("nen", [20, 8])
+@pytest.mark.parametrize("aspect", [1.0, 100.0, 1e4])
+def test_accepted_elements_have_the_parallelepipeds_matrix(patches, aspect, nen):
+    """What is accepted has the matrix of its parallelepiped: with J (I + E),
+    E one row of at most three parts of 1e-12, ||E|| < 6e-12, and K moves by
+    at most (2 + sqrt 3) ||E|| of its norm: 2e-11."""
+    def matrix(x):
+        d = P.column_deck(1, 1, 1, nen=nen)
+        d.x[:] = x
+        d.idv[:] = 0
+        st = O.build_structure(d)
+        m = O.OracleModel(d, st)
+        m.assemble(isw=2, lhs=True, rhs=False)
+        return np.concatenate([m.ad, np.sqrt(2.0) * m.al[: st["nad"]]])
+
+    ix, x = P.box_mesh(1, 1, 1, h=(1.0, 1.0, 1.0 / aspect))
+    k0 = matrix(x)
+    accepted = 0
+    for axis in range(3):
+        for e in np.arange(-18.0, -5.0, 0.5):
+            y = x.copy()
+            y[ix[0, 6] - 1, axis] = 10.0 ** e  # the vertex at the origin
+            if _parallelepiped(patches, ix[0], y):
+                accepted += 1
+                assert np.linalg.norm(matrix(y) - k0) <= 2e-11 * np.linalg.norm(k0), (axis, e)
+    assert accepted >= 3
