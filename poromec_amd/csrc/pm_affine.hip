@@ -25,10 +25,7 @@
 // result every time.
 #include <algorithm>
 #include <cstring>
-#include <functional>
 #include <new>
-#include <system_error>
-#include <thread>
 
 #include "pm_affine.h"
 #include "pm_elemlib.h"
@@ -1175,102 +1172,6 @@ void pm_affine_free(PmAffine *a) {
   delete a;
 }
 
-// Slots and patches: the elements of each connected part of the mesh split in
-// two along its longest side (in mean element sizes), again and again, at
-// multiples of L elements, so that only a part's last patch is not full.
-static void element_patches(const PmHostMesh &m, const double *x, int L, std::vector<int> &ord,
-                            std::vector<int> &ps) {
-  const int numel = m.numel;
-  std::vector<float> cen((size_t)numel * 3);
-  double size[3] = {0, 0, 0};
-  std::vector<int> part((size_t)m.nnodev);
-  for (int n = 0; n < m.nnodev; n++) part[n] = n;
-  auto root = [&](int n) {
-    while (part[n] != n) n = part[n] = part[part[n]];
-    return n;
-  };
-  for (int e = 0; e < numel; e++) {
-    const int *v = m.ix20.data() + (size_t)e * 21;
-    const int r = root(v[0] - 1);
-    for (int k = 1; k < 8; k++) {
-      const int q = root(v[k] - 1);
-      if (q != r) part[q] = r;
-    }
-    for (int d = 0; d < 3; d++) {
-      double lo = x[(size_t)(v[0] - 1) * 3 + d], hi = lo, sum = 0.0;
-      for (int k = 0; k < 8; k++) {
-        const double xk = x[(size_t)(v[k] - 1) * 3 + d];
-        lo = std::min(lo, xk);
-        hi = std::max(hi, xk);
-        sum += xk;
-      }
-      cen[(size_t)e * 3 + d] = (float)(0.125 * sum);
-      size[d] += hi - lo;
-    }
-  }
-  for (int d = 0; d < 3; d++)
-    if (!(size[d] > 0.0)) size[d] = 1.0;
-  for (int e = 0; e < numel; e++)
-    for (int d = 0; d < 3; d++) cen[(size_t)e * 3 + d] *= (float)(numel / size[d]);
-  // parts in the order of their lowest equation, as the matrix has them
-  std::vector<int> key((size_t)m.nnodev, INT32_MAX);
-  for (int e = 0; e < numel; e++) {
-    int lo = INT32_MAX;
-    for (int k = 0; k < m.nen; k++)
-      for (int d = 0; d < 4; d++) {
-        const int q = m.id[(size_t)(m.ix20[(size_t)e * 21 + k] - 1) * 4 + d];
-        if (q > 0) lo = std::min(lo, q);
-      }
-    int &kr = key[root(m.ix20[(size_t)e * 21] - 1)];
-    kr = std::min(kr, lo);
-  }
-  ord.resize((size_t)numel);
-  std::vector<std::pair<int, int>> pk((size_t)numel);
-  for (int e = 0; e < numel; e++) {
-    const int r = root(m.ix20[(size_t)e * 21] - 1);
-    pk[e] = {key[r] == INT32_MAX ? INT32_MAX : key[r], r};
-    ord[e] = e;
-  }
-  std::stable_sort(ord.begin(), ord.end(), [&](int a, int b) { return pk[a] < pk[b]; });
-  std::function<void(int, int, int)> split = [&](int lo, int hi, int fork) {
-    const int n = hi - lo;
-    if (n <= L) return;
-    float mn[3] = {1e30f, 1e30f, 1e30f}, mx[3] = {-1e30f, -1e30f, -1e30f};
-    for (int i = lo; i < hi; i++)
-      for (int d = 0; d < 3; d++) {
-        const float v = cen[(size_t)ord[i] * 3 + d];
-        mn[d] = std::min(mn[d], v);
-        mx[d] = std::max(mx[d], v);
-      }
-    int ax = 0;
-    for (int d = 1; d < 3; d++)
-      if (mx[d] - mn[d] > (mx[ax] - mn[ax]) * 1.001f + 0.01f) ax = d;
-    const int mid = lo + ((n + L - 1) / L) / 2 * L;
-    std::nth_element(ord.begin() + lo, ord.begin() + mid, ord.begin() + hi, [&](int a, int b) {
-      const float va = cen[(size_t)a * 3 + ax], vb = cen[(size_t)b * 3 + ax];
-      return va != vb ? va < vb : a < b;
-    });
-    std::thread t;
-    if (fork > 0 && n > 20000) {
-      try {
-        t = std::thread([&] { split(lo, mid, fork - 1); });
-      } catch (const std::system_error &) {  // no more threads: this one does both halves
-      }
-    }
-    if (!t.joinable()) split(lo, mid, fork - 1);
-    split(mid, hi, fork - 1);
-    if (t.joinable()) t.join();
-  };
-  ps.assign(1, 0);
-  for (int a = 0; a < numel;) {
-    int b = a + 1;
-    while (b < numel && pk[ord[b]] == pk[ord[a]]) b++;
-    split(a, b, 3);
-    for (int q = a; q < b; q += L) ps.push_back(std::min(q + L, b));
-    a = b;
-  }
-}
-
 static int affine_setup(pm_ctx *c, const double *x, const PmHostPattern &pat) {
   const std::vector<int> &eq_block = pat.eq_block;
   const PmHostMesh &m = c->mesh;
@@ -1308,7 +1209,7 @@ static int affine_setup(pm_ctx *c, const double *x, const PmHostPattern &pat) {
   // 24^3 21.1 / 26.1, 32^3 30.6 / 33.2, 40^3 50.8 / 46.4, 48^3 79.8 / 76.3.
   // (With the patches' nodes in the order of their equations 64^3 takes 48.7, 48^3 69.9.)
   const int lpe = numel >= 50000 ? 1 : 4;
-  element_patches(m, x, 64 / lpe, ord, ps);
+  pm_element_patches(numel, nen, m.nnodev, m.ix20.data(), m.id.data(), x, 64 / lpe, ord, ps);
   const int npatch = (int)ps.size() - 1;
   // patch nodes; restrained nodes share the dummy after the last
   std::vector<unsigned int> en((size_t)numel * nen), pn((size_t)npatch + 1, 0), pw;

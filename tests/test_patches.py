@@ -13,6 +13,15 @@ from poromec_amd import problem as P
 CSRC = Path(__file__).resolve().parents[1] / "poromec_amd" / "csrc"
 WRAP = r"""
 #include "pm_patches.h"
+#include <cstring>
+extern "C" int element_patches(int numel, int nen, int nnodev, const int *ix, const int *id,
+                               const double *x, int L, int *ord, int *ps) {
+  std::vector<int> o, p;
+  pm_element_patches(numel, nen, nnodev, ix, id, x, L, o, p);
+  std::memcpy(ord, o.data(), o.size() * sizeof(int));
+  std::memcpy(ps, p.data(), p.size() * sizeof(int));
+  return (int)p.size() - 1;
+}
 extern "C" int parallelepiped(const int *v, const double *x) { return pm_is_parallelepiped(v, x); }
 """
 
@@ -31,6 +40,17 @@ def _parallelepiped(lib, ix, x):
     v = np.ascontiguousarray(ix[:8], np.int32)
     x = np.ascontiguousarray(x, np.float64)
     return bool(lib.parallelepiped(v.ctypes.data_as(C.c_void_p), x.ctypes.data_as(C.c_void_p)))
+
+
+def _patches(lib, nx, ny, nz, x, lanes):
+    """(ord, ps) of a box of vertex-numbered Q1/Q1 elements at coordinates x."""
+    ix = np.ascontiguousarray(P.box_mesh(nx, ny, nz)[0])
+    idm = np.arange(1, 4 * len(x) + 1, dtype=np.int32)
+    x = np.ascontiguousarray(x, np.float64)
+    ord_, ps = np.zeros(len(ix), np.int32), np.zeros(len(ix) + 1, np.int32)
+    p = lambda a: a.ctypes.data_as(C.c_void_p)  # noqa: E731
+    n = lib.element_patches(len(ix), 8, len(x), p(ix), p(idm), p(x), lanes, p(ord_), p(ps))
+    return ord_, ps[: n + 1]
 
 
 SHEAR = np.array([[1.0, 0.2, -0.1], [0.15, 0.8, 0.25], [-0.2, 0.1, 1.2]])
@@ -83,3 +103,19 @@ def test_accepted_elements_have_the_parallelepipeds_matrix(patches, aspect, nen)
                 accepted += 1
                 assert np.linalg.norm(matrix(y) - k0) <= 2e-11 * np.linalg.norm(k0), (axis, e)
     assert accepted >= 3
+
+
+@pytest.mark.parametrize("lanes", [16, 64])
+def test_patches_are_bricks_at_any_offset(patches, lanes):
+    """The patches of a mesh at map coordinates are those of the same mesh at
+    the origin: full, and bricks of 4 x 4 x 4 (4 x 2 x 2) cells."""
+    n, h = 16, 0.25
+    _, x = P.box_mesh(n, n, n, h=(h, h, h))
+    ord0, ps0 = _patches(patches, n, n, n, x, lanes)
+    assert np.array_equal(np.sort(ord0), np.arange(n ** 3))
+    assert np.array_equal(ps0, np.arange(0, n ** 3 + 1, lanes))
+    for a, b in zip(ps0[:-1], ps0[1:]):
+        cell = ord0[a:b, None] // np.array([1, n, n * n]) % n
+        assert np.prod(cell.max(0) - cell.min(0) + 1) == lanes
+    ord1, ps1 = _patches(patches, n, n, n, x + np.array([7.0e6, -7.0e6, 2.0e3]), lanes)
+    assert np.array_equal(ord0, ord1) and np.array_equal(ps0, ps1)
