@@ -10,6 +10,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <new>
 #include <thread>
 
 #include "pm_internal.h"
@@ -34,7 +35,8 @@ void pm_stage_free(PmStage *s) { delete s; }
 
 static PmStage *stage(pm_ctx *c) {
   if (c->stage) return c->stage;
-  PmStage *s = new PmStage();
+  PmStage *s = new (std::nothrow) PmStage();
+  if (!s) return nullptr;  // the plain copy
   bool ok = true;
   for (int i = 0; i < kThreads && ok; i++)
     ok = hipHostMalloc((void **)&s->buf[i], kPiece, hipHostMallocDefault) == hipSuccess &&

@@ -6,8 +6,8 @@
 #include <cmath>
 #include <cstddef>
 #include <cstdint>
+#include <exception>
 #include <functional>
-#include <system_error>
 #include <thread>
 #include <utility>
 
@@ -131,9 +131,10 @@ void pm_element_patches(int numel, int nen, int nnodev, const int *ix, const int
     if (fork > 0 && n > 20000) {
       try {
         t = std::thread([&] { split(lo, mid, fork - 1); });
-      } catch (const std::system_error &) {  // no more threads: this one does both halves
+      } catch (const std::exception &) {  // no thread, or no memory for one
       }
     }
+    // nothing below allocates but threads, so nothing throws past a running one
     if (!t.joinable()) split(lo, mid, fork - 1);
     split(mid, hi, fork - 1);
     if (t.joinable()) t.join();

@@ -119,3 +119,77 @@ def test_patches_are_bricks_at_any_offset(patches, lanes):
         assert np.prod(cell.max(0) - cell.min(0) + 1) == lanes
     ord1, ps1 = _patches(patches, n, n, n, x + np.array([7.0e6, -7.0e6, 2.0e3]), lanes)
     assert np.array_equal(ord0, ord1) and np.array_equal(ps0, ps1)
+
+
+# operator new fails in one call: the `at`-th that is made while `patches` runs
+# on the calling thread (at < 0: on any other thread)
+ALLOC = r"""
+#include <atomic>
+#include <cstdlib>
+#include <new>
+#include <thread>
+static std::atomic<int> g_at{0};
+static std::atomic<bool> g_on{false};
+static std::thread::id g_caller;
+void *operator new(std::size_t n) {
+  if (g_on.load()) {
+    const bool caller = std::this_thread::get_id() == g_caller;
+    if (g_at.load() < 0 ? !caller : caller && g_at.fetch_sub(1) == 1) throw std::bad_alloc();
+  }
+  if (void *p = std::malloc(n ? n : 1)) return p;
+  throw std::bad_alloc();
+}
+void operator delete(void *p) noexcept { std::free(p); }
+void operator delete(void *p, std::size_t) noexcept { std::free(p); }
+
+#include "pm_patches.h"
+#include <cstdio>
+int main(int argc, char **argv) {
+  const int n = 60, nv = n + 1, numel = n * n * n;
+  std::vector<int> ix((size_t)numel * 21, 0), id((size_t)nv * nv * nv * 4), ord, ps, ref, rps;
+  std::vector<double> x((size_t)nv * nv * nv * 3);
+  for (size_t i = 0; i < id.size(); i++) id[i] = (int)i + 1;
+  for (int i = 0; i < nv * nv * nv; i++) {
+    x[3 * (size_t)i] = i % nv;
+    x[3 * (size_t)i + 1] = i / nv % nv;
+    x[3 * (size_t)i + 2] = i / nv / nv;
+  }
+  for (int e = 0; e < numel; e++)
+    for (int k = 0; k < 8; k++)
+      ix[(size_t)e * 21 + k] = 1 + (e % n + (k & 1)) + nv * ((e / n % n + (k >> 1 & 1)) +
+                                                             nv * (e / n / n + (k >> 2)));
+  auto run = [&](std::vector<int> &o, std::vector<int> &p) {
+    pm_element_patches(numel, 8, nv * nv * nv, ix.data(), id.data(), x.data(), 64, o, p);
+  };
+  run(ref, rps);
+  g_caller = std::this_thread::get_id();
+  int refused = 0;
+  for (int at = -1; at < 64; at++) {
+    if (at == 0) continue;
+    g_at = at;
+    g_on = true;
+    try {
+      run(ord, ps);
+      g_on = false;
+      if (ord != ref || ps != rps) return 1;
+    } catch (const std::bad_alloc &) {  // pm_affine_setup keeps the stored matrix
+      g_on = false;
+      refused++;
+    }
+  }
+  std::printf("%d refused\n", refused);
+  return 0;
+}
+"""
+
+
+def test_patches_without_memory(tmp_path):
+    """Memory may end anywhere while patches are made: the call comes back, with
+    the patches or std::bad_alloc, and the process stays."""
+    (tmp_path / "alloc.cpp").write_text(ALLOC)
+    exe = tmp_path / "alloc"
+    subprocess.run(["g++", "-std=c++17", "-O2", "-pthread", f"-I{CSRC}",
+                    str(tmp_path / "alloc.cpp"), str(CSRC / "pm_patches.cpp"), "-o", str(exe)],
+                   check=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, (r.returncode, r.stderr)
