@@ -209,8 +209,9 @@ int pm_solve(pm_ctx *ctx, const pm_solver_cfg *cfg, const double *b, double *x,
  * pm_values_upload).  Limits: neq <= PM_NOALLOC_MAX_NEQ (PM_ERR_ARG beyond),
  * not GMRES and no SQMR -> GMRES fallback (SQMR at maxit returns
  * PM_ERR_MAXIT), not the batching form (PM_ERR_UNSUPPORTED), FP32IR only
- * once the FP32 values exist (PM_ERR_STATE otherwise; a pm_solve with
- * FP32IR or pm_tune_spmv(use32 = 1) makes them).  b / x as in pm_solve; NULL
+ * once the FP32 values exist (PM_ERR_STATE otherwise; pm_tune_spmv(use32 = 1)
+ * makes them, or a pm_solve with FP32IR, which does without them where its
+ * products go through the elements).  b / x as in pm_solve; NULL
  * needs the context's device vectors to exist (PM_ERR_STATE otherwise).
  * Every call on one GPU shares that GPU's array: calls that overlap on one
  * GPU race. */

@@ -436,6 +436,7 @@ int pm_batch_krylov(pm_ctx *c, int solver, int maxit, double tol, const double *
       return worst;
     }
   }
+  if (use32 && !c->A.have32) PM_TRY(pm_make_val32(c));  // the elements were expected to serve
   PM_TRY(breset(c));
   if (solver == PM_SOLVER_PCG) {
     double *r = c->d_wk[0], *z = c->d_wk[1], *p = c->d_wk[2];

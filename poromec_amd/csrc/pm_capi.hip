@@ -298,6 +298,22 @@ int pm_make_val32(pm_ctx *c) {
   return PM_OK;
 }
 
+// what an FP32+IR solve needs of the matrix: its FP32 values, unless every
+// inner product goes through the elements, which hold FP64 coefficients only
+int pm_ready_fp32ir(pm_ctx *c) {
+  if (!c->A.have32 && !pm_affine_product(c, 1)) PM_TRY(pm_make_val32(c));
+  c->A.ir_ready = true;
+  return PM_OK;
+}
+
+// before a setting that takes the products from the elements: a matrix that
+// pm_solve_noalloc could solve in FP32+IR stays one
+static int leave_elements(pm_ctx *c) {
+  if (!c->A.ir_ready || c->A.have32) return PM_OK;
+  PM_CHECK_HIP(hipSetDevice(c->device));
+  return pm_make_val32(c);
+}
+
 // CSRC values -> node-block values: every strict-lower entry (r, c) goes to
 // (r, c) and (c, r), the diagonal to (r, r)
 __global__ void k_csrc_values(int neq, const int64_t *ia, const int *ja, const double *ad,
@@ -737,7 +753,7 @@ extern "C" int pm_values_upload(pm_ctx *c, const double *ad, const double *al) {
   PM_TRY(pm_extract_diag(c));
   PM_CHECK_HIP(hipStreamSynchronize(c->stream));
   A.values_valid = true;
-  A.have32 = false;
+  A.have32 = A.ir_ready = false;
   if (c->affine) c->affine->op_valid = false;  // no longer the elements' matrix
   return PM_OK;
 }
@@ -956,6 +972,7 @@ extern "C" int pm_set_vprop(pm_ctx *c, const int *ie, const int *vprop) {
   PM_TRY(dupload(c, &c->d_e, e.data(), e.size()));
   PM_TRY(dupload(c, &c->d_vp, vp.data(), vp.size()));
   PM_TRY(dupload(c, &c->d_ie, ie, (size_t)numat));
+  PM_TRY(leave_elements(c));
   PM_CHECK_HIP(hipStreamSynchronize(c->stream));
   for (int i = 0; i < 4; i++) c->vprop[i] = f[i];
   return PM_OK;
@@ -979,6 +996,7 @@ extern "C" int pm_tform(pm_ctx *c, double *tx, double *txe, double *txb, double 
 
 extern "C" int pm_set_ordered(pm_ctx *c, int on) {
   if (!c) return PM_ERR_ARG;
+  if (on) PM_TRY(leave_elements(c));
   c->ordered = on != 0;
   return PM_OK;
 }

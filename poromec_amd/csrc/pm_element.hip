@@ -746,7 +746,7 @@ int pm_pform_dev(pm_ctx *c, int isw, int lhs, int rhs, double dt, double t, doub
       PM_CHECK_HIP(hipMemsetAsync(c->A.val, 0, sizeof(double) * (size_t)c->A.nnz, c->stream));
     if (c->affine) c->affine->op_valid = false;
     c->A.values_valid = false;
-    c->A.have32 = false;
+    c->A.have32 = c->A.ir_ready = false;
   }
   ElemArgs A = elem_args(c, dt, t, bvec, lhs, rhs);
   const bool q1 = c->mesh.nen == 8;

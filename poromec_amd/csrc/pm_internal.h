@@ -118,6 +118,7 @@ struct PmDevMatrix {
   double *diag = nullptr;  // ad
   int64_t *diagpos = nullptr; // position of the diagonal entry of each row
   bool have32 = false;
+  bool ir_ready = false;  // FP32+IR was solved: the FP32 values exist, or the elements do without
   bool values_valid = false;
 };
 
@@ -263,6 +264,7 @@ int pm_tform_dev(pm_ctx *c, double *tx, double *txe, double *txb, double *flux);
 int pm_update_prop_dev(pm_ctx *c, double dt);
 int pm_extract_diag(pm_ctx *c);
 int pm_make_val32(pm_ctx *c);
+int pm_ready_fp32ir(pm_ctx *c);
 int pm_step_dev(pm_ctx *c, double dt, const pm_solver_cfg *cfg, pm_step_info *info);
 double pm_dot_host(pm_ctx *c, const double *a, const double *b, int n, int *rc);
 int pm_batch_define_dev(pm_ctx *c, int nbox, const int *elem_off);

@@ -1626,7 +1626,7 @@ int pm_solve_dev(pm_ctx *c, const pm_solver_cfg *cfg, const double *b, double *x
     if (cfg->precision == PM_PREC_FP64) {
       PM_TRY(pm_batch_krylov(c, cfg->solver, cfg->maxit, cfg->tol, b, x, c->d_m, 0, info));
     } else {
-      if (!c->A.have32) PM_TRY(pm_make_val32(c));
+      PM_TRY(pm_ready_fp32ir(c));
       double *rr = c->d_wk[13], *dx = c->d_wk[14], *m32 = c->d_wk[15];
       launch_vec<0>(c, n, c->d_scal, RoundM32{c->d_m, m32}, NoEpi{}, 1);
       launch_vec<0>(c, n, c->d_scal, CopyBody{rr, b}, NoEpi{}, 1);
@@ -1700,7 +1700,7 @@ int pm_solve_dev(pm_ctx *c, const pm_solver_cfg *cfg, const double *b, double *x
   if (cfg->precision == PM_PREC_FP64) {
     PM_TRY(krylov(c, cfg, n, b, x, c->d_m, cfg->tol, 0, info));
   } else if (cfg->precision == PM_PREC_FP32IR) {
-    if (!c->A.have32) PM_TRY(pm_make_val32(c));
+    PM_TRY(pm_ready_fp32ir(c));
     double *rr = c->d_wk[13], *dx = c->d_wk[14], *m32 = c->d_wk[15];
     launch_vec<0>(c, n, c->d_scal, RoundM32{c->d_m, m32}, NoEpi{}, 1);
     launch_vec<0>(c, n, c->d_scal, CopyBody{rr, b}, NoEpi{}, 1);

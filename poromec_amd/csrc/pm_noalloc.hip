@@ -15,7 +15,7 @@
 #include <cstring>
 #include <mutex>
 
-#include "pm_internal.h"
+#include "pm_affine.h"
 
 int pm_solve_dev(pm_ctx *c, const pm_solver_cfg *cfg, const double *b, double *x,
                  pm_solve_info *info);
@@ -60,7 +60,9 @@ extern "C" int pm_solve_noalloc(pm_ctx *c, const pm_solver_cfg *cfg, const doubl
   if (n <= 0 || (int64_t)n > kMaxNeq) return PM_ERR_ARG;  // beyond the scratch's vectors
   if (c->batch) return PM_ERR_UNSUPPORTED;                 // the batching form has its own buffers
   if (cfg->solver == PM_SOLVER_GMRES) return PM_ERR_UNSUPPORTED;  // its basis is (ngram + 1) x neq
-  if (cfg->precision == PM_PREC_FP32IR && !c->A.have32) return PM_ERR_STATE;  // FP32 values not made
+  if (cfg->precision == PM_PREC_FP32IR && !c->A.have32 &&
+      !(c->A.ir_ready && pm_affine_product(c, 1)))
+    return PM_ERR_STATE;  // FP32 values not made
   if (!b && !c->d_b) return PM_ERR_STATE;
   if (!x && !c->d_x0) return PM_ERR_STATE;
   PM_CHECK_HIP(hipSetDevice(c->device));

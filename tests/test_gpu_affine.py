@@ -236,18 +236,56 @@ def test_batch_through_elements(nen, ns, solver, prec):
 # every twelve layers keep the system's condition that of a short column.
 def test_batch_boxes_sharing_restrained_nodes():
     from poromec_amd.solver import MefSolver, SolverConfig
-    shape, cut = (3, 3, 1400), 501
+    shape, cut = (3, 3, 1700), 501
     d = P.heterogeneous_box_deck(3, seed=6, shape=shape, corr_len=4.0, dt=0.1, nen=8)
     d.idv[d.x[:, 2] % 12 == 0, :3] = 1
     d.idv[d.x[:, 2] == cut] = 1
     s = MefSolver(d, reorder=False)  # as read: one box's equations after the other's
     s.pform(2, True, False, d.dt, d.dt)
-    assert s.matrix_info()["nnz"] > 3_600_000 and s.products_through_elements(False)
+    assert s.products_through_elements(False) and s.products_through_elements(True)
     b = np.random.default_rng(10).standard_normal(s.neq)
     cs = _stored(s)
     x0, _ = cs.solve(b, SolverConfig(tol=1e-12))
     s.batch_define([0, 9 * cut, d.numel])
     x, info = s.solve(b, SolverConfig(tol=1e-12))
     assert _rel(x, x0) < 1e-9, info
+    x, info = s.solve(b, SolverConfig(tol=1e-10, precision="fp32ir"))
+    assert info["true_rel"] < 1e-10, info
     s.close()
     cs.close()
+
+
+# FP32+IR through the elements reads no FP32 values: none are made, and the
+# solve without allocations takes the same matrix
+def test_fp32ir_through_elements_makes_no_fp32_values():
+    import ctypes as C
+    from poromec_amd import _lib as L
+    from poromec_amd.solver import MefSolver, SolverConfig
+    d = _deck((14, 14, 14), 20, shear=False)
+    s = MefSolver(d)
+    s.pform(2, True, False, d.dt, d.dt)
+    assert s.products_through_elements(True)
+    b = np.random.default_rng(5).standard_normal(s.neq)
+    s.solve(b, SolverConfig(tol=1e-6))  # the work vectors
+    cfg = SolverConfig(tol=1e-8, precision="fp32ir")
+
+    def free():
+        f, total = C.c_size_t(), C.c_size_t()
+        assert s.lib.hipMemGetInfo(C.byref(f), C.byref(total)) == 0
+        return f.value
+
+    def noalloc():
+        x = np.zeros(s.neq)
+        rc = s.lib.pm_solve_noalloc(s.ctx, C.byref(cfg.c()), L.ptr(b), L.ptr(x), None)
+        return rc, x
+
+    assert noalloc()[0] == -8  # no FP32+IR solve of this matrix yet
+    before = free()
+    x, info = s.solve(b, cfg)
+    assert info["true_rel"] < 1e-8
+    assert before - free() < 2 * s.matrix_info()["nnz"]
+    rc, y = noalloc()
+    assert rc == 0 and np.array_equal(x, y)
+    s.pform(2, True, False, d.dt, d.dt)
+    assert noalloc()[0] == -8
+    s.close()
