@@ -23,8 +23,9 @@
 // ---------------------------------------------------------------------------
 // pass A on the stored matrix: a wavefront per node block, UNR columns a lane
 // ---------------------------------------------------------------------------
-template <typename VT, int UNR>
+template <typename VT>
 struct PmStoredPart {  // UNR columns a lane of a node block: values, t and q
+  static constexpr int UNR = 3;
   VT w[UNR][4];
   double t[UNR], q[UNR];
   __device__ __forceinline__ void load(const PmBlockMeta &m, int j0, int lane, const int *ncol,
@@ -58,7 +59,7 @@ struct PmStoredPart {  // UNR columns a lane of a node block: values, t and q
 };
 
 // The first block's loads are in flight while the scalars form.
-template <typename VT, int UNR, PmMethod MT>
+template <typename VT, PmMethod MT>
 __global__ __launch_bounds__(PM_WG) void k_stored_pass(
     int nrn, const int *__restrict__ fr, const int *__restrict__ nr,
     const int64_t *__restrict__ colptr, const int64_t *__restrict__ valptr,
@@ -72,7 +73,8 @@ __global__ __launch_bounds__(PM_WG) void k_stored_pass(
   pm_chunk(nrn, lb, gridDim.x, k0, k1);
   int64_t k = k0 + grp;
   PmBlockMeta m = pm_uniform<64>(pm_block_meta(k, k1, colptr, valptr, nr));
-  PmStoredPart<VT, UNR> D;
+  constexpr int UNR = PmStoredPart<VT>::UNR;
+  PmStoredPart<VT> D;
   int f = 0;
   if (k < k1) {
     D.load(m, 0, lane, ncol, val, V);
@@ -370,7 +372,7 @@ static int stored_pass(pm_ctx *c, const VT *val, const PmVecs &V, PmIterState *s
   }
   int g = (A.nrn + PM_WG / 64 - 1) / (PM_WG / 64);
   g = (std::min(g, PM_MAX_GRID) + 7) & ~7;
-  hipLaunchKernelGGL((k_stored_pass<VT, 3, MT>), dim3(g), dim3(PM_WG), 0, c->stream, A.nrn, A.fr,
+  hipLaunchKernelGGL((k_stored_pass<VT, MT>), dim3(g), dim3(PM_WG), 0, c->stream, A.nrn, A.fr,
                      A.nr, A.colptr, A.valptr, A.ncol, val, V, st, cur, first, tol, nblk, pb, pa);
   return g;
 }

@@ -804,9 +804,10 @@ static void launch_spmv(pm_ctx *c, int use32, const double *x, double *y, const 
   pm_spmv_time_end(c, use32);
 }
 
-// The product of the Krylov loops: through the elements where the mesh allows
-// it (pm_affine.hip; FP64 throughout, also in place of the FP32 values), from
-// the stored matrix otherwise.
+// The product of BiCGSTAB, MINRES and GMRES: through the elements where the
+// mesh allows it (pm_affine.hip; FP64 throughout, also in place of the FP32
+// values), from the stored matrix otherwise.  PCG and SQMR run fused wherever
+// the elements serve.
 template <int NV, bool SCALE_M, class Epi>
 static void launch_product(pm_ctx *c, int use32, const double *x, double *y, const double *w,
                            const double *m, PmScalars *S, Epi epi) {
@@ -1292,7 +1293,7 @@ static int run_pcg(pm_ctx *c, int n, const double *b, double *x, const double *m
     int chunk = std::min(next_chunk(launched), maxit - launched);
     for (int it = 0; it < chunk; it++) {
       c->cur_iter = launched + it + 1;
-      launch_product<1, false>(c, use32, p, z, p, nullptr, S, PcgAlpha{});
+      launch_spmv<1, false>(c, use32, p, z, p, nullptr, S, PcgAlpha{});
       (use32 ? info->spmv32 : info->spmv64)++;
       launch_vec<1>(c, n, S, PcgUpd{x, r, z, p, m}, PcgUpdEpi{});
       launch_vec<0>(c, n, S, PcgP{p, z}, FinishEpi{});
@@ -1330,7 +1331,7 @@ static int run_sqmr(pm_ctx *c, int n, const double *b, double *x, const double *
     int chunk = std::min(next_chunk(launched), maxit - launched);
     for (int it = 0; it < chunk; it++) {
       c->cur_iter = launched + it + 1;
-      launch_product<1, false>(c, use32, q, t, q, nullptr, S, SqmrSigma{});
+      launch_spmv<1, false>(c, use32, q, t, q, nullptr, S, SqmrSigma{});
       (use32 ? info->spmv32 : info->spmv64)++;
       launch_vec<2>(c, n, S, SqmrRT{r, t, m}, SqmrRTEpi{});
       launch_vec<0>(c, n, S, SqmrDXQ{d, x, q, t}, SqmrFinishEpi{});
