@@ -1,5 +1,6 @@
 """Parallelepiped meshes, whose element loops and Krylov products run in the
-element's Legendre modes (pm_affine.hip), against the oracle's Gauss loops.
+element's Legendre modes (pm_affine.hip), against the oracle's Gauss loops; the
+loops of distorted meshes, which keep the Gauss points, on the same decks.
 
 Bars: the element loops' own (matrix within 1e-13 of the row's largest entry,
 right-hand sides within 1e-13 of max|b|); solutions within 1e-9 of those from
@@ -39,8 +40,24 @@ def _deck(shape, nen, shear=True, seed=3):
 @pytest.mark.parametrize("nen", [20, 8])
 @pytest.mark.parametrize("shape", [(1, 1, 1), (3, 7, 3), (4, 4, 4), (5, 13, 1), (9, 5, 6)])
 def test_element_loops(shape, nen):
+    _check_loops(_deck(shape, nen))
+
+
+# the Gauss loops in colours, which meshes of other elements keep: every
+# interior vertex moved, and one vertex of a box alone
+@pytest.mark.parametrize("nen", [20, 8])
+@pytest.mark.parametrize("shape,one", [((3, 4, 3), False), ((6, 5, 4), False), ((4, 4, 4), True)])
+def test_element_loops_distorted(shape, one, nen):
+    d = _deck(shape, nen, shear=False)
+    x = d.x.copy()
+    inner = np.nonzero(np.all((x > 0) & (x < np.array(shape)), axis=1))[0]
+    inner = inner[:1] if one else inner
+    x[inner] += 0.08 * np.random.default_rng(2).standard_normal((len(inner), 3))
+    _check_loops(dataclasses.replace(d, x=x))
+
+
+def _check_loops(d):
     from poromec_amd.solver import MefSolver
-    d = _deck(shape, nen)
     st = O.build_structure(d)
     m = O.OracleModel(d, st)
     s = MefSolver(d)
@@ -123,6 +140,8 @@ def test_products_sqmr(nen, shape, moved):
     s = MefSolver(d)
     s.pform(2, True, False, d.dt, d.dt)
     assert s.matrix_info()["nnz"] > 4_500_000
+    for use32 in (False, True):
+        assert s.products_through_elements(use32) == (not moved)
     b = np.random.default_rng(5).standard_normal(s.neq)
     cs = _stored(s)
     x0, _ = cs.solve(b, SolverConfig(tol=1e-11))
@@ -141,7 +160,7 @@ def test_products_other_solvers():
     d.idv[:, 3] = 1  # K = K_uu, positive definite
     s = MefSolver(d)
     s.pform(2, True, False, d.dt, d.dt)
-    assert s.matrix_info()["nnz"] > 4_500_000
+    assert s.products_through_elements(False)
     b = np.random.default_rng(6).standard_normal(s.neq)
     cs = _stored(s)
     x0, _ = cs.solve(b, SolverConfig(solver="pcg", tol=1e-12))
@@ -201,9 +220,9 @@ def test_batch_through_elements(nen, ns, solver, prec):
     decks = [P.heterogeneous_box_deck(n, seed=n, corr_len=n / 2, dt=0.1, nen=nen) for n in ns]
     big, off = P.concat_decks(decks)
     s = MefSolver(big)
-    assert s.matrix_info()["nnz"] > 4_500_000
     s.batch_define(off)
     s.pform(2, True, False, big.dt, big.dt)
+    assert s.products_through_elements(prec == "fp32ir")
     rng = np.random.default_rng(9)
     singles = [MefSolver(d) for d in decks]
     bs = [rng.standard_normal(o.neq) if k != 1 else np.zeros(o.neq) for k, o in enumerate(singles)]
@@ -228,6 +247,56 @@ def test_batch_through_elements(nen, ns, solver, prec):
     else:
         assert info["true_rel"] < 1e-10
     s.close()
+
+
+# one lane an element (from 50,000 on): the solvers' products against the
+# residual recomputed from the stored matrix; K = K_uu, positive definite.
+# MINRES and GMRES stop on a scaled residual; the rows' scales differ by < 100
+@pytest.mark.parametrize("nen", [20, 8])
+def test_products_one_lane(nen):
+    from poromec_amd.solver import MefSolver, SolverConfig
+    d = _deck((37, 38, 36), nen)
+    assert d.numel >= 50000
+    d.idv[:, 3] = 1
+    s = MefSolver(d)
+    s.pform(2, True, False, d.dt, d.dt)
+    assert s.products_through_elements(False) and s.products_through_elements(True)
+    b = np.random.default_rng(6).standard_normal(s.neq)
+    for solver, precond, prec, tol, bar in (("pcg", 2, "fp64", 1e-11, 1e-9),
+                                            ("pcg", 2, "fp32ir", 1e-10, 1e-10),
+                                            ("bicgstab", 2, "fp64", 1e-11, 1e-9),
+                                            ("minres", 5, "fp64", 1e-10, 1e-8),
+                                            ("gmres", 2, "fp64", 1e-6, 1e-4)):
+        x, info = s.solve(b, SolverConfig(solver=solver, precond=precond, tol=tol, precision=prec))
+        assert info["true_rel"] < bar, (solver, prec, info)
+    s.close()
+
+
+# the batched passes with one lane an element, the two boxes' element counts
+# (27,000 and 24,389) each below that line: against each box alone
+@pytest.mark.parametrize("nen", [20, 8])
+@pytest.mark.parametrize("solver", ["sqmr", "pcg"])
+def test_batch_one_lane(nen, solver):
+    from poromec_amd.solver import MefSolver, SolverConfig
+    decks = [P.heterogeneous_box_deck(n, seed=n, corr_len=8.0, dt=0.1, nen=nen) for n in (30, 29)]
+    big, off = P.concat_decks(decks)
+    assert big.numel >= 50000
+    s = MefSolver(big)
+    s.batch_define(off)
+    s.pform(2, True, False, big.dt, big.dt)
+    assert s.products_through_elements(False)
+    rng = np.random.default_rng(9)
+    singles = [MefSolver(d) for d in decks]
+    bs = [rng.standard_normal(o.neq) for o in singles]
+    x, _ = s.solve(np.concatenate(bs), SolverConfig(solver=solver, tol=1e-12))
+    s.close()
+    at = 0
+    for k, o in enumerate(singles):
+        o.pform(2, True, False, big.dt, big.dt)
+        ref, _ = o.solve(bs[k], SolverConfig(tol=1e-12))
+        assert _rel(x[at: at + o.neq], ref) < 1e-9, k
+        at += o.neq
+        o.close()
 
 
 # two boxes that meet in a plane of restrained nodes: no equation couples them,

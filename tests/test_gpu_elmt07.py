@@ -180,9 +180,10 @@ def test_q1_stabilized_column():
 def test_q1_every_spmv_shape():
     """Every SpMV shape on a Q1/Q1 box (interior node blocks of 4 rows x 108
     columns, 27 runs): FP64 against the exported CSRC matrix applied on the
-    host, FP32+IR to the FP64 solution."""
+    host, FP32 by FP32+IR solves."""
     import scipy.sparse as sp
-    from poromec_amd.solver import SPMV_SHAPES, MefSolver, SolverConfig
+    from poromec_amd.solver import SPMV_SHAPES, MefSolver
+    from test_gpu_spmv import check_fp32_shapes
     d = q1_deck(6, 3, loads=False)
     s = MefSolver(d)
     s.pform(2, True, False, d.dt, d.dt)
@@ -192,16 +193,11 @@ def test_q1_every_spmv_shape():
     Lm = sp.csr_matrix((al, (rows, ja - 1)), shape=(n, n))
     x = np.random.default_rng(8).standard_normal(n)
     y0 = ad * x + Lm @ x + Lm.T @ x
-    b = np.random.default_rng(6).standard_normal(n)
-    x64, _ = s.solve(b, SolverConfig(tol=1e-10))
     for shape in range(SPMV_SHAPES):
         s.set_spmv_shape(False, shape)
         y = s.spmv(x)
         assert np.abs(y - y0).max() <= 1e-13 * np.abs(y0).max(), shape
-        s.set_spmv_shape(True, shape)
-        x32, i32 = s.solve(b, SolverConfig(tol=1e-10, precision="fp32ir"))
-        assert i32["true_rel"] < 1e-10, shape
-        assert np.abs(x32 - x64).max() <= 1e-8 * np.abs(x64).max(), shape
+    check_fp32_shapes(s)
     s.close()
 
 

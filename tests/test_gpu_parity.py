@@ -137,28 +137,15 @@ def test_fp32ir_reaches_tolerance(column):
 
 
 def test_fp32ir_every_spmv_shape():
-    """Every SpMV shape, the index-prefetch ones included, on a box whose
-    interior node blocks are wider than one pass of the narrower shapes
-    (270 columns): FP32+IR reaches the FP64 solution, and the shapes' inner
-    iteration counts agree up to the drift that their different summation
-    orders cause (an operator that is not the FP32 matrix, or not the same
-    one every iteration, shows as a far larger count)."""
-    from poromec_amd.solver import SPMV_SHAPES, SolverConfig
+    """Every SpMV shape, the index-prefetch ones included, with FP32 values on
+    the pattern of a box whose interior node blocks are wider than one pass of
+    the narrower shapes (270 columns)."""
+    from test_gpu_spmv import check_fp32_shapes
     d = P.heterogeneous_box_deck(4, seed=2, sigma_lnk=0.5, corr_len=2.0)
     s = _solver(d)
     s.pform(2, True, False, d.dt, d.dt)
     assert s.matrix_info()["ncols"] > 0
-    b = np.random.default_rng(6).standard_normal(s.neq)
-    x64, _ = s.solve(b, SolverConfig(tol=1e-10))
-    iters = []
-    for shape in range(SPMV_SHAPES):
-        s.set_spmv_shape(True, shape)
-        x32, i32 = s.solve(b, SolverConfig(tol=1e-10, precision="fp32ir"))
-        assert i32["true_rel"] < 1e-10, shape
-        assert np.abs(x32 - x64).max() <= 1e-8 * np.abs(x64).max(), shape
-        iters.append(i32["iters"])
-    for shape, it in enumerate(iters):
-        assert abs(it - iters[0]) <= 0.1 * iters[0] + 5, (shape, iters)
+    check_fp32_shapes(s)
 
 
 def test_fp64_spmv_every_shape():
