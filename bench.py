@@ -109,6 +109,14 @@ def through_elements(solver, use32):
     return bool(q and q(use32))
 
 
+def tune_stored(solver):
+    """The stored product's shape, tuned for the value precisions whose solves
+    read it (pform before): name -> (shape, ms of every shape), (None, None)
+    where the products go through the elements."""
+    return {name: (None, None) if through_elements(solver, use32)
+            else solver.tune_spmv(use32, reps=5) for use32, name in ((False, "fp64"), (True, "fp32"))}
+
+
 def element_pass_bytes(nen, numel, neq):
     """Bytes the pass "q = t + beta q, d and x updated, y = A q, q.y" of an SQMR
     iteration cannot do without when the product goes through the elements:
@@ -244,7 +252,7 @@ def batch_form(args):
         s.batch_graphs(False)
     setup_s = time.perf_counter() - t0
     s.pform(2, True, False, big.dt, big.dt)
-    shapes = {name: s.tune_spmv(use32, reps=5)[0] for use32, name in ((False, "fp64"), (True, "fp32"))}
+    shapes = {name: best for name, (best, _) in tune_stored(s).items()}
     log(f"batch ({args.element}): {args.nbox} boxes, neq {s.neq}, setup {setup_s:.1f} s, "
         f"shapes {shapes}")
     out = {}
@@ -576,10 +584,10 @@ def main():
     # SpMV shape tuner on this matrix (lanes per node block x columns in flight)
     solver.pform(2, True, False, deck.dt, deck.dt)
     shapes = {}
-    for use32, name in ((False, "fp64"), (True, "fp32")):
-        best, ms = solver.tune_spmv(use32, reps=5)
-        shapes[name] = {"best": best, "ms": [round(v, 4) for v in ms]}
-        log(f"SpMV shapes {name}: " + ", ".join(f"{v:.3f}" for v in ms) + f" ms -> shape {best}")
+    for name, (best, ms) in tune_stored(solver).items():
+        shapes[name] = {"best": best, "ms": None if ms is None else [round(v, 4) for v in ms]}
+        log(f"SpMV shapes {name}: " + ("through the elements" if ms is None else
+                                       ", ".join(f"{v:.3f}" for v in ms) + f" ms -> shape {best}"))
 
     cfg64 = SolverConfig(precision="fp64", tol=1e-10, stop_crit=1)
     cfg32 = SolverConfig(precision="fp32ir", tol=1e-10, ir_inner_tol=1e-5, stop_crit=1)
@@ -797,7 +805,7 @@ def q1_nominal_leg(args, cfg32, cfg64, left, margin):
     s = MefSolver(d)
     info = s.matrix_info()
     s.pform(2, True, False, d.dt, d.dt)
-    shapes = {name: s.tune_spmv(use32, reps=5)[0] for use32, name in ((False, "fp64"), (True, "fp32"))}
+    shapes = {name: best for name, (best, _) in tune_stored(s).items()}
     res = {"workload": f"Biot u-p Q1/Q1 hexa8 box 128^3 cells ({s.neq} equations), "
                        "heterogeneous log-k, 10% patch load, dt 0.1 s, SQMR+Jacobi 1e-10",
            "neq": s.neq, "nnz": info["nnz"], "setup_s": time.perf_counter() - t0,
