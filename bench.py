@@ -127,8 +127,8 @@ def element_pass_bytes(nen, numel, neq):
 
 def element_pass_flops(nen, numel):
     """FP64 operations of the element vectors (one lane an element; a
-    multiply-add counts two), as the compiled kernel has them."""
-    return numel * (2435 if nen == 20 else 1005)
+    multiply-add counts two), as the compiled k_affine_elements has them."""
+    return numel * (2211 if nen == 20 else 835)
 
 
 def measured_traffic(prec, shape, info):

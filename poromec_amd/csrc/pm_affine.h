@@ -3,8 +3,8 @@
 #include "pm_elemargs.h"
 
 // Device data of a mesh whose elements are all parallelepipeds (constant
-// Jacobian).  Elements are kept in slots (ord), a patch of up to 16 neighbours
-// after the other.
+// Jacobian).  Elements are kept in slots (ord), a patch of up to 64 / lpe
+// neighbours after the other.
 struct PmAffine {
   int numel = 0, nen = 0, nrn = 0;
   int *ord = nullptr;            // (numel) element of each slot

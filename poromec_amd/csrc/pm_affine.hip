@@ -12,17 +12,18 @@
 //   * a derivative moves a coefficient one degree down (P1' = P0, P2' = 3 P1),
 //   * the 4^3 (2^3) Gauss rule is exact for every product that occurs, so the
 //     17 derivative modes are orthogonal and D acts on each mode alone.
-// An element's K_e u_e is then ~2800 FP64 instructions (Q1/Q1 ~1300) instead
-// of the 64-point loops' ~2 million operations, and needs its 15 coefficients
+// An element's K_e u_e is then 1,624 FP64 instructions (Q1/Q1 637) instead of
+// the 64-point loops' ~2 million operations, and needs its 15 coefficients
 // (128 B) instead of the matrix's 37 KB of stored values.
 //
-// In small meshes four lanes take an element: lanes 0-2 one displacement
-// component each, lane 3 the pressure; the stress of a mode exchanges
-// gradients inside the quad by DPP (6500 instructions per 64 elements, but
-// four times the wavefronts).  A wavefront sums the vectors of its 64 or 16
-// neighbouring elements in LDS and writes the patch's nodes to ye; a second
-// kernel sums every node's patches in a fixed order: no colours, the same
-// result every time.
+// In large meshes a lane takes an element (2,800 vector instructions a
+// wavefront of 64, patch and scalars included).  In small ones four lanes do:
+// lanes 0-2 one displacement component each, lane 3 the pressure; the stress of
+// a mode exchanges gradients inside the quad by DPP (four wavefronts of 1,600
+// for the same 64).  A wavefront sums the vectors of its 64 or 16 neighbouring
+// elements in LDS and writes the patch's nodes to ye; a second kernel sums
+// every node's patches in a fixed order: no colours, the same result every
+// time.
 #include <algorithm>
 #include <cstring>
 #include <new>
@@ -1205,9 +1206,10 @@ static int affine_setup(pm_ctx *c, const double *x, const PmHostPattern &pat) {
   std::vector<int> ord, ps;
   // one lane an element from 50,000 elements (800 wavefronts): below, four
   // times the wavefronts hide more latency.  SQMR iteration, four lanes / one:
-  // Q1/Q1 32^3 18.1 / 18.3 us, 40^3 24.1 / 22.9, 64^3 65.7 / 51.9; hexa20/8
-  // 24^3 21.1 / 26.1, 32^3 30.6 / 33.2, 40^3 50.8 / 46.4, 48^3 79.8 / 76.3.
-  // (With the patches' nodes in the order of their equations 64^3 takes 48.7, 48^3 69.9.)
+  // Q1/Q1 32^3 17.5 / 18.3 us, 36^3 20.5 / 19.7, 40^3 22.8 / 21.6, 48^3 32.9 /
+  // 28.7, 64^3 62.6 / 48.9; hexa20/8 24^3 20.0 / 25.1, 32^3 28.8 / 31.1, 36^3
+  // 38.3 / 37.2, 40^3 47.8 / 43.3, 48^3 74.1 / 69.8.  Between the crossing,
+  // near 40,000, and the line the two are within 4 %.
   const int lpe = numel >= 50000 ? 1 : 4;
   pm_element_patches(numel, nen, m.nnodev, m.ix20.data(), m.id.data(), x, 64 / lpe, ord, ps);
   const int npatch = (int)ps.size() - 1;
@@ -1341,10 +1343,10 @@ static bool affine_elements(const pm_ctx *c) {
 // From 3.6 million stored values on with FP64 values, 4.5 with FP32: below,
 // the stored product is the shorter chain (one pass against two).  An SQMR
 // iteration on boxes, stored / elements, FP64 and FP32: hexa20/8 11^3 (3.2 M
-// values) 14.2 / 17.2 us and 13.6 / 16.6, 12^3 (4.2 M) 17.5 / 16.9 and 15.3 /
-// 16.3, 14^3 (6.7 M) 22.3 / 16.5 and 20.1 / 16.6; Q1/Q1 18^3 (2.4 M) 12.6 /
-// 15.6 and 12.7 / 15.7, 20^3 (3.3 M) 14.9 / 16.0 and 14.0 / 16.3, 24^3 (5.8 M)
-// 20.4 / 16.0 and 18.3 / 15.8.
+// values) 13.9 / 16.4 us and 13.5 / 16.1, 12^3 (4.2 M) 17.6 / 16.1 and 15.2 /
+// 16.1, 14^3 (6.7 M) 22.7 / 16.1 and 20.2 / 16.3; Q1/Q1 18^3 (2.4 M) 12.1 /
+// 14.6 and 12.3 / 15.2, 20^3 (3.3 M) 14.7 / 15.4 and 13.7 / 14.8, 22^3 (4.4 M)
+// 17.7 / 14.8 and 14.9 / 14.7, 24^3 (5.8 M) 20.7 / 15.0 and 17.8 / 15.3.
 bool pm_affine_product(const pm_ctx *c, int use32) {
   return affine_elements(c) && c->affine->op_valid && c->A.values_valid &&
          c->A.nnz >= (use32 ? 4500000 : 3600000);
