@@ -307,11 +307,10 @@ int pm_ready_fp32ir(pm_ctx *c) {
 }
 
 // before a setting that takes the products from the elements: a matrix that
-// pm_solve_noalloc could solve in FP32+IR stays one
-static int leave_elements(pm_ctx *c) {
-  if (!c->A.ir_ready || c->A.have32) return PM_OK;
-  PM_CHECK_HIP(hipSetDevice(c->device));
-  return pm_make_val32(c);
+// pm_solve_noalloc could solve in FP32+IR stays one where memory allows
+static void leave_elements(pm_ctx *c) {
+  if (!c->A.ir_ready || c->A.have32) return;
+  if (hipSetDevice(c->device) != hipSuccess || pm_make_val32(c) != PM_OK) (void)hipGetLastError();
 }
 
 // CSRC values -> node-block values: every strict-lower entry (r, c) goes to
@@ -972,7 +971,7 @@ extern "C" int pm_set_vprop(pm_ctx *c, const int *ie, const int *vprop) {
   PM_TRY(dupload(c, &c->d_e, e.data(), e.size()));
   PM_TRY(dupload(c, &c->d_vp, vp.data(), vp.size()));
   PM_TRY(dupload(c, &c->d_ie, ie, (size_t)numat));
-  PM_TRY(leave_elements(c));
+  leave_elements(c);
   PM_CHECK_HIP(hipStreamSynchronize(c->stream));
   for (int i = 0; i < 4; i++) c->vprop[i] = f[i];
   return PM_OK;
@@ -996,7 +995,7 @@ extern "C" int pm_tform(pm_ctx *c, double *tx, double *txe, double *txb, double 
 
 extern "C" int pm_set_ordered(pm_ctx *c, int on) {
   if (!c) return PM_ERR_ARG;
-  if (on) PM_TRY(leave_elements(c));
+  if (on) leave_elements(c);
   c->ordered = on != 0;
   return PM_OK;
 }

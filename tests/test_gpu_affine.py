@@ -355,6 +355,9 @@ def test_fp32ir_through_elements_makes_no_fp32_values():
     assert before - free() < 2 * s.matrix_info()["nnz"]
     rc, y = noalloc()
     assert rc == 0 and np.array_equal(x, y)
+    s.set_ordered(True)  # takes the stored values: made now, for the call that cannot
+    assert before - free() > 3 * s.matrix_info()["nnz"]
+    s.set_ordered(False)
     s.pform(2, True, False, d.dt, d.dt)
     assert noalloc()[0] == -8
     s.close()
